@@ -451,7 +451,7 @@ static int launch_pack(mbs_ctx *ctx, int nb, const mbs_consts &c, double scale, 
 {
     // small-phase area limit: (legacy ? invComplWave : -invComplWave) * area
     const double sg = c.legacy_sign ? 1.0 : -1.0;
-    pack_beams_kernel<<<(nb + 127) / 128, 128, 0, ctx->stream>>>(
+    pack_beams_kernel<<<(nb + PACK_BEAMS - 1) / PACK_BEAMS, PACK_THREADS, 0, ctx->stream>>>(
         nb, ctx->bs_in.p, ctx->nv.p, ctx->ext.p, ctx->voff.p, ctx->vx_in.p, ctx->vy_in.p,
         ctx->syx_in.p, ctx->sxy_in.p, ctx->ef_in.p, c.wave_index, sg * c.inv_compl_wave[0],
         sg * c.inv_compl_wave[1], c.compl_wave[0], c.compl_wave[1], rescale ? scale : 1.0,

@@ -128,139 +128,126 @@ __global__ void grid_tables_kernel(const double *__restrict__ theta,
 }
 
 // ---------------------------------------------------------------------------
-// Beam packing: one thread per beam, from the C-ABI input arrays to the
-// kernel record (po_layout.h).  Small-phase moments follow
-// small_phase_polygon_factor (src/handler/HandlerPO_fast.h:154-216).
+// Beam packing, from the C-ABI input arrays to the kernel record
+// (po_layout.h): eight lanes per beam, sixteen beams per workgroup.  Small-phase
+// moments follow small_phase_polygon_factor (src/handler/HandlerPO_fast.h:154-216).
+//
+// What bounds it is latency for small batches and issue for large ones.  One
+// thread per beam, with the moments of orders 3-5 from binomial sums of pow()
+// (about 1,800 calls for a 4-vertex beam), took 0.73 ms for 185 beams, 1.74 ms
+// for 59,000 and 2.57 ms for 137,000; this form takes 13, 53 and 105 us.  The
+// polygon is staged in LDS, the lanes of a group
+// take the vertices in turn and add their sums by butterflies, and an edge's
+// share of a moment is a 3-point Gauss rule: over the triangle (0, P, Q) a
+// monomial of degree n integrates to det(P, Q) / (n + 2) times its mean along
+// PQ, which three nodes give exactly to degree 5.  The record goes through LDS
+// so that its stores are contiguous.
 // ---------------------------------------------------------------------------
-__global__ void pack_beams_kernel(int n_beams, const double *__restrict__ bs,
-                                  const int32_t *__restrict__ nv_in,
-                                  const int32_t *__restrict__ ext_in,
-                                  const int64_t *__restrict__ voff,
-                                  const double *__restrict__ vx,
-                                  const double *__restrict__ vy,
-                                  const double *__restrict__ syx,
-                                  const double *__restrict__ sxy,
-                                  const uint8_t *__restrict__ ef, double k,
-                                  double al_re, double al_im, double cw_re,
-                                  double cw_im, double sc,
-                                  const double *__restrict__ raw_j,
-                                  const double *__restrict__ path,
-                                  const double *__restrict__ sign,
-                                  const int64_t *__restrict__ abs_off,
-                                  const double *__restrict__ abs_path, double c_abs,
-                                  double k_j,
-                                  double *__restrict__ hdr,
-                                  float *__restrict__ hdr32,
-                                  double *__restrict__ vtx,
-                                  double *__restrict__ vdd,
-                                  int32_t *__restrict__ vflag,
-                                  float *__restrict__ wb)
+enum { PACK_GROUP = 8, PACK_BEAMS = 16, PACK_THREADS = PACK_GROUP * PACK_BEAMS };
+
+__device__ __forceinline__ double group_sum(double v)
 {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= n_beams)
-        return;
-    const double *s = bs + (size_t)b * 36;
+    for (int off = 1; off < PACK_GROUP; off <<= 1)
+        v += __shfl_xor(v, off, PACK_GROUP);
+    return v;
+}
+
+__device__ __forceinline__ double group_min(double v)
+{
+    for (int off = 1; off < PACK_GROUP; off <<= 1)
+        v = fmin(v, __shfl_xor(v, off, PACK_GROUP));
+    return v;
+}
+
+__global__ void __launch_bounds__(PACK_THREADS) pack_beams_kernel(
+    int n_beams, const double *__restrict__ bs, const int32_t *__restrict__ nv_in,
+    const int32_t *__restrict__ ext_in, const int64_t *__restrict__ voff,
+    const double *__restrict__ vx, const double *__restrict__ vy,
+    const double *__restrict__ syx, const double *__restrict__ sxy,
+    const uint8_t *__restrict__ ef, double k, double al_re, double al_im, double cw_re,
+    double cw_im, double sc, const double *__restrict__ raw_j,
+    const double *__restrict__ path, const double *__restrict__ sign,
+    const int64_t *__restrict__ abs_off, const double *__restrict__ abs_path, double c_abs,
+    double k_j, double *__restrict__ hdr, float *__restrict__ hdr32,
+    double *__restrict__ vtx, double *__restrict__ vdd, int32_t *__restrict__ vflag,
+    float *__restrict__ wb)
+{
+    __shared__ double s_bs[PACK_BEAMS * 36];
+    __shared__ double s_x[PACK_BEAMS][33], s_y[PACK_BEAMS][33];  // odd stride: no bank conflicts
+    __shared__ double s_h[PACK_BEAMS * HDR_STRIDE];
+    const int g = threadIdx.x / PACK_GROUP, q = threadIdx.x % PACK_GROUP;
+    const int first = blockIdx.x * PACK_BEAMS;
+    const int count = min((int)PACK_BEAMS, n_beams - first);  // beams of this workgroup
+    const int b = first + min(g, count - 1);  // spare groups repeat the last beam
+    for (int i = threadIdx.x; i < count * 36; i += PACK_THREADS)
+        s_bs[i] = bs[(size_t)first * 36 + i];
     const int nv = nv_in[b];
     const int64_t v0 = voff[b];
     // size rescaling (raw_j set): vertices and centre times sc, area times
     // sc^2, J_phased rebuilt below; sc = 1 leaves every value as it is
-    auto X = [&](int i) { return vx[v0 + i] * sc; };
-    auto Y = [&](int i) { return vy[v0 + i] * sc; };
-    double *h = hdr + (size_t)b * HDR_STRIDE;
-    float *h32 = hdr32 + (size_t)b * HDR32_STRIDE;
-    const double *hor = s + 0, *ver = s + 3, *bd = s + 6;
-    const double cen[3] = {s[9] * sc, s[10] * sc, s[11] * sc};
-    h[H_HOR + 0] = hor[0];
-    h[H_HOR + 1] = hor[1];
-    h[H_HOR + 2] = hor[2];
-    h[H_A0] = bd[0] * hor[0] + bd[1] * hor[1] + bd[2] * hor[2];
-    h[H_VER + 0] = ver[0];
-    h[H_VER + 1] = ver[1];
-    h[H_VER + 2] = ver[2];
-    h[H_B0] = bd[0] * ver[0] + bd[1] * ver[1] + bd[2] * ver[2];
-    const bool ext = ext_in[b] != 0;
-    // psi = -k d.c for internal beams; external beams carry no direction phase
-    h[H_KC + 0] = ext ? 0.0 : -k * cen[0];
-    h[H_KC + 1] = ext ? 0.0 : -k * cen[1];
-    h[H_KC + 2] = ext ? 0.0 : -k * cen[2];
-    // complWave is folded into J_phased below; the small-phase area limit is
-    // therefore stored divided by complWave.
-    const double area = s[12] * (sc * sc);
-    const double cw2 = cw_re * cw_re + cw_im * cw_im;
-    const double lr = al_re * area, li = al_im * area;
-    h[H_AL + 0] = (lr * cw_re + li * cw_im) / cw2;
-    h[H_AL + 1] = (li * cw_re - lr * cw_im) / cw2;
-    // polygon moments about the aperture origin
-    double tw = 0, fx6 = 0, fy6 = 0, sx12 = 0, sy12 = 0, sxy24 = 0;
+    for (int i = q; i < nv; i += PACK_GROUP) {
+        s_x[g][i] = vx[v0 + i] * sc;
+        s_y[g][i] = vy[v0 + i] * sc;
+    }
+    __syncthreads();
+    const double *s = s_bs + (b - first) * 36, *px = s_x[g], *py = s_y[g];
+    double *h = s_h + g * HDR_STRIDE;
+    // polygon sums about the aperture origin, and the bounding box
+    double sum[6] = {0, 0, 0, 0, 0, 0}, m3[4] = {0, 0, 0, 0}, m4[5] = {0, 0, 0, 0, 0},
+           m5[6] = {0, 0, 0, 0, 0, 0};
     double minX = 1e300, maxX = -1e300, minY = 1e300, maxY = -1e300;
-    for (int i = 0; i < nv; ++i) {
+    for (int i = q; i < nv; i += PACK_GROUP) {
         const int j = (i + 1 < nv) ? i + 1 : 0;
-        const double xi = X(i), yi = Y(i);
-        const double xj = X(j), yj = Y(j);
+        const double xi = px[i], yi = py[i], xj = px[j], yj = py[j];
         const double cr = xi * yj - xj * yi;
-        tw += cr;
-        fx6 += (xi + xj) * cr;
-        fy6 += (yi + yj) * cr;
-        sx12 += (xi * xi + xi * xj + xj * xj) * cr;
-        sy12 += (yi * yi + yi * yj + yj * yj) * cr;
-        sxy24 += (2.0 * xi * yi + xi * yj + xj * yi + 2.0 * xj * yj) * cr;
+        sum[0] += cr;
+        sum[1] += (xi + xj) * cr;
+        sum[2] += (yi + yj) * cr;
+        sum[3] += (xi * xi + xi * xj + xj * xj) * cr;
+        sum[4] += (yi * yi + yi * yj + yj * yj) * cr;
+        sum[5] += (2.0 * xi * yi + xi * yj + xj * yi + 2.0 * xj * yj) * cr;
         minX = fmin(minX, xi);
         maxX = fmax(maxX, xi);
         minY = fmin(minY, yi);
         maxY = fmax(maxY, yi);
-    }
-    const double areaScale = fmax((maxX - minX) * (maxY - minY), 2.2250738585072014e-308);
-    double mX = 0, mY = 0, mXX = 0, mYY = 0, mXY = 0;
-    if (!(fabs(tw) <= 0x1p-40 * areaScale)) {
-        const double inv = 2.0 / tw;
-        mX = (fx6 / 6.0) * inv;
-        mY = (fy6 / 6.0) * inv;
-        mXX = (sx12 / 12.0) * inv;
-        mYY = (sy12 / 12.0) * inv;
-        mXY = (sxy24 / 24.0) * inv;
-    }
-    h[H_MOM + 0] = k * mX;
-    h[H_MOM + 1] = k * mY;
-    h[H_MOM + 2] = k * k * mXX;
-    h[H_MOM + 3] = 2.0 * k * k * mXY;
-    h[H_MOM + 4] = k * k * mYY;
-    // Orders 3-5.  Over the triangle (0, P, Q) of each edge, with x = s Px +
-    // t Qx, y = s Py + t Qy and the simplex integral of s^i t^j equal to
-    // i! j! / (i + j + 2)!, the integral of x^a y^b is det(P, Q) times
-    //   sum_{i<=a, j<=b} C(a,i) C(b,j) Px^i Qx^(a-i) Py^j Qy^(b-j)
-    //                    (i+j)! (a+b-i-j)! / (a+b+2)!.
-    // Summed over the edges it is the polygon's moment; divided by the area
-    // (tw / 2), the mean <x^a y^b>.
-    {
-        const double fact[8] = {1, 1, 2, 6, 24, 120, 720, 5040};
-        const double binom[6][6] = {{1, 0, 0, 0, 0, 0}, {1, 1, 0, 0, 0, 0},
-                                    {1, 2, 1, 0, 0, 0}, {1, 3, 3, 1, 0, 0},
-                                    {1, 4, 6, 4, 1, 0}, {1, 5, 10, 10, 5, 1}};
-        const bool ok = !(fabs(tw) <= 0x1p-40 * areaScale);
-        const int base_of[6] = {0, 0, 0, H_MOM3, H_MOM4, H_MOM5};
-        double kn = k * k;
-        for (int n = 3; n <= 5; ++n) {
-            kn *= k;
-            for (int a = 0; a <= n; ++a) {
-                const int b2 = n - a;
-                double sum = 0.0;
-                for (int e = 0; e < nv; ++e) {
-                    const int f = (e + 1 < nv) ? e + 1 : 0;
-                    const double px = X(e), py = Y(e), qx = X(f), qy = Y(f);
-                    const double det = px * qy - qx * py;
-                    double acc = 0.0;
-                    for (int i = 0; i <= a; ++i)
-                        for (int j = 0; j <= b2; ++j)
-                            acc += binom[a][i] * binom[b2][j] * pow(px, i) * pow(qx, a - i) *
-                                   pow(py, j) * pow(qy, b2 - j) * fact[i + j] *
-                                   fact[n - i - j];
-                    sum += det * acc;
-                }
-                const double mean = ok ? sum / fact[n + 2] * (2.0 / tw) : 0.0;
-                h[base_of[n] + a] = kn * binom[n][a] * mean / fact[n];
-            }
+        const double node[3] = {0.5 - 0.38729833462074168852, 0.5, 0.5 + 0.38729833462074168852};
+        const double weight[3] = {5.0 / 18.0, 8.0 / 18.0, 5.0 / 18.0};
+        for (int n = 0; n < 3; ++n) {
+            const double x = xi + node[n] * (xj - xi), y = yi + node[n] * (yj - yi);
+            const double w = weight[n] * cr;
+            const double x2 = x * x, y2 = y * y, wx3 = w * x * x2, wy3 = w * y * y2;
+            m3[0] += wy3;
+            m3[1] += w * x * y2;
+            m3[2] += w * x2 * y;
+            m3[3] += wx3;
+            m4[0] += wy3 * y;
+            m4[1] += wy3 * x;
+            m4[2] += w * x2 * y2;
+            m4[3] += wx3 * y;
+            m4[4] += wx3 * x;
+            m5[0] += wy3 * y2;
+            m5[1] += wy3 * x * y;
+            m5[2] += wy3 * x2;
+            m5[3] += wx3 * y2;
+            m5[4] += wx3 * x * y;
+            m5[5] += wx3 * x2;
         }
     }
+    for (double &v : sum)
+        v = group_sum(v);
+    for (double &v : m3)
+        v = group_sum(v);
+    for (double &v : m4)
+        v = group_sum(v);
+    for (double &v : m5)
+        v = group_sum(v);
+    minX = group_min(minX);
+    minY = group_min(minY);
+    maxX = -group_min(-maxX);
+    maxY = -group_min(-maxY);
+    const double tw = sum[0];
+    const double areaScale = fmax((maxX - minX) * (maxY - minY), 2.2250738585072014e-308);
+    const double inv = !(fabs(tw) <= 0x1p-40 * areaScale) ? 2.0 / tw : 0.0;
     // Small-phase bound.  The vertex phases k (A x + B y) spread over at
     // least k |(A, B)| w, w the least width of the vertex set, so some phase
     // exceeds 1e-3 rad once max(|A|, |B|) > 2e-3 / (k w); the kernels test
@@ -269,104 +256,147 @@ __global__ void pack_beams_kernel(int n_beams, const double *__restrict__ bs,
     // across the line through the pair: every edge of the convex hull is such
     // a pair, and the hull's least width lies across one of its edges.
     double wmin = __builtin_inf();
-    if (nv <= 32) {
-        for (int i = 0; i < nv; ++i) {
-            const double xi = X(i), yi = Y(i);
-            for (int j = i + 1; j < nv; ++j) {
-                const double ex = X(j) - xi, ey = Y(j) - yi;
-                const double len = sqrt(ex * ex + ey * ey);
-                if (!(len > 0.0))
-                    continue;
-                double lo = 0.0, hi = 0.0;
-                for (int l = 0; l < nv; ++l) {
-                    const double c = ex * (Y(l) - yi) - ey * (X(l) - xi);
-                    lo = fmin(lo, c);
-                    hi = fmax(hi, c);
-                }
-                wmin = fmin(wmin, (hi - lo) / len);
+    for (int i = q; i < nv; i += PACK_GROUP) {
+        const double xi = px[i], yi = py[i];
+        for (int j = i + 1; j < nv; ++j) {
+            const double ex = px[j] - xi, ey = py[j] - yi;
+            const double len = sqrt(ex * ex + ey * ey);
+            if (!(len > 0.0))
+                continue;
+            double lo = 0.0, hi = 0.0;
+            for (int l = 0; l < nv; ++l) {
+                const double c = ex * (py[l] - yi) - ey * (px[l] - xi);
+                lo = fmin(lo, c);
+                hi = fmax(hi, c);
             }
+            wmin = fmin(wmin, (hi - lo) / len);
         }
     }
-    // a degenerate or very large polygon keeps the per-vertex test everywhere
-    h[H_PHB] = (wmin > 0.0 && wmin < __builtin_inf()) ? 2.04e-3 / (k * wmin)
-                                                      : __builtin_inf();
-    // the mixed kernels compare in FP32: the bound is kept as an FP32 value
-    // in the slot's low word, so no conversion is needed per beam
-    h[H_PHBM] = __builtin_bit_cast(
-        double, (uint64_t)__builtin_bit_cast(
-                    uint32_t, (float)(h[H_PHB] * (kSmallPhaseMixed / kSmallPhase))));
-    // rotation vectors, pre-scaled by 1/2 (exact)
-    for (int q = 0; q < 3; ++q) {
-        h[H_T0 + q] = 0.5 * s[13 + q];      // NT
-        h[H_T0 + 3 + q] = 0.5 * s[19 + q];  // nxDT
-        h[H_T1 + q] = 0.5 * s[16 + q];      // NP
-        h[H_T1 + 3 + q] = 0.5 * s[22 + q];  // nxDP
+    wmin = group_min(wmin);
+    const bool ext = ext_in[b] != 0;
+    if (q == 0) {
+        const double *hor = s + 0, *ver = s + 3, *bd = s + 6;
+        for (int i = 0; i < 3; ++i) {
+            h[H_HOR + i] = hor[i];
+            h[H_VER + i] = ver[i];
+            // psi = -k d.c for internal beams; external beams carry no
+            // direction phase
+            h[H_KC + i] = ext ? 0.0 : -k * (s[9 + i] * sc);
+        }
+        h[H_A0] = bd[0] * hor[0] + bd[1] * hor[1] + bd[2] * hor[2];
+        h[H_B0] = bd[0] * ver[0] + bd[1] * ver[1] + bd[2] * ver[2];
+        // complWave is folded into J_phased below; the small-phase area limit is
+        // therefore stored divided by complWave.
+        const double area = s[12] * (sc * sc);
+        const double cw2 = cw_re * cw_re + cw_im * cw_im;
+        const double lr = al_re * area, li = al_im * area;
+        h[H_AL + 0] = (lr * cw_re + li * cw_im) / cw2;
+        h[H_AL + 1] = (li * cw_re - lr * cw_im) / cw2;
+        // a degenerate or very large polygon keeps the per-vertex test everywhere
+        const double phb =
+            (wmin > 0.0 && wmin < __builtin_inf()) ? 2.04e-3 / (k * wmin) : __builtin_inf();
+        h[H_PHB] = phb;
+        // the mixed kernels compare in FP32: the bound is kept as an FP32 value
+        // in the slot's low word, so no conversion is needed per beam
+        h[H_PHBM] = __builtin_bit_cast(
+            double, (uint64_t)__builtin_bit_cast(
+                        uint32_t, (float)(phb * (kSmallPhaseMixed / kSmallPhase))));
+        for (int i = HDR_USED; i < HDR_STRIDE; ++i)
+            h[i] = 0.0;
+    } else if (q == 1) {
+        // entry a of order n: k^n C(n, a) <x^a y^(n-a)> / n!, the mean being
+        // the integral over the polygon divided by its area tw / 2
+        h[H_MOM + 0] = k * ((sum[1] / 6.0) * inv);
+        h[H_MOM + 1] = k * ((sum[2] / 6.0) * inv);
+        h[H_MOM + 2] = k * k * ((sum[3] / 12.0) * inv);
+        h[H_MOM + 3] = 2.0 * k * k * ((sum[5] / 24.0) * inv);
+        h[H_MOM + 4] = k * k * ((sum[4] / 12.0) * inv);
+        const double k3 = k * k * k;
+        const double c3[4] = {1, 3, 3, 1}, c4[5] = {1, 4, 6, 4, 1}, c5[6] = {1, 5, 10, 10, 5, 1};
+        for (int a = 0; a < 4; ++a)
+            h[H_MOM3 + a] = k3 * c3[a] * (m3[a] / 5.0 * inv) / 6.0;
+        for (int a = 0; a < 5; ++a)
+            h[H_MOM4 + a] = k3 * k * c4[a] * (m4[a] / 6.0 * inv) / 24.0;
+        for (int a = 0; a < 6; ++a)
+            h[H_MOM5 + a] = k3 * k * k * c5[a] * (m5[a] / 7.0 * inv) / 120.0;
+    } else if (q == 2) {
+        // rotation vectors, pre-scaled by 1/2 (exact)
+        for (int i = 0; i < 3; ++i) {
+            h[H_T0 + i] = 0.5 * s[13 + i];      // NT
+            h[H_T0 + 3 + i] = 0.5 * s[19 + i];  // nxDT
+            h[H_T1 + i] = 0.5 * s[16 + i];      // NP
+            h[H_T1 + 3 + i] = 0.5 * s[22 + i];  // nxDP
+        }
     }
     // J_phased, or for a rescaled set sign * a(sc) * J * exp(i k_j path sc),
     // a(sc) the mean of exp(c_abs p sc) over the absorption paths p (1 for
     // p <= DBL_EPSILON): the host rule of the multi-size pack
-    double jpv[8];
+    double amp = 1.0, sn = 0.0, cs = 1.0;
     if (raw_j) {
-        double amp = sign[b];
+        amp = sign[b];
         const int64_t a0 = abs_off[b], a1 = abs_off[b + 1];
         if (a1 > a0) {
-            double sum = 0.0;
-            for (int64_t a = a0; a < a1; ++a)
-                sum += abs_path[a] > 2.220446049250313e-16 ? exp(c_abs * abs_path[a] * sc) : 1.0;
-            amp *= sum / (double)(a1 - a0);
+            double total = 0.0;
+            for (int64_t a = a0 + q; a < a1; a += PACK_GROUP)
+                total +=
+                    abs_path[a] > 2.220446049250313e-16 ? exp(c_abs * abs_path[a] * sc) : 1.0;
+            amp *= group_sum(total) / (double)(a1 - a0);
         }
-        double sn, cs;
         sincos(k_j * (path[b] * sc), &sn, &cs);
-        for (int q = 0; q < 4; ++q) {
-            const double jr = raw_j[(size_t)b * 8 + 2 * q] * amp;
-            const double ji = raw_j[(size_t)b * 8 + 2 * q + 1] * amp;
-            jpv[2 * q] = jr * cs - ji * sn;
-            jpv[2 * q + 1] = jr * sn + ji * cs;
-        }
-    } else {
-        for (int q = 0; q < 8; ++q)
-            jpv[q] = s[25 + q];
     }
-    for (int q = 0; q < 4; ++q) {  // complWave * J_phased
-        const double jr = jpv[2 * q], ji = jpv[2 * q + 1];
+    if (q < 4) {  // complWave * J_phased, one complex element a lane
+        double jr, ji;
+        if (raw_j) {
+            const double rr = raw_j[(size_t)b * 8 + 2 * q] * amp;
+            const double ri = raw_j[(size_t)b * 8 + 2 * q + 1] * amp;
+            jr = rr * cs - ri * sn;
+            ji = rr * sn + ri * cs;
+        } else {
+            jr = s[25 + 2 * q];
+            ji = s[26 + 2 * q];
+        }
         h[H_JP + 2 * q] = cw_re * jr - cw_im * ji;
         h[H_JP + 2 * q + 1] = cw_re * ji + cw_im * jr;
     }
-    // MFMA operand: W[m][c] = T0[m] Jp[0][c] + T1[m] Jp[1][c] (FP64, then FP32)
-    float *w = wb + (size_t)b * WB_STRIDE;
-    for (int n = 0; n < 32; ++n) {
-        double re = 0.0, im = 0.0;
-        if (n < WB_COLS) {
-            const int m = n >> 2, c = (n >> 1) & 1;
-            const double t0 = h[H_T0 + m], t1 = h[H_T1 + m];
-            const double wr = t0 * h[H_JP + 2 * c] + t1 * h[H_JP + 4 + 2 * c];
-            const double wi = t0 * h[H_JP + 2 * c + 1] + t1 * h[H_JP + 4 + 2 * c + 1];
-            const bool imag_col = n & 1;
-            re = imag_col ? wi : wr;   // row 0 multiplies Re F
-            im = imag_col ? wr : -wi;  // row 1 multiplies Im F
+    if (g < count)
+        for (int i = q; i < nv; i += PACK_GROUP) {
+            double *v = vtx + (size_t)(v0 + i) * VTX_STRIDE;
+            const uint8_t f = ef[v0 + i];
+            v[V_KX] = k * px[i];
+            v[V_KY] = k * py[i];
+            v[V_SYX] = (f & 1) ? syx[v0 + i] : kInvalidSlope;
+            v[V_SXY] = (f & 2) ? sxy[v0 + i] : kInvalidSlope;
+            const int j = (i + 1 < nv) ? i + 1 : 0;
+            double *w = vdd + (size_t)(v0 + i) * VDD_STRIDE;
+            w[D_DX] = px[j] - px[i];
+            w[D_DY] = py[j] - py[i];
+            vflag[v0 + i] = f;
         }
-        w[n] = (float)re;
-        w[32 + n] = (float)im;
+    __syncthreads();
+    // the records of the workgroup's beams are contiguous
+    for (int i = threadIdx.x; i < count * HDR_STRIDE; i += PACK_THREADS)
+        hdr[(size_t)first * HDR_STRIDE + i] = s_h[i];
+    // FP32 copy of the rotation data the vector-ALU mixed kernel uses: T0, T1
+    // and complWave J_phased lie together from H_T0 on
+    static_assert(H32_T0 == 0 && H32_T1 == H_T1 - H_T0 && H32_JP == H_JP - H_T0, "");
+    for (int i = threadIdx.x; i < count * HDR32_STRIDE; i += PACK_THREADS) {
+        const int c = i / HDR32_STRIDE, e = i - c * HDR32_STRIDE;
+        hdr32[(size_t)first * HDR32_STRIDE + i] = (float)s_h[c * HDR_STRIDE + H_T0 + e];
     }
-    // FP32 copy of the rotation data the vector-ALU mixed kernel uses
-    for (int q = 0; q < 6; ++q) {
-        h32[H32_T0 + q] = (float)h[H_T0 + q];
-        h32[H32_T1 + q] = (float)h[H_T1 + q];
-    }
-    for (int q = 0; q < 8; ++q)
-        h32[H32_JP + q] = (float)h[H_JP + q];
-    for (int i = 0; i < nv; ++i) {
-        double *v = vtx + (size_t)(v0 + i) * VTX_STRIDE;
-        const uint8_t f = ef[v0 + i];
-        v[V_KX] = k * X(i);
-        v[V_KY] = k * Y(i);
-        v[V_SYX] = (f & 1) ? syx[v0 + i] : kInvalidSlope;
-        v[V_SXY] = (f & 2) ? sxy[v0 + i] : kInvalidSlope;
-        const int j = (i + 1 < nv) ? i + 1 : 0;
-        double *w = vdd + (size_t)(v0 + i) * VDD_STRIDE;
-        w[D_DX] = X(j) - X(i);
-        w[D_DY] = Y(j) - Y(i);
-        vflag[v0 + i] = f;
+    // MFMA operand: W[m][c] = T0[m] Jp[0][c] + T1[m] Jp[1][c] (FP64, then FP32)
+    for (int i = threadIdx.x; i < count * WB_STRIDE; i += PACK_THREADS) {
+        const int c = i / WB_STRIDE, e = i - c * WB_STRIDE, n = e & 31;
+        float out = 0.0f;
+        if (n < WB_COLS) {
+            const double *hb = s_h + c * HDR_STRIDE;
+            const int m = n >> 2, col = (n >> 1) & 1;
+            const double t0 = hb[H_T0 + m], t1 = hb[H_T1 + m];
+            const double wr = t0 * hb[H_JP + 2 * col] + t1 * hb[H_JP + 4 + 2 * col];
+            const double wi = t0 * hb[H_JP + 2 * col + 1] + t1 * hb[H_JP + 4 + 2 * col + 1];
+            // rows 0 and 1 multiply Re F and Im F
+            out = e < 32 ? (float)((n & 1) ? wi : wr) : (float)((n & 1) ? wr : -wi);
+        }
+        wb[(size_t)first * WB_STRIDE + i] = out;
     }
 }
 

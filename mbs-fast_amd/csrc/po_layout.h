@@ -25,6 +25,7 @@ enum {
     H_MOM3 = 40,  // (4)
     H_MOM4 = 44,  // (5)
     H_MOM5 = 49,  // (6)
+    HDR_USED = 55,
     HDR_STRIDE = 56
 };
 

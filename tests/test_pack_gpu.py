@@ -1,0 +1,70 @@
+"""The device pack and the aperture integral over every vertex count the ABI
+takes (3..31), at beam counts around the pack's sixteen beams per workgroup,
+against the FP64 oracle.  Half of the beams leave along a pole, so cells near
+it take the small-phase moment forms with the packed moments to fifth order.
+Bars: those of tests/test_engine_gpu.py for the path (FP64 grid L2 1e-10,
+mixed P11 grid L2 1e-4).  No per-cell bar: a single beam's grid has zeros.
+"""
+import numpy as np
+import pytest
+
+import metrics as M
+from conftest import load_fixture
+
+pytestmark = pytest.mark.gpu
+
+
+def polygon_batch(abi, n_beams, seed, scale=1.0):
+    """One orientation of n_beams convex polygons with 3, 4, ... 31, 3, ...
+    vertices on random ellipses, in the frames and with the polarisation data
+    of traced beams; even beams leave along theta = 0."""
+    rng = np.random.default_rng(seed)
+    src = abi.BeamBatch.from_fixture(load_fixture("sobol_average"))
+    bs = src.beam_scalars[rng.integers(0, src.n_beams, n_beams)].copy()
+    nv = 3 + np.arange(n_beams) % 29
+    vo = np.r_[0, np.cumsum(nv)]
+    x, y, syx, sxy, fl = (np.zeros(vo[-1]) for _ in range(5))
+    for b in range(n_beams):
+        a, c = scale * rng.uniform(0.5, 3.0, 2)
+        t = np.sort(rng.uniform(0.0, 2 * np.pi, nv[b]))
+        while np.max(np.diff(np.r_[t, t[0] + 2 * np.pi])) > 3.0 or np.min(np.diff(t)) < 1e-3:
+            t = np.sort(rng.uniform(0.0, 2 * np.pi, nv[b]))
+        v = slice(vo[b], vo[b + 1])
+        x[v], y[v] = a * np.cos(t), c * np.sin(t)
+        dx, dy = np.roll(x[v], -1) - x[v], np.roll(y[v], -1) - y[v]
+        syx[v], sxy[v], fl[v] = dy / dx, dx / dy, 3
+        bs[b, abi.B_AREA] = 0.5 * np.sum(x[v] * np.roll(y[v], -1) - np.roll(x[v], -1) * y[v])
+        if b % 2 == 0:  # rotate the frame so that the beam leaves along theta = 0
+            d = bs[b, abi.B_DIR:abi.B_DIR + 3] / np.linalg.norm(bs[b, abi.B_DIR:abi.B_DIR + 3])
+            u = np.array([0.0, 0.0, -1.0]) - d
+            n2 = u @ u
+            if n2 > 1e-24:  # a reflection is as good as a rotation here
+                for col in (abi.B_HOR, abi.B_VER, abi.B_DIR, abi.B_NT, abi.B_NP, abi.B_NXDT,
+                            abi.B_NXDP, abi.B_NORMAL):
+                    w = bs[b, col:col + 3]
+                    bs[b, col:col + 3] = w - 2.0 * u * (u @ w) / n2
+    ext = (np.arange(n_beams) % 7 == 6).astype(np.int32)
+    return abi.BeamBatch([0, n_beams], [1.0], bs, nv, ext, vo, x, y, syx, sxy, fl)
+
+
+@pytest.mark.parametrize("n_beams", [1, 15, 16, 17, 31, 64])
+def test_every_vertex_count(pkg, oracle, n_beams):
+    abi = pkg.abi
+    consts = abi.consts_from_fixture(load_fixture("sobol_average"))
+    batch = polygon_batch(abi, n_beams, seed=40 + n_beams)
+    theta = np.r_[0.0, np.logspace(-6, -1, 21), np.linspace(0.2, np.pi, 40)]
+    grid = abi.Grid.build(theta, 7)
+    with pkg.engine.Context(0) as ctx:
+        ctx.set_grid(grid)
+        ctx.upload(batch, consts)
+        o, on, _ = oracle.diffract(grid, batch, consts, noshadow=True)
+        m, mn = ctx.mueller(abi.PREC_FP64, noshadow=True)
+        for a, b in ((m, o), (mn, on)):
+            print("%d beams FP64: %s" % (n_beams, M.summary(a, b, theta)))
+            assert M.grid_l2(a, b, theta) < 1e-10
+        for extra in (0, abi.NO_MFMA):
+            m, mn = ctx.mueller(abi.PREC_MIXED | extra, noshadow=True)
+            for a, b in ((m, o), (mn, on)):
+                e = M.grid_l2(a[..., :1], b[..., :1], theta)
+                print("%d beams mixed (%d): P11 grid_l2 %.2e" % (n_beams, extra, e))
+                assert e < 1e-4
