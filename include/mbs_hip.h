@@ -112,12 +112,15 @@ typedef struct mbs_consts {
 
 /* Flags of mbs_diffract. */
 #define MBS_PREC_FP64 0u      /* FP64 throughout                                */
-#define MBS_PREC_MIXED 1u     /* FP64 phase arguments, their reduction, edge
-                                 coefficients and polygon moments; FP32
-                                 phasors, edge sums, rotation and Jones sums.
-                                 Edges with |C| <= max(eps1, 3e-5) take the
-                                 exact half-angle form in FP64, as the
-                                 reference FP32 build does                    */
+#define MBS_PREC_MIXED 1u     /* FP64 phase arguments (to 2^-30 turn), phase
+                                 steps and polygon moments; FP32 phasors, edge
+                                 sums and Jones sums, the contraction on
+                                 three-part BF16 factors (24 bits) with FP32
+                                 accumulation.  An edge whose phase step the sum
+                                 divides by, and with MBS_EDGE_* data that
+                                 differ from the vertices any edge, with |C| <=
+                                 max(eps1, 3e-5) takes the exact half-angle form
+                                 in FP64, as the reference FP32 build does    */
 #define MBS_NOSHADOW 4u       /* also accumulate the no-shadow Mueller grid     */
 #define MBS_PER_ORIENT 8u     /* also keep one Mueller grid per orientation     */
 #define MBS_NO_MFMA 16u       /* mixed precision: rotation and coherent sum on

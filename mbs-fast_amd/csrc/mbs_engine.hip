@@ -85,7 +85,10 @@ struct mbs_ctx {
     DevBuf<int64_t> voff, ooff;
     DevBuf<uint8_t> ef_in;
     DevBuf<double> hdr, vtx, vdd;
-    DevBuf<float> hdr32, wb;
+    DevBuf<uint32_t> wb;          // MFMA operand of the mixed kernels
+    DevBuf<double> ebeam, evert;  // aperture records of the mixed kernels
+    DevBuf<PhasorNode> phasor;        // their phasor nodes
+    bool phasor_ok = false;
     // size rescaling data of the batch (mbs_upload_beam_scaling)
     bool scaling_ok = false;
     double sc_cabs = 0.0, sc_k = 0.0;
@@ -336,7 +339,9 @@ int mbs_ctx_destroy(mbs_ctx *ctx)
     ctx->vtx.release();
     ctx->vdd.release();
     ctx->wb.release();
-    ctx->hdr32.release();
+    ctx->ebeam.release();
+    ctx->evert.release();
+    ctx->phasor.release();
     ctx->items.release();
     ctx->queue.release();
     ctx->part.release();
@@ -418,11 +423,17 @@ int mbs_set_grid(mbs_ctx *ctx, const mbs_grid *g)
     HIP_TRY(ctx, ctx->vf.ensure((size_t)cells * 3));
     HIP_TRY(ctx, ctx->tab.ensure((size_t)cells * DT_COUNT));
     HIP_TRY(ctx, ctx->tab32.ensure((size_t)cells * DT32_COUNT));
+    HIP_TRY(ctx, ctx->phasor.ensure(kPhasorN));
     HIP_TRY(ctx, hipMemcpyAsync(ctx->theta.p, g->theta, sizeof(double) * ctx->n_zen1,
                                 hipMemcpyHostToDevice, ctx->stream));
     HIP_TRY(ctx, hipMemcpyAsync(ctx->vf.p, g->vf, sizeof(double) * cells * 3,
                                 hipMemcpyHostToDevice, ctx->stream));
+    if (!ctx->phasor_ok) {  // once per context
+        phasor_node_kernel<<<kPhasorN, 64, 0, ctx->stream>>>(ctx->phasor.p);
+        HIP_TRY(ctx, hipGetLastError());
+    }
     HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+    ctx->phasor_ok = true;
     ctx->tab_mode = -1;
     ctx->grid_ok = true;
     return MBS_OK;
@@ -444,6 +455,11 @@ static int ensure_tables(mbs_ctx *ctx)
     return MBS_OK;
 }
 
+// The mixed kernels form edge phasor differences in FP32, so their switch to
+// the exact half-angle edge form happens at |C| <= 3e-5, the floor the
+// reference applies to its FP32 build (GpuDiffraction.cu:498-512).
+static double mixed_eps(const mbs_consts &c) { return std::max(c.eps1, 3e-5); }
+
 // Device records from the uploaded inputs: pack_beams_kernel on the
 // context's stream, for size scale `scale` with the scaling data when
 // `rescale`, else as uploaded.
@@ -456,8 +472,8 @@ static int launch_pack(mbs_ctx *ctx, int nb, const mbs_consts &c, double scale, 
         ctx->syx_in.p, ctx->sxy_in.p, ctx->ef_in.p, c.wave_index, sg * c.inv_compl_wave[0],
         sg * c.inv_compl_wave[1], c.compl_wave[0], c.compl_wave[1], rescale ? scale : 1.0,
         rescale ? ctx->sc_raw.p : nullptr, ctx->sc_path.p, ctx->sc_sign.p, ctx->sc_aoff.p,
-        ctx->sc_apath.p, ctx->sc_cabs, ctx->sc_k, ctx->hdr.p, ctx->hdr32.p, ctx->vtx.p,
-        ctx->vdd.p, ctx->vflag.p, ctx->wb.p);
+        ctx->sc_apath.p, ctx->sc_cabs, ctx->sc_k, mixed_eps(c), ctx->hdr.p, ctx->vtx.p,
+        ctx->vdd.p, ctx->vflag.p, ctx->wb.p, ctx->ebeam.p, ctx->evert.p);
     HIP_TRY(ctx, hipGetLastError());
     return MBS_OK;
 }
@@ -492,8 +508,6 @@ static int upload_impl(mbs_ctx *ctx, const mbs_beam_batch *bt, const mbs_consts 
     for (int o = 0; o < no; ++o) {
         if (bt->orient_offsets[o + 1] < bt->orient_offsets[o])
             return fail(ctx, MBS_ERR_INVALID, "orient_offsets decrease at %d", o);
-        // the MFMA kernel addresses a beam range's operands with 32-bit byte
-        // offsets (WB_STRIDE floats per beam)
         if (bt->orient_offsets[o + 1] - bt->orient_offsets[o] > MBS_MAX_BEAMS_PER_ORIENT)
             return fail(ctx, MBS_ERR_CAPACITY,
                         "orientation %d holds %lld beams; at most %d per orientation", o,
@@ -531,7 +545,8 @@ static int upload_impl(mbs_ctx *ctx, const mbs_beam_batch *bt, const mbs_consts 
     HIP_TRY(ctx, ctx->sxy_in.ensure(nvert));
     HIP_TRY(ctx, ctx->ef_in.ensure(nvert));
     HIP_TRY(ctx, ctx->hdr.ensure((size_t)nb * HDR_STRIDE));
-    HIP_TRY(ctx, ctx->hdr32.ensure((size_t)nb * HDR32_STRIDE));
+    HIP_TRY(ctx, ctx->ebeam.ensure((size_t)nb * EB_STRIDE));
+    HIP_TRY(ctx, ctx->evert.ensure((size_t)nvert * EV_STRIDE));
     HIP_TRY(ctx, ctx->vtx.ensure((size_t)nvert * VTX_STRIDE));
     HIP_TRY(ctx, ctx->vdd.ensure((size_t)nvert * VDD_STRIDE));
     HIP_TRY(ctx, ctx->wb.ensure((size_t)std::max(nb, 1) * WB_STRIDE));
@@ -827,8 +842,8 @@ static void launch_one(const KernelArgs &a, int blocks, hipStream_t s)
     if constexpr (PREC == 4)
         diffract_mfma_kernel<NS, JONES, PER, Q, 1><<<blocks, 256, 0, s>>>(
             a.items, a.n_items, a.n_tiles, a.cells, a.n_az, a.tab, a.hdr, a.wb, a.vtx, a.vdd,
-            a.vflag, a.nv, a.voff, a.ext, a.ooff, a.weights, a.k, a.eps1, a.out, a.out_ns,
-            a.per_orient, a.queue, a.tab32, a.sidx, a.fbuf);
+            a.vflag, a.ebeam, a.evert, a.phasor, a.ooff, a.weights, a.k,
+            a.eps1, a.out, a.out_ns, a.per_orient, a.queue, a.tab32, a.sidx, a.fbuf);
     else if constexpr (PREC == 3)
         diffract_incoherent_kernel<<<blocks, 256, 0, s>>>(
             a.items, a.n_items, a.n_tiles, a.cells, a.tab, a.hdr, a.vtx, a.vdd, a.vflag, a.nv,
@@ -836,14 +851,13 @@ static void launch_one(const KernelArgs &a, int blocks, hipStream_t s)
     else if constexpr (PREC == 2)
         diffract_mfma_kernel<NS, JONES, PER, Q><<<blocks, 256, 0, s>>>(
             a.items, a.n_items, a.n_tiles, a.cells, a.n_az, a.tab, a.hdr, a.wb, a.vtx, a.vdd,
-            a.vflag,
-            a.nv, a.voff, a.ext, a.ooff, a.weights, a.k, a.eps1, a.out, a.out_ns,
+            a.vflag, a.ebeam, a.evert, a.phasor, a.ooff, a.weights, a.k, a.eps1, a.out, a.out_ns,
             a.per_orient, a.queue, a.tab32);
     else
         diffract_kernel<PREC, NS, JONES, PER, Q><<<blocks, 256, 0, s>>>(
-            a.items, a.n_items, a.n_tiles, a.cells, a.n_az, a.tab, a.hdr, a.hdr32, a.vtx, a.vdd,
-            a.vflag, a.nv, a.voff, a.ext, a.ooff, a.weights, a.k, a.eps1, a.out, a.out_ns,
-            a.per_orient, a.queue, a.tab32);
+            a.items, a.n_items, a.n_tiles, a.cells, a.n_az, a.tab, a.hdr, a.vtx, a.vdd, a.vflag,
+            a.nv, a.voff, a.ext, a.ooff, a.weights, a.k, a.eps1, a.out, a.out_ns, a.per_orient,
+            a.queue, a.tab32, a.ebeam, a.evert, a.phasor);
 }
 
 // queue: the persistent work-queue kernels (beam segments, no per-orientation
@@ -856,12 +870,12 @@ static void launch_diffract(int prec, int ns, int jones, int per, bool queue,
         if (a.waves == 4)
             diffract_mfma_kernel<0, 1, 0, 0, 0, 4><<<blocks, 256, 0, s>>>(
                 a.items, a.n_items, a.n_tiles, a.cells, a.n_az, a.tab, a.hdr, a.wb, a.vtx,
-                a.vdd, a.vflag, a.nv, a.voff, a.ext, a.ooff, a.weights, a.k, a.eps1, a.out,
+                a.vdd, a.vflag, a.ebeam, a.evert, a.phasor, a.ooff, a.weights, a.k, a.eps1, a.out,
                 a.out_ns, a.per_orient, a.queue, a.tab32);
         else
             diffract_mfma_kernel<0, 1, 0, 0, 0, 6><<<blocks, 256, 0, s>>>(
                 a.items, a.n_items, a.n_tiles, a.cells, a.n_az, a.tab, a.hdr, a.wb, a.vtx,
-                a.vdd, a.vflag, a.nv, a.voff, a.ext, a.ooff, a.weights, a.k, a.eps1, a.out,
+                a.vdd, a.vflag, a.ebeam, a.evert, a.phasor, a.ooff, a.weights, a.k, a.eps1, a.out,
                 a.out_ns, a.per_orient, a.queue, a.tab32);
         return;
     }
@@ -952,7 +966,9 @@ static void batch_args(const mbs_ctx *ctx, int prec, int n_items, int n_tiles, K
     a.tab = ctx->tab.p;
     a.tab32 = ctx->tab32.p;
     a.hdr = ctx->hdr.p;
-    a.hdr32 = ctx->hdr32.p;
+    a.ebeam = ctx->ebeam.p;
+    a.evert = ctx->evert.p;
+    a.phasor = ctx->phasor.p;
     a.wb = ctx->wb.p;
     a.vtx = ctx->vtx.p;
     a.vdd = ctx->vdd.p;
@@ -963,14 +979,9 @@ static void batch_args(const mbs_ctx *ctx, int prec, int n_items, int n_tiles, K
     a.ooff = ctx->ooff.p;
     a.weights = ctx->weights.p;
     a.k = ctx->consts.wave_index;
-    // The mixed kernel forms edge phasor differences in FP32, so its
-    // switch to the exact half-angle edge form happens at |C| <= 3e-5, the
-    // floor the reference applies to its FP32 build (GpuDiffraction.cu:498-512).
-    // The FP64 kernels (prec 0, and 3 = the FP64 incoherent sum) keep the
-    // handler's eps1.  (prec 4: the mixed MFMA kernel with the spectrum
-    // source.)
-    a.eps1 = (prec == 1 || prec == 2 || prec == 4) ? std::max(ctx->consts.eps1, 3e-5)
-                                                   : ctx->consts.eps1;
+    // the FP64 kernels (prec 0, and 3 = the FP64 incoherent sum) keep the
+    // handler's eps1 (prec 4: the mixed MFMA kernel with the spectrum source)
+    a.eps1 = (prec == 1 || prec == 2 || prec == 4) ? mixed_eps(ctx->consts) : ctx->consts.eps1;
     if (prec == 4) {
         a.sidx = ctx->spec_sidx.p;
         a.fbuf = ctx->spec_f.p;

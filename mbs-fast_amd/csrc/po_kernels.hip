@@ -23,6 +23,8 @@
 //   max|phi_v| <= 1e-3 and the half-angle form when |C_e| <= eps1;
 //   r_ij = u_i(d).T_j(beam) (the Jones rotation of HandlerPO_fast.h:580-683
 //   rewritten exactly with per-direction vectors u_i), d = F R J_phased.
+// The mixed kernels evaluate the same integral from other sums: see "mixed
+// precision" below.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -39,14 +41,13 @@
 #define MBS_MIN_WAVES 4
 #endif
 #define MBS_OCCUPANCY __attribute__((amdgpu_waves_per_eu(MBS_MIN_WAVES, 8)))
-// The MFMA kernel is held to WAVES waves per SIMD (default 5: 96 VGPRs)
-// when it keeps one accumulator set -- its 20.5 KB of LDS per workgroup lets
-// seven workgroups share a CU; the no-shadow variant (two sets) gets 2.  The
-// autotuner also tries 4 and 6 for the default beam-segment kernel.
+// The MFMA kernel is held to WAVES waves per SIMD (default 5: 96 VGPRs); its
+// 29 KB of LDS per workgroup lets five workgroups share a CU.  The autotuner
+// also tries 4 and 6 for the default beam-segment kernel.
 #ifndef MBS_MFMA_WAVES
 #define MBS_MFMA_WAVES 5
 #endif
-#define MBS_MFMA_OCCUPANCY __attribute__((amdgpu_waves_per_eu(NS ? 2 : WAVES, 8)))
+#define MBS_MFMA_OCCUPANCY __attribute__((amdgpu_waves_per_eu(WAVES, 8)))
 
 namespace mbs {
 
@@ -73,6 +74,44 @@ __device__ __forceinline__ size_t abi_cell(int cell, int n_az, int cells)
 // rotate_jones_inline does).  Then cpT.vt = NT.(vt x d) + nxDT.(vt - d(d.vt))
 // for cpT = d x NT + nxDT - d (d.nxDT), and likewise for cpP, vf.
 // ---------------------------------------------------------------------------
+// Phasor nodes (po_math.h), one wave per node: of the angles within
+// kNodeTries / 2 steps of 2e-7 rad around the nominal one, the angle whose
+// cosine and sine / sqrt(2) are nearest to FP32 numbers (the least of the
+// larger error, the first of equal ones).
+constexpr int kNodeTries = 2048;
+__global__ void __launch_bounds__(64) phasor_node_kernel(PhasorNode *__restrict__ tab)
+{
+    const int j = blockIdx.x;
+    const double nominal = (j + 0.5) * (2.0 * kPi / kPhasorN);
+    double best = 1.0;
+    int at = 0;
+    for (int i = threadIdx.x; i < kNodeTries; i += 64) {
+        double s, c;
+        sincos(nominal + (i - kNodeTries / 2) * 2e-7, &s, &c);
+        s *= 0.70710678118654752440;
+        const double e = fmax(fabs(c - (float)c), fabs(s - (float)s));
+        if (e < best) {
+            best = e;
+            at = i;
+        }
+    }
+    for (int off = 1; off < 64; off <<= 1) {
+        const double e = __shfl_xor(best, off, 64);
+        const int i = __shfl_xor(at, off, 64);
+        if (e < best || (e == best && i < at)) {
+            best = e;
+            at = i;
+        }
+    }
+    if (threadIdx.x == 0) {
+        const double delta = (at - kNodeTries / 2) * 2e-7;
+        double s, c;
+        sincos(nominal + delta, &s, &c);
+        tab[j] = PhasorNode{(float)c, (float)(s * 0.70710678118654752440),
+                            (float)(-kPhasorHalf - delta * 0.70710678118654752440), 0.0f};
+    }
+}
+
 __global__ void grid_tables_kernel(const double *__restrict__ theta,
                                    const double *__restrict__ vf, int n_az,
                                    int n_zen1, double az_step,
@@ -133,14 +172,14 @@ __global__ void grid_tables_kernel(const double *__restrict__ theta,
 // moments follow small_phase_polygon_factor (src/handler/HandlerPO_fast.h:154-216).
 //
 // What bounds it is latency for small batches and issue for large ones.  One
-// thread per beam, with the moments of orders 3-5 from binomial sums of pow()
+// thread per beam, with the moments (orders 3-5 then) from binomial sums of pow()
 // (about 1,800 calls for a 4-vertex beam), took 0.73 ms for 185 beams, 1.74 ms
 // for 59,000 and 2.57 ms for 137,000; this form takes 13, 53 and 105 us.  The
 // polygon is staged in LDS, the lanes of a group
 // take the vertices in turn and add their sums by butterflies, and an edge's
-// share of a moment is a 3-point Gauss rule: over the triangle (0, P, Q) a
+// share of a moment is a 4-point Gauss rule: over the triangle (0, P, Q) a
 // monomial of degree n integrates to det(P, Q) / (n + 2) times its mean along
-// PQ, which three nodes give exactly to degree 5.  The record goes through LDS
+// PQ, which four nodes give exactly to degree 7.  The record goes through LDS
 // so that its stores are contiguous.
 // ---------------------------------------------------------------------------
 enum { PACK_GROUP = 8, PACK_BEAMS = 16, PACK_THREADS = PACK_GROUP * PACK_BEAMS };
@@ -159,6 +198,40 @@ __device__ __forceinline__ double group_min(double v)
     return v;
 }
 
+// FP32 -> BF16 bits, nearest (ties to even), and back.
+__device__ __forceinline__ uint32_t bf16_bits(float x)
+{
+    const uint32_t u = __float_as_uint(x);
+    return (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
+}
+__device__ __forceinline__ float bf16_value(uint32_t b) { return __uint_as_float(b << 16); }
+
+// Two 32-bit values in one FP64 slot (low word first).
+__device__ __forceinline__ double pack_words(uint32_t lo, uint32_t hi)
+{
+    return __builtin_bit_cast(double, (uint64_t)lo | (uint64_t)hi << 32);
+}
+__device__ __forceinline__ double pack_floats(float lo, float hi)
+{
+    return pack_words(__float_as_uint(lo), __float_as_uint(hi));
+}
+__device__ __forceinline__ int low_word(double slot)
+{
+    return (int)(uint32_t)__builtin_bit_cast(uint64_t, slot);
+}
+__device__ __forceinline__ int high_word(double slot)
+{
+    return (int)(uint32_t)(__builtin_bit_cast(uint64_t, slot) >> 32);
+}
+__device__ __forceinline__ float low_float(double slot)
+{
+    return __uint_as_float((uint32_t)__builtin_bit_cast(uint64_t, slot));
+}
+__device__ __forceinline__ float high_float(double slot)
+{
+    return __uint_as_float((uint32_t)(__builtin_bit_cast(uint64_t, slot) >> 32));
+}
+
 __global__ void __launch_bounds__(PACK_THREADS) pack_beams_kernel(
     int n_beams, const double *__restrict__ bs, const int32_t *__restrict__ nv_in,
     const int32_t *__restrict__ ext_in, const int64_t *__restrict__ voff,
@@ -168,13 +241,14 @@ __global__ void __launch_bounds__(PACK_THREADS) pack_beams_kernel(
     double cw_im, double sc, const double *__restrict__ raw_j,
     const double *__restrict__ path, const double *__restrict__ sign,
     const int64_t *__restrict__ abs_off, const double *__restrict__ abs_path, double c_abs,
-    double k_j, double *__restrict__ hdr, float *__restrict__ hdr32,
-    double *__restrict__ vtx, double *__restrict__ vdd, int32_t *__restrict__ vflag,
-    float *__restrict__ wb)
+    double k_j, double eps_mixed, double *__restrict__ hdr, double *__restrict__ vtx,
+    double *__restrict__ vdd, int32_t *__restrict__ vflag, uint32_t *__restrict__ wb,
+    double *__restrict__ ebeam, double *__restrict__ evert)
 {
     __shared__ double s_bs[PACK_BEAMS * 36];
     __shared__ double s_x[PACK_BEAMS][33], s_y[PACK_BEAMS][33];  // odd stride: no bank conflicts
     __shared__ double s_h[PACK_BEAMS * HDR_STRIDE];
+    __shared__ double s_scale[PACK_BEAMS];
     const int g = threadIdx.x / PACK_GROUP, q = threadIdx.x % PACK_GROUP;
     const int first = blockIdx.x * PACK_BEAMS;
     const int count = min((int)PACK_BEAMS, n_beams - first);  // beams of this workgroup
@@ -194,8 +268,11 @@ __global__ void __launch_bounds__(PACK_THREADS) pack_beams_kernel(
     double *h = s_h + g * HDR_STRIDE;
     // polygon sums about the aperture origin, and the bounding box
     double sum[6] = {0, 0, 0, 0, 0, 0}, m3[4] = {0, 0, 0, 0}, m4[5] = {0, 0, 0, 0, 0},
-           m5[6] = {0, 0, 0, 0, 0, 0};
+           m5[6] = {0, 0, 0, 0, 0, 0}, m6[7] = {0, 0, 0, 0, 0, 0, 0},
+           m7[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     double minX = 1e300, maxX = -1e300, minY = 1e300, maxY = -1e300;
+    double longest = -1.0;  // squared length of this lane's longest edge, and
+    int start = 0;          // the edge (the least index of equal ones)
     for (int i = q; i < nv; i += PACK_GROUP) {
         const int j = (i + 1 < nv) ? i + 1 : 0;
         const double xi = px[i], yi = py[i], xj = px[j], yj = py[j];
@@ -210,27 +287,34 @@ __global__ void __launch_bounds__(PACK_THREADS) pack_beams_kernel(
         maxX = fmax(maxX, xi);
         minY = fmin(minY, yi);
         maxY = fmax(maxY, yi);
-        const double node[3] = {0.5 - 0.38729833462074168852, 0.5, 0.5 + 0.38729833462074168852};
-        const double weight[3] = {5.0 / 18.0, 8.0 / 18.0, 5.0 / 18.0};
-        for (int n = 0; n < 3; ++n) {
+        const double l2 = (xj - xi) * (xj - xi) + (yj - yi) * (yj - yi);
+        if (l2 > longest) {
+            longest = l2;
+            start = i;
+        }
+        const double node[4] = {0.5 - 0.43056815579702628761, 0.5 - 0.16999052179242813240,
+                                0.5 + 0.16999052179242813240, 0.5 + 0.43056815579702628761};
+        const double weight[4] = {0.17392742256872692869, 0.32607257743127307131,
+                                  0.32607257743127307131, 0.17392742256872692869};
+        for (int n = 0; n < 4; ++n) {
             const double x = xi + node[n] * (xj - xi), y = yi + node[n] * (yj - yi);
-            const double w = weight[n] * cr;
-            const double x2 = x * x, y2 = y * y, wx3 = w * x * x2, wy3 = w * y * y2;
-            m3[0] += wy3;
-            m3[1] += w * x * y2;
-            m3[2] += w * x2 * y;
-            m3[3] += wx3;
-            m4[0] += wy3 * y;
-            m4[1] += wy3 * x;
-            m4[2] += w * x2 * y2;
-            m4[3] += wx3 * y;
-            m4[4] += wx3 * x;
-            m5[0] += wy3 * y2;
-            m5[1] += wy3 * x * y;
-            m5[2] += wy3 * x2;
-            m5[3] += wx3 * y2;
-            m5[4] += wx3 * x * y;
-            m5[5] += wx3 * x2;
+            double px7[8], py7[8];  // powers, the weight in those of x
+            px7[0] = weight[n] * cr;
+            py7[0] = 1.0;
+            for (int e = 1; e < 8; ++e) {
+                px7[e] = px7[e - 1] * x;
+                py7[e] = py7[e - 1] * y;
+            }
+            for (int e = 0; e < 4; ++e)
+                m3[e] += px7[e] * py7[3 - e];
+            for (int e = 0; e < 5; ++e)
+                m4[e] += px7[e] * py7[4 - e];
+            for (int e = 0; e < 6; ++e)
+                m5[e] += px7[e] * py7[5 - e];
+            for (int e = 0; e < 7; ++e)
+                m6[e] += px7[e] * py7[6 - e];
+            for (int e = 0; e < 8; ++e)
+                m7[e] += px7[e] * py7[7 - e];
         }
     }
     for (double &v : sum)
@@ -241,6 +325,18 @@ __global__ void __launch_bounds__(PACK_THREADS) pack_beams_kernel(
         v = group_sum(v);
     for (double &v : m5)
         v = group_sum(v);
+    for (double &v : m6)
+        v = group_sum(v);
+    for (double &v : m7)
+        v = group_sum(v);
+    for (int off = 1; off < PACK_GROUP; off <<= 1) {
+        const double l2 = __shfl_xor(longest, off, PACK_GROUP);
+        const int at = __shfl_xor(start, off, PACK_GROUP);
+        if (l2 > longest || (l2 == longest && at < start)) {
+            longest = l2;
+            start = at;
+        }
+    }
     minX = group_min(minX);
     minY = group_min(minY);
     maxX = -group_min(-maxX);
@@ -274,8 +370,8 @@ __global__ void __launch_bounds__(PACK_THREADS) pack_beams_kernel(
     }
     wmin = group_min(wmin);
     const bool ext = ext_in[b] != 0;
+    const double *hor = s + 0, *ver = s + 3, *bd = s + 6;
     if (q == 0) {
-        const double *hor = s + 0, *ver = s + 3, *bd = s + 6;
         for (int i = 0; i < 3; ++i) {
             h[H_HOR + i] = hor[i];
             h[H_VER + i] = ver[i];
@@ -296,11 +392,7 @@ __global__ void __launch_bounds__(PACK_THREADS) pack_beams_kernel(
         const double phb =
             (wmin > 0.0 && wmin < __builtin_inf()) ? 2.04e-3 / (k * wmin) : __builtin_inf();
         h[H_PHB] = phb;
-        // the mixed kernels compare in FP32: the bound is kept as an FP32 value
-        // in the slot's low word, so no conversion is needed per beam
-        h[H_PHBM] = __builtin_bit_cast(
-            double, (uint64_t)__builtin_bit_cast(
-                        uint32_t, (float)(phb * (kSmallPhaseMixed / kSmallPhase))));
+        h[H_SPARE] = 0.0;
         for (int i = HDR_USED; i < HDR_STRIDE; ++i)
             h[i] = 0.0;
     } else if (q == 1) {
@@ -319,6 +411,11 @@ __global__ void __launch_bounds__(PACK_THREADS) pack_beams_kernel(
             h[H_MOM4 + a] = k3 * k * c4[a] * (m4[a] / 6.0 * inv) / 24.0;
         for (int a = 0; a < 6; ++a)
             h[H_MOM5 + a] = k3 * k * k * c5[a] * (m5[a] / 7.0 * inv) / 120.0;
+        const double c6[7] = {1, 6, 15, 20, 15, 6, 1}, c7[8] = {1, 7, 21, 35, 35, 21, 7, 1};
+        for (int a = 0; a < 7; ++a)
+            h[H_MOM6 + a] = k3 * k3 * c6[a] * (m6[a] / 8.0 * inv) / 720.0;
+        for (int a = 0; a < 8; ++a)
+            h[H_MOM7 + a] = k3 * k3 * k * c7[a] * (m7[a] / 9.0 * inv) / 5040.0;
     } else if (q == 2) {
         // rotation vectors, pre-scaled by 1/2 (exact)
         for (int i = 0; i < 3; ++i) {
@@ -358,45 +455,172 @@ __global__ void __launch_bounds__(PACK_THREADS) pack_beams_kernel(
         h[H_JP + 2 * q] = cw_re * jr - cw_im * ji;
         h[H_JP + 2 * q + 1] = cw_re * ji + cw_im * jr;
     }
-    if (g < count)
-        for (int i = q; i < nv; i += PACK_GROUP) {
-            double *v = vtx + (size_t)(v0 + i) * VTX_STRIDE;
-            const uint8_t f = ef[v0 + i];
-            v[V_KX] = k * px[i];
-            v[V_KY] = k * py[i];
-            v[V_SYX] = (f & 1) ? syx[v0 + i] : kInvalidSlope;
-            v[V_SXY] = (f & 2) ? sxy[v0 + i] : kInvalidSlope;
-            const int j = (i + 1 < nv) ? i + 1 : 0;
-            double *w = vdd + (size_t)(v0 + i) * VDD_STRIDE;
-            w[D_DX] = px[j] - px[i];
-            w[D_DY] = py[j] - py[i];
-            vflag[v0 + i] = f;
+    // The beam's class.  The formulas of the mixed kernels work from the
+    // vertices alone, so the slopes and flags have to agree with them (an edge
+    // left out of one branch of the reference's sum must be negligible in it),
+    // and the phases have to fit the fixed-point range; any other beam keeps
+    // the sum over the slopes.
+    const double lmax = sqrt(longest);
+    const double cx = ext ? 0.0 : s[9] * sc, cy = ext ? 0.0 : s[10] * sc,
+                 cz = ext ? 0.0 : s[11] * sc;
+    const double k_turn = k * kInvTwoPi;
+    const double tol = 1e-9 * lmax;
+    double agree = 1.0, reach = 0.0;  // every edge agrees; the largest |vertex|
+    for (int i = q; i < nv; i += PACK_GROUP) {
+        const int to = (i + 1 < nv) ? i + 1 : 0;
+        const double x = px[i], y = py[i], dx = px[to] - x, dy = py[to] - y;
+        const uint8_t f = ef[v0 + i];
+        const bool okx = (f & 1) ? fabs(syx[v0 + i] * dx - dy) <= tol : fabs(dx) <= tol;
+        const bool oky = (f & 2) ? fabs(sxy[v0 + i] * dy - dx) <= tol : fabs(dy) <= tol;
+        if (!(okx && oky && sqrt(dx * dx + dy * dy) > tol && (f & 3)))
+            agree = 0.0;
+        reach = fmax(reach, sqrt(x * x + y * y));
+    }
+    agree = group_min(agree);
+    reach = -group_min(-reach);
+    const double n_hor = hor[0] * hor[0] + hor[1] * hor[1] + hor[2] * hor[2];
+    const double n_ver = ver[0] * ver[0] + ver[1] * ver[1] + ver[2] * ver[2];
+    const double n_bd = bd[0] * bd[0] + bd[1] * bd[1] + bd[2] * bd[2];
+    const double skew = hor[0] * ver[0] + hor[1] * ver[1] + hor[2] * ver[2];
+    // |phase| <= |Q| |d - b| with axes no longer than 1; comparisons written
+    // so that a value that is not a number fails them
+    const bool unit = n_hor <= 1.0 + 1e-6 && n_ver <= 1.0 + 1e-6 && n_bd <= 1.0 + 1e-6;
+    const bool fits = 2.5 * k_turn * (sqrt(cx * cx + cy * cy + cz * cz) + reach) < 0x1p20;
+    int cls = BEAM_VERTICES;
+    double scale = 1.0;  // F / F' of the class's formula
+    if (!(unit && fits && agree == 1.0)) {
+        cls = BEAM_SLOPES;
+    } else if (fabs(skew) <= 1e-6 && 2.01 * k * reach <= kSmallPhaseMixed) {
+        cls = BEAM_MOMENTS;
+    } else if (nv <= 4) {
+        // parallel edges, to 1e-9 of the area's own products (a traced
+        // hexagonal particle: nineteen quadrilaterals in twenty have a
+        // parallel pair, to 1e-12)
+        const auto cross = [&](int i, int j) {
+            const int i1 = (i + 1) % nv, j1 = (j + 1) % nv;
+            return (px[i1] - px[i]) * (py[j1] - py[j]) - (py[i1] - py[i]) * (px[j1] - px[j]);
+        };
+        const auto len2 = [&](int i) {
+            const int i1 = (i + 1) % nv;
+            return (px[i1] - px[i]) * (px[i1] - px[i]) + (py[i1] - py[i]) * (py[i1] - py[i]);
+        };
+        int from = start;
+        if (nv == 3) {
+            cls = BEAM_TRAPEZOID;
+        } else {
+            const double c01 = fabs(cross(0, 1)), c03 = fabs(cross(0, 3)), c21 = fabs(cross(2, 1));
+            const bool p02 = fabs(cross(0, 2)) <= 1e-9 * fmin(c01, c03);
+            const bool p13 = fabs(cross(1, 3)) <= 1e-9 * fmin(c01, c21);
+            const double gx = px[0] - px[1] + px[2] - px[3], gy = py[0] - py[1] + py[2] - py[3];
+            if (p02 && p13 && k * sqrt(gx * gx + gy * gy) <= 1e-8) {
+                cls = BEAM_PARALLEL;
+            } else if (p02 || p13) {
+                cls = BEAM_TRAPEZOID;
+                from = p02 ? (len2(0) >= len2(2) ? 0 : 2) : (len2(1) >= len2(3) ? 1 : 3);
+            }
         }
+        if (cls != BEAM_VERTICES) {
+            // w_1 = -(t_0 x t_1) (k / 2 pi)^2; the sines carry 1/sqrt(2) each
+            const double w1 = -cross(from, (from + 1) % nv) * k_turn * k_turn;
+            scale = cls == BEAM_PARALLEL ? -2.0 * w1 : 1.41421356237309504880 * w1;
+            if (fabs(scale) >= 1e-30 && fabs(scale) <= 1e30) {
+                start = from;
+            } else {
+                cls = nv == 3 ? BEAM_SLOPES : BEAM_VERTICES;
+            }
+        }
+    }
+    if (cls == BEAM_VERTICES)
+        scale = 1.41421356237309504880;
+    else if (cls == BEAM_SLOPES)
+        scale = 1.0;
+    // phase vector in turns of a point of the aperture plane, from the beam
+    // centre or from the particle's origin
+    const auto turns = [&](double x, double y, bool centred, double *out) {
+        for (int i = 0; i < 3; ++i)
+            out[i] = -k_turn * ((centred ? 0.0 : i == 0 ? cx : i == 1 ? cy : cz) + x * hor[i] +
+                                y * ver[i]);
+    };
+    const auto vert = [&](int i) {  // vertex i of the record
+        const int at = start + i;
+        return at < nv ? at : at - nv;
+    };
+    const double t0x = px[vert(1)] - px[vert(0)], t0y = py[vert(1)] - py[vert(0)];
+    for (int i = q; i < nv && g < count; i += PACK_GROUP) {
+        const int at = vert(i), to = (at + 1 < nv) ? at + 1 : 0;
+        const double x = px[at], y = py[at], dx = px[to] - x, dy = py[to] - y;
+        const uint8_t f = ef[v0 + at];
+        double *v = vtx + (size_t)(v0 + i) * VTX_STRIDE;
+        v[V_KX] = k * x;
+        v[V_KY] = k * y;
+        v[V_SYX] = (f & 1) ? syx[v0 + at] : kInvalidSlope;
+        v[V_SXY] = (f & 2) ? sxy[v0 + at] : kInvalidSlope;
+        double *w = vdd + (size_t)(v0 + i) * VDD_STRIDE;
+        w[D_DX] = dx;
+        w[D_DY] = dy;
+        vflag[v0 + i] = f;
+        if (cls == BEAM_VERTICES) {
+            const double cross = i == 0 ? 0.0 : t0x * dy - t0y * dx;
+            double *ev = evert + (size_t)(v0 + i) * EV_STRIDE;
+            turns(x, y, false, ev + EV_Q);
+            ev[EV_W] = nv == 4 ? pack_floats((float)(-cross * k_turn * k_turn), 0.0f)
+                               : pack_floats((float)(k_turn * dx), (float)(-k_turn * dy));
+        }
+    }
+    if (q == 0 && g < count) {
+        const auto X = [&](int i) { return px[vert(i % nv)]; };
+        const auto Y = [&](int i) { return py[vert(i % nv)]; };
+        double *eb = ebeam + (size_t)b * EB_STRIDE, *eq = eb + EB_Q;
+        for (int i = 0; i < EB_STRIDE - EB_Q; ++i)
+            eq[i] = 0.0;
+        if (cls == BEAM_TRAPEZOID) {  // edge 1 and the last one
+            turns(0.5 * (X(1) + X(2)), 0.5 * (Y(1) + Y(2)), false, eq);
+            turns(0.5 * (X(2) - X(1)), 0.5 * (Y(2) - Y(1)), true, eq + 3);
+            turns(0.5 * (X(nv - 1) + X(0)), 0.5 * (Y(nv - 1) + Y(0)), false, eq + 6);
+            turns(0.5 * (X(0) - X(nv - 1)), 0.5 * (Y(0) - Y(nv - 1)), true, eq + 9);
+        } else if (cls == BEAM_PARALLEL) {
+            turns(0.5 * (X(0) + X(2)), 0.5 * (Y(0) + Y(2)), false, eq);
+            turns(0.5 * (X(1) - X(0)), 0.5 * (Y(1) - Y(0)), true, eq + 3);
+            turns(0.5 * (X(2) - X(1)), 0.5 * (Y(2) - Y(1)), true, eq + 6);
+        }
+        const double offset = -k_turn * (cx * bd[0] + cy * bd[1] + cz * bd[2]) +
+                              (cls == BEAM_TRAPEZOID || cls == BEAM_VERTICES ? 0.25 : 0.0);
+        const double sing = eps_mixed * k_turn * sqrt(t0x * t0x + t0y * t0y);
+        for (int i = 0; i < 3; ++i)
+            eb[EB_DIR + i] = bd[i];
+        eb[EB_PHASE] = (offset - rint(offset)) + kTurnMagic;
+        eb[EB_LIM] = pack_floats((float)fmax(sing, kLookStep), (float)sing);
+        eb[EB_SCALE] = pack_floats((float)scale, (float)(1.0 / scale));
+        eb[EB_KIND] = pack_words(nv + BEAM_CLASS * cls, ext ? 1 : 0);
+        eb[EB_VOFF] = __builtin_bit_cast(double, v0);
+        s_scale[g] = scale;
+    }
     __syncthreads();
     // the records of the workgroup's beams are contiguous
     for (int i = threadIdx.x; i < count * HDR_STRIDE; i += PACK_THREADS)
         hdr[(size_t)first * HDR_STRIDE + i] = s_h[i];
-    // FP32 copy of the rotation data the vector-ALU mixed kernel uses: T0, T1
-    // and complWave J_phased lie together from H_T0 on
-    static_assert(H32_T0 == 0 && H32_T1 == H_T1 - H_T0 && H32_JP == H_JP - H_T0, "");
-    for (int i = threadIdx.x; i < count * HDR32_STRIDE; i += PACK_THREADS) {
-        const int c = i / HDR32_STRIDE, e = i - c * HDR32_STRIDE;
-        hdr32[(size_t)first * HDR32_STRIDE + i] = (float)s_h[c * HDR_STRIDE + H_T0 + e];
-    }
-    // MFMA operand: W[m][c] = T0[m] Jp[0][c] + T1[m] Jp[1][c] (FP64, then FP32)
-    for (int i = threadIdx.x; i < count * WB_STRIDE; i += PACK_THREADS) {
-        const int c = i / WB_STRIDE, e = i - c * WB_STRIDE, n = e & 31;
-        float out = 0.0f;
-        if (n < WB_COLS) {
-            const double *hb = s_h + c * HDR_STRIDE;
-            const int m = n >> 2, col = (n >> 1) & 1;
-            const double t0 = hb[H_T0 + m], t1 = hb[H_T1 + m];
-            const double wr = t0 * hb[H_JP + 2 * col] + t1 * hb[H_JP + 4 + 2 * col];
-            const double wi = t0 * hb[H_JP + 2 * col + 1] + t1 * hb[H_JP + 4 + 2 * col + 1];
-            // rows 0 and 1 multiply Re F and Im F
-            out = e < 32 ? (float)((n & 1) ? wi : wr) : (float)((n & 1) ? wr : -wi);
-        }
-        wb[(size_t)first * WB_STRIDE + i] = out;
+    // MFMA operand: W[m][c] = s (T0[m] Jp[0][c] + T1[m] Jp[1][c]) in FP64,
+    // split into three BF16 parts
+    for (int i = threadIdx.x; i < count * (2 * WB_COLS); i += PACK_THREADS) {
+        const int c = i / (2 * WB_COLS), e = i - c * (2 * WB_COLS);
+        const int row = e / WB_COLS, n = e - row * WB_COLS;
+        const double *hb = s_h + c * HDR_STRIDE;
+        const int m = n >> 2, col = (n >> 1) & 1;
+        const double t0 = hb[H_T0 + m], t1 = hb[H_T1 + m];
+        const double wr = t0 * hb[H_JP + 2 * col] + t1 * hb[H_JP + 4 + 2 * col];
+        const double wi = t0 * hb[H_JP + 2 * col + 1] + t1 * hb[H_JP + 4 + 2 * col + 1];
+        // rows 0 and 1 multiply Re F and Im F / sqrt(2)
+        const double w = s_scale[c] * (row == 0 ? ((n & 1) ? wi : wr)
+                                                : 1.41421356237309504880 *
+                                                      ((n & 1) ? wr : -wi));
+        const uint32_t ph = bf16_bits((float)w);
+        const double r1 = w - (double)bf16_value(ph);
+        const uint32_t pm = bf16_bits((float)r1);
+        const uint32_t pl = bf16_bits((float)(r1 - (double)bf16_value(pm)));
+        uint32_t *out = wb + (size_t)first * WB_STRIDE + (size_t)i * WB_WORDS;
+        out[0] = out[1] = ph | pm << 16;
+        out[2] = ph << 16;
+        out[3] = pl << 16;
     }
 }
 
@@ -692,311 +916,401 @@ __device__ __forceinline__ void beam_dir_f64(
     }
 }
 
-// One edge of the aperture sum, mixed precision: phase arguments, their
-// reduction and the edge coefficient in FP64, phasors and sums in FP32.
-__device__ __forceinline__ void edge_mixed(int e, int n, const double *__restrict__ vtx,
-                                           const double *__restrict__ vdd,
-                                           const int32_t *__restrict__ vflag, double A,
-                                           double B, double psi, bool useB, int vmask,
-                                           const float4 *__restrict__ tab, double k,
-                                           double eps1, float s0, float c0, float &sp,
-                                           float &cp, float &sr, float &si, bool small)
-{
-    const double *v = vtx + (size_t)e * VTX_STRIDE;
-    const double syx = uniform_f64(v[V_SYX]), sxy = uniform_f64(v[V_SXY]);
-    const int f = __builtin_amdgcn_readfirstlane(vflag[e]);
-    float sn = s0, cn = c0;
-    if (e + 1 < n) {
-        const double xn = __builtin_fma(B, v[VTX_STRIDE + V_KY], psi);
-        sincos_table_f32(__builtin_fma(A, v[VTX_STRIDE + V_KX], xn), tab, sn, cn);
-    }
-    // the edge coefficient is cancellation-prone: FP64
-    const double cc = useB ? __builtin_fma(syx, B, A) : __builtin_fma(sxy, A, B);
-    const bool big = __builtin_fabs(cc) > eps1;
-    // hardware reciprocal (1 ulp): the FP32 phasor differences it scales
-    // carry more rounding than that; an invalid edge's stored slope makes
-    // it exactly zero
-    const float r = __builtin_amdgcn_rcpf((float)cc);
-    const float inv = big ? r : 0.0f;
-    sr = __builtin_fmaf(cn - cp, inv, sr);
-    si = __builtin_fmaf(sn - sp, inv, si);
-    if (__builtin_expect(!big && !small && (f & vmask) != 0, 0)) {
-        const double *w = vdd + (size_t)e * VDD_STRIDE;
-        const double dd = useB ? uniform_f64(w[D_DX]) : uniform_f64(w[D_DY]);
-        const double2 q =
-            stable_edge_quotient((double)cp, (double)sp, (double)cn, (double)sn, dd, cc, k);
-        sr += (float)q.x;
-        si += (float)q.y;
-    }
-    sp = sn;
-    cp = cn;
-}
-
-// The end of the mixed aperture integral: the 1/B or -1/A normalisation,
-// the small-phase moment form when every vertex phase is within 0.25 rad,
-// and a NaN result (degenerate beam) returned as 0, i.e. the beam skipped.
-// The normaliser is the hardware reciprocal (1 ulp), as for the edge
-// coefficients: the FP32 edge sum it scales carries more rounding than that.
-// Word 3 of a raw buffer resource on gfx9-family devices (32-bit data
-// format; the element and index fields unused).
-constexpr int kBufferRsrcWord3 = 0x00020000;
-
-// The FP32 small-phase bound stored in the low word of header slot H_PHBM.
-__device__ __forceinline__ float phase_bound_f32(double slot)
-{
-    return __builtin_bit_cast(float, low_bits(slot));
-}
-
-__device__ __forceinline__ void aperture_mixed_finish(const double *__restrict__ h, double A,
-                                                      double B, double psi, float nin,
-                                                      bool small, float sr, float si,
-                                                      const float4 *__restrict__ tab,
-                                                      float &out_r, float &out_i)
-{
-    const float nrm = __builtin_amdgcn_rcpf(nin);  // nin: B or -A
-    float fr = sr * nrm, fi = si * nrm;
-    if (__builtin_expect(small, 0)) {
-        // <e^{i phi}> = sum_n i^n <phi^n> / n! to fifth order
-        const double p1 = A * h[H_MOM] + B * h[H_MOM + 1];
-        const double p2 = A * A * h[H_MOM + 2] + A * B * h[H_MOM + 3] + B * B * h[H_MOM + 4];
-        const double A2 = A * A, B2 = B * B, AB = A * B;
-        const double *c3 = h + H_MOM3, *c4 = h + H_MOM4, *c5 = h + H_MOM5;
-        const double q3 = B * (B2 * c3[0] + AB * c3[1]) + A * (AB * c3[2] + A2 * c3[3]);
-        const double q4 = B2 * (B2 * c4[0] + AB * c4[1]) + A2 * (B2 * c4[2] + AB * c4[3] + A2 * c4[4]);
-        const double q5 = B * B2 * (B2 * c5[0] + AB * c5[1] + A2 * c5[2]) +
-                          A * A2 * (B2 * c5[3] + AB * c5[4] + A2 * c5[5]);
-        const double gr = 1.0 - 0.5 * p2 + q4, gi = p1 - q3 + q5;
-        const double ar = h[H_AL] * gr - h[H_AL + 1] * gi;
-        const double ai = h[H_AL] * gi + h[H_AL + 1] * gr;
-        float sd, cd;
-        sincos_table_f32(psi, tab, sd, cd);
-        fr = (float)ar * cd - (float)ai * sd;
-        fi = (float)ar * sd + (float)ai * cd;
-    }
-    // a NaN F (degenerate polygon) counts as zero; the selects only in
-    // waves that have one
-    out_r = fr;
-    out_i = fi;
-    const bool bad = __builtin_isnan(fr);
-    if (__builtin_expect(__builtin_amdgcn_ballot_w64(bad) != 0, 0)) {
-        out_r = bad ? 0.0f : fr;
-        out_i = bad ? 0.0f : fi;
-    }
-}
-
-// The edge sum of aperture_mixed_nv.  Both coefficients come from scalar
-// slopes, then a per-lane select of the result (selecting the slope first
-// costs two moves and a select per half of the FP64 operand).  An edge that
-// is invalid for the lane's branch carries kInvalidSlope, so its reciprocal
-// is zero and the sum needs no validity test.  A separate pass for waves
-// whose lanes all take one branch of the reference's sum (one coefficient
-// per edge; about half the waves of an orientation average) gained 0.4 %
-// for three copies of the loop, and none in the FP64 sum.  Near-singular edges
-// (|C| <= eps1, their term below zero) are evaluated in one pass after the
-// sum, taken only when some lane has one; the validity test lives there.
-template <int NV>
-__device__ __forceinline__ void edge_sum_mixed_nv(
-    const double *syx, const double *sxy, const int *fl, const float *sv, const float *cv,
-    const double *__restrict__ vdd, double A, double B, bool useB, int vmask, double k,
-    double eps1, bool small, float &sr, float &si)
-{
-    bool rare[NV];
-    bool any_rare = false;
-    // every term taken as it comes: a lane with a near-singular edge (its
-    // reciprocal huge or infinite) sums again below, so the common sum
-    // carries no select
-#pragma unroll
-    for (int e = 0; e < NV; ++e) {
-        const int f = e + 1 < NV ? e + 1 : 0;
-        const double cx = __builtin_fma(syx[e], B, A);
-        const double cy = __builtin_fma(sxy[e], A, B);
-        const double cc = useB ? cx : cy;
-        const bool big = __builtin_fabs(cc) > eps1;
-        // hardware reciprocal (1 ulp): the FP32 phasor differences it scales
-        // carry more rounding than that
-        const float r = __builtin_amdgcn_rcpf((float)cc);
-        sr = __builtin_fmaf(cv[f] - cv[e], r, sr);
-        si = __builtin_fmaf(sv[f] - sv[e], r, si);
-        // near-singular lanes as scalar mask arithmetic (a second vector
-        // compare for !big otherwise)
-        rare[e] = __builtin_amdgcn_inverse_ballot_w64(~__builtin_amdgcn_ballot_w64(big));
-        any_rare = any_rare || rare[e];
-    }
-    // (lanes on the moment form discard the sum)
-    if (__builtin_expect(any_rare && !small, 0)) {
-        // the sum without the near-singular terms (the same operations, so
-        // the same bits as a masked first pass) ...
-        sr = 0.0f;
-        si = 0.0f;
-#pragma unroll
-        for (int e = 0; e < NV; ++e) {
-            const int f = e + 1 < NV ? e + 1 : 0;
-            const double cc =
-                useB ? __builtin_fma(syx[e], B, A) : __builtin_fma(sxy[e], A, B);
-            const float inv = rare[e] ? 0.0f : __builtin_amdgcn_rcpf((float)cc);
-            sr = __builtin_fmaf(cv[f] - cv[e], inv, sr);
-            si = __builtin_fmaf(sv[f] - sv[e], inv, si);
-        }
-        // ... and those terms in the stable form
-#pragma unroll
-        for (int e = 0; e < NV; ++e) {
-            if (rare[e] && (fl[e] & vmask) != 0) {
-                const int f = e + 1 < NV ? e + 1 : 0;
-                const double cc =
-                    useB ? __builtin_fma(syx[e], B, A) : __builtin_fma(sxy[e], A, B);
-                const double *w = vdd + (size_t)e * VDD_STRIDE;
-                const double dx = uniform_f64(w[D_DX]), dy = uniform_f64(w[D_DY]);
-                const double2 q = stable_edge_quotient((double)cv[e], (double)sv[e],
-                                                       (double)cv[f], (double)sv[f],
-                                                       useB ? dx : dy, cc, k);
-                sr += (float)q.x;
-                si += (float)q.y;
-            }
-        }
-    }
-}
-
-// Aperture integral F(beam, direction) / complWave, mixed precision: A, B,
-// the phases and their reduction, the edge coefficients and the moments in
-// FP64; phasors and edge sums in FP32.
+// ---- mixed precision ----------------------------------------------------
 //
-// NV > 0: the vertex count is known at compile time.  The phases of all
-// vertices are reduced and their table reads issued together, so the LDS
-// latency of one vertex overlaps the arithmetic of the others; the edges
-// follow.
-template <int NV>
-__device__ __forceinline__ void aperture_mixed_nv(
-    const double *__restrict__ h, const double *__restrict__ vtx,
-    const double *__restrict__ vdd, const int32_t *__restrict__ vflag, int nv,
-    const double *d, const float4 *__restrict__ tab, double k, double eps1, float &out_r,
-    float &out_i)
+// The aperture integral over a polygon with edges t_e, phases phi_v at its
+// vertices and phase steps D_e = phi_{e+1} - phi_e is, for ANY direction q,
+//   F = -(k / K.q) sum_e (q x t_e) (e^{i phi_{e+1}} - e^{i phi_e}) / D_e,
+// K = k (A, B) / k the projected wave vector: the reference's two branches are
+// q = y (divide by B, weights dx) and q = x (divide by -A, weights dy).  With q
+// = t_0 the weights are constants of the beam, K.q is edge 0's own phase step,
+// edge 0 drops out of the sum, and no lane chooses a branch:
+//   F = sum_{e>0} w_e (e^{i phi_{e+1}} - e^{i phi_e}) / D_e / D_0.
+// Nothing but phases at points of the aperture is needed of the direction, so
+// A, B and psi are not formed either: a phase is three FMAs from d - b and a
+// packed vector, its constant term (with the fixed-point offset of kTurnMagic)
+// the accumulator they start from.  And with an edge's middle phase m_e and half
+// step h_e = D_e / 2, (e^{i phi_{e+1}} - e^{i phi_e}) / D_e = i e^{i m_e} sin(h_e)
+// / h_e / 2, which does not cancel as D_e goes to zero: no edge but edge 0 is
+// ever singular.
+//
+// An edge parallel to t_0 has no weight, and then the other two edges of a
+// quadrilateral have opposite weights; a triangle is the same with that edge
+// shrunk to a point (l: the last edge):
+//   F = 2 i w_1 (e^{i m_1} sin(h_1) / D_1 - e^{i m_l} sin(h_l) / D_l) / D_0,
+// and for a parallelogram with centre phase m
+//   F = -4 w_1 e^{i m} sin(h_0) sin(h_1) / (D_0 D_1).
+// The constants go into the packed W, so these take 60 and 40 vector
+// instructions where the reference's branches (A, B, psi, two FP64 coefficients
+// and a select per edge, an FP64 reduction per vertex) took 109, and other
+// quadrilaterals 95 (137,000 beams of 2,000-15,000 an orientation on 541 x 96
+// directions: 17.3 ms against 27.3 for the kernel, contraction included).  A traced column's beams are 0.32 parallelograms, 0.61
+// trapezoids and triangles; the 8-column aggregate's 0.09 and 0.63.  From five
+// vertices on (shadow beams, 4 to 15 in 100 others) the weights are the
+// reference's dx or dy, by the larger of |A| and |B|, since one edge's own step
+// is too often small against K there.
+//
+// Lanes where D_0 is small leave the sums: fix_lanes below.  Forms that were
+// shorter and lost precision: one coefficient per vertex, X_v / (D_{v-1} D_v)
+// (twice the error: its coefficients multiply phasors, not differences), and the
+// sum over edge 0 on phasor differences (1.3 times the error of the branches).
+
+// The moment form: F of a cell whose vertex phases are all within
+// kSmallPhaseMixed: <e^{i phi}> = sum_n i^n <phi^n> / n! to
+// seventh order, times the area limit and e^{i psi}.  Returns Re F and
+// Im F / sqrt(2).
+__device__ __forceinline__ void moments_mixed(const double *__restrict__ h, double A, double B,
+                                              double psi, const PhasorNode *__restrict__ tab,
+                                              float &out_r, float &out_s)
 {
-    // a product sum, then one subtraction: an FMA chain ending on A0 would
-    // pair two scalar operands in one instruction and cost two moves
-    const double A = h[H_A0] - (d[0] * h[H_HOR] + d[1] * h[H_HOR + 1] + d[2] * h[H_HOR + 2]);
-    const double B = h[H_B0] - (d[0] * h[H_VER] + d[1] * h[H_VER + 1] + d[2] * h[H_VER + 2]);
-    const double psi = d[0] * h[H_KC] + d[1] * h[H_KC + 1] + d[2] * h[H_KC + 2];
+    const double A2 = A * A, B2 = B * B, AB = A * B;
+    const double *c3 = h + H_MOM3, *c4 = h + H_MOM4, *c5 = h + H_MOM5, *c6 = h + H_MOM6,
+                 *c7 = h + H_MOM7;
+    const double p1 = A * h[H_MOM] + B * h[H_MOM + 1];
+    const double p2 = A2 * h[H_MOM + 2] + AB * h[H_MOM + 3] + B2 * h[H_MOM + 4];
+    const double q3 = B * (B2 * c3[0] + AB * c3[1]) + A * (AB * c3[2] + A2 * c3[3]);
+    const double q4 =
+        B2 * (B2 * c4[0] + AB * c4[1]) + A2 * (B2 * c4[2] + AB * c4[3] + A2 * c4[4]);
+    const double A3 = A * A2, B3 = B * B2;
+    const double q5 = B3 * (B2 * c5[0] + AB * c5[1] + A2 * c5[2]) +
+                      A3 * (B2 * c5[3] + AB * c5[4] + A2 * c5[5]);
+    const double q6 = B3 * (B3 * c6[0] + A * (B2 * c6[1] + AB * c6[2])) +
+                      A3 * (B3 * c6[3] + A * (B2 * c6[4] + AB * c6[5] + A2 * c6[6]));
+    const double q7 =
+        B2 * B2 * (B3 * c7[0] + A * (B2 * c7[1] + AB * c7[2] + A2 * c7[3])) +
+        A2 * A2 * (B3 * c7[4] + A * (B2 * c7[5] + AB * c7[6] + A2 * c7[7]));
+    const double gr = 1.0 - 0.5 * p2 + (q4 - q6), gi = p1 - q3 + (q5 - q7);
+    const float ar = (float)(h[H_AL] * gr - h[H_AL + 1] * gi);
+    const float ai = (float)(h[H_AL] * gi + h[H_AL + 1] * gr);
+    float c, s;
+    phasor_rad(psi, tab, c, s);
+    out_r = __builtin_fmaf(-ai * kSqrt2, s, ar * c);
+    out_s = __builtin_fmaf(ar, s, ai * kInvSqrt2 * c);
+}
+
+// The edge sum over the reference's branches, as the ABI's slopes and flags
+// define it, for any vertex count and any phase: beams of class BEAM_GENERAL,
+// and single lanes of other beams next to a singular edge.  The edge
+// coefficient is cancellation-prone and stays in FP64; edges with |C| <=
+// eps1 take the half-angle form.
+__device__ __forceinline__ void edges_mixed(const double *__restrict__ vtx,
+                                            const double *__restrict__ vdd,
+                                            const int32_t *__restrict__ vflag, int nv, double A,
+                                            double B, double psi,
+                                            const PhasorNode *__restrict__ tab, double k,
+                                            double eps1, float &out_r, float &out_s)
+{
     const bool useB = __builtin_fabs(B) > __builtin_fabs(A);
     const int vmask = useB ? EDGE_VX : EDGE_VY;
-    const float nin = useB ? (float)B : -(float)A;
-    float sr = 0.0f, si = 0.0f;
-    bool small;
-    if constexpr (NV > 0) {
-        // scalar loads first: LDS reads and scalar loads share one wait
-        // counter, so a scalar load between two table reads would drain both
-        double kx[NV], ky[NV];
-#pragma unroll
-        for (int e = 0; e < NV; ++e) {
-            kx[e] = uniform_f64(vtx[(size_t)e * VTX_STRIDE + V_KX]);
-            ky[e] = uniform_f64(vtx[(size_t)e * VTX_STRIDE + V_KY]);
+    float c0, s0;
+    phasor_rad(__builtin_fma(A, vtx[V_KX], __builtin_fma(B, vtx[V_KY], psi)), tab, c0, s0);
+    float cp = c0, sp = s0, sr = 0.0f, ss = 0.0f;
+    for (int e = 0; e < nv; ++e) {
+        const double *v = vtx + (size_t)e * VTX_STRIDE;
+        const double syx = uniform_f64(v[V_SYX]), sxy = uniform_f64(v[V_SXY]);
+        const int f = __builtin_amdgcn_readfirstlane(vflag[e]);
+        float cn = c0, sn = s0;
+        if (e + 1 < nv) {
+            const double xn = __builtin_fma(B, v[VTX_STRIDE + V_KY], psi);
+            phasor_rad(__builtin_fma(A, v[VTX_STRIDE + V_KX], xn), tab, cn, sn);
         }
-        // the moment form's bound (loaded with the header's first fields,
-        // so no scalar load waits among the table reads)
-        const float bnd = phase_bound_f32(uniform_f64(h[H_PHBM]));
-        float dv[NV];
-        float4 ev[NV];
-#pragma unroll
-        for (int e = 0; e < NV; ++e)
-            sincos_reduce_f32(__builtin_fma(A, kx[e], __builtin_fma(B, ky[e], psi)), tab, dv[e],
-                              ev[e]);
-        float sv[NV], cv[NV];
-#pragma unroll
-        for (int e = 0; e < NV; ++e)
-            sincos_finish_f32(dv[e], ev[e], sv[e], cv[e]);
-        // the vertex phases one by one only in waves where the beam's bound
-        // leaves the moment form possible for some lane
-        small = false;
-        const bool maybe = __builtin_fabsf(nin) <= bnd;
-        if (__builtin_expect(__builtin_amdgcn_ballot_w64(maybe) != 0, 0))
-            small = maybe && all_phases_small_nv<NV>(kx, ky, A, B, kSmallPhaseMixed);
-        double syx[NV], sxy[NV];
-        int fl[NV];
-#pragma unroll
-        for (int e = 0; e < NV; ++e) {
-            syx[e] = uniform_f64(vtx[(size_t)e * VTX_STRIDE + V_SYX]);
-            sxy[e] = uniform_f64(vtx[(size_t)e * VTX_STRIDE + V_SXY]);
-            fl[e] = __builtin_amdgcn_readfirstlane(vflag[e]);
+        const double cc = useB ? __builtin_fma(syx, B, A) : __builtin_fma(sxy, A, B);
+        const bool big = __builtin_fabs(cc) > eps1;
+        // an invalid edge's stored slope makes the reciprocal exactly zero
+        const float r = __builtin_amdgcn_rcpf((float)cc);
+        const float inv = big ? r : 0.0f;
+        sr = __builtin_fmaf(cn - cp, inv, sr);
+        ss = __builtin_fmaf(sn - sp, inv, ss);
+        if (__builtin_expect(!big && (f & vmask) != 0, 0)) {
+            const double *w = vdd + (size_t)e * VDD_STRIDE;
+            const double dd = useB ? uniform_f64(w[D_DX]) : uniform_f64(w[D_DY]);
+            const double2 q = stable_edge_quotient((double)cp, (double)(sp * kSqrt2), (double)cn,
+                                                   (double)(sn * kSqrt2), dd, cc, k);
+            sr += (float)q.x;
+            ss += (float)(q.y * (double)kInvSqrt2);
         }
-        edge_sum_mixed_nv<NV>(syx, sxy, fl, sv, cv, vdd, A, B, useB, vmask, k, eps1, small, sr,
-                              si);
-    } else {
-        small = false;
-        if (__builtin_expect(__builtin_fabsf(nin) <= phase_bound_f32(h[H_PHBM]), 0))
-            small = all_phases_small(vtx, nv, A, B, kSmallPhaseMixed);
-        float s0, c0;
-        sincos_table_f32(__builtin_fma(A, vtx[V_KX], __builtin_fma(B, vtx[V_KY], psi)), tab, s0,
-                         c0);
-        float sp = s0, cp = c0;
-        for (int e = 0; e < nv; ++e)
-            edge_mixed(e, nv, vtx, vdd, vflag, A, B, psi, useB, vmask, tab, k, eps1,
-                       s0, c0, sp, cp, sr, si, small);
+        cp = cn;
+        sp = sn;
     }
-    aperture_mixed_finish(h, A, B, psi, nin, small, sr, si, tab, out_r, out_i);
+    const float nrm = __builtin_amdgcn_rcpf(useB ? (float)B : -(float)A);
+    out_r = sr * nrm;
+    out_s = ss * nrm;
 }
 
+// F' of the lanes that the formulas over edge 0 leave: those with small phases
+// (`maybe` those to be tested for it) by the moments, those next to a singular
+// edge, and every lane of a BEAM_SLOPES beam, by the reference's branches.
+__device__ __forceinline__ void fix_lanes(const double *eb, const double *__restrict__ h,
+                                          const double *__restrict__ vtx,
+                                          const double *__restrict__ vdd,
+                                          const int32_t *__restrict__ vflag, int nv, int cls,
+                                          const double *d, bool singular, bool maybe,
+                                          const PhasorNode *__restrict__ tab, double k,
+                                          double eps1, float &out_r, float &out_s)
+{
+    // A, B: projections of k - k0 = b - d on the aperture axes
+    const double k0 = eb[EB_DIR] - d[0], k1 = eb[EB_DIR + 1] - d[1], k2 = eb[EB_DIR + 2] - d[2];
+    const double A = k0 * h[H_HOR] + k1 * h[H_HOR + 1] + k2 * h[H_HOR + 2];
+    const double B = k0 * h[H_VER] + k1 * h[H_VER + 1] + k2 * h[H_VER + 2];
+    const double psi = d[0] * h[H_KC] + d[1] * h[H_KC + 1] + d[2] * h[H_KC + 2];
+    const bool small =
+        maybe && (cls == BEAM_MOMENTS || all_phases_small(vtx, nv, A, B, kSmallPhaseMixed));
+    if (singular && !small)
+        edges_mixed(vtx, vdd, vflag, nv, A, B, psi, tab, k, eps1, out_r, out_s);
+    if (small)
+        moments_mixed(h, A, B, psi, tab, out_r, out_s);
+    if (singular || small) {
+        const float inv = high_float(eb[EB_SCALE]);
+        // a NaN F (degenerate polygon) counts as zero
+        const bool bad = __builtin_isnan(out_r);
+        out_r = bad ? 0.0f : out_r * inv;
+        out_s = bad ? 0.0f : out_s * inv;
+    }
+}
+
+// sin(2 pi f) / sqrt(2) / f from the series, for a small half step f.
+__device__ __forceinline__ float sine_ratio_series(float f)
+{
+    const float x = 6.28318530717958648f * f, z = x * x;
+    return 4.44288293815836625f *
+           __builtin_fmaf(z, __builtin_fmaf(z, 1.0f / 120.0f, -1.0f / 6.0f), 1.0f);
+}
+
+// Triangles and trapezoids.
+__device__ __forceinline__ void aperture_trapezoid(const double *eb, const double *d,
+                                                   const PhasorNode *__restrict__ tab,
+                                                   float &out_r, float &out_s, bool &singular,
+                                                   bool &maybe)
+{
+    const double k0 = d[0] - eb[EB_DIR], k1 = d[1] - eb[EB_DIR + 1], k2 = d[2] - eb[EB_DIR + 2];
+    const auto phase = [&](const double *q, double c) {
+        return __builtin_fma(k2, q[2], __builtin_fma(k1, q[1], __builtin_fma(k0, q[0], c)));
+    };
+    const double *q = eb + EB_Q;
+    const double m1 = phase(q, eb[EB_PHASE]), a1 = phase(q + 3, kTurnMagic);
+    const double m3 = phase(q + 6, eb[EB_PHASE]), a3 = phase(q + 9, kTurnMagic);
+    const PhasorNode em1 = phasor_read(low_bits(m1), tab), ea1 = phasor_read(low_bits(a1), tab),
+                     em3 = phasor_read(low_bits(m3), tab), ea3 = phasor_read(low_bits(a3), tab);
+    const double h1 = a1 - kTurnMagic, h3 = a3 - kTurnMagic;
+    const float f1 = (float)h1, f3 = (float)h3;
+    const float step = (float)((m1 - m3) - (h1 + h3));  // edge 0
+    const float r0 = __builtin_amdgcn_rcpf(step);
+    float c1, s1, c3, s3;
+    phasor_finish(low_bits(m1), em1, c1, s1);
+    phasor_finish(low_bits(m3), em3, c3, s3);
+    float q1 = sine_finish(low_bits(a1), ea1) * __builtin_amdgcn_rcpf(f1);
+    float q3 = sine_finish(low_bits(a3), ea3) * __builtin_amdgcn_rcpf(f3);
+    const bool series =
+        __builtin_fminf(__builtin_fabsf(f1), __builtin_fabsf(f3)) < kSeriesStep;
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(series) != 0, 0)) {
+        q1 = __builtin_fabsf(f1) < kSeriesStep ? sine_ratio_series(f1) : q1;
+        q3 = __builtin_fabsf(f3) < kSeriesStep ? sine_ratio_series(f3) : q3;
+    }
+    out_r = __builtin_fmaf(q1, c1, -(q3 * c3)) * r0;
+    out_s = __builtin_fmaf(q1, s1, -(q3 * s3)) * r0;
+    const bool look = !(__builtin_fabsf(step) >= low_float(eb[EB_LIM]));
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(look) != 0, 0)) {
+        singular = !(__builtin_fabsf(step) >= high_float(eb[EB_LIM]));
+        maybe = look &&
+                __builtin_fmaxf(__builtin_fabsf(f1), __builtin_fabsf(f3)) <= (float)kLookStep;
+    }
+}
+
+// Parallelograms.
+__device__ __forceinline__ void aperture_parallelogram(const double *eb, const double *d,
+                                                       const PhasorNode *__restrict__ tab,
+                                                       float &out_r, float &out_s)
+{
+    const double k0 = d[0] - eb[EB_DIR], k1 = d[1] - eb[EB_DIR + 1], k2 = d[2] - eb[EB_DIR + 2];
+    const auto phase = [&](const double *q, double c) {
+        return __builtin_fma(k2, q[2], __builtin_fma(k1, q[1], __builtin_fma(k0, q[0], c)));
+    };
+    const double m = phase(eb + EB_Q, eb[EB_PHASE]);
+    const double a0 = phase(eb + EB_Q + 3, kTurnMagic), a1 = phase(eb + EB_Q + 6, kTurnMagic);
+    const PhasorNode em = phasor_read(low_bits(m), tab), e0 = phasor_read(low_bits(a0), tab),
+                     e1 = phasor_read(low_bits(a1), tab);
+    const float f0 = (float)(a0 - kTurnMagic), f1 = (float)(a1 - kTurnMagic);
+    float c, s;
+    phasor_finish(low_bits(m), em, c, s);
+    const float s0 = sine_finish(low_bits(a0), e0), s1 = sine_finish(low_bits(a1), e1);
+    float q = s0 * s1 * __builtin_amdgcn_rcpf(f0 * f1);
+    const bool series =
+        __builtin_fminf(__builtin_fabsf(f0), __builtin_fabsf(f1)) < kSeriesStep;
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(series) != 0, 0)) {
+        if (series) {
+            const float q0 = __builtin_fabsf(f0) < kSeriesStep
+                                 ? sine_ratio_series(f0)
+                                 : s0 * __builtin_amdgcn_rcpf(f0);
+            const float q1 = __builtin_fabsf(f1) < kSeriesStep
+                                 ? sine_ratio_series(f1)
+                                 : s1 * __builtin_amdgcn_rcpf(f1);
+            q = q0 * q1;
+        }
+    }
+    out_r = q * c;
+    out_s = q * s;
+}
+
+// One edge's (cos, sin / sqrt 2) of the middle phase and sin(2 pi h) / sqrt(2) / h
+// of its half step h, from the phases p, n (with kTurnMagic) of its ends.
+__device__ __forceinline__ void edge_terms(double p, double n,
+                                           const PhasorNode *__restrict__ tab, float &c,
+                                           float &s, float &q, float &f)
+{
+    const double m = 0.5 * (p + n), a = __builtin_fma(0.5, n - p, kTurnMagic);
+    const PhasorNode em = phasor_read(low_bits(m), tab), ea = phasor_read(low_bits(a), tab);
+    f = (float)(a - kTurnMagic);
+    phasor_finish(low_bits(m), em, c, s);
+    q = sine_finish(low_bits(a), ea) * __builtin_amdgcn_rcpf(f);
+    const bool series = __builtin_fabsf(f) < kSeriesStep;
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(series) != 0, 0))
+        q = series ? sine_ratio_series(f) : q;
+}
+
+// The sum over edge 0 for the other quadrilaterals.
+__device__ __forceinline__ void aperture_quad(const double *eb, const double *__restrict__ ev,
+                                              const double *d,
+                                              const PhasorNode *__restrict__ tab, float &out_r,
+                                              float &out_s, bool &singular, bool &maybe)
+{
+    const double k0 = d[0] - eb[EB_DIR], k1 = d[1] - eb[EB_DIR + 1], k2 = d[2] - eb[EB_DIR + 2];
+    double ph[4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        const double *q = ev + v * EV_STRIDE;
+        ph[v] = __builtin_fma(k2, q[2], __builtin_fma(k1, q[1], __builtin_fma(k0, q[0],
+                                                                              eb[EB_PHASE])));
+    }
+    const float step = (float)(ph[1] - ph[0]);
+    float sr = 0.0f, ss = 0.0f, legs = 0.0f;
+#pragma unroll
+    for (int e = 1; e < 4; ++e) {
+        float c, s, q, f;
+        edge_terms(ph[e], ph[(e + 1) % 4], tab, c, s, q, f);
+        const float coef = q * low_float(ev[e * EV_STRIDE + EV_W]);
+        sr = __builtin_fmaf(c, coef, sr);
+        ss = __builtin_fmaf(s, coef, ss);
+        legs = __builtin_fmaxf(legs, __builtin_fabsf(f));
+    }
+    const float r0 = __builtin_amdgcn_rcpf(step);
+    out_r = sr * r0;
+    out_s = ss * r0;
+    singular = !(__builtin_fabsf(step) >= high_float(eb[EB_LIM]));
+    maybe = __builtin_fmaxf(legs, __builtin_fabsf(step)) <= (float)kLookStep;
+}
+
+// Five vertices and more, one at a time, with the reference's weights.
+__device__ __forceinline__ void aperture_loop(const double *eb, const double *__restrict__ ev,
+                                              const double *__restrict__ h, int nv,
+                                              const double *d,
+                                              const PhasorNode *__restrict__ tab, float &out_r,
+                                              float &out_s, bool &maybe)
+{
+    const double k0 = d[0] - eb[EB_DIR], k1 = d[1] - eb[EB_DIR + 1], k2 = d[2] - eb[EB_DIR + 2];
+    const double base = eb[EB_PHASE];
+    const float A = -(float)(k0 * h[H_HOR] + k1 * h[H_HOR + 1] + k2 * h[H_HOR + 2]);
+    const float B = -(float)(k0 * h[H_VER] + k1 * h[H_VER + 1] + k2 * h[H_VER + 2]);
+    const bool useB = __builtin_fabsf(B) > __builtin_fabsf(A);
+    const double p0 = __builtin_fma(k2, ev[2], __builtin_fma(k1, ev[1],
+                                                             __builtin_fma(k0, ev[0], base)));
+    double pp = p0;
+    float sr = 0.0f, ss = 0.0f, steps = 0.0f;
+    for (int e = 0; e < nv; ++e) {
+        const double *q = ev + e * EV_STRIDE;
+        const float wx = low_float(q[EV_W]), wy = high_float(q[EV_W]);
+        double pn = p0;
+        if (e + 1 < nv) {
+            q += EV_STRIDE;
+            pn = __builtin_fma(k2, q[2], __builtin_fma(k1, q[1], __builtin_fma(k0, q[0], base)));
+        }
+        float c, s, ratio, f;
+        edge_terms(pp, pn, tab, c, s, ratio, f);
+        const float coef = ratio * (useB ? wx : wy);
+        sr = __builtin_fmaf(c, coef, sr);
+        ss = __builtin_fmaf(s, coef, ss);
+        steps = __builtin_fmaxf(steps, __builtin_fabsf(f));
+        pp = pn;
+    }
+    const float r = __builtin_amdgcn_rcpf(useB ? B : A);
+    out_r = sr * r;
+    out_s = ss * r;
+    maybe = steps <= (float)kLookStep;
+}
+
+// F' = F / complWave / s of a beam in a direction, s its EB_SCALE, mixed
+// precision: FP64 phases and moments, FP32 phasors and sums.  eb: the beam's
+// record (in registers), v0 its vertex offset.  Returns the real part and the
+// imaginary part / sqrt(2).
 __device__ __forceinline__ void aperture_mixed(
-    const double *__restrict__ h, const double *__restrict__ vtx,
-    const double *__restrict__ vdd, const int32_t *__restrict__ vflag, int nv,
-    const double *d, const float4 *__restrict__ tab, double k, double eps1, float &out_r,
-    float &out_i)
+    const double *eb, const double *__restrict__ evert, const double *__restrict__ h,
+    const double *__restrict__ vtxs, const double *__restrict__ vdds,
+    const int32_t *__restrict__ vflags, const double *d, const PhasorNode *__restrict__ tab,
+    double k, double eps1, float &out_r, float &out_s)
 {
-    if (nv == 4)
-        aperture_mixed_nv<4>(h, vtx, vdd, vflag, 4, d, tab, k, eps1, out_r, out_i);
-    else if (nv == 3)
-        aperture_mixed_nv<3>(h, vtx, vdd, vflag, 3, d, tab, k, eps1, out_r, out_i);
-    else
-        aperture_mixed_nv<0>(h, vtx, vdd, vflag, nv, d, tab, k, eps1, out_r, out_i);
+    const int kind = low_word(eb[EB_KIND]);
+    const int nv = kind & BEAM_NV, cls = kind / BEAM_CLASS;
+    const int64_t v0 = __builtin_bit_cast(int64_t, eb[EB_VOFF]);
+    bool singular = false, maybe = false;
+    out_r = out_s = 0.0f;
+    if (cls == BEAM_TRAPEZOID) {
+        aperture_trapezoid(eb, d, tab, out_r, out_s, singular, maybe);
+    } else if (cls == BEAM_PARALLEL) {
+        aperture_parallelogram(eb, d, tab, out_r, out_s);
+    } else if (cls == BEAM_VERTICES) {
+        const double *ev = evert + (size_t)v0 * EV_STRIDE;
+        if (nv == 4)
+            aperture_quad(eb, ev, d, tab, out_r, out_s, singular, maybe);
+        else
+            aperture_loop(eb, ev, h, nv, d, tab, out_r, out_s, maybe);
+    } else {
+        singular = cls == BEAM_SLOPES;
+        maybe = true;
+    }
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(singular || maybe) != 0, 0)) {
+        if (singular || maybe)
+            fix_lanes(eb, h, vtxs + (size_t)v0 * VTX_STRIDE, vdds + (size_t)v0 * VDD_STRIDE,
+                      vflags + v0, nv, cls, d, singular, maybe, tab, k, eps1, out_r, out_s);
+    }
 }
 
-// Mixed precision with the rotation and coherent sum on the vector ALU.
-template <int ACC_NS>
-__device__ __forceinline__ void beam_dir_mixed(
-    const double *__restrict__ h, const float *__restrict__ h32,
-    const double *__restrict__ vtx, const double *__restrict__ vdd,
-    const int32_t *__restrict__ vflag, int nv, const double *d,
-    const float *__restrict__ su, const float4 *__restrict__ tab, double k, double eps1,
-    float *j, float *jn)
+// A beam's record in scalar registers.
+struct BeamRecord {
+    double v[EB_STRIDE];
+};
+__device__ __forceinline__ BeamRecord load_record(const double *__restrict__ ebeam, int64_t b)
 {
-    float fr, fi;
-    aperture_mixed(h, vtx, vdd, vflag, nv, d, tab, k, eps1, fr, fi);
-    if (fr == 0.0f && fi == 0.0f)
-        return;
-    const int l = threadIdx.x;
-    float u0[6], u1[6];
+    BeamRecord r;
+    for (int i = 0; i < EB_STRIDE; ++i)
+        r.v[i] = ebeam[(size_t)b * EB_STRIDE + i];
+    return r;
+}
+
+// Adds F times R Jp to j[8]: the rotation and the sum on the vector ALU, the
+// beam's rotation data converted from its FP64 header; fr, fs as
+// aperture_mixed returns them, scale the beam's F / F'.
+__device__ __forceinline__ void rotate_add_mixed(const double *__restrict__ h,
+                                                 const float *u0, const float *u1, float scale,
+                                                 float fr, float fs, float *j)
+{
+    const float fi = fs * (kSqrt2 * scale);
+    fr *= scale;
+    float r[2][2] = {{0, 0}, {0, 0}};  // r[i][m]: u_i . T_m
     for (int q = 0; q < 6; ++q) {
-        u0[q] = su[q * 256 + l];
-        u1[q] = su[(6 + q) * 256 + l];
+        const float t0 = (float)h[H_T0 + q], t1 = (float)h[H_T1 + q];
+        r[0][0] = __builtin_fmaf(u0[q], t0, r[0][0]);
+        r[0][1] = __builtin_fmaf(u0[q], t1, r[0][1]);
+        r[1][0] = __builtin_fmaf(u1[q], t0, r[1][0]);
+        r[1][1] = __builtin_fmaf(u1[q], t1, r[1][1]);
     }
-    const float *T0 = h32 + H32_T0, *T1 = h32 + H32_T1;
-    const float r00 = u0[0] * T0[0] + u0[1] * T0[1] + u0[2] * T0[2] + u0[3] * T0[3] + u0[4] * T0[4] + u0[5] * T0[5];
-    const float r01 = u0[0] * T1[0] + u0[1] * T1[1] + u0[2] * T1[2] + u0[3] * T1[3] + u0[4] * T1[4] + u0[5] * T1[5];
-    const float r10 = u1[0] * T0[0] + u1[1] * T0[1] + u1[2] * T0[2] + u1[3] * T0[3] + u1[4] * T0[4] + u1[5] * T0[5];
-    const float r11 = u1[0] * T1[0] + u1[1] * T1[1] + u1[2] * T1[2] + u1[3] * T1[3] + u1[4] * T1[4] + u1[5] * T1[5];
-    const float *jp = h32 + H32_JP;
-    float q[8];
-    q[0] = r00 * jp[0] + r01 * jp[4];
-    q[1] = r00 * jp[1] + r01 * jp[5];
-    q[2] = r00 * jp[2] + r01 * jp[6];
-    q[3] = r00 * jp[3] + r01 * jp[7];
-    q[4] = r10 * jp[0] + r11 * jp[4];
-    q[5] = r10 * jp[1] + r11 * jp[5];
-    q[6] = r10 * jp[2] + r11 * jp[6];
-    q[7] = r10 * jp[3] + r11 * jp[7];
-    if constexpr (ACC_NS) {
-        for (int t = 0; t < 4; ++t) {
-            const float dr = fr * q[2 * t] - fi * q[2 * t + 1];
-            const float di = fr * q[2 * t + 1] + fi * q[2 * t];
-            j[2 * t] += dr;
-            j[2 * t + 1] += di;
-            jn[2 * t] += dr;
-            jn[2 * t + 1] += di;
+    for (int i = 0; i < 2; ++i)
+        for (int c = 0; c < 2; ++c) {
+            const double *p = h + H_JP + 2 * c;  // complWave * J_phased
+            const float qr = r[i][0] * (float)p[0] + r[i][1] * (float)p[4];
+            const float qi = r[i][0] * (float)p[1] + r[i][1] * (float)p[5];
+            float *o = j + 2 * (2 * i + c);
+            o[0] = __builtin_fmaf(fr, qr, __builtin_fmaf(-fi, qi, o[0]));
+            o[1] = __builtin_fmaf(fr, qi, __builtin_fmaf(fi, qr, o[1]));
         }
-    } else {
-        for (int t = 0; t < 4; ++t) {
-            j[2 * t] = __builtin_fmaf(fr, q[2 * t], __builtin_fmaf(-fi, q[2 * t + 1], j[2 * t]));
-            j[2 * t + 1] = __builtin_fmaf(fr, q[2 * t + 1], __builtin_fmaf(fi, q[2 * t], j[2 * t + 1]));
-        }
-    }
 }
 
 // XCD-aware block -> (item, tile): consecutive workgroup ids land on the 8
@@ -1119,8 +1433,10 @@ struct KernelArgs {
     int n_items, n_tiles, cells, n_az;
     const double *tab;       // grid tables [DT_COUNT][cells]
     const double *hdr;       // [n_beams][HDR_STRIDE]
-    const float *hdr32;      // [n_beams][HDR32_STRIDE]
-    const float *wb;         // [n_beams][WB_STRIDE]
+    const uint32_t *wb;      // [n_beams][WB_STRIDE]
+    const double *ebeam;     // [n_beams][EB_STRIDE]
+    const double *evert;     // [n_vert][EV_STRIDE]
+    const PhasorNode *phasor;  // [kPhasorN] phasor nodes of the mixed kernels
     const double *vtx;       // [n_vert][VTX_STRIDE]
     const double *vdd;       // [n_vert][VDD_STRIDE]
     const int32_t *vflag;    // [n_vert]
@@ -1171,20 +1487,22 @@ template <int PREC, int NS, int JONES, int PER, int QUEUE>
 __global__ __launch_bounds__(256) MBS_OCCUPANCY void diffract_kernel(
     const WorkItem *__restrict__ items, int n_items, int n_tiles, int cells, int n_az,
     const double *__restrict__ tab, const double *__restrict__ hdr,
-    const float *__restrict__ hdr32, const double *__restrict__ vtx,
+    const double *__restrict__ vtx,
     const double *__restrict__ vdd, const int32_t *__restrict__ vflag,
     const int32_t *__restrict__ nv,
     const int64_t *__restrict__ voff, const int32_t *__restrict__ ext,
     const int64_t *__restrict__ ooff, const double *__restrict__ weights, double k,
     double eps1, double *__restrict__ out, double *__restrict__ out_ns,
-    double *__restrict__ per_orient, int *__restrict__ queue, const float *__restrict__ tab32)
+    double *__restrict__ per_orient, int *__restrict__ queue, const float *__restrict__ tab32,
+    const double *__restrict__ ebeam, const double *__restrict__ evert,
+    const PhasorNode *__restrict__ phasor)
 {
     using U = typename std::conditional<PREC == 1, float, double>::type;
-    using U2 = typename std::conditional<PREC == 1, float4, double2>::type;
+    using U2 = typename std::conditional<PREC == 1, PhasorNode, double2>::type;
     // LDS: this lane's rotation vectors u0, u1 ([12][256], read once per beam
     // after the vertex loop instead of occupying 12-24 VGPRs through it) and
-    // the phasor table e^{i 2 pi j/TN} (512 FP32 entries, 256 FP64 ones)
-    constexpr int TN = PREC == 1 ? kTabN32 : kTabN;
+    // the phasor table (1024 FP32 nodes, 256 FP64 ones)
+    constexpr int TN = PREC == 1 ? kPhasorN : kTabN;
     __shared__ U s_u[12 * 256];
     __shared__ U2 s_tab[TN];
     __shared__ int s_unit;
@@ -1195,7 +1513,7 @@ __global__ __launch_bounds__(256) MBS_OCCUPANCY void diffract_kernel(
     }
     for (int i = threadIdx.x; i < TN; i += blockDim.x) {
         if constexpr (PREC == 1) {
-            s_tab[i] = tab32_entry(i);
+            s_tab[i] = phasor[i];
         } else {
             double ts, tc;
             sincospi((double)i / (TN / 2), &ts, &tc);
@@ -1230,6 +1548,7 @@ __global__ __launch_bounds__(256) MBS_OCCUPANCY void diffract_kernel(
         }
         U j[8] = {0, 0, 0, 0, 0, 0, 0, 0};
         U jn[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+        U jx[8] = {0, 0, 0, 0, 0, 0, 0, 0};
         // the next beam's vertex offset and count are loaded one beam
         // ahead, so a beam's header and vertex loads issue together
         int64_t v0_next = b0 < b1 ? voff[b0] : 0;
@@ -1253,13 +1572,25 @@ __global__ __launch_bounds__(256) MBS_OCCUPANCY void diffract_kernel(
                     beam_dir_f64<0>(h, bv, bd, vflag + v0, nvb, d, s_u, s_tab, k, eps1, j,
                                     nullptr);
             } else {
-                const float *h32 = hdr32 + (size_t)b * HDR32_STRIDE;
-                if (NS && ext[b] == 0)
-                    beam_dir_mixed<1>(h, h32, bv, bd, vflag + v0, nvb, d, s_u, s_tab, k, eps1,
-                                      j, jn);
+                float fr, fs;
+                const BeamRecord rec = load_record(ebeam, b);
+                aperture_mixed(rec.v, evert, h, vtx, vdd, vflag, d, s_tab, k, eps1, fr, fs);
+                float u0[6], u1[6];
+                for (int q = 0; q < 6; ++q) {
+                    u0[q] = s_u[q * 256 + threadIdx.x];
+                    u1[q] = s_u[(6 + q) * 256 + threadIdx.x];
+                }
+                const float scale = low_float(rec.v[EB_SCALE]);
+                if (NS && ext[b] != 0)
+                    rotate_add_mixed(h, u0, u1, scale, fr, fs, jx);
                 else
-                    beam_dir_mixed<0>(h, h32, bv, bd, vflag + v0, nvb, d, s_u, s_tab, k, eps1,
-                                      j, nullptr);
+                    rotate_add_mixed(h, u0, u1, scale, fr, fs, j);
+            }
+        }
+        if constexpr (PREC == 1 && NS) {  // j: the other beams, jx: the shadow beams
+            for (int q = 0; q < 8; ++q) {
+                jn[q] = j[q];
+                j[q] += jx[q];
             }
         }
         if (!live)
@@ -1356,17 +1687,43 @@ __global__ __launch_bounds__(256) MBS_OCCUPANCY void diffract_incoherent_kernel(
 // W[m][c] = T0[m] Jp[0][c] + T1[m] Jp[1][c],
 //   J[i][c](dir) = sum_b F_b(dir) (R_b Jp_b)[i][c]
 //                = sum_m u_i[m](dir) G[m][c](dir),  G = sum_b F_b(dir) W_b[m][c].
-// G is a complex [64 directions x beams] . [beams x 12] product per wave,
-// done as a real one with K = 2 per beam (Re F, Im F) and N = 24 columns on
-// v_mfma_f32_32x32x2f32 (two 32-direction blocks per wave).  The vector ALU
-// keeps only the aperture integral; the rotation (4 six-term dot products),
-// R.Jp and the accumulation (56 operations per beam and direction) move to
-// the matrix cores.  The 24 columns pad to 32; the unpadded form on
-// v_mfma_f32_4x4x1f32 (16 blocks of 4 directions, 12 instructions and 48
-// bytes of operands per lane and beam) measured 30.0 ms against 28.4: its
-// operand registers cost the occupancy more than the matrix-core cycles it
-// saves.
+// G is a complex [64 directions x beams] . [beams x 12] product per wave, a
+// real one with two rows (Re F, Im F) per beam and N = 24 columns.
+//
+// It runs on v_mfma_f32_32x32x16_bf16 with both factors split into three BF16
+// parts (x = h + m + l, 24 significant bits): the six products down to 2^-16
+// relative, hh hm hl mh mm lh, are summed in FP32; the first one left out is
+// ~2^-25.  The matrix cores run BF16 beside the vector ALU (64 FMAs plus two of
+// these: 281 cycles a wave, against 257 for the FMAs alone), while the FP32
+// form does not overlap with it at all on this device (64 FMAs plus two
+// v_mfma_f32_32x32x2f32: 396 cycles), so the split costs its 12 vector
+// instructions and saves 128 cycles a beam.
+//
+// One v_permlane32_swap gives lane l of both halves the two parts of direction
+// l (block 0) and l + 32 (block 1): Re F in lanes 0-31, Im F in lanes 32-63, as
+// K rows 0-7 and 8-15.  Each lane then holds 8 K entries in four words, (h, h)
+// (m, m) (0, l) (0, h), against the record's words (h, m) (h, m) (0, h) (0, l).
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+// Word 3 of a raw buffer resource on gfx9-family devices (32-bit data
+// format; the element and index fields unused).
+constexpr int kBufferRsrcWord3 = 0x00020000;
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+// The A words of one value: its three BF16 parts by truncation (each exact:
+// h + m + l == x), as (h, h) (m, m) (0, l) (0, h).  The remainders are FP32
+// numbers whose top halves are the parts.
+__device__ __forceinline__ bf16x8 split_words(uint32_t x)
+{
+    const uint32_t h = x & 0xffff0000u;
+    const uint32_t r = __float_as_uint(__uint_as_float(x) - __uint_as_float(h));
+    const uint32_t m = r & 0xffff0000u;
+    const uint32_t l = __float_as_uint(__uint_as_float(r) - __uint_as_float(m));
+    constexpr uint32_t kTops = 0x07060302;  // the top halves of both operands
+    const u32x4 w = {__builtin_amdgcn_perm(x, x, kTops), __builtin_amdgcn_perm(r, r, kTops), l, h};
+    return __builtin_bit_cast(bf16x8, w);
+}
+
 enum { G_LD = 25 };  // LDS row stride (floats) of the per-wave G transpose
 
 // G (this wave's accumulators) -> this lane's Jones sum.  Accumulator v of
@@ -1415,16 +1772,16 @@ template <int NS, int JONES, int PER, int QUEUE, int FSRC = 0, int WAVES = MBS_M
 __global__ __launch_bounds__(256) MBS_MFMA_OCCUPANCY void diffract_mfma_kernel(
     const WorkItem *__restrict__ items, int n_items, int n_tiles, int cells, int n_az,
     const double *__restrict__ tab, const double *__restrict__ hdr,
-    const float *__restrict__ wb, const double *__restrict__ vtx,
+    const uint32_t *__restrict__ wb, const double *__restrict__ vtx,
     const double *__restrict__ vdd, const int32_t *__restrict__ vflag,
-    const int32_t *__restrict__ nv, const int64_t *__restrict__ voff,
-    const int32_t *__restrict__ ext, const int64_t *__restrict__ ooff,
+    const double *__restrict__ ebeam, const double *__restrict__ evert,
+    const PhasorNode *__restrict__ phasor, const int64_t *__restrict__ ooff,
     const double *__restrict__ weights, double k, double eps1, double *__restrict__ out,
     double *__restrict__ out_ns, double *__restrict__ per_orient, int *__restrict__ queue,
     const float *__restrict__ tab32, const int32_t *__restrict__ sidx = nullptr,
     const float2 *__restrict__ fbuf = nullptr)
 {
-    __shared__ float4 s_tab[kTabN32];
+    __shared__ PhasorNode s_tab[kPhasorN];
     __shared__ float s_g[4 * 32 * G_LD];
     __shared__ int s_unit;
     int item = 0, tile = 0;
@@ -1432,8 +1789,8 @@ __global__ __launch_bounds__(256) MBS_MFMA_OCCUPANCY void diffract_mfma_kernel(
         if (!map_block(n_items, n_tiles, item, tile))
             return;
     }
-    for (int i = threadIdx.x; i < kTabN32; i += blockDim.x)
-        s_tab[i] = tab32_entry(i);
+    for (int i = threadIdx.x; i < kPhasorN; i += blockDim.x)
+        s_tab[i] = phasor[i];
     QueueCursor qc;
     for (;;) {
     if constexpr (QUEUE) {
@@ -1460,61 +1817,70 @@ __global__ __launch_bounds__(256) MBS_MFMA_OCCUPANCY void diffract_mfma_kernel(
             b0 = it.b_begin;
             b1 = it.b_end;
         }
-        f32x16 g0 = {}, g1 = {}, n0 = {}, n1 = {};
-        // the next beam's vertex offset and count are loaded one beam
-        // ahead, so a beam's header and vertex loads issue together
-        int64_t v0_next = b0 < b1 ? voff[b0] : 0;
-        int nv_next = b0 < b1 ? nv[b0] : 0;
+        f32x16 g0 = {}, g1 = {};
+        float jx[8] = {0, 0, 0, 0, 0, 0, 0, 0};  // shadow beams (NS)
         // a 32-bit trip count: the scalar unit has no 64-bit ordered compare,
         // so a 64-bit loop test would go to the vector unit
         const int nbeam = (int)(b1 - b0);
-        // B operand rows through a buffer resource based at the range's first
-        // beam: the beam's offset is a scalar register and the lane's a loop-
-        // invariant vector register, so no per-lane 64-bit address is formed
-        // or kept (a range holds far fewer than 2^24 beams; reads past it
-        // return zero)
-        const __amdgpu_buffer_rsrc_t wres = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<float *>(wb + (size_t)b0 * WB_STRIDE), 0,
-            nbeam * (int)(WB_STRIDE * sizeof(float)), kBufferRsrcWord3);
-        const int lane_off = lane * (int)sizeof(float);
+        BeamRecord rec{};
+        if (nbeam > 0)
+            rec = load_record(ebeam, b0);
+        // this lane's B words: row lane / 32, column lane % 32; the columns
+        // past 24 lie outside the record and read as zero
+        const int col = lane & 31;
+        const int lane_off = col < WB_COLS
+                                 ? ((lane >> 5) * WB_COLS + col) * WB_WORDS * (int)sizeof(uint32_t)
+                                 : WB_STRIDE * (int)sizeof(uint32_t);
+        const uint32_t *w = wb + (size_t)b0 * WB_STRIDE;
         for (int ib = 0; ib < nbeam; ++ib) {
             const int64_t b = b0 + ib;
-            const float bop = __builtin_bit_cast(
-                float, __builtin_amdgcn_raw_buffer_load_b32(
-                           wres, lane_off, ib * (int)(WB_STRIDE * sizeof(float)), 0));
-            const int64_t v0 = v0_next;
-            const int nvb = nv_next;
-            if (ib + 1 < nbeam) {
-                v0_next = voff[b + 1];
-                nv_next = nv[b + 1];
-            }
-            float fr, fi;
+            const __amdgpu_buffer_rsrc_t wres = __builtin_amdgcn_make_buffer_rsrc(
+                const_cast<uint32_t *>(w), 0, WB_STRIDE * (int)sizeof(uint32_t),
+                kBufferRsrcWord3);
+            w += WB_STRIDE;
+            const u32x4 bw = __builtin_amdgcn_raw_buffer_load_b128(wres, lane_off, 0, 0);
+            float fr, fs;  // Re F', Im F' / sqrt(2)
+            const double *h = hdr + (size_t)b * HDR_STRIDE;
             const int slot = FSRC ? __builtin_amdgcn_readfirstlane(sidx[b]) : -1;
             if (FSRC && slot >= 0) {
                 const float2 f = fbuf[(size_t)slot * cells + c];
-                fr = f.x;
-                fi = f.y;
+                const float inv = high_float(rec.v[EB_SCALE]);
+                fr = f.x * inv;
+                fs = f.y * (kInvSqrt2 * inv);
             } else {
-                aperture_mixed(hdr + (size_t)b * HDR_STRIDE, vtx + (size_t)v0 * VTX_STRIDE,
-                               vdd + (size_t)v0 * VDD_STRIDE, vflag + v0, nvb, d, s_tab, k,
-                               eps1, fr, fi);
+                aperture_mixed(rec.v, evert, h, vtx, vdd, vflag, d, s_tab, k, eps1, fr, fs);
             }
-            // A operands: lanes 0-31 (Re F), lanes 32-63 (Im F) of the
-            // wave's directions 0-31, then the same for directions 32-63
+            const float scale = low_float(rec.v[EB_SCALE]);
+            const bool shadow = NS && high_word(rec.v[EB_KIND]) != 0;
+            // the next beam's record: after this one's last table read (LDS
+            // reads and scalar loads share one wait counter), so that it
+            // arrives while the contraction issues
+            rec = load_record(ebeam, b0 + min(ib + 1, nbeam - 1));
+            if (shadow) {
+                // shadow beams (one an orientation) stay out of the no-shadow
+                // sum: added on the vector ALU to sums of their own, so that
+                // one accumulator set serves both grids
+                float u0[6], u1[6];
+                for (int q = 0; q < 6; ++q) {
+                    u0[q] = u[q];
+                    u1[q] = u[6 + q];
+                }
+                rotate_add_mixed(h, u0, u1, scale, fr, fs, jx);
+                continue;
+            }
             const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(fr),
-                                                             __float_as_uint(fi), false, false);
-            const float a0 = __uint_as_float(sw[0]), a1 = __uint_as_float(sw[1]);
-            g0 = __builtin_amdgcn_mfma_f32_32x32x2f32(a0, bop, g0, 0, 0, 0);
-            g1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a1, bop, g1, 0, 0, 0);
-            if (NS && ext[b] == 0) {
-                n0 = __builtin_amdgcn_mfma_f32_32x32x2f32(a0, bop, n0, 0, 0, 0);
-                n1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a1, bop, n1, 0, 0, 0);
-            }
+                                                             __float_as_uint(fs), false, false);
+            const bf16x8 bop = __builtin_bit_cast(bf16x8, bw);
+            g0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(split_words(sw[0]), bop, g0, 0, 0, 0);
+            g1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(split_words(sw[1]), bop, g1, 0, 0, 0);
         }
         float j[8], jn[8];
         mfma_epilogue(g0, g1, sg, u, cells, j);
         if constexpr (NS)
-            mfma_epilogue(n0, n1, sg, u, cells, jn);
+            for (int q = 0; q < 8; ++q) {
+                jn[q] = j[q];
+                j[q] += jx[q];
+            }
         if (!live)
             continue;
         if constexpr (JONES) {

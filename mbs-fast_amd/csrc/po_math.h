@@ -5,9 +5,7 @@
 // reduction against a 256-entry LDS table of e^{2 pi i j / 256} and short
 // Taylor polynomials (see sincos_table below).  Phases reach ~1e4 rad for the
 // largest particles; the reduction is exact to an ulp for |x| < 2^20.
-// The FP32 variant used by the mixed-precision kernels reduces in FP64 the
-// same way against a 512-entry table and needs only first- and second-order
-// corrections in FP32 (error ~1 ulp of FP32).
+// The mixed-precision kernels' FP32 phasors are further down.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -19,13 +17,11 @@ constexpr double kPi = 3.141592653589793116;            // double(pi) = M_PI
 // Small-phase switch: every vertex phase within 1e-3 rad
 // (HandlerPO_fast.h:161-216).
 constexpr double kSmallPhase = 1e-3;
-// The mixed-precision kernels' switch.  Their edge sum differences FP32
-// phasors (error ~1e-7 each) whose sum cancels to O(phase^2) of a single
-// term, so its relative error grows like 1e-7 / phase^2 -- 1e-1 at 1e-3 rad.
-// They take the moment form up to 0.25 rad instead, with polygon moments to
-// fifth order (truncation below max|phase|^6 / 6! = 3.4e-7 there), where the
-// edge sum's error has fallen to ~1e-5.
-constexpr double kSmallPhaseMixed = 0.25;
+// The mixed-precision kernels' switch.  Their sums cancel to O(phase) of a
+// single term where a lane's phase steps are small (kLookStep), so such lanes
+// take the moment form where every phase is within 0.5 rad, with polygon moments
+// to seventh order (truncation below max|phase|^8 / 8! = 9.7e-8 there).
+constexpr double kSmallPhaseMixed = 0.5;
 
 // Slope stored for an edge that is not valid in that direction (|dx| or
 // |dy| below the reference's geometric tolerance).  Its coefficient
@@ -70,8 +66,9 @@ __device__ __forceinline__ uint32_t low_bits(double t)
     return (uint32_t)__builtin_bit_cast(uint64_t, t);
 }
 
-// In two halves, as for the FP32 variant below: reduction and table read,
-// then polynomials and product.
+// In two halves, so that callers can issue the table reads of several arguments
+// before using any of them: reduction and table read, then polynomials and
+// product.
 __device__ __forceinline__ void sincos_reduce(double x, const double2 *__restrict__ tab,
                                               double &d, double2 &e)
 {
@@ -104,60 +101,88 @@ __device__ __forceinline__ void sincos_table(double x, const double2 *__restrict
     sincos_finish(d, e, s, c);
 }
 
-// FP32 result from an FP64 argument against a 512-entry FP32 table of
-// e^{2 pi i j / 512}, in two halves so that callers can issue the table
-// reads of several arguments before using any of them: the FP64 reduction
-// and table read, then the FP32 correction and the product with the table
-// entry.  One FMA reduces: kTab32Step = double(pi)/256 differs from 2 pi/512
-// by 4.8e-19, so x - j kTab32Step is off by j 4.8e-19 = |x| 3.9e-17 at most,
-// below half an ulp of x itself (the FP64 kernels add the second term of
-// the split; an FP32 result cannot see it).  Against the 256-entry table the
-// index costs one more instruction (a mask and a shift instead of one shift
-// of the low byte) and the correction two fewer.
+// ---------------------------------------------------------------------------
+// FP32 phasors of the mixed kernels.  A phase is held in turns as an FP64
+// number with 1.5 2^22 added (kTurnMagic, carried by the phase's constant
+// term, so the addition costs nothing): the low word of the sum is then the
+// phase modulo 4 turns in units of 2^-30 turn (5.9e-9 rad), exact to that unit
+// for phases within 2^21 turns.  Bits 20..29 select one of 1024 nodes, the 20
+// bits below are the place between nodes.
 //
-// An entry holds (cos, sin, cos/2, sin/2) of its angle (16 bytes, one LDS
-// read): with the halves at hand the correction and the product are four
-// FMAs (see sincos_finish_f32).
-constexpr int kTabN32 = 512;
-constexpr double kTab32InvStep = 81.487330863050411912;  // 512 / (2 pi)
-constexpr double kTab32Step = 3.141592653589793116 / 256.0;
+// Node j lies near (j + 1/2) / 1024 turn, at an angle whose cosine and
+// sine / sqrt(2) both happen to be FP32 numbers to ~1/50 ulp (phasor_node_kernel
+// looks for it), so that the table adds no rounding; its third word is
+// the offset that belongs to that angle.
+//
+// The rotation by the distance d from the node is three shears, x1 = c - t s,
+// s' = s + 2t x1, c' = x1 - t s' with t = d / 2, which is (1 - d^2/2, d) to
+// d^3/6 < 5e-9.  With the sine scaled by 1/sqrt(2), in the table and in the
+// result, all three take the same factor g = d / sqrt(2): one FMA for g and
+// three for the phasor.  (Sine results keep the 1/sqrt(2); the consumers'
+// constants absorb the sqrt(2).)  Per vertex this is six vector instructions
+// after the phase, where a 512-entry table of (cos, sin, cos/2, sin/2) with an
+// FP64 reduction to radians took ten.
+// ---------------------------------------------------------------------------
+constexpr int kPhasorN = 1024;
+constexpr double kTurnMagic = 6291456.0;                 // 1.5 * 2^22
+constexpr double kInvTwoPi = 0.15915494309189533577;
+constexpr float kSqrt2 = 1.41421356237309504880f;
+constexpr float kInvSqrt2 = 0.70710678118654752440f;
+// g = sqrt(2) pi (r - 2^19) 2^-30 - (node offset) / sqrt(2) for the 20-bit place
+// r, whose bits taken as an FP32 number are r 2^-149
+constexpr double kPhasorHalf = 4.44288293815836624702 / 2048.0;  // at r = 2^19
+constexpr float kPhasorG1 = (float)(4.44288293815836624702 * 0x1p+119);
+struct __align__(16) PhasorNode {
+    float c, s, g0, unused;
+};
 
-// Entry j of the FP32 table.
-__device__ __forceinline__ float4 tab32_entry(int j)
+// The table entry of phase word u (byte offset of a 16-byte entry: bits
+// 20..29 of u moved to 4..13, one instruction).
+__device__ __forceinline__ PhasorNode phasor_read(uint32_t u, const PhasorNode *__restrict__ tab)
 {
-    double ts, tc;
-    sincospi((double)j / (kTabN32 / 2), &ts, &tc);
-    return make_float4((float)tc, (float)ts, (float)(0.5 * tc), (float)(0.5 * ts));
+    const uint32_t off = (u >> 16) & (uint32_t)((kPhasorN - 1) * sizeof(PhasorNode));
+    return *reinterpret_cast<const PhasorNode *>(reinterpret_cast<const char *>(tab) + off);
 }
 
-__device__ __forceinline__ void sincos_reduce_f32(double x, const float4 *__restrict__ tab,
-                                                  float &d, float4 &e)
+__device__ __forceinline__ float phasor_angle(uint32_t u, PhasorNode e)
 {
-    const double t = __builtin_fma(x, kTab32InvStep, kRoundMagic);
-    const double j = t - kRoundMagic;
-    d = (float)__builtin_fma(-j, kTab32Step, x);
-    e = tab[low_bits(t) & (kTabN32 - 1)];
+    // keeps the read at 16 bytes: one of 12 takes 1.6 times the LDS cycles (19.7
+    // against 12.0 a wave at random nodes)
+    asm volatile("" ::"v"(e.unused));
+    return __builtin_fmaf(__uint_as_float(u & 0xfffffu), kPhasorG1, e.g0);
 }
 
-// |d| <= pi/512 = 6.14e-3, so e^{i d} = (1 - d^2/2) + i d to FP32 accuracy:
-// the dropped terms are below 3.9e-8 (d^3/6) and 6e-11 (d^4/24), within an
-// ulp of FP32 near 1 (6e-8) -- the phasor rounding the mixed kernels carry
-// anyway.  With T = (c, s) the entry,
-//   Im T e^{id} = s + d (c - d s/2),   Re T e^{id} = c - d (s + d c/2),
-// two FMAs each on the stored halves.
-__device__ __forceinline__ void sincos_finish_f32(float d, float4 e, float &s, float &c)
+// (cos, sin / sqrt 2) of phase word u from its table entry.
+__device__ __forceinline__ void phasor_finish(uint32_t u, PhasorNode e, float &c, float &s)
 {
-    s = __builtin_fmaf(d, __builtin_fmaf(-d, e.w, e.x), e.y);
-    c = __builtin_fmaf(-d, __builtin_fmaf(d, e.z, e.y), e.x);
+    const float g = phasor_angle(u, e);
+    const float x1 = __builtin_fmaf(-g, e.s, e.c);
+    s = __builtin_fmaf(g, x1, e.s);
+    c = __builtin_fmaf(-g, s, x1);
 }
 
-__device__ __forceinline__ void sincos_table_f32(double x, const float4 *__restrict__ tab,
-                                                 float &s, float &c)
+// sin / sqrt 2 alone.
+__device__ __forceinline__ float sine_finish(uint32_t u, PhasorNode e)
 {
-    float d;
-    float4 e;
-    sincos_reduce_f32(x, tab, d, e);
-    sincos_finish_f32(d, e, s, c);
+    const float g = phasor_angle(u, e);
+    return __builtin_fmaf(g, __builtin_fmaf(-g, e.s, e.c), e.s);
+}
+
+// Phase steps (in turns) up to which a lane is looked at one by one for the
+// moment form: 0.25 rad, by edge 0's step and then the other edges' half steps.
+constexpr double kLookStep = 0.25 * kInvTwoPi;
+// Half steps (in turns) up to which sin(h) / h is taken from its series; the
+// table's relative error grows like 3e-10 / h below.
+constexpr float kSeriesStep = 1.0f / 512.0f;
+
+// The phasor of an angle in radians, of any size: reduced to half a turn
+// first.
+__device__ __forceinline__ void phasor_rad(double x, const PhasorNode *__restrict__ tab,
+                                           float &c, float &s)
+{
+    const double y = x * kInvTwoPi;
+    const uint32_t u = low_bits((y - __builtin_rint(y)) + kTurnMagic);
+    phasor_finish(u, phasor_read(u, tab), c, s);
 }
 
 // 1/x to full FP64 precision: hardware estimate + two Newton steps.

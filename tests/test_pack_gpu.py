@@ -68,3 +68,93 @@ def test_every_vertex_count(pkg, oracle, n_beams):
                 e = M.grid_l2(a[..., :1], b[..., :1], theta)
                 print("%d beams mixed (%d): P11 grid_l2 %.2e" % (n_beams, extra, e))
                 assert e < 1e-4
+
+
+def _shapes(rng):
+    """Polygons of every class of the mixed kernels (and both orientations):
+    (name, vertices)."""
+    def turn(p, a):
+        c, s = np.cos(a), np.sin(a)
+        return np.asarray(p) @ np.array([[c, s], [-s, c]])
+    out = []
+    for _ in range(4):
+        a = rng.uniform(0, 2 * np.pi)
+        w, h, sk, top = rng.uniform(0.3, 3.0, 4)
+        out += [("triangle", turn([(-w, -h), (w, -h), (sk - w, h)], a)),
+                ("parallelogram", turn([(-w - sk, -h), (w - sk, -h), (w + sk, h), (sk - w, h)], a)),
+                ("trapezoid", turn([(-w, -h), (w, -h), (sk, h), (sk - top, h)], a)),
+                ("quadrilateral", turn([(-w, -h), (w, -1.2 * h), (0.9 * w, h), (-w, 0.7 * h)], a)),
+                ("rectangle on the axes", np.array([(-w, -h), (w, -h), (w, h), (-w, h)])),
+                ("point on an edge", turn([(-w, -h), (0.2 * w, -h), (w, -h), (0.5 * w, h)], a)),
+                ("sliver", turn([(-w, -h), (w, -h), (w, 1e-3 - h), (2e-3 - w, 1e-3 - h)], a)),
+                ("pentagon", turn([(-w, -h), (w, -h), (1.3 * w, 0), (0, h), (-w, 0.8 * h)], a)),
+                ("hexagon", turn([(w * np.cos(t), h * np.sin(t)) for t in np.arange(6) * np.pi / 3],
+                                 a))]
+    return out
+
+
+@pytest.mark.parametrize("variant", ["plain", "clockwise", "tiny", "small", "far", "slopes",
+                                     "doubled", "long axes"])
+def test_polygon_classes(pkg, oracle, variant):
+    """Shapes of every class on a grid with near-forward rows, as they are; with
+    the vertices reversed; scaled to where every direction (tiny) or some
+    (small) take the moments; with centres so far out that the phases leave
+    the fixed-point range; with slopes that differ from the vertices' by 1e-4;
+    with a repeated vertex; with an aperture axis longer than 1."""
+    abi = pkg.abi
+    fx = load_fixture("sobol_average")
+    consts = abi.consts_from_fixture(fx)
+    src = abi.BeamBatch.from_fixture(fx)
+    rng = np.random.default_rng(77)
+    shapes = _shapes(rng)
+    bs = src.beam_scalars[rng.integers(0, src.n_beams, len(shapes))].copy()
+    cols = {k: [] for k in ("x", "y", "syx", "sxy", "fl")}
+    nv = []
+    for b, (_, p) in enumerate(shapes):
+        p = p * {"tiny": 0.004, "small": 0.1}.get(variant, 1.0)
+        if variant == "clockwise":
+            p = p[::-1]
+        if variant == "doubled":
+            p = np.insert(p, 1, p[1], axis=0)
+        dx, dy = (np.roll(p, -1, 0) - p).T
+        okx, oky = np.abs(dx) > 1e-12, np.abs(dy) > 1e-12
+        syx = np.divide(dy, dx, out=np.zeros_like(dx), where=okx)
+        sxy = np.divide(dx, dy, out=np.zeros_like(dx), where=oky)
+        if variant == "slopes":
+            syx, sxy = syx * (1 + 1e-4), sxy * (1 + 1e-4)
+        for k, v in zip(("x", "y", "syx", "sxy", "fl"),
+                        (p[:, 0], p[:, 1], syx, sxy, okx + 2 * oky)):
+            cols[k].append(v)
+        nv.append(len(p))
+        bs[b, abi.B_AREA] = 0.5 * np.sum(p[:, 0] * np.roll(p[:, 1], -1)
+                                         - np.roll(p[:, 0], -1) * p[:, 1])
+        if b % 3 == 0:  # leaves along theta = 0 (reflect the frame)
+            u = np.array([0.0, 0.0, -1.0]) - bs[b, abi.B_DIR:abi.B_DIR + 3]
+            for col in (abi.B_HOR, abi.B_VER, abi.B_DIR, abi.B_NT, abi.B_NP, abi.B_NXDT,
+                        abi.B_NXDP, abi.B_NORMAL):
+                w = bs[b, col:col + 3]
+                bs[b, col:col + 3] = w - 2.0 * u * (u @ w) / max(u @ u, 1e-30)
+    if variant == "far":
+        bs[:, abi.B_CEN:abi.B_CEN + 3] *= 3e5 / np.linalg.norm(bs[:, abi.B_CEN:abi.B_CEN + 3],
+                                                               axis=1, keepdims=True)
+    if variant == "long axes":
+        bs[:, abi.B_HOR:abi.B_HOR + 3] *= 1.5
+    nb = len(shapes)
+    batch = abi.BeamBatch([0, nb], [1.0], bs, nv, np.arange(nb) % 5 == 4,
+                          np.r_[0, np.cumsum(nv)],
+                          *[np.concatenate(cols[k]) for k in ("x", "y", "syx", "sxy", "fl")])
+    theta = np.r_[0.0, np.logspace(-4, -1, 25), np.linspace(0.2, np.pi, 40)]
+    grid = abi.Grid.build(theta, 9)
+    o, on, _ = oracle.diffract(grid, batch, consts, noshadow=True)
+    with pkg.engine.Context(0) as ctx:
+        ctx.set_grid(grid)
+        ctx.upload(batch, consts)
+        for extra in (0, abi.NO_MFMA):
+            m, mn = ctx.mueller(abi.PREC_MIXED | extra, noshadow=True)
+            for a, b in ((m, o), (mn, on)):
+                e = M.grid_l2(a, b, theta)
+                e11 = M.grid_l2(a[..., :1], b[..., :1], theta)
+                print("%s (%d): grid_l2 %.2e, P11 %.2e" % (variant, extra, e, e11))
+                # the path's bar; a far centre's phases of 4e6 rad carry 1e-9
+                # rad of their own rounding
+                assert e11 < 1e-4 and e < 1e-4
