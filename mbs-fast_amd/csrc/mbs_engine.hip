@@ -81,13 +81,14 @@ struct mbs_ctx {
     double mean_edges = 0;
     mbs_consts consts{};
     DevBuf<double> bs_in, vx_in, vy_in, syx_in, sxy_in, weights;
-    DevBuf<int32_t> nv, ext, vflag;
+    DevBuf<int32_t> nv, ext;
     DevBuf<int64_t> voff, ooff;
     DevBuf<uint8_t> ef_in;
-    DevBuf<double> hdr, vtx, vdd;
+    DevBuf<double> hdr, w64, vtx, vx;
     DevBuf<uint32_t> wb;          // MFMA operand of the mixed kernels
-    DevBuf<double> ebeam, evert;  // aperture records of the mixed kernels
-    DevBuf<PhasorNode> phasor;        // their phasor nodes
+    DevBuf<double> ebeam;         // aperture records
+    DevBuf<PhasorNode> phasor;    // phasor nodes of the mixed kernels
+    DevBuf<double2> turns;        // phasors of the FP64 kernels
     bool phasor_ok = false;
     // size rescaling data of the batch (mbs_upload_beam_scaling)
     bool scaling_ok = false;
@@ -331,16 +332,16 @@ int mbs_ctx_destroy(mbs_ctx *ctx)
     ctx->weights.release();
     ctx->nv.release();
     ctx->ext.release();
-    ctx->vflag.release();
+    ctx->w64.release();
     ctx->voff.release();
     ctx->ooff.release();
     ctx->ef_in.release();
     ctx->hdr.release();
     ctx->vtx.release();
-    ctx->vdd.release();
+    ctx->vx.release();
     ctx->wb.release();
     ctx->ebeam.release();
-    ctx->evert.release();
+    ctx->turns.release();
     ctx->phasor.release();
     ctx->items.release();
     ctx->queue.release();
@@ -424,12 +425,15 @@ int mbs_set_grid(mbs_ctx *ctx, const mbs_grid *g)
     HIP_TRY(ctx, ctx->tab.ensure((size_t)cells * DT_COUNT));
     HIP_TRY(ctx, ctx->tab32.ensure((size_t)cells * DT32_COUNT));
     HIP_TRY(ctx, ctx->phasor.ensure(kPhasorN));
+    HIP_TRY(ctx, ctx->turns.ensure(kTabN));
     HIP_TRY(ctx, hipMemcpyAsync(ctx->theta.p, g->theta, sizeof(double) * ctx->n_zen1,
                                 hipMemcpyHostToDevice, ctx->stream));
     HIP_TRY(ctx, hipMemcpyAsync(ctx->vf.p, g->vf, sizeof(double) * cells * 3,
                                 hipMemcpyHostToDevice, ctx->stream));
     if (!ctx->phasor_ok) {  // once per context
         phasor_node_kernel<<<kPhasorN, 64, 0, ctx->stream>>>(ctx->phasor.p);
+        HIP_TRY(ctx, hipGetLastError());
+        turn_table_kernel<<<kTabN / 256, 256, 0, ctx->stream>>>(ctx->turns.p);
         HIP_TRY(ctx, hipGetLastError());
     }
     HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
@@ -472,8 +476,8 @@ static int launch_pack(mbs_ctx *ctx, int nb, const mbs_consts &c, double scale, 
         ctx->syx_in.p, ctx->sxy_in.p, ctx->ef_in.p, c.wave_index, sg * c.inv_compl_wave[0],
         sg * c.inv_compl_wave[1], c.compl_wave[0], c.compl_wave[1], rescale ? scale : 1.0,
         rescale ? ctx->sc_raw.p : nullptr, ctx->sc_path.p, ctx->sc_sign.p, ctx->sc_aoff.p,
-        ctx->sc_apath.p, ctx->sc_cabs, ctx->sc_k, mixed_eps(c), ctx->hdr.p, ctx->vtx.p,
-        ctx->vdd.p, ctx->vflag.p, ctx->wb.p, ctx->ebeam.p, ctx->evert.p);
+        ctx->sc_apath.p, ctx->sc_cabs, ctx->sc_k, c.eps1, mixed_eps(c), ctx->hdr.p, ctx->w64.p,
+        ctx->vtx.p, ctx->vx.p, ctx->wb.p, ctx->ebeam.p);
     HIP_TRY(ctx, hipGetLastError());
     return MBS_OK;
 }
@@ -546,11 +550,10 @@ static int upload_impl(mbs_ctx *ctx, const mbs_beam_batch *bt, const mbs_consts 
     HIP_TRY(ctx, ctx->ef_in.ensure(nvert));
     HIP_TRY(ctx, ctx->hdr.ensure((size_t)nb * HDR_STRIDE));
     HIP_TRY(ctx, ctx->ebeam.ensure((size_t)nb * EB_STRIDE));
-    HIP_TRY(ctx, ctx->evert.ensure((size_t)nvert * EV_STRIDE));
+    HIP_TRY(ctx, ctx->w64.ensure((size_t)nb * W64_STRIDE));
     HIP_TRY(ctx, ctx->vtx.ensure((size_t)nvert * VTX_STRIDE));
-    HIP_TRY(ctx, ctx->vdd.ensure((size_t)nvert * VDD_STRIDE));
+    HIP_TRY(ctx, ctx->vx.ensure((size_t)nvert * VX_STRIDE));
     HIP_TRY(ctx, ctx->wb.ensure((size_t)std::max(nb, 1) * WB_STRIDE));
-    HIP_TRY(ctx, ctx->vflag.ensure(nvert));
     hipStream_t s = ctx->stream;
     if (ctx->timing)
         HIP_TRY(ctx, hipEventRecord(ctx->ev[0], s));
@@ -841,23 +844,23 @@ static void launch_one(const KernelArgs &a, int blocks, hipStream_t s)
 {
     if constexpr (PREC == 4)
         diffract_mfma_kernel<NS, JONES, PER, Q, 1><<<blocks, 256, 0, s>>>(
-            a.items, a.n_items, a.n_tiles, a.cells, a.n_az, a.tab, a.hdr, a.wb, a.vtx, a.vdd,
-            a.vflag, a.ebeam, a.evert, a.phasor, a.ooff, a.weights, a.k,
+            a.items, a.n_items, a.n_tiles, a.cells, a.n_az, a.tab, a.hdr, a.w64, a.wb,
+            a.vtx, a.vx, a.ebeam, a.phasor, a.ooff, a.weights, a.k,
             a.eps1, a.out, a.out_ns, a.per_orient, a.queue, a.tab32, a.sidx, a.fbuf);
     else if constexpr (PREC == 3)
         diffract_incoherent_kernel<<<blocks, 256, 0, s>>>(
-            a.items, a.n_items, a.n_tiles, a.cells, a.tab, a.hdr, a.vtx, a.vdd, a.vflag, a.nv,
-            a.voff, a.ooff, a.weights, a.k, a.eps1, a.out);
+            a.items, a.n_items, a.n_tiles, a.cells, a.tab, a.hdr, a.w64, a.vtx, a.vx,
+            a.ebeam, a.turns, a.ooff, a.weights, a.k, a.eps1, a.out);
     else if constexpr (PREC == 2)
         diffract_mfma_kernel<NS, JONES, PER, Q><<<blocks, 256, 0, s>>>(
-            a.items, a.n_items, a.n_tiles, a.cells, a.n_az, a.tab, a.hdr, a.wb, a.vtx, a.vdd,
-            a.vflag, a.ebeam, a.evert, a.phasor, a.ooff, a.weights, a.k, a.eps1, a.out, a.out_ns,
+            a.items, a.n_items, a.n_tiles, a.cells, a.n_az, a.tab, a.hdr, a.w64, a.wb,
+            a.vtx, a.vx, a.ebeam, a.phasor, a.ooff, a.weights, a.k, a.eps1, a.out, a.out_ns,
             a.per_orient, a.queue, a.tab32);
     else
         diffract_kernel<PREC, NS, JONES, PER, Q><<<blocks, 256, 0, s>>>(
-            a.items, a.n_items, a.n_tiles, a.cells, a.n_az, a.tab, a.hdr, a.vtx, a.vdd, a.vflag,
-            a.nv, a.voff, a.ext, a.ooff, a.weights, a.k, a.eps1, a.out, a.out_ns, a.per_orient,
-            a.queue, a.tab32, a.ebeam, a.evert, a.phasor);
+            a.items, a.n_items, a.n_tiles, a.cells, a.n_az, a.tab, a.hdr, a.w64, a.vtx, a.vx,
+            a.ebeam, a.phasor, a.turns, a.ooff, a.weights, a.k, a.eps1, a.out, a.out_ns,
+            a.per_orient, a.queue, a.tab32);
 }
 
 // queue: the persistent work-queue kernels (beam segments, no per-orientation
@@ -869,13 +872,13 @@ static void launch_diffract(int prec, int ns, int jones, int per, bool queue,
     if (prec == 2 && !ns && jones && !per && !queue && (a.waves == 4 || a.waves == 6)) {
         if (a.waves == 4)
             diffract_mfma_kernel<0, 1, 0, 0, 0, 4><<<blocks, 256, 0, s>>>(
-                a.items, a.n_items, a.n_tiles, a.cells, a.n_az, a.tab, a.hdr, a.wb, a.vtx,
-                a.vdd, a.vflag, a.ebeam, a.evert, a.phasor, a.ooff, a.weights, a.k, a.eps1, a.out,
+                a.items, a.n_items, a.n_tiles, a.cells, a.n_az, a.tab, a.hdr, a.w64, a.wb,
+                a.vtx, a.vx, a.ebeam, a.phasor, a.ooff, a.weights, a.k, a.eps1, a.out,
                 a.out_ns, a.per_orient, a.queue, a.tab32);
         else
             diffract_mfma_kernel<0, 1, 0, 0, 0, 6><<<blocks, 256, 0, s>>>(
-                a.items, a.n_items, a.n_tiles, a.cells, a.n_az, a.tab, a.hdr, a.wb, a.vtx,
-                a.vdd, a.vflag, a.ebeam, a.evert, a.phasor, a.ooff, a.weights, a.k, a.eps1, a.out,
+                a.items, a.n_items, a.n_tiles, a.cells, a.n_az, a.tab, a.hdr, a.w64, a.wb,
+                a.vtx, a.vx, a.ebeam, a.phasor, a.ooff, a.weights, a.k, a.eps1, a.out,
                 a.out_ns, a.per_orient, a.queue, a.tab32);
         return;
     }
@@ -967,15 +970,12 @@ static void batch_args(const mbs_ctx *ctx, int prec, int n_items, int n_tiles, K
     a.tab32 = ctx->tab32.p;
     a.hdr = ctx->hdr.p;
     a.ebeam = ctx->ebeam.p;
-    a.evert = ctx->evert.p;
+    a.w64 = ctx->w64.p;
     a.phasor = ctx->phasor.p;
+    a.turns = ctx->turns.p;
     a.wb = ctx->wb.p;
     a.vtx = ctx->vtx.p;
-    a.vdd = ctx->vdd.p;
-    a.vflag = ctx->vflag.p;
-    a.nv = ctx->nv.p;
-    a.voff = ctx->voff.p;
-    a.ext = ctx->ext.p;
+    a.vx = ctx->vx.p;
     a.ooff = ctx->ooff.p;
     a.weights = ctx->weights.p;
     a.k = ctx->consts.wave_index;

@@ -33,9 +33,11 @@
 #include "po_math.h"
 #include "po_layout.h"
 
-// Occupancy of the vector-ALU kernels: at least 4 waves per SIMD (128
-// VGPRs).  The FP64 kernel, whose batched vertex phasors would otherwise take
-// ~140 VGPRs and 3 waves, spills only a few scalars per beam to keep it.
+// Occupancy of the vector-ALU kernels: at least 4 waves per SIMD (128 VGPRs).
+// The FP64 kernel's common path takes about 120 with its 24 sums; the other
+// polygons' spill there.  With 3 waves and no spills it is slower (11.7 ms
+// against 9.3 for 35,800 beams on 541 x 96 directions): it waits on LDS and
+// scalar loads.
 // Builds may pass -DMBS_MIN_WAVES=N for tuning.
 #ifndef MBS_MIN_WAVES
 #define MBS_MIN_WAVES 4
@@ -112,6 +114,15 @@ __global__ void __launch_bounds__(64) phasor_node_kernel(PhasorNode *__restrict_
     }
 }
 
+// e^{2 pi i j / 1024}, the table of the FP64 phasors.
+__global__ void turn_table_kernel(double2 *__restrict__ turns)
+{
+    const int j = blockIdx.x * blockDim.x + threadIdx.x;
+    double s, c;
+    sincospi((double)j / (kTabN / 2), &s, &c);
+    turns[j] = make_double2(c, s);
+}
+
 __global__ void grid_tables_kernel(const double *__restrict__ theta,
                                    const double *__restrict__ vf, int n_az,
                                    int n_zen1, double az_step,
@@ -179,7 +190,7 @@ __global__ void grid_tables_kernel(const double *__restrict__ theta,
 // take the vertices in turn and add their sums by butterflies, and an edge's
 // share of a moment is a 4-point Gauss rule: over the triangle (0, P, Q) a
 // monomial of degree n integrates to det(P, Q) / (n + 2) times its mean along
-// PQ, which four nodes give exactly to degree 7.  The record goes through LDS
+// PQ, which three nodes give exactly to degree 5.  The record goes through LDS
 // so that its stores are contiguous.
 // ---------------------------------------------------------------------------
 enum { PACK_GROUP = 8, PACK_BEAMS = 16, PACK_THREADS = PACK_GROUP * PACK_BEAMS };
@@ -241,14 +252,15 @@ __global__ void __launch_bounds__(PACK_THREADS) pack_beams_kernel(
     double cw_im, double sc, const double *__restrict__ raw_j,
     const double *__restrict__ path, const double *__restrict__ sign,
     const int64_t *__restrict__ abs_off, const double *__restrict__ abs_path, double c_abs,
-    double k_j, double eps_mixed, double *__restrict__ hdr, double *__restrict__ vtx,
-    double *__restrict__ vdd, int32_t *__restrict__ vflag, uint32_t *__restrict__ wb,
-    double *__restrict__ ebeam, double *__restrict__ evert)
+    double k_j, double eps1, double eps_mixed, double *__restrict__ hdr,
+    double *__restrict__ w64, double *__restrict__ vtx, double *__restrict__ vx_out,
+    uint32_t *__restrict__ wb, double *__restrict__ ebeam)
 {
     __shared__ double s_bs[PACK_BEAMS * 36];
     __shared__ double s_x[PACK_BEAMS][33], s_y[PACK_BEAMS][33];  // odd stride: no bank conflicts
     __shared__ double s_h[PACK_BEAMS * HDR_STRIDE];
-    __shared__ double s_scale[PACK_BEAMS];
+    __shared__ double s_jp[PACK_BEAMS][8];  // complWave * J_phased
+    __shared__ double s_s64[PACK_BEAMS], s_scale[PACK_BEAMS];
     const int g = threadIdx.x / PACK_GROUP, q = threadIdx.x % PACK_GROUP;
     const int first = blockIdx.x * PACK_BEAMS;
     const int count = min((int)PACK_BEAMS, n_beams - first);  // beams of this workgroup
@@ -268,8 +280,7 @@ __global__ void __launch_bounds__(PACK_THREADS) pack_beams_kernel(
     double *h = s_h + g * HDR_STRIDE;
     // polygon sums about the aperture origin, and the bounding box
     double sum[6] = {0, 0, 0, 0, 0, 0}, m3[4] = {0, 0, 0, 0}, m4[5] = {0, 0, 0, 0, 0},
-           m5[6] = {0, 0, 0, 0, 0, 0}, m6[7] = {0, 0, 0, 0, 0, 0, 0},
-           m7[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+           m5[6] = {0, 0, 0, 0, 0, 0};
     double minX = 1e300, maxX = -1e300, minY = 1e300, maxY = -1e300;
     double longest = -1.0;  // squared length of this lane's longest edge, and
     int start = 0;          // the edge (the least index of equal ones)
@@ -292,29 +303,24 @@ __global__ void __launch_bounds__(PACK_THREADS) pack_beams_kernel(
             longest = l2;
             start = i;
         }
-        const double node[4] = {0.5 - 0.43056815579702628761, 0.5 - 0.16999052179242813240,
-                                0.5 + 0.16999052179242813240, 0.5 + 0.43056815579702628761};
-        const double weight[4] = {0.17392742256872692869, 0.32607257743127307131,
-                                  0.32607257743127307131, 0.17392742256872692869};
-        for (int n = 0; n < 4; ++n) {
+        const double node[3] = {0.5 - 0.38729833462074168852, 0.5,
+                                0.5 + 0.38729833462074168852};
+        const double weight[3] = {5.0 / 18.0, 8.0 / 18.0, 5.0 / 18.0};
+        for (int n = 0; n < 3; ++n) {
             const double x = xi + node[n] * (xj - xi), y = yi + node[n] * (yj - yi);
-            double px7[8], py7[8];  // powers, the weight in those of x
-            px7[0] = weight[n] * cr;
-            py7[0] = 1.0;
-            for (int e = 1; e < 8; ++e) {
-                px7[e] = px7[e - 1] * x;
-                py7[e] = py7[e - 1] * y;
+            double powx[6], powy[6];  // the weight in those of x
+            powx[0] = weight[n] * cr;
+            powy[0] = 1.0;
+            for (int e = 1; e < 6; ++e) {
+                powx[e] = powx[e - 1] * x;
+                powy[e] = powy[e - 1] * y;
             }
             for (int e = 0; e < 4; ++e)
-                m3[e] += px7[e] * py7[3 - e];
+                m3[e] += powx[e] * powy[3 - e];
             for (int e = 0; e < 5; ++e)
-                m4[e] += px7[e] * py7[4 - e];
+                m4[e] += powx[e] * powy[4 - e];
             for (int e = 0; e < 6; ++e)
-                m5[e] += px7[e] * py7[5 - e];
-            for (int e = 0; e < 7; ++e)
-                m6[e] += px7[e] * py7[6 - e];
-            for (int e = 0; e < 8; ++e)
-                m7[e] += px7[e] * py7[7 - e];
+                m5[e] += powx[e] * powy[5 - e];
         }
     }
     for (double &v : sum)
@@ -324,10 +330,6 @@ __global__ void __launch_bounds__(PACK_THREADS) pack_beams_kernel(
     for (double &v : m4)
         v = group_sum(v);
     for (double &v : m5)
-        v = group_sum(v);
-    for (double &v : m6)
-        v = group_sum(v);
-    for (double &v : m7)
         v = group_sum(v);
     for (int off = 1; off < PACK_GROUP; off <<= 1) {
         const double l2 = __shfl_xor(longest, off, PACK_GROUP);
@@ -392,7 +394,6 @@ __global__ void __launch_bounds__(PACK_THREADS) pack_beams_kernel(
         const double phb =
             (wmin > 0.0 && wmin < __builtin_inf()) ? 2.04e-3 / (k * wmin) : __builtin_inf();
         h[H_PHB] = phb;
-        h[H_SPARE] = 0.0;
         for (int i = HDR_USED; i < HDR_STRIDE; ++i)
             h[i] = 0.0;
     } else if (q == 1) {
@@ -411,19 +412,6 @@ __global__ void __launch_bounds__(PACK_THREADS) pack_beams_kernel(
             h[H_MOM4 + a] = k3 * k * c4[a] * (m4[a] / 6.0 * inv) / 24.0;
         for (int a = 0; a < 6; ++a)
             h[H_MOM5 + a] = k3 * k * k * c5[a] * (m5[a] / 7.0 * inv) / 120.0;
-        const double c6[7] = {1, 6, 15, 20, 15, 6, 1}, c7[8] = {1, 7, 21, 35, 35, 21, 7, 1};
-        for (int a = 0; a < 7; ++a)
-            h[H_MOM6 + a] = k3 * k3 * c6[a] * (m6[a] / 8.0 * inv) / 720.0;
-        for (int a = 0; a < 8; ++a)
-            h[H_MOM7 + a] = k3 * k3 * k * c7[a] * (m7[a] / 9.0 * inv) / 5040.0;
-    } else if (q == 2) {
-        // rotation vectors, pre-scaled by 1/2 (exact)
-        for (int i = 0; i < 3; ++i) {
-            h[H_T0 + i] = 0.5 * s[13 + i];      // NT
-            h[H_T0 + 3 + i] = 0.5 * s[19 + i];  // nxDT
-            h[H_T1 + i] = 0.5 * s[16 + i];      // NP
-            h[H_T1 + 3 + i] = 0.5 * s[22 + i];  // nxDP
-        }
     }
     // J_phased, or for a rescaled set sign * a(sc) * J * exp(i k_j path sc),
     // a(sc) the mean of exp(c_abs p sc) over the absorption paths p (1 for
@@ -452,28 +440,34 @@ __global__ void __launch_bounds__(PACK_THREADS) pack_beams_kernel(
             jr = s[25 + 2 * q];
             ji = s[26 + 2 * q];
         }
-        h[H_JP + 2 * q] = cw_re * jr - cw_im * ji;
-        h[H_JP + 2 * q + 1] = cw_re * ji + cw_im * jr;
+        s_jp[g][2 * q] = cw_re * jr - cw_im * ji;
+        s_jp[g][2 * q + 1] = cw_re * ji + cw_im * jr;
     }
-    // The beam's class.  The formulas of the mixed kernels work from the
-    // vertices alone, so the slopes and flags have to agree with them (an edge
-    // left out of one branch of the reference's sum must be negligible in it),
-    // and the phases have to fit the fixed-point range; any other beam keeps
-    // the sum over the slopes.
+    // The beam's class.  The formulas work from the vertices alone, so the
+    // slopes and flags have to agree with them (an edge left out of one branch of
+    // the reference's sum must be negligible in it), and in the mixed kernels the
+    // phases have to fit the fixed-point range; any other beam keeps the sum over
+    // the slopes.  "Agree" and "parallel" are 1e-9 for the mixed kernels and 1e-13
+    // for the FP64 ones, the size of their own rounding for phases of 1e2-1e3 rad.
+    // (Of a traced hexagonal column's quadrilaterals 0.945 have a parallel pair
+    // to 1e-13 and 0.964 to 1e-12 or any tolerance up to 1e-6.)
     const double lmax = sqrt(longest);
     const double cx = ext ? 0.0 : s[9] * sc, cy = ext ? 0.0 : s[10] * sc,
                  cz = ext ? 0.0 : s[11] * sc;
-    const double k_turn = k * kInvTwoPi;
+    const double k_turn = k * kInvTwoPi, k_node = kPhasorN * k_turn;
     const double tol = 1e-9 * lmax;
-    double agree = 1.0, reach = 0.0;  // every edge agrees; the largest |vertex|
+    // 2 where every edge agrees closely, 1 where every edge does; the largest |vertex|
+    double agree = 2.0, reach = 0.0;
     for (int i = q; i < nv; i += PACK_GROUP) {
         const int to = (i + 1 < nv) ? i + 1 : 0;
         const double x = px[i], y = py[i], dx = px[to] - x, dy = py[to] - y;
         const uint8_t f = ef[v0 + i];
-        const bool okx = (f & 1) ? fabs(syx[v0 + i] * dx - dy) <= tol : fabs(dx) <= tol;
-        const bool oky = (f & 2) ? fabs(sxy[v0 + i] * dy - dx) <= tol : fabs(dy) <= tol;
-        if (!(okx && oky && sqrt(dx * dx + dy * dy) > tol && (f & 3)))
-            agree = 0.0;
+        const double offx = fabs((f & 1) ? syx[v0 + i] * dx - dy : dx);
+        const double offy = fabs((f & 2) ? sxy[v0 + i] * dy - dx : dy);
+        const bool edge = sqrt(dx * dx + dy * dy) > tol && (f & 3);
+        const double here = !(edge && offx <= tol && offy <= tol) ? 0.0
+                            : offx <= 1e-4 * tol && offy <= 1e-4 * tol ? 2.0 : 1.0;
+        agree = fmin(agree, here);
         reach = fmax(reach, sqrt(x * x + y * y));
     }
     agree = group_min(agree);
@@ -486,53 +480,68 @@ __global__ void __launch_bounds__(PACK_THREADS) pack_beams_kernel(
     // so that a value that is not a number fails them
     const bool unit = n_hor <= 1.0 + 1e-6 && n_ver <= 1.0 + 1e-6 && n_bd <= 1.0 + 1e-6;
     const bool fits = 2.5 * k_turn * (sqrt(cx * cx + cy * cy + cz * cz) + reach) < 0x1p20;
-    int cls = BEAM_VERTICES;
-    double scale = 1.0;  // F / F' of the class's formula
-    if (!(unit && fits && agree == 1.0)) {
-        cls = BEAM_SLOPES;
-    } else if (fabs(skew) <= 1e-6 && 2.01 * k * reach <= kSmallPhaseMixed) {
-        cls = BEAM_MOMENTS;
-    } else if (nv <= 4) {
-        // parallel edges, to 1e-9 of the area's own products (a traced
-        // hexagonal particle: nineteen quadrilaterals in twenty have a
-        // parallel pair, to 1e-12)
-        const auto cross = [&](int i, int j) {
-            const int i1 = (i + 1) % nv, j1 = (j + 1) % nv;
-            return (px[i1] - px[i]) * (py[j1] - py[j]) - (py[i1] - py[i]) * (px[j1] - px[j]);
-        };
-        const auto len2 = [&](int i) {
-            const int i1 = (i + 1) % nv;
-            return (px[i1] - px[i]) * (px[i1] - px[i]) + (py[i1] - py[i]) * (py[i1] - py[i]);
-        };
-        int from = start;
-        if (nv == 3) {
-            cls = BEAM_TRAPEZOID;
-        } else {
-            const double c01 = fabs(cross(0, 1)), c03 = fabs(cross(0, 3)), c21 = fabs(cross(2, 1));
-            const bool p02 = fabs(cross(0, 2)) <= 1e-9 * fmin(c01, c03);
-            const bool p13 = fabs(cross(1, 3)) <= 1e-9 * fmin(c01, c21);
-            const double gx = px[0] - px[1] + px[2] - px[3], gy = py[0] - py[1] + py[2] - py[3];
-            if (p02 && p13 && k * sqrt(gx * gx + gy * gy) <= 1e-8) {
-                cls = BEAM_PARALLEL;
-            } else if (p02 || p13) {
-                cls = BEAM_TRAPEZOID;
-                from = p02 ? (len2(0) >= len2(2) ? 0 : 2) : (len2(1) >= len2(3) ? 1 : 3);
-            }
-        }
-        if (cls != BEAM_VERTICES) {
-            // w_1 = -(t_0 x t_1) (k / 2 pi)^2; the sines carry 1/sqrt(2) each
-            const double w1 = -cross(from, (from + 1) % nv) * k_turn * k_turn;
-            scale = cls == BEAM_PARALLEL ? -2.0 * w1 : 1.41421356237309504880 * w1;
-            if (fabs(scale) >= 1e-30 && fabs(scale) <= 1e30) {
-                start = from;
-            } else {
-                cls = nv == 3 ? BEAM_SLOPES : BEAM_VERTICES;
-            }
+    // the polygon's own form, and edge 0 for it
+    int form = BEAM_VERTICES, from = start;
+    bool close = agree == 2.0;  // to the FP64 kernels' tolerance
+    const auto cross = [&](int i, int j) {
+        const int i1 = (i + 1) % nv, j1 = (j + 1) % nv;
+        return (px[i1] - px[i]) * (py[j1] - py[j]) - (py[i1] - py[i]) * (px[j1] - px[j]);
+    };
+    const auto len2 = [&](int i) {
+        const int i1 = (i + 1) % nv;
+        return (px[i1] - px[i]) * (px[i1] - px[i]) + (py[i1] - py[i]) * (py[i1] - py[i]);
+    };
+    if (nv == 3) {
+        form = BEAM_TRAPEZOID;
+    } else if (nv == 4) {
+        // parallel edges, against the area's own products
+        const double c02 = fabs(cross(0, 2)) / fmin(fabs(cross(0, 1)), fabs(cross(0, 3)));
+        const double c13 = fabs(cross(1, 3)) / fmin(fabs(cross(0, 1)), fabs(cross(2, 1)));
+        const double gx = px[0] - px[1] + px[2] - px[3], gy = py[0] - py[1] + py[2] - py[3];
+        const double gap = k * sqrt(gx * gx + gy * gy);
+        const bool para = c02 <= 1e-9 && c13 <= 1e-9 && gap <= 1e-8;
+        const bool para64 = para && gap <= 4e-15 * k * (reach + sqrt(cx * cx + cy * cy + cz * cz));
+        const double c = fmin(c02, c13);
+        if (para && (para64 || !(c <= 1e-13))) {
+            form = BEAM_PARALLEL;
+            close = close && para64;
+        } else if (c <= 1e-9) {
+            form = BEAM_TRAPEZOID;
+            close = close && c <= 1e-13;
+            // the pair that is parallel, the nearer to it of two
+            from = c02 <= c13 ? (len2(0) >= len2(2) ? 0 : 2) : (len2(1) >= len2(3) ? 1 : 3);
         }
     }
+    double s64 = 1.0, scale = 1.0;  // F / F' of the formulas, FP64 and mixed
+    int cls64 = BEAM_SLOPES, cls = BEAM_VERTICES;
+    if (form != BEAM_VERTICES) {
+        // w_1 = -(t_0 x t_1) (1024 k / 2 pi)^2, steps being in nodes
+        const double w1 = -cross(from, (from + 1) % nv) * k_node * k_node;
+        if (fabs(w1) >= 1e-30 && fabs(w1) <= 1e30) {
+            if (unit && agree >= 1.0)
+                start = from;
+            if (unit && close) {
+                cls64 = form;  // else the sum over vertices, below
+                s64 = form == BEAM_PARALLEL ? -w1 : w1;
+            }
+            // the mixed kernels' sines carry 1/sqrt(2) each
+            scale = form == BEAM_PARALLEL ? -2.0 * w1 : 1.41421356237309504880 * w1;
+            cls = form;
+        } else if (nv == 3) {
+            cls = BEAM_SLOPES;
+        }
+    }
+    if (cls64 == BEAM_SLOPES && unit && agree == 2.0) {
+        cls64 = BEAM_VERTICES;
+        s64 = k_node * (kPhasorN * kInvTwoPi);
+    }
+    if (!(unit && fits && agree >= 1.0))
+        cls = BEAM_SLOPES;
+    else if (fabs(skew) <= 1e-6 && 2.01 * k * reach <= kSmallPhaseMixed)
+        cls = BEAM_MOMENTS;
     if (cls == BEAM_VERTICES)
         scale = 1.41421356237309504880;
-    else if (cls == BEAM_SLOPES)
+    else if (cls == BEAM_SLOPES || cls == BEAM_MOMENTS)
         scale = 1.0;
     // phase vector in turns of a point of the aperture plane, from the beam
     // centre or from the particle's origin
@@ -555,60 +564,94 @@ __global__ void __launch_bounds__(PACK_THREADS) pack_beams_kernel(
         v[V_KY] = k * y;
         v[V_SYX] = (f & 1) ? syx[v0 + at] : kInvalidSlope;
         v[V_SXY] = (f & 2) ? sxy[v0 + at] : kInvalidSlope;
-        double *w = vdd + (size_t)(v0 + i) * VDD_STRIDE;
-        w[D_DX] = dx;
-        w[D_DY] = dy;
-        vflag[v0 + i] = f;
-        if (cls == BEAM_VERTICES) {
-            const double cross = i == 0 ? 0.0 : t0x * dy - t0y * dx;
-            double *ev = evert + (size_t)(v0 + i) * EV_STRIDE;
-            turns(x, y, false, ev + EV_Q);
-            ev[EV_W] = nv == 4 ? pack_floats((float)(-cross * k_turn * k_turn), 0.0f)
-                               : pack_floats((float)(k_turn * dx), (float)(-k_turn * dy));
-        }
+        double *w = vx_out + (size_t)(v0 + i) * VX_STRIDE;
+        w[VX_DX] = dx;
+        w[VX_DY] = dy;
+        const double tx = t0x * k_node, ty = t0y * k_node;
+        const double kw = k_node * (kPhasorN * kInvTwoPi);
+        w[VX_W] = nv == 4 ? pack_floats(i == 0 ? 0.0f : (float)((ty * dx - tx * dy) * k_node), 0.0f)
+                          : pack_floats((float)(kw * dx), (float)(-kw * dy));
+        w[VX_FLAG] = pack_words(f, 0);
     }
     if (q == 0 && g < count) {
         const auto X = [&](int i) { return px[vert(i % nv)]; };
         const auto Y = [&](int i) { return py[vert(i % nv)]; };
         double *eb = ebeam + (size_t)b * EB_STRIDE, *eq = eb + EB_Q;
-        for (int i = 0; i < EB_STRIDE - EB_Q; ++i)
-            eq[i] = 0.0;
-        if (cls == BEAM_TRAPEZOID) {  // edge 1 and the last one
+        const bool trapezoid = cls == BEAM_TRAPEZOID || cls64 == BEAM_TRAPEZOID;
+        const bool parallel = cls == BEAM_PARALLEL || cls64 == BEAM_PARALLEL;
+        if (trapezoid) {  // edge 1 and the last one
             turns(0.5 * (X(1) + X(2)), 0.5 * (Y(1) + Y(2)), false, eq);
             turns(0.5 * (X(2) - X(1)), 0.5 * (Y(2) - Y(1)), true, eq + 3);
             turns(0.5 * (X(nv - 1) + X(0)), 0.5 * (Y(nv - 1) + Y(0)), false, eq + 6);
             turns(0.5 * (X(0) - X(nv - 1)), 0.5 * (Y(0) - Y(nv - 1)), true, eq + 9);
-        } else if (cls == BEAM_PARALLEL) {
-            turns(0.5 * (X(0) + X(2)), 0.5 * (Y(0) + Y(2)), false, eq);
-            turns(0.5 * (X(1) - X(0)), 0.5 * (Y(1) - Y(0)), true, eq + 3);
-            turns(0.5 * (X(2) - X(1)), 0.5 * (Y(2) - Y(1)), true, eq + 6);
+        } else if (parallel) {
+            // means over opposite vertices and edges: what the polygon lacks to a
+            // parallelogram then enters in pairs of opposite sign
+            const double ux = X(1) - X(0) + (X(2) - X(3)), uy = Y(1) - Y(0) + (Y(2) - Y(3));
+            const double wx = X(2) - X(1) + (X(3) - X(0)), wy = Y(2) - Y(1) + (Y(3) - Y(0));
+            turns(0.25 * (X(0) + X(2) + (X(1) + X(3))), 0.25 * (Y(0) + Y(2) + (Y(1) + Y(3))), false,
+                  eq);
+            turns(0.25 * ux, 0.25 * uy, true, eq + 3);
+            turns(0.25 * wx, 0.25 * wy, true, eq + 6);
+            eq[9] = eq[10] = eq[11] = 0.0;
+        } else {
+            for (int i = 0; i < 3; ++i) {
+                eq[i] = -kInvTwoPi * hor[i];
+                eq[3 + i] = -kInvTwoPi * ver[i];
+                eq[9 + i] = 0.0;
+            }
+            turns(0.0, 0.0, false, eq + 6);
         }
-        const double offset = -k_turn * (cx * bd[0] + cy * bd[1] + cz * bd[2]) +
-                              (cls == BEAM_TRAPEZOID || cls == BEAM_VERTICES ? 0.25 : 0.0);
-        const double sing = eps_mixed * k_turn * sqrt(t0x * t0x + t0y * t0y);
+        const double offset = -k_turn * (cx * bd[0] + cy * bd[1] + cz * bd[2]);
+        const double part = kPhasorN * (offset - rint(offset));
+        const double edge = k_node * sqrt(t0x * t0x + t0y * t0y);
         for (int i = 0; i < 3; ++i)
-            eb[EB_DIR + i] = bd[i];
-        eb[EB_PHASE] = (offset - rint(offset)) + kTurnMagic;
+            eb[EB_DIR + i] = kPhasorN * bd[i];
+        eb[EB_PHASE] =
+            part + (cls == BEAM_TRAPEZOID || cls == BEAM_VERTICES ? kPhasorN / 4 : 0) + kNodeMagic;
+        const double sing = eps_mixed * edge;
         eb[EB_LIM] = pack_floats((float)fmax(sing, kLookStep), (float)sing);
-        eb[EB_SCALE] = pack_floats((float)scale, (float)(1.0 / scale));
-        eb[EB_KIND] = pack_words(nv + BEAM_CLASS * cls, ext ? 1 : 0);
+        eb[EB_SCALE] = pack_floats((float)(scale / s64), (float)(1.0 / scale));
+        eb[EB_KIND] = pack_words(nv + BEAM_CLASS * cls, 2 * cls64 + (ext ? 1 : 0));
         eb[EB_VOFF] = __builtin_bit_cast(double, v0);
+        eb[EB_PHASE64] = part + (cls64 == BEAM_TRAPEZOID ? kPhasorN / 4 : 0);
+        eb[EB_S64] = s64;
+        // every vertex phase within 1e-3 rad: half of edge 0's step is within that,
+        // or the projections within the bound below (see H_PHB)
+        const double small = 1.02 * kSmallPhase * (kPhasorN * kInvTwoPi);
+        eb[EB_LOOK64] = cls64 == BEAM_VERTICES   ? h[H_PHB] * kPhasorN
+                        : cls64 == BEAM_PARALLEL ? small
+                                                 : fmax(eps1 * edge, 2.0 * small);
+        eb[EB_SING64] = cls64 == BEAM_VERTICES ? eps1 * k_node * lmax
+                        : cls64 == BEAM_TRAPEZOID ? eps1 * edge : 0.0;
         s_scale[g] = scale;
+        s_s64[g] = s64;
     }
     __syncthreads();
     // the records of the workgroup's beams are contiguous
     for (int i = threadIdx.x; i < count * HDR_STRIDE; i += PACK_THREADS)
         hdr[(size_t)first * HDR_STRIDE + i] = s_h[i];
-    // MFMA operand: W[m][c] = s (T0[m] Jp[0][c] + T1[m] Jp[1][c]) in FP64,
-    // split into three BF16 parts
+    // W[m][c] = T0[m] Jp[0][c] + T1[m] Jp[1][c], T the rotation vectors halved
+    // (exact): column n of beam c
+    const auto rotation = [&](int c, int n, double &wr, double &wi) {
+        const int m = n >> 2, col = (n >> 1) & 1;
+        const double *v = s_bs + c * 36 + (m < 3 ? 13 + m : 16 + m);  // NT NP nxDT nxDP
+        const double t0 = 0.5 * v[0], t1 = 0.5 * v[3], *jp = s_jp[c] + 2 * col;
+        wr = t0 * jp[0] + t1 * jp[4];
+        wi = t0 * jp[1] + t1 * jp[5];
+    };
+    for (int i = threadIdx.x; i < count * W64_STRIDE; i += PACK_THREADS) {
+        const int c = i / W64_STRIDE, n = i - c * W64_STRIDE;
+        double wr, wi;
+        rotation(c, n, wr, wi);
+        w64[(size_t)first * W64_STRIDE + i] = s_s64[c] * ((n & 1) ? wi : wr);
+    }
+    // MFMA operand, split into three BF16 parts
     for (int i = threadIdx.x; i < count * (2 * WB_COLS); i += PACK_THREADS) {
         const int c = i / (2 * WB_COLS), e = i - c * (2 * WB_COLS);
         const int row = e / WB_COLS, n = e - row * WB_COLS;
-        const double *hb = s_h + c * HDR_STRIDE;
-        const int m = n >> 2, col = (n >> 1) & 1;
-        const double t0 = hb[H_T0 + m], t1 = hb[H_T1 + m];
-        const double wr = t0 * hb[H_JP + 2 * col] + t1 * hb[H_JP + 4 + 2 * col];
-        const double wi = t0 * hb[H_JP + 2 * col + 1] + t1 * hb[H_JP + 4 + 2 * col + 1];
+        double wr, wi;
+        rotation(c, n, wr, wi);
         // rows 0 and 1 multiply Re F and Im F / sqrt(2)
         const double w = s_scale[c] * (row == 0 ? ((n & 1) ? wi : wr)
                                                 : 1.41421356237309504880 *
@@ -646,6 +689,12 @@ __device__ __forceinline__ double uniform_f64(double x)
     const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)b);
     const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(b >> 32));
     return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+
+// The edge flags of a vertex, in a scalar register.
+__device__ __forceinline__ int vertex_flags(const double *__restrict__ vx, int e)
+{
+    return __builtin_amdgcn_readfirstlane(low_word(vx[(size_t)e * VX_STRIDE + VX_FLAG]));
 }
 
 // Every vertex phase within 1e-3 rad: the cell takes the small-phase moment
@@ -694,8 +743,7 @@ __device__ __forceinline__ uint64_t edge_valid_mask(int flags, uint64_t mB)
 // contribution (e^{i phi_{e+1}} - e^{i phi_e}) / C, or the exact half-angle
 // form when |C| <= eps1.
 __device__ __forceinline__ void edge_f64(int e, int n, const double *__restrict__ vtx,
-                                         const double *__restrict__ vdd,
-                                         const int32_t *__restrict__ vflag, double A, double B,
+                                         const double *__restrict__ vx, double A, double B,
                                          double psi, bool useB, uint64_t mB,
                                          const double2 *__restrict__ tab, double k,
                                          double eps1, double s0, double c0, double &sp,
@@ -706,7 +754,7 @@ __device__ __forceinline__ void edge_f64(int e, int n, const double *__restrict_
     // (a select between the two loads becomes a divergent branch around each
     // scalar load)
     const double syx = uniform_f64(v[V_SYX]), sxy = uniform_f64(v[V_SXY]);
-    const int f = __builtin_amdgcn_readfirstlane(vflag[e]);
+    const int f = vertex_flags(vx, e);
     double sn = s0, cn = c0;
     if (e + 1 < n) {
         const double xn = __builtin_fma(B, v[VTX_STRIDE + V_KY], psi);
@@ -720,8 +768,8 @@ __device__ __forceinline__ void edge_f64(int e, int n, const double *__restrict_
     sr = __builtin_fma(cn - cp, inv, sr);
     si = __builtin_fma(sn - sp, inv, si);
     if (__builtin_expect(__builtin_amdgcn_inverse_ballot_w64(mvalid & ~mbig) && !small, 0)) {
-        const double *w = vdd + (size_t)e * VDD_STRIDE;
-        const double dd = useB ? uniform_f64(w[D_DX]) : uniform_f64(w[D_DY]);
+        const double *w = vx + (size_t)e * VX_STRIDE;
+        const double dd = useB ? uniform_f64(w[VX_DX]) : uniform_f64(w[VX_DY]);
         const double2 q = stable_edge_quotient(cp, sp, cn, sn, dd, cc, k);
         sr += q.x;
         si += q.y;
@@ -735,7 +783,7 @@ __device__ __forceinline__ void edge_f64(int e, int n, const double *__restrict_
 template <int NV>
 __device__ __forceinline__ void edge_sum_f64_nv(
     const double *syx, const double *sxy, const int *fl, const double *sv, const double *cv,
-    const double *__restrict__ vdd, double A, double B, bool useB, uint64_t mB, double k,
+    const double *__restrict__ vx, double A, double B, bool useB, uint64_t mB, double k,
     double eps1, bool small, double &sr, double &si)
 {
 #pragma unroll
@@ -752,8 +800,8 @@ __device__ __forceinline__ void edge_sum_f64_nv(
         si = __builtin_fma(sv[f] - sv[e], inv, si);
         const bool rare = __builtin_amdgcn_inverse_ballot_w64(mvalid & ~mbig) && !small;
         if (__builtin_expect(rare, 0)) {
-            const double *w = vdd + (size_t)e * VDD_STRIDE;
-            const double dx = uniform_f64(w[D_DX]), dy = uniform_f64(w[D_DY]);
+            const double *w = vx + (size_t)e * VX_STRIDE;
+            const double dx = uniform_f64(w[VX_DX]), dy = uniform_f64(w[VX_DY]);
             const double2 q =
                 stable_edge_quotient(cv[e], sv[e], cv[f], sv[f], useB ? dx : dy, cc, k);
             sr += q.x;
@@ -761,6 +809,10 @@ __device__ __forceinline__ void edge_sum_f64_nv(
         }
     }
 }
+
+// A lane holds its direction d as 1024 d, so that phases come out in nodes.
+constexpr double kNode = 1.0 / kPhasorN;
+static_assert(kPhasorN == kTabN, "both precisions count phases in the same nodes");
 
 // Aperture integral F(beam, direction) / complWave in FP64 (A4).  NV > 0
 // is the vertex count known at compile time (the loops are unrolled, the
@@ -770,15 +822,15 @@ __device__ __forceinline__ void edge_sum_f64_nv(
 template <int NV>
 __device__ __forceinline__ bool aperture_f64(const double *__restrict__ h,
                                              const double *__restrict__ vtx,
-                                             const double *__restrict__ vdd,
-                                             const int32_t *__restrict__ vflag, int nv,
+                                             const double *__restrict__ vx, int nv,
                                              const double *d, const double2 *__restrict__ tab,
                                              double k, double eps1, double &fr, double &fi)
 {
     // A, B: projections of k - k0 = b - d on the aperture axes
-    const double A = h[H_A0] - (d[0] * h[H_HOR] + d[1] * h[H_HOR + 1] + d[2] * h[H_HOR + 2]);
-    const double B = h[H_B0] - (d[0] * h[H_VER] + d[1] * h[H_VER + 1] + d[2] * h[H_VER + 2]);
-    const double psi = d[0] * h[H_KC] + d[1] * h[H_KC + 1] + d[2] * h[H_KC + 2];
+    const double d0 = d[0] * kNode, d1 = d[1] * kNode, d2 = d[2] * kNode;
+    const double A = h[H_A0] - (d0 * h[H_HOR] + d1 * h[H_HOR + 1] + d2 * h[H_HOR + 2]);
+    const double B = h[H_B0] - (d0 * h[H_VER] + d1 * h[H_VER + 1] + d2 * h[H_VER + 2]);
+    const double psi = d0 * h[H_KC] + d1 * h[H_KC + 1] + d2 * h[H_KC + 2];
     const bool useB = __builtin_fabs(B) > __builtin_fabs(A);
     const uint64_t mB = __builtin_amdgcn_ballot_w64(useB);  // lanes summing the dx-valid edges
     // psi is folded into the vertex phasors (the integral is linear in each
@@ -804,7 +856,7 @@ __device__ __forceinline__ bool aperture_f64(const double *__restrict__ h,
         double sv[NV], cv[NV];
 #pragma unroll
         for (int e = 0; e < NV; ++e)
-            sincos_finish(dv[e], ev[e], sv[e], cv[e]);
+            node_finish(dv[e], ev[e], sv[e], cv[e]);
         // the vertex phases one by one only where the beam's bound leaves
         // the small-phase form possible, after the table reads are consumed
         small = false;
@@ -816,9 +868,9 @@ __device__ __forceinline__ bool aperture_f64(const double *__restrict__ h,
         for (int e = 0; e < NV; ++e) {
             syx[e] = uniform_f64(vtx[(size_t)e * VTX_STRIDE + V_SYX]);
             sxy[e] = uniform_f64(vtx[(size_t)e * VTX_STRIDE + V_SXY]);
-            fl[e] = __builtin_amdgcn_readfirstlane(vflag[e]);
+            fl[e] = vertex_flags(vx, e);
         }
-        edge_sum_f64_nv<NV>(syx, sxy, fl, sv, cv, vdd, A, B, useB, mB, k, eps1, small, sr, si);
+        edge_sum_f64_nv<NV>(syx, sxy, fl, sv, cv, vx, A, B, useB, mB, k, eps1, small, sr, si);
     } else {
         small = false;
         if (__builtin_expect(__builtin_fabs(useB ? B : -A) <= h[H_PHB], 0))
@@ -827,8 +879,8 @@ __device__ __forceinline__ bool aperture_f64(const double *__restrict__ h,
         sincos_table(__builtin_fma(A, vtx[V_KX], __builtin_fma(B, vtx[V_KY], psi)), tab, s0, c0);
         double sp = s0, cp = c0;
         for (int e = 0; e < nv; ++e)
-            edge_f64(e, nv, vtx, vdd, vflag, A, B, psi, useB, mB, tab, k, eps1, s0,
-                     c0, sp, cp, sr, si, small);
+            edge_f64(e, nv, vtx, vx, A, B, psi, useB, mB, tab, k, eps1, s0, c0, sp, cp, sr, si,
+                     small);
     }
     const double nrm = rcp_f64(useB ? B : -A);
     fr = sr * nrm;
@@ -849,74 +901,7 @@ __device__ __forceinline__ bool aperture_f64(const double *__restrict__ h,
     return !__builtin_isnan(fr);
 }
 
-// Per-beam aperture integral dispatched on the vertex count (3 and 4 cover
-// most beams of a hexagonal particle).
-__device__ __forceinline__ bool aperture_f64_any(const double *__restrict__ h,
-                                                 const double *__restrict__ vtx,
-                                                 const double *__restrict__ vdd,
-                                                 const int32_t *__restrict__ vflag, int nv,
-                                                 const double *d,
-                                                 const double2 *__restrict__ tab, double k,
-                                                 double eps1, double &fr, double &fi)
-{
-    if (nv == 4)
-        return aperture_f64<4>(h, vtx, vdd, vflag, 4, d, tab, k, eps1, fr, fi);
-    if (nv == 3)
-        return aperture_f64<3>(h, vtx, vdd, vflag, 3, d, tab, k, eps1, fr, fi);
-    return aperture_f64<0>(h, vtx, vdd, vflag, nv, d, tab, k, eps1, fr, fi);
-}
-
-template <int ACC_NS>
-__device__ __forceinline__ void beam_dir_f64(
-    const double *__restrict__ h, const double *__restrict__ vtx,
-    const double *__restrict__ vdd, const int32_t *__restrict__ vflag, int nv,
-    const double *d, const double *__restrict__ su, const double2 *__restrict__ tab,
-    double k, double eps1, double *j, double *jn)
-{
-    double fr, fi;
-    if (!aperture_f64_any(h, vtx, vdd, vflag, nv, d, tab, k, eps1, fr, fi))
-        return;
-    // rotation vectors of this lane's direction, from LDS ([12][256])
-    const int l = threadIdx.x;
-    double u0[6], u1[6];
-    for (int q = 0; q < 6; ++q) {
-        u0[q] = su[q * 256 + l];
-        u1[q] = su[(6 + q) * 256 + l];
-    }
-    const double *T0 = h + H_T0, *T1 = h + H_T1;
-    const double r00 = u0[0] * T0[0] + u0[1] * T0[1] + u0[2] * T0[2] + u0[3] * T0[3] + u0[4] * T0[4] + u0[5] * T0[5];
-    const double r01 = u0[0] * T1[0] + u0[1] * T1[1] + u0[2] * T1[2] + u0[3] * T1[3] + u0[4] * T1[4] + u0[5] * T1[5];
-    const double r10 = u1[0] * T0[0] + u1[1] * T0[1] + u1[2] * T0[2] + u1[3] * T0[3] + u1[4] * T0[4] + u1[5] * T0[5];
-    const double r11 = u1[0] * T1[0] + u1[1] * T1[1] + u1[2] * T1[2] + u1[3] * T1[3] + u1[4] * T1[4] + u1[5] * T1[5];
-    const double *jp = h + H_JP;  // complWave * J_phased
-    // q = R Jp (real 2x2 times complex 2x2), then d = F q
-    double q[8];
-    q[0] = r00 * jp[0] + r01 * jp[4];
-    q[1] = r00 * jp[1] + r01 * jp[5];
-    q[2] = r00 * jp[2] + r01 * jp[6];
-    q[3] = r00 * jp[3] + r01 * jp[7];
-    q[4] = r10 * jp[0] + r11 * jp[4];
-    q[5] = r10 * jp[1] + r11 * jp[5];
-    q[6] = r10 * jp[2] + r11 * jp[6];
-    q[7] = r10 * jp[3] + r11 * jp[7];
-    if constexpr (ACC_NS) {
-        for (int t = 0; t < 4; ++t) {
-            const double dr = fr * q[2 * t] - fi * q[2 * t + 1];
-            const double di = fr * q[2 * t + 1] + fi * q[2 * t];
-            j[2 * t] += dr;
-            j[2 * t + 1] += di;
-            jn[2 * t] += dr;
-            jn[2 * t + 1] += di;
-        }
-    } else {
-        for (int t = 0; t < 4; ++t) {
-            j[2 * t] = __builtin_fma(fr, q[2 * t], __builtin_fma(-fi, q[2 * t + 1], j[2 * t]));
-            j[2 * t + 1] = __builtin_fma(fr, q[2 * t + 1], __builtin_fma(fi, q[2 * t], j[2 * t + 1]));
-        }
-    }
-}
-
-// ---- mixed precision ----------------------------------------------------
+// ---- polygon classes ------------------------------------------------------
 //
 // The aperture integral over a polygon with edges t_e, phases phi_v at its
 // vertices and phase steps D_e = phi_{e+1} - phi_e is, for ANY direction q,
@@ -928,11 +913,10 @@ __device__ __forceinline__ void beam_dir_f64(
 //   F = sum_{e>0} w_e (e^{i phi_{e+1}} - e^{i phi_e}) / D_e / D_0.
 // Nothing but phases at points of the aperture is needed of the direction, so
 // A, B and psi are not formed either: a phase is three FMAs from d - b and a
-// packed vector, its constant term (with the fixed-point offset of kTurnMagic)
-// the accumulator they start from.  And with an edge's middle phase m_e and half
-// step h_e = D_e / 2, (e^{i phi_{e+1}} - e^{i phi_e}) / D_e = i e^{i m_e} sin(h_e)
-// / h_e / 2, which does not cancel as D_e goes to zero: no edge but edge 0 is
-// ever singular.
+// packed vector, its constant term the accumulator they start from.  And with an
+// edge's middle phase m_e and half step h_e = D_e / 2, (e^{i phi_{e+1}} -
+// e^{i phi_e}) / D_e = i e^{i m_e} sin(h_e) / h_e / 2, which does not cancel as
+// D_e goes to zero: no edge but edge 0 is ever singular.
 //
 // An edge parallel to t_0 has no weight, and then the other two edges of a
 // quadrilateral have opposite weights; a triangle is the same with that edge
@@ -940,15 +924,214 @@ __device__ __forceinline__ void beam_dir_f64(
 //   F = 2 i w_1 (e^{i m_1} sin(h_1) / D_1 - e^{i m_l} sin(h_l) / D_l) / D_0,
 // and for a parallelogram with centre phase m
 //   F = -4 w_1 e^{i m} sin(h_0) sin(h_1) / (D_0 D_1).
-// The constants go into the packed W, so these take 60 and 40 vector
-// instructions where the reference's branches (A, B, psi, two FP64 coefficients
-// and a select per edge, an FP64 reduction per vertex) took 109, and other
-// quadrilaterals 95 (137,000 beams of 2,000-15,000 an orientation on 541 x 96
-// directions: 17.3 ms against 27.3 for the kernel, contraction included).  A traced column's beams are 0.32 parallelograms, 0.61
-// trapezoids and triangles; the 8-column aggregate's 0.09 and 0.63.  From five
-// vertices on (shadow beams, 4 to 15 in 100 others) the weights are the
-// reference's dx or dy, by the larger of |A| and |B|, since one edge's own step
-// is too often small against K there.
+// The constants go into the packed W.  A traced column's beams are 0.32
+// parallelograms, 0.61 trapezoids and triangles; the 8-column aggregate's 0.09
+// and 0.63.
+//
+// FP64: a parallelogram takes 112 vector instructions and a trapezoid 138, the
+// sum into G included, where the reference's branches (A, B, psi, two
+// coefficients and a select per edge, four phasors with an extra constant and a
+// longer polynomial each) took 214; other polygons the sum over their vertices with
+// the reference's weights.  35,800 beams of 2,000-15,000 an orientation on 541 x 96
+// directions: 8.8 ms against 12.7 for the kernel, which the vector ALU bounds (150
+// instructions a beam and wave on average; four waves a SIMD leave it 80 % busy).
+// The error against extended precision is 0.25 to 0.4 of the branches'.
+
+// 1/x to full FP64 precision from the hardware estimate e (1 + e + e^2).
+__device__ __forceinline__ double rcp_f64_cubic(double x)
+{
+    const double r = __builtin_amdgcn_rcp(x);
+    const double e = __builtin_fma(-x, r, 1.0);
+    return __builtin_fma(__builtin_fma(e, e, e), r, r);
+}
+
+// F' = sum over the edges of (dx or dy) (e^{i phi_{e+1}} - e^{i phi_e}) / D_e, over
+// b or -a: a polygon that is neither triangle, trapezoid nor parallelogram, by the
+// reference's weights.  `reach` is |b| or |a|, `step` the least |D_e|.
+template <int NV>
+__device__ __forceinline__ void aperture_vertices_f64(const double *__restrict__ h,
+                                                      const double *__restrict__ vtx,
+                                                      const double *__restrict__ vx, int nv,
+                                                      double k0, double k1, double k2,
+                                                      const double *d,
+                                                      const double2 *__restrict__ tab,
+                                                      double &fr, double &fi, double &reach,
+                                                      double &step)
+{
+    const double A = k0 * h[H_HOR] + k1 * h[H_HOR + 1] + k2 * h[H_HOR + 2];
+    const double B = k0 * h[H_VER] + k1 * h[H_VER + 1] + k2 * h[H_VER + 2];
+    const double a = -kInvTwoPi * A, b = -kInvTwoPi * B;
+    const double c = kInvTwoPi * (d[0] * h[H_KC] + d[1] * h[H_KC + 1] + d[2] * h[H_KC + 2]);
+    // the weights over K.q: dx / b, or -dy / a
+    const bool useB = __builtin_fabs(B) > __builtin_fabs(A);
+    const double over = rcp_f64_cubic(useB ? b : -a);
+    const double ux = useB ? over : 0.0, uy = useB ? 0.0 : over;
+    reach = __builtin_fabs(useB ? B : A);
+    const auto vertex = [&](int v, double &p, double &sn, double &cs) {
+        const double *q = vtx + v * VTX_STRIDE;
+        p = __builtin_fma(a, q[V_KX], __builtin_fma(b, q[V_KY], c));
+        double r;
+        double2 e;
+        node_reduce(p, tab, r, e);
+        node_finish(r, e, sn, cs);
+    };
+    double p0, s0, c0;
+    vertex(0, p0, s0, c0);
+    double pp = p0, sp = s0, cp = c0, sr = 0.0, si = 0.0;
+    step = __builtin_inf();
+    const int n = NV > 0 ? NV : nv;
+#pragma unroll
+    for (int e = 0; e < n; ++e) {
+        const double dx = uniform_f64(vx[e * VX_STRIDE + VX_DX]),
+                     dy = uniform_f64(vx[e * VX_STRIDE + VX_DY]);
+        double pn = p0, sn = s0, cn = c0;
+        if (e + 1 < n)
+            vertex(e + 1, pn, sn, cn);
+        const double D = pn - pp;
+        const double w = __builtin_fma(dy, uy, dx * ux) * rcp_f64_cubic(D);
+        sr = __builtin_fma(cn - cp, w, sr);
+        si = __builtin_fma(sn - sp, w, si);
+        step = __builtin_fmin(step, __builtin_fabs(D));
+        pp = pn;
+        sp = sn;
+        cp = cn;
+    }
+    fr = sr;
+    fi = si;
+}
+
+// F' = F / complWave / s of a beam in a direction, s its EB_S64.  Returns the
+// lanes (a mask) whose F is NaN: there the beam does not count (HandlerPO.cpp:2742).
+// Lane conditions are kept as scalar masks: as bools they would cross the
+// blocks in vector registers.
+__device__ __forceinline__ uint64_t aperture_any_f64(const double *eb, const double *__restrict__ h,
+                                                 const double *__restrict__ vtxs,
+                                                 const double *__restrict__ vxs, const double *d,
+                                                 const double2 *__restrict__ tab, double k,
+                                                 double eps1, double &fr, double &fi)
+{
+    const int cls = high_word(eb[EB_KIND]) >> 1;
+    const int nv = low_word(eb[EB_KIND]) & BEAM_NV;
+    const int64_t v0 = __builtin_bit_cast(int64_t, eb[EB_VOFF]);
+    const double *vtx = vtxs + (size_t)v0 * VTX_STRIDE, *vx = vxs + (size_t)v0 * VX_STRIDE;
+    const double k0 = d[0] - eb[EB_DIR], k1 = d[1] - eb[EB_DIR + 1], k2 = d[2] - eb[EB_DIR + 2];
+    const auto half = [&](const double *q) {
+        return __builtin_fma(k2, q[2], __builtin_fma(k1, q[1], k0 * q[0]));
+    };
+    const auto phase = [&](const double *q) {
+        return __builtin_fma(k2, q[2], __builtin_fma(k1, q[1], __builtin_fma(k0, q[0],
+                                                                             eb[EB_PHASE64])));
+    };
+    const double *q = eb + EB_Q;
+    uint64_t look = 0, general = 0, dead = 0;
+    // edge 0's step (the least step), and the divisor, which may be zero without it
+    double step = 1.0, div = 1.0;
+    if (cls == BEAM_TRAPEZOID) {
+        const double m1 = phase(q), h1 = half(q + 3), m3 = phase(q + 6), h3 = half(q + 9);
+        double rm1, rh1, rm3, rh3;
+        double2 em1, eh1, em3, eh3;
+        node_reduce(m1, tab, rm1, em1);
+        node_reduce(h1, tab, rh1, eh1);
+        node_reduce(m3, tab, rm3, em3);
+        node_reduce(h3, tab, rh3, eh3);
+        step = (m1 - m3) - (h1 + h3);
+        div = h1 * h3 * step;
+        const double r = rcp_f64_cubic(div);
+        const double q1 = node_sine(rh1, eh1) * h3, q3 = node_sine(rh3, eh3) * h1;
+        double s1, c1, s3, c3;
+        node_finish(rm1, em1, s1, c1);
+        node_finish(rm3, em3, s3, c3);
+        fr = __builtin_fma(q1, c1, -(q3 * c3)) * r;
+        fi = __builtin_fma(q1, s1, -(q3 * s3)) * r;
+        look = __builtin_amdgcn_ballot_w64(!(__builtin_fabs(step) >= eb[EB_LOOK64])) |
+               __builtin_amdgcn_ballot_w64(div == 0.0);
+    } else if (cls == BEAM_PARALLEL) {
+        const double m = phase(q), h1 = half(q + 6);
+        step = half(q + 3);
+        double rm, r0, r1;
+        double2 em, e0, e1;
+        node_reduce(m, tab, rm, em);
+        node_reduce(step, tab, r0, e0);
+        node_reduce(h1, tab, r1, e1);
+        div = step * h1;
+        const double f = node_sine(r0, e0) * node_sine(r1, e1) * rcp_f64_cubic(div);
+        double s, c;
+        node_finish(rm, em, s, c);
+        fr = c * f;
+        fi = s * f;
+        look = __builtin_amdgcn_ballot_w64(!(__builtin_fabs(step) >= eb[EB_LOOK64])) |
+               __builtin_amdgcn_ballot_w64(div == 0.0);
+    } else if (cls == BEAM_VERTICES) {
+        double reach;
+        if (nv == 4)
+            aperture_vertices_f64<4>(h, vtx, vx, 4, k0, k1, k2, d, tab, fr, fi, reach, step);
+        else
+            aperture_vertices_f64<0>(h, vtx, vx, nv, k0, k1, k2, d, tab, fr, fi, reach, step);
+        look = __builtin_amdgcn_ballot_w64(!(reach > eb[EB_LOOK64])) |
+               __builtin_amdgcn_ballot_w64(!(step > eb[EB_SING64]));
+    } else {
+        general = ~0ull;
+    }
+    // next to a singular edge, and where every phase is small: the branches
+    if (__builtin_expect(look != 0, 0)) {
+        const double A = -kNode * (k0 * h[H_HOR] + k1 * h[H_HOR + 1] + k2 * h[H_HOR + 2]);
+        const double B = -kNode * (k0 * h[H_VER] + k1 * h[H_VER + 1] + k2 * h[H_VER + 2]);
+        const bool leaves = !(__builtin_fabs(step) > eb[EB_SING64]) || div == 0.0 ||
+                            all_phases_small(vtx, nv, A, B);
+        general = look & __builtin_amdgcn_ballot_w64(leaves);
+    }
+    if (__builtin_expect(general != 0, 0)) {
+        bool ok = true;
+        if (__builtin_amdgcn_inverse_ballot_w64(general)) {
+            if (nv == 4)
+                ok = aperture_f64<4>(h, vtx, vx, 4, d, tab, k, eps1, fr, fi);
+            else if (nv == 3)
+                ok = aperture_f64<3>(h, vtx, vx, 3, d, tab, k, eps1, fr, fi);
+            else
+                ok = aperture_f64<0>(h, vtx, vx, nv, d, tab, k, eps1, fr, fi);
+            const double inv = 1.0 / eb[EB_S64];
+            fr *= inv;
+            fi *= inv;
+        }
+        dead = __builtin_amdgcn_ballot_w64(!ok);
+    }
+    return dead;
+}
+
+// G += F' W: entry 4m + 2c + r of G and of W (po_layout.h).
+__device__ __forceinline__ void add_rotated_f64(const double *__restrict__ w, double fr, double fi,
+                                                double *g)
+{
+#pragma unroll
+    for (int n = 0; n < W64_STRIDE; n += 2) {
+        g[n] = __builtin_fma(fr, w[n], __builtin_fma(-fi, w[n + 1], g[n]));
+        g[n + 1] = __builtin_fma(fr, w[n + 1], __builtin_fma(fi, w[n], g[n + 1]));
+    }
+}
+
+// The Jones sum of a lane from its G: J[i][c] = sum_m u_i[m] G[m][c]; entry m of u0,
+// u1 at m * ld.
+__device__ __forceinline__ void add_jones(const double *g, const double *u, size_t ld, double *j)
+{
+#pragma unroll
+    for (int m = 0; m < 12; ++m) {
+        const double um = u[m * ld];
+        for (int n = 0; n < 4; ++n)
+            j[4 * (m / 6) + n] = __builtin_fma(um, g[4 * (m % 6) + n], j[4 * (m / 6) + n]);
+    }
+}
+
+// ---- mixed precision ----------------------------------------------------
+//
+// The polygon classes above, with phases in fixed-point nodes (the constant term
+// of a phase carries the offset kNodeMagic) and FP32 phasors.  Trapezoids take 60
+// and parallelograms 40 vector instructions, where the reference's branches (A,
+// B, psi, two FP64 coefficients and a select per edge, an FP64 reduction per
+// vertex) took 109, and other quadrilaterals 100 (137,000 beams of 2,000-15,000
+// an orientation on 541 x 96 directions: 17.3 ms against 27.3 for the kernel,
+// contraction included).  From five vertices on (shadow beams, 4 to 15 in 100
+// others) the weights are the reference's dx or dy, by the larger of |A| and |B|,
+// since one edge's own step is too often small against K there.
 //
 // Lanes where D_0 is small leave the sums: fix_lanes below.  Forms that were
 // shorter and lost precision: one coefficient per vertex, X_v / (D_{v-1} D_v)
@@ -957,15 +1140,14 @@ __device__ __forceinline__ void beam_dir_f64(
 
 // The moment form: F of a cell whose vertex phases are all within
 // kSmallPhaseMixed: <e^{i phi}> = sum_n i^n <phi^n> / n! to
-// seventh order, times the area limit and e^{i psi}.  Returns Re F and
+// fifth order, times the area limit and e^{i psi}.  Returns Re F and
 // Im F / sqrt(2).
 __device__ __forceinline__ void moments_mixed(const double *__restrict__ h, double A, double B,
                                               double psi, const PhasorNode *__restrict__ tab,
                                               float &out_r, float &out_s)
 {
     const double A2 = A * A, B2 = B * B, AB = A * B;
-    const double *c3 = h + H_MOM3, *c4 = h + H_MOM4, *c5 = h + H_MOM5, *c6 = h + H_MOM6,
-                 *c7 = h + H_MOM7;
+    const double *c3 = h + H_MOM3, *c4 = h + H_MOM4, *c5 = h + H_MOM5;
     const double p1 = A * h[H_MOM] + B * h[H_MOM + 1];
     const double p2 = A2 * h[H_MOM + 2] + AB * h[H_MOM + 3] + B2 * h[H_MOM + 4];
     const double q3 = B * (B2 * c3[0] + AB * c3[1]) + A * (AB * c3[2] + A2 * c3[3]);
@@ -974,12 +1156,7 @@ __device__ __forceinline__ void moments_mixed(const double *__restrict__ h, doub
     const double A3 = A * A2, B3 = B * B2;
     const double q5 = B3 * (B2 * c5[0] + AB * c5[1] + A2 * c5[2]) +
                       A3 * (B2 * c5[3] + AB * c5[4] + A2 * c5[5]);
-    const double q6 = B3 * (B3 * c6[0] + A * (B2 * c6[1] + AB * c6[2])) +
-                      A3 * (B3 * c6[3] + A * (B2 * c6[4] + AB * c6[5] + A2 * c6[6]));
-    const double q7 =
-        B2 * B2 * (B3 * c7[0] + A * (B2 * c7[1] + AB * c7[2] + A2 * c7[3])) +
-        A2 * A2 * (B3 * c7[4] + A * (B2 * c7[5] + AB * c7[6] + A2 * c7[7]));
-    const double gr = 1.0 - 0.5 * p2 + (q4 - q6), gi = p1 - q3 + (q5 - q7);
+    const double gr = 1.0 - 0.5 * p2 + q4, gi = p1 - q3 + q5;
     const float ar = (float)(h[H_AL] * gr - h[H_AL + 1] * gi);
     const float ai = (float)(h[H_AL] * gi + h[H_AL + 1] * gr);
     float c, s;
@@ -989,13 +1166,12 @@ __device__ __forceinline__ void moments_mixed(const double *__restrict__ h, doub
 }
 
 // The edge sum over the reference's branches, as the ABI's slopes and flags
-// define it, for any vertex count and any phase: beams of class BEAM_GENERAL,
+// define it, for any vertex count and any phase: beams of class BEAM_SLOPES,
 // and single lanes of other beams next to a singular edge.  The edge
 // coefficient is cancellation-prone and stays in FP64; edges with |C| <=
 // eps1 take the half-angle form.
 __device__ __forceinline__ void edges_mixed(const double *__restrict__ vtx,
-                                            const double *__restrict__ vdd,
-                                            const int32_t *__restrict__ vflag, int nv, double A,
+                                            const double *__restrict__ vx, int nv, double A,
                                             double B, double psi,
                                             const PhasorNode *__restrict__ tab, double k,
                                             double eps1, float &out_r, float &out_s)
@@ -1008,7 +1184,7 @@ __device__ __forceinline__ void edges_mixed(const double *__restrict__ vtx,
     for (int e = 0; e < nv; ++e) {
         const double *v = vtx + (size_t)e * VTX_STRIDE;
         const double syx = uniform_f64(v[V_SYX]), sxy = uniform_f64(v[V_SXY]);
-        const int f = __builtin_amdgcn_readfirstlane(vflag[e]);
+        const int f = vertex_flags(vx, e);
         float cn = c0, sn = s0;
         if (e + 1 < nv) {
             const double xn = __builtin_fma(B, v[VTX_STRIDE + V_KY], psi);
@@ -1022,8 +1198,8 @@ __device__ __forceinline__ void edges_mixed(const double *__restrict__ vtx,
         sr = __builtin_fmaf(cn - cp, inv, sr);
         ss = __builtin_fmaf(sn - sp, inv, ss);
         if (__builtin_expect(!big && (f & vmask) != 0, 0)) {
-            const double *w = vdd + (size_t)e * VDD_STRIDE;
-            const double dd = useB ? uniform_f64(w[D_DX]) : uniform_f64(w[D_DY]);
+            const double *w = vx + (size_t)e * VX_STRIDE;
+            const double dd = useB ? uniform_f64(w[VX_DX]) : uniform_f64(w[VX_DY]);
             const double2 q = stable_edge_quotient((double)cp, (double)(sp * kSqrt2), (double)cn,
                                                    (double)(sn * kSqrt2), dd, cc, k);
             sr += (float)q.x;
@@ -1042,21 +1218,21 @@ __device__ __forceinline__ void edges_mixed(const double *__restrict__ vtx,
 // edge, and every lane of a BEAM_SLOPES beam, by the reference's branches.
 __device__ __forceinline__ void fix_lanes(const double *eb, const double *__restrict__ h,
                                           const double *__restrict__ vtx,
-                                          const double *__restrict__ vdd,
-                                          const int32_t *__restrict__ vflag, int nv, int cls,
+                                          const double *__restrict__ vx, int nv, int cls,
                                           const double *d, bool singular, bool maybe,
                                           const PhasorNode *__restrict__ tab, double k,
                                           double eps1, float &out_r, float &out_s)
 {
     // A, B: projections of k - k0 = b - d on the aperture axes
-    const double k0 = eb[EB_DIR] - d[0], k1 = eb[EB_DIR + 1] - d[1], k2 = eb[EB_DIR + 2] - d[2];
+    const double k0 = kNode * (eb[EB_DIR] - d[0]), k1 = kNode * (eb[EB_DIR + 1] - d[1]),
+                 k2 = kNode * (eb[EB_DIR + 2] - d[2]);
     const double A = k0 * h[H_HOR] + k1 * h[H_HOR + 1] + k2 * h[H_HOR + 2];
     const double B = k0 * h[H_VER] + k1 * h[H_VER + 1] + k2 * h[H_VER + 2];
-    const double psi = d[0] * h[H_KC] + d[1] * h[H_KC + 1] + d[2] * h[H_KC + 2];
+    const double psi = kNode * (d[0] * h[H_KC] + d[1] * h[H_KC + 1] + d[2] * h[H_KC + 2]);
     const bool small =
         maybe && (cls == BEAM_MOMENTS || all_phases_small(vtx, nv, A, B, kSmallPhaseMixed));
     if (singular && !small)
-        edges_mixed(vtx, vdd, vflag, nv, A, B, psi, tab, k, eps1, out_r, out_s);
+        edges_mixed(vtx, vx, nv, A, B, psi, tab, k, eps1, out_r, out_s);
     if (small)
         moments_mixed(h, A, B, psi, tab, out_r, out_s);
     if (singular || small) {
@@ -1068,30 +1244,30 @@ __device__ __forceinline__ void fix_lanes(const double *eb, const double *__rest
     }
 }
 
-// sin(2 pi f) / sqrt(2) / f from the series, for a small half step f.
+// sin(h) / sqrt(2) / f from the series, for a small half step of f nodes (h rad).
 __device__ __forceinline__ float sine_ratio_series(float f)
 {
-    const float x = 6.28318530717958648f * f, z = x * x;
-    return 4.44288293815836625f *
+    const float x = (float)(6.28318530717958648 / kPhasorN) * f, z = x * x;
+    return (float)(4.44288293815836625 / kPhasorN) *
            __builtin_fmaf(z, __builtin_fmaf(z, 1.0f / 120.0f, -1.0f / 6.0f), 1.0f);
 }
 
 // Triangles and trapezoids.
 __device__ __forceinline__ void aperture_trapezoid(const double *eb, const double *d,
                                                    const PhasorNode *__restrict__ tab,
-                                                   float &out_r, float &out_s, bool &singular,
-                                                   bool &maybe)
+                                                   float &out_r, float &out_s,
+                                                   uint64_t &singular, uint64_t &maybe)
 {
     const double k0 = d[0] - eb[EB_DIR], k1 = d[1] - eb[EB_DIR + 1], k2 = d[2] - eb[EB_DIR + 2];
     const auto phase = [&](const double *q, double c) {
         return __builtin_fma(k2, q[2], __builtin_fma(k1, q[1], __builtin_fma(k0, q[0], c)));
     };
     const double *q = eb + EB_Q;
-    const double m1 = phase(q, eb[EB_PHASE]), a1 = phase(q + 3, kTurnMagic);
-    const double m3 = phase(q + 6, eb[EB_PHASE]), a3 = phase(q + 9, kTurnMagic);
+    const double m1 = phase(q, eb[EB_PHASE]), a1 = phase(q + 3, kNodeMagic);
+    const double m3 = phase(q + 6, eb[EB_PHASE]), a3 = phase(q + 9, kNodeMagic);
     const PhasorNode em1 = phasor_read(low_bits(m1), tab), ea1 = phasor_read(low_bits(a1), tab),
                      em3 = phasor_read(low_bits(m3), tab), ea3 = phasor_read(low_bits(a3), tab);
-    const double h1 = a1 - kTurnMagic, h3 = a3 - kTurnMagic;
+    const double h1 = a1 - kNodeMagic, h3 = a3 - kNodeMagic;
     const float f1 = (float)h1, f3 = (float)h3;
     const float step = (float)((m1 - m3) - (h1 + h3));  // edge 0
     const float r0 = __builtin_amdgcn_rcpf(step);
@@ -1110,9 +1286,11 @@ __device__ __forceinline__ void aperture_trapezoid(const double *eb, const doubl
     out_s = __builtin_fmaf(q1, s1, -(q3 * s3)) * r0;
     const bool look = !(__builtin_fabsf(step) >= low_float(eb[EB_LIM]));
     if (__builtin_expect(__builtin_amdgcn_ballot_w64(look) != 0, 0)) {
-        singular = !(__builtin_fabsf(step) >= high_float(eb[EB_LIM]));
-        maybe = look &&
-                __builtin_fmaxf(__builtin_fabsf(f1), __builtin_fabsf(f3)) <= (float)kLookStep;
+        singular =
+            __builtin_amdgcn_ballot_w64(!(__builtin_fabsf(step) >= high_float(eb[EB_LIM])));
+        maybe = __builtin_amdgcn_ballot_w64(
+            look &&
+            __builtin_fmaxf(__builtin_fabsf(f1), __builtin_fabsf(f3)) <= (float)kLookStep);
     }
 }
 
@@ -1126,10 +1304,10 @@ __device__ __forceinline__ void aperture_parallelogram(const double *eb, const d
         return __builtin_fma(k2, q[2], __builtin_fma(k1, q[1], __builtin_fma(k0, q[0], c)));
     };
     const double m = phase(eb + EB_Q, eb[EB_PHASE]);
-    const double a0 = phase(eb + EB_Q + 3, kTurnMagic), a1 = phase(eb + EB_Q + 6, kTurnMagic);
+    const double a0 = phase(eb + EB_Q + 3, kNodeMagic), a1 = phase(eb + EB_Q + 6, kNodeMagic);
     const PhasorNode em = phasor_read(low_bits(m), tab), e0 = phasor_read(low_bits(a0), tab),
                      e1 = phasor_read(low_bits(a1), tab);
-    const float f0 = (float)(a0 - kTurnMagic), f1 = (float)(a1 - kTurnMagic);
+    const float f0 = (float)(a0 - kNodeMagic), f1 = (float)(a1 - kNodeMagic);
     float c, s;
     phasor_finish(low_bits(m), em, c, s);
     const float s0 = sine_finish(low_bits(a0), e0), s1 = sine_finish(low_bits(a1), e1);
@@ -1151,15 +1329,15 @@ __device__ __forceinline__ void aperture_parallelogram(const double *eb, const d
     out_s = q * s;
 }
 
-// One edge's (cos, sin / sqrt 2) of the middle phase and sin(2 pi h) / sqrt(2) / h
-// of its half step h, from the phases p, n (with kTurnMagic) of its ends.
+// One edge's (cos, sin / sqrt 2) of the middle phase and sin / sqrt(2) / f of its
+// half step, f nodes, from the phases p, n (with kNodeMagic) of its ends.
 __device__ __forceinline__ void edge_terms(double p, double n,
                                            const PhasorNode *__restrict__ tab, float &c,
                                            float &s, float &q, float &f)
 {
-    const double m = 0.5 * (p + n), a = __builtin_fma(0.5, n - p, kTurnMagic);
+    const double m = 0.5 * (p + n), a = __builtin_fma(0.5, n - p, kNodeMagic);
     const PhasorNode em = phasor_read(low_bits(m), tab), ea = phasor_read(low_bits(a), tab);
-    f = (float)(a - kTurnMagic);
+    f = (float)(a - kNodeMagic);
     phasor_finish(low_bits(m), em, c, s);
     q = sine_finish(low_bits(a), ea) * __builtin_amdgcn_rcpf(f);
     const bool series = __builtin_fabsf(f) < kSeriesStep;
@@ -1167,27 +1345,43 @@ __device__ __forceinline__ void edge_terms(double p, double n,
         q = series ? sine_ratio_series(f) : q;
 }
 
-// The sum over edge 0 for the other quadrilaterals.
-__device__ __forceinline__ void aperture_quad(const double *eb, const double *__restrict__ ev,
-                                              const double *d,
-                                              const PhasorNode *__restrict__ tab, float &out_r,
-                                              float &out_s, bool &singular, bool &maybe)
+// The projections -A / 2 pi, -B / 2 pi ... of d - b for the classes with vertices:
+// a vertex's phase is a k x + b k y + c.
+struct Projection {
+    double a, b, c;
+};
+__device__ __forceinline__ Projection project(const double *eb, const double *d)
 {
     const double k0 = d[0] - eb[EB_DIR], k1 = d[1] - eb[EB_DIR + 1], k2 = d[2] - eb[EB_DIR + 2];
+    const double *q = eb + EB_Q;
+    return {__builtin_fma(k2, q[2], __builtin_fma(k1, q[1], k0 * q[0])),
+            __builtin_fma(k2, q[5], __builtin_fma(k1, q[4], k0 * q[3])),
+            __builtin_fma(k2, q[8], __builtin_fma(k1, q[7], __builtin_fma(k0, q[6],
+                                                                          eb[EB_PHASE])))};
+}
+__device__ __forceinline__ double vertex_phase(const Projection &p, const double *v)
+{
+    return __builtin_fma(p.a, v[V_KX], __builtin_fma(p.b, v[V_KY], p.c));
+}
+
+// The sum over edge 0 for the other quadrilaterals.
+__device__ __forceinline__ void aperture_quad(const double *eb, const double *__restrict__ vtx,
+                                              const double *__restrict__ vx, const double *d,
+                                              const PhasorNode *__restrict__ tab, float &out_r,
+                                              float &out_s, uint64_t &singular, uint64_t &maybe)
+{
+    const Projection p = project(eb, d);
     double ph[4];
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        const double *q = ev + v * EV_STRIDE;
-        ph[v] = __builtin_fma(k2, q[2], __builtin_fma(k1, q[1], __builtin_fma(k0, q[0],
-                                                                              eb[EB_PHASE])));
-    }
+    for (int v = 0; v < 4; ++v)
+        ph[v] = vertex_phase(p, vtx + v * VTX_STRIDE);
     const float step = (float)(ph[1] - ph[0]);
     float sr = 0.0f, ss = 0.0f, legs = 0.0f;
 #pragma unroll
     for (int e = 1; e < 4; ++e) {
         float c, s, q, f;
         edge_terms(ph[e], ph[(e + 1) % 4], tab, c, s, q, f);
-        const float coef = q * low_float(ev[e * EV_STRIDE + EV_W]);
+        const float coef = q * low_float(vx[e * VX_STRIDE + VX_W]);
         sr = __builtin_fmaf(c, coef, sr);
         ss = __builtin_fmaf(s, coef, ss);
         legs = __builtin_fmaxf(legs, __builtin_fabsf(f));
@@ -1195,34 +1389,29 @@ __device__ __forceinline__ void aperture_quad(const double *eb, const double *__
     const float r0 = __builtin_amdgcn_rcpf(step);
     out_r = sr * r0;
     out_s = ss * r0;
-    singular = !(__builtin_fabsf(step) >= high_float(eb[EB_LIM]));
-    maybe = __builtin_fmaxf(legs, __builtin_fabsf(step)) <= (float)kLookStep;
+    singular = __builtin_amdgcn_ballot_w64(!(__builtin_fabsf(step) >= high_float(eb[EB_LIM])));
+    maybe = __builtin_amdgcn_ballot_w64(__builtin_fmaxf(legs, __builtin_fabsf(step)) <=
+                                        (float)kLookStep);
 }
 
 // Five vertices and more, one at a time, with the reference's weights.
-__device__ __forceinline__ void aperture_loop(const double *eb, const double *__restrict__ ev,
-                                              const double *__restrict__ h, int nv,
+__device__ __forceinline__ void aperture_loop(const double *eb, const double *__restrict__ vtx,
+                                              const double *__restrict__ vx, int nv,
                                               const double *d,
                                               const PhasorNode *__restrict__ tab, float &out_r,
-                                              float &out_s, bool &maybe)
+                                              float &out_s, uint64_t &maybe)
 {
-    const double k0 = d[0] - eb[EB_DIR], k1 = d[1] - eb[EB_DIR + 1], k2 = d[2] - eb[EB_DIR + 2];
-    const double base = eb[EB_PHASE];
-    const float A = -(float)(k0 * h[H_HOR] + k1 * h[H_HOR + 1] + k2 * h[H_HOR + 2]);
-    const float B = -(float)(k0 * h[H_VER] + k1 * h[H_VER + 1] + k2 * h[H_VER + 2]);
-    const bool useB = __builtin_fabsf(B) > __builtin_fabsf(A);
-    const double p0 = __builtin_fma(k2, ev[2], __builtin_fma(k1, ev[1],
-                                                             __builtin_fma(k0, ev[0], base)));
+    const Projection p = project(eb, d);
+    const bool useB = __builtin_fabs(p.b) > __builtin_fabs(p.a);
+    const double p0 = vertex_phase(p, vtx);
     double pp = p0;
     float sr = 0.0f, ss = 0.0f, steps = 0.0f;
     for (int e = 0; e < nv; ++e) {
-        const double *q = ev + e * EV_STRIDE;
-        const float wx = low_float(q[EV_W]), wy = high_float(q[EV_W]);
+        const double w = vx[e * VX_STRIDE + VX_W];
+        const float wx = low_float(w), wy = high_float(w);
         double pn = p0;
-        if (e + 1 < nv) {
-            q += EV_STRIDE;
-            pn = __builtin_fma(k2, q[2], __builtin_fma(k1, q[1], __builtin_fma(k0, q[0], base)));
-        }
+        if (e + 1 < nv)
+            pn = vertex_phase(p, vtx + (e + 1) * VTX_STRIDE);
         float c, s, ratio, f;
         edge_terms(pp, pn, tab, c, s, ratio, f);
         const float coef = ratio * (useB ? wx : wy);
@@ -1231,45 +1420,45 @@ __device__ __forceinline__ void aperture_loop(const double *eb, const double *__
         steps = __builtin_fmaxf(steps, __builtin_fabsf(f));
         pp = pn;
     }
-    const float r = __builtin_amdgcn_rcpf(useB ? B : A);
+    const float r = __builtin_amdgcn_rcpf((float)(useB ? p.b : p.a));
     out_r = sr * r;
     out_s = ss * r;
-    maybe = steps <= (float)kLookStep;
+    maybe = __builtin_amdgcn_ballot_w64(steps <= (float)kLookStep);
 }
 
-// F' = F / complWave / s of a beam in a direction, s its EB_SCALE, mixed
-// precision: FP64 phases and moments, FP32 phasors and sums.  eb: the beam's
-// record (in registers), v0 its vertex offset.  Returns the real part and the
-// imaginary part / sqrt(2).
-__device__ __forceinline__ void aperture_mixed(
-    const double *eb, const double *__restrict__ evert, const double *__restrict__ h,
-    const double *__restrict__ vtxs, const double *__restrict__ vdds,
-    const int32_t *__restrict__ vflags, const double *d, const PhasorNode *__restrict__ tab,
-    double k, double eps1, float &out_r, float &out_s)
+// F' = F / complWave / s of a beam in a direction, s = 1 / the second half of its
+// EB_SCALE, mixed precision: FP64 phases and moments, FP32 phasors and sums.  eb: the
+// beam's record (in registers).  Returns the real part and the imaginary part /
+// sqrt(2).
+__device__ __forceinline__ void aperture_mixed(const double *eb, const double *__restrict__ h,
+                                               const double *__restrict__ vtxs,
+                                               const double *__restrict__ vxs, const double *d,
+                                               const PhasorNode *__restrict__ tab, double k,
+                                               double eps1, float &out_r, float &out_s)
 {
     const int kind = low_word(eb[EB_KIND]);
     const int nv = kind & BEAM_NV, cls = kind / BEAM_CLASS;
     const int64_t v0 = __builtin_bit_cast(int64_t, eb[EB_VOFF]);
-    bool singular = false, maybe = false;
+    const double *vtx = vtxs + (size_t)v0 * VTX_STRIDE, *vx = vxs + (size_t)v0 * VX_STRIDE;
+    uint64_t singular = 0, maybe = 0;  // lanes
     out_r = out_s = 0.0f;
     if (cls == BEAM_TRAPEZOID) {
         aperture_trapezoid(eb, d, tab, out_r, out_s, singular, maybe);
     } else if (cls == BEAM_PARALLEL) {
         aperture_parallelogram(eb, d, tab, out_r, out_s);
     } else if (cls == BEAM_VERTICES) {
-        const double *ev = evert + (size_t)v0 * EV_STRIDE;
         if (nv == 4)
-            aperture_quad(eb, ev, d, tab, out_r, out_s, singular, maybe);
+            aperture_quad(eb, vtx, vx, d, tab, out_r, out_s, singular, maybe);
         else
-            aperture_loop(eb, ev, h, nv, d, tab, out_r, out_s, maybe);
+            aperture_loop(eb, vtx, vx, nv, d, tab, out_r, out_s, maybe);
     } else {
-        singular = cls == BEAM_SLOPES;
-        maybe = true;
+        singular = cls == BEAM_SLOPES ? ~0ull : 0;
+        maybe = ~0ull;
     }
-    if (__builtin_expect(__builtin_amdgcn_ballot_w64(singular || maybe) != 0, 0)) {
-        if (singular || maybe)
-            fix_lanes(eb, h, vtxs + (size_t)v0 * VTX_STRIDE, vdds + (size_t)v0 * VDD_STRIDE,
-                      vflags + v0, nv, cls, d, singular, maybe, tab, k, eps1, out_r, out_s);
+    if (__builtin_expect((singular | maybe) != 0, 0)) {
+        if (__builtin_amdgcn_inverse_ballot_w64(singular | maybe))
+            fix_lanes(eb, h, vtx, vx, nv, cls, d, __builtin_amdgcn_inverse_ballot_w64(singular),
+                      __builtin_amdgcn_inverse_ballot_w64(maybe), tab, k, eps1, out_r, out_s);
     }
 }
 
@@ -1277,40 +1466,52 @@ __device__ __forceinline__ void aperture_mixed(
 struct BeamRecord {
     double v[EB_STRIDE];
 };
-__device__ __forceinline__ BeamRecord load_record(const double *__restrict__ ebeam, int64_t b)
+__device__ __forceinline__ BeamRecord load_record(const double *__restrict__ eb)
 {
     BeamRecord r;
     for (int i = 0; i < EB_STRIDE; ++i)
-        r.v[i] = ebeam[(size_t)b * EB_STRIDE + i];
+        r.v[i] = eb[i];
     return r;
 }
 
-// Adds F times R Jp to j[8]: the rotation and the sum on the vector ALU, the
-// beam's rotation data converted from its FP64 header; fr, fs as
-// aperture_mixed returns them, scale the beam's F / F'.
-__device__ __forceinline__ void rotate_add_mixed(const double *__restrict__ h,
-                                                 const float *u0, const float *u1, float scale,
-                                                 float fr, float fs, float *j)
-{
-    const float fi = fs * (kSqrt2 * scale);
-    fr *= scale;
-    float r[2][2] = {{0, 0}, {0, 0}};  // r[i][m]: u_i . T_m
-    for (int q = 0; q < 6; ++q) {
-        const float t0 = (float)h[H_T0 + q], t1 = (float)h[H_T1 + q];
-        r[0][0] = __builtin_fmaf(u0[q], t0, r[0][0]);
-        r[0][1] = __builtin_fmaf(u0[q], t1, r[0][1]);
-        r[1][0] = __builtin_fmaf(u1[q], t0, r[1][0]);
-        r[1][1] = __builtin_fmaf(u1[q], t1, r[1][1]);
+// One word of each cache line of a beam's W: brings it into the scalar cache a
+// beam ahead.  W (48 registers) and the next record (40) do not fit the scalar
+// registers together, so W is read in three parts, each of them waited for; from
+// L2 these waits were 6 % of the FP64 kernel's time.  `arrived` ends it.
+struct Lines {
+    float v[3];
+    __device__ __forceinline__ void touch(const double *__restrict__ w)
+    {
+        for (int i = 0; i < 3; ++i)
+            v[i] = *reinterpret_cast<const float *>(w + 8 * i);
     }
-    for (int i = 0; i < 2; ++i)
-        for (int c = 0; c < 2; ++c) {
-            const double *p = h + H_JP + 2 * c;  // complWave * J_phased
-            const float qr = r[i][0] * (float)p[0] + r[i][1] * (float)p[4];
-            const float qi = r[i][0] * (float)p[1] + r[i][1] * (float)p[5];
-            float *o = j + 2 * (2 * i + c);
-            o[0] = __builtin_fmaf(fr, qr, __builtin_fmaf(-fi, qi, o[0]));
-            o[1] = __builtin_fmaf(fr, qi, __builtin_fmaf(fi, qr, o[1]));
+    __device__ __forceinline__ void arrived() const
+    {
+        asm volatile("" ::"s"(v[0]), "s"(v[1]), "s"(v[2]));
+    }
+};
+static_assert(W64_STRIDE == 24, "three lines of 64 bytes");
+
+// Adds F R Jp to j[8], w the beam's rotation data, u (entry m at m * ld) the lane's
+// rotation vectors u0, u1; a loop, to hold few registers.
+template <typename T>
+__device__ __forceinline__ void rotate_add(const double *__restrict__ w, const T *u, size_t ld,
+                                           T fr, T fi, T *j)
+{
+    T q[8] = {0, 0, 0, 0, 0, 0, 0, 0};  // R Jp
+#pragma unroll 1
+    for (int m = 0; m < 6; ++m) {
+        const T u0 = u[m * ld], u1 = u[(6 + m) * ld];
+        for (int n = 0; n < 4; ++n) {
+            const T wn = (T)w[4 * m + n];
+            q[n] = u0 * wn + q[n];
+            q[4 + n] = u1 * wn + q[4 + n];
         }
+    }
+    for (int n = 0; n < 8; n += 2) {
+        j[n] = fr * q[n] + (j[n] - fi * q[n + 1]);
+        j[n + 1] = fr * q[n + 1] + (j[n + 1] + fi * q[n]);
+    }
 }
 
 // XCD-aware block -> (item, tile): consecutive workgroup ids land on the 8
@@ -1435,14 +1636,11 @@ struct KernelArgs {
     const double *hdr;       // [n_beams][HDR_STRIDE]
     const uint32_t *wb;      // [n_beams][WB_STRIDE]
     const double *ebeam;     // [n_beams][EB_STRIDE]
-    const double *evert;     // [n_vert][EV_STRIDE]
+    const double *w64;       // [n_beams][W64_STRIDE]
     const PhasorNode *phasor;  // [kPhasorN] phasor nodes of the mixed kernels
+    const double2 *turns;    // [kTabN] phasors of the FP64 kernels
     const double *vtx;       // [n_vert][VTX_STRIDE]
-    const double *vdd;       // [n_vert][VDD_STRIDE]
-    const int32_t *vflag;    // [n_vert]
-    const int32_t *nv;       // [n_beams]
-    const int64_t *voff;     // [n_beams+1]
-    const int32_t *ext;      // [n_beams]
+    const double *vx;        // [n_vert][VX_STRIDE]
     const int64_t *ooff;     // [n_orient+1]
     const double *weights;   // [n_orient]
     double k, eps1;
@@ -1483,28 +1681,30 @@ __device__ __forceinline__ void flush_mueller(const T *j, double w, double *dst,
 // All pointers are separate __restrict__ kernel arguments: the per-orientation
 // stores into `out` must be provably disjoint from the beam records for the
 // compiler to keep reading those through the scalar cache.
+//
+// FP64 (PREC 0): the sum is kept in the directions' frame, G[m][c] += F W[m][c]
+// (24 FP64 accumulators, 48 FMAs a beam with W in scalar registers), and turned
+// into the Jones sum once per orientation or segment.  Rotating each beam (R =
+// u . T, R Jp, F R Jp) took 56 and twelve LDS reads.  PREC 1, the mixed kernel on
+// the vector ALU: FP32 sums, each beam rotated.
 template <int PREC, int NS, int JONES, int PER, int QUEUE>
 __global__ __launch_bounds__(256) MBS_OCCUPANCY void diffract_kernel(
     const WorkItem *__restrict__ items, int n_items, int n_tiles, int cells, int n_az,
     const double *__restrict__ tab, const double *__restrict__ hdr,
-    const double *__restrict__ vtx,
-    const double *__restrict__ vdd, const int32_t *__restrict__ vflag,
-    const int32_t *__restrict__ nv,
-    const int64_t *__restrict__ voff, const int32_t *__restrict__ ext,
-    const int64_t *__restrict__ ooff, const double *__restrict__ weights, double k,
-    double eps1, double *__restrict__ out, double *__restrict__ out_ns,
-    double *__restrict__ per_orient, int *__restrict__ queue, const float *__restrict__ tab32,
-    const double *__restrict__ ebeam, const double *__restrict__ evert,
-    const PhasorNode *__restrict__ phasor)
+    const double *__restrict__ w64, const double *__restrict__ vtx,
+    const double *__restrict__ vx, const double *__restrict__ ebeam,
+    const PhasorNode *__restrict__ phasor, const double2 *__restrict__ turns,
+    const int64_t *__restrict__ ooff, const double *__restrict__ weights, double k, double eps1,
+    double *__restrict__ out, double *__restrict__ out_ns, double *__restrict__ per_orient,
+    int *__restrict__ queue, const float *__restrict__ tab32)
 {
     using U = typename std::conditional<PREC == 1, float, double>::type;
     using U2 = typename std::conditional<PREC == 1, PhasorNode, double2>::type;
-    // LDS: this lane's rotation vectors u0, u1 ([12][256], read once per beam
-    // after the vertex loop instead of occupying 12-24 VGPRs through it) and
-    // the phasor table (1024 FP32 nodes, 256 FP64 ones)
+    // LDS: the phasor table (1024 entries of 16 bytes), and the sums over the
+    // shadow beams of an orientation (NS), a column per lane
     constexpr int TN = PREC == 1 ? kPhasorN : kTabN;
-    __shared__ U s_u[12 * 256];
     __shared__ U2 s_tab[TN];
+    __shared__ U s_jx[NS ? 8 * 256 : 1];
     __shared__ int s_unit;
     int item = 0, tile = 0;
     if constexpr (!QUEUE) {
@@ -1512,14 +1712,12 @@ __global__ __launch_bounds__(256) MBS_OCCUPANCY void diffract_kernel(
             return;
     }
     for (int i = threadIdx.x; i < TN; i += blockDim.x) {
-        if constexpr (PREC == 1) {
+        if constexpr (PREC == 1)
             s_tab[i] = phasor[i];
-        } else {
-            double ts, tc;
-            sincospi((double)i / (TN / 2), &ts, &tc);
-            s_tab[i] = make_double2(tc, ts);
-        }
+        else
+            s_tab[i] = turns[i];
     }
+    __syncthreads();
     QueueCursor qc;
     for (;;) {
     if constexpr (QUEUE) {
@@ -1531,14 +1729,25 @@ __global__ __launch_bounds__(256) MBS_OCCUPANCY void diffract_kernel(
     const int c = live ? cell : cells - 1;  // dead lanes compute, never store
     double d[3];
     for (int q = 0; q < 3; ++q)
-        d[q] = tab[(size_t)(DT_DIR + q) * cells + c];
-    for (int q = 0; q < 12; ++q) {
-        if constexpr (PREC == 1)
-            s_u[q * 256 + threadIdx.x] = tab32[(size_t)c * DT32_COUNT + q];
-        else
-            s_u[q * 256 + threadIdx.x] = tab[(size_t)(DT_U0 + q) * cells + c];
+        d[q] = kPhasorN * tab[(size_t)(DT_DIR + q) * cells + c];
+    // this lane's rotation vectors u0, u1 (6 each)
+    const U *u;
+    size_t ld;
+    if constexpr (PREC == 1) {
+        u = tab32 + (size_t)c * DT32_COUNT;
+        ld = 1;
+    } else {
+        u = tab + (size_t)DT_U0 * cells + c;
+        ld = cells;
     }
-    __syncthreads();
+    const auto add_shadow = [&](const double *w, U fr, U fi) {
+        U jx[8];
+        for (int q = 0; q < 8; ++q)
+            jx[q] = s_jx[q * 256 + threadIdx.x];
+        rotate_add<U>(w, u, ld, fr, fi, jx);
+        for (int q = 0; q < 8; ++q)
+            s_jx[q * 256 + threadIdx.x] = jx[q];
+    };
     const WorkItem it = items[item];
     for (int o = it.o_begin; o < it.o_end; ++o) {
         int64_t b0 = ooff[o], b1 = ooff[o + 1];
@@ -1546,53 +1755,64 @@ __global__ __launch_bounds__(256) MBS_OCCUPANCY void diffract_kernel(
             b0 = it.b_begin;
             b1 = it.b_end;
         }
-        U j[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-        U jn[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-        U jx[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-        // the next beam's vertex offset and count are loaded one beam
-        // ahead, so a beam's header and vertex loads issue together
-        int64_t v0_next = b0 < b1 ? voff[b0] : 0;
-        int nv_next = b0 < b1 ? nv[b0] : 0;
+        constexpr int SUMS = PREC == 1 ? 8 : W64_STRIDE;  // J, or G
+        U sum[SUMS];
+        for (int q = 0; q < SUMS; ++q)
+            sum[q] = 0;
+        if constexpr (NS)
+            for (int q = 0; q < 8; ++q)
+                s_jx[q * 256 + threadIdx.x] = 0;
         const int nbeam = (int)(b1 - b0);  // 32-bit loop test (scalar unit)
-        for (int ib = 0; ib < nbeam; ++ib) {
-            const int64_t b = b0 + ib;
-            const double *h = hdr + (size_t)b * HDR_STRIDE;
-            const int64_t v0 = v0_next;
-            const int nvb = nv_next;
-            if (ib + 1 < nbeam) {
-                v0_next = voff[b + 1];
-                nv_next = nv[b + 1];
-            }
-            const double *bv = vtx + (size_t)v0 * VTX_STRIDE;
-            const double *bd = vdd + (size_t)v0 * VDD_STRIDE;
+        const double *eb = ebeam + (size_t)b0 * EB_STRIDE;
+        const double *w = w64 + (size_t)b0 * W64_STRIDE;
+        BeamRecord rec{};
+        Lines ahead{};
+        if (nbeam > 0)
+            rec = load_record(eb);
+        for (int ib = 0; ib < nbeam; ++ib, w += W64_STRIDE) {
+            const double *h = hdr + (size_t)(b0 + ib) * HDR_STRIDE;
+            const bool shadow = NS && (high_word(rec.v[EB_KIND]) & 1) != 0;
             if constexpr (PREC == 0) {
-                if (NS && ext[b] == 0)
-                    beam_dir_f64<1>(h, bv, bd, vflag + v0, nvb, d, s_u, s_tab, k, eps1, j, jn);
-                else
-                    beam_dir_f64<0>(h, bv, bd, vflag + v0, nvb, d, s_u, s_tab, k, eps1, j,
-                                    nullptr);
+                double fr, fi;
+                const uint64_t dead =
+                    aperture_any_f64(rec.v, h, vtx, vx, d, s_tab, k, eps1, fr, fi);
+                ahead.arrived();
+                const bool counts = __builtin_amdgcn_inverse_ballot_w64(~dead);
+                if (shadow) {
+                    if (counts)
+                        add_shadow(w, fr, fi);
+                } else if (counts) {
+                    add_rotated_f64(w, fr, fi, sum);
+                }
+                ahead.touch(w + (ib + 1 < nbeam ? W64_STRIDE : 0));
+                eb += ib + 1 < nbeam ? EB_STRIDE : 0;
+                rec = load_record(eb);
             } else {
                 float fr, fs;
-                const BeamRecord rec = load_record(ebeam, b);
-                aperture_mixed(rec.v, evert, h, vtx, vdd, vflag, d, s_tab, k, eps1, fr, fs);
-                float u0[6], u1[6];
-                for (int q = 0; q < 6; ++q) {
-                    u0[q] = s_u[q * 256 + threadIdx.x];
-                    u1[q] = s_u[(6 + q) * 256 + threadIdx.x];
-                }
+                aperture_mixed(rec.v, h, vtx, vx, d, s_tab, k, eps1, fr, fs);
                 const float scale = low_float(rec.v[EB_SCALE]);
-                if (NS && ext[b] != 0)
-                    rotate_add_mixed(h, u0, u1, scale, fr, fs, jx);
+                eb += ib + 1 < nbeam ? EB_STRIDE : 0;
+                rec = load_record(eb);
+                fr *= scale;
+                fs *= kSqrt2 * scale;
+                if (shadow)
+                    add_shadow(w, fr, fs);
                 else
-                    rotate_add_mixed(h, u0, u1, scale, fr, fs, j);
+                    rotate_add<U>(w, u, ld, fr, fs, sum);
             }
         }
-        if constexpr (PREC == 1 && NS) {  // j: the other beams, jx: the shadow beams
+        U j[8] = {0, 0, 0, 0, 0, 0, 0, 0}, jn[8];
+        if constexpr (PREC == 1) {
+            for (int q = 0; q < 8; ++q)
+                j[q] = sum[q];
+        } else {
+            add_jones(sum, u, ld, j);
+        }
+        if constexpr (NS)  // the sum without and with the shadow beams
             for (int q = 0; q < 8; ++q) {
                 jn[q] = j[q];
-                j[q] += jx[q];
+                j[q] += s_jx[q * 256 + threadIdx.x];
             }
-        }
         if (!live)
             continue;
         if constexpr (JONES) {
@@ -1619,7 +1839,6 @@ __global__ __launch_bounds__(256) MBS_OCCUPANCY void diffract_kernel(
     }
     if constexpr (!QUEUE)
         return;
-    __syncthreads();  // the next unit overwrites s_u
     }
 }
 
@@ -1627,15 +1846,16 @@ __global__ __launch_bounds__(256) MBS_OCCUPANCY void diffract_kernel(
 // matrices of the single beams are added -- sum_b Mueller(d_b) rather than
 // Mueller(sum_b d_b) -- so beams do not interfere.  Its M11 element, the sum
 // of |d_b|^2 / 2, is what the reference's theta probe accumulates
-// (theta_m11_kernel, src/cuda/GpuDiffraction.cu:1909-1957).  Orientation
+// (theta_m11_kernel, src/cuda/GpuDiffraction.cu:1909-1957).  With d = F q, q = R Jp,
+// a beam's matrix is |F|^2 Mueller(q).  Orientation
 // items as in diffract_kernel's orientation mode: each item writes the
 // weighted sum of its orientations, which reduce_mueller_kernel adds.
 __global__ __launch_bounds__(256) MBS_OCCUPANCY void diffract_incoherent_kernel(
     const WorkItem *__restrict__ items, int n_items, int n_tiles, int cells,
     const double *__restrict__ tab, const double *__restrict__ hdr,
-    const double *__restrict__ vtx, const double *__restrict__ vdd,
-    const int32_t *__restrict__ vflag, const int32_t *__restrict__ nv,
-    const int64_t *__restrict__ voff, const int64_t *__restrict__ ooff,
+    const double *__restrict__ w64, const double *__restrict__ vtx,
+    const double *__restrict__ vx, const double *__restrict__ ebeam,
+    const double2 *__restrict__ turns, const int64_t *__restrict__ ooff,
     const double *__restrict__ weights, double k, double eps1, double *__restrict__ out)
 {
     int item, tile;
@@ -1644,39 +1864,55 @@ __global__ __launch_bounds__(256) MBS_OCCUPANCY void diffract_incoherent_kernel(
     const int cell = tile * 256 + threadIdx.x;
     const bool live = cell < cells;
     const int c = live ? cell : cells - 1;  // dead lanes compute, never store
-    double d[3];
+    double d[3], u[12];
     for (int q = 0; q < 3; ++q)
-        d[q] = tab[(size_t)(DT_DIR + q) * cells + c];
-    __shared__ double s_u[12 * 256];
+        d[q] = kPhasorN * tab[(size_t)(DT_DIR + q) * cells + c];
     __shared__ double2 s_tab[kTabN];
     for (int q = 0; q < 12; ++q)
-        s_u[q * 256 + threadIdx.x] = tab[(size_t)(DT_U0 + q) * cells + c];
-    {
-        double ts, tc;
-        sincospi((double)threadIdx.x / (kTabN / 2), &ts, &tc);
-        s_tab[threadIdx.x] = make_double2(tc, ts);
-    }
+        u[q] = tab[(size_t)(DT_U0 + q) * cells + c];
+    for (int i = threadIdx.x; i < kTabN; i += blockDim.x)
+        s_tab[i] = turns[i];
     __syncthreads();
     const WorkItem it = items[item];
     for (int o = it.o_begin; o < it.o_end; ++o) {
         double m[16];
         for (int q = 0; q < 16; ++q)
             m[q] = 0.0;
-        for (int64_t b = ooff[o]; b < ooff[o + 1]; ++b) {
-            const int64_t v0 = voff[b];
-            double dj[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-            beam_dir_f64<0>(hdr + (size_t)b * HDR_STRIDE, vtx + (size_t)v0 * VTX_STRIDE,
-                            vdd + (size_t)v0 * VDD_STRIDE, vflag + v0, nv[b], d, s_u, s_tab, k,
-                            eps1, dj, nullptr);
-            add_mueller(m, dj, 1.0);
+        const int64_t b0 = ooff[o];
+        const int nbeam = (int)(ooff[o + 1] - b0);
+        const double *eb = ebeam + (size_t)b0 * EB_STRIDE;
+        const double *w = w64 + (size_t)b0 * W64_STRIDE;
+        BeamRecord rec{};
+        Lines ahead{};
+        if (nbeam > 0)
+            rec = load_record(eb);
+        for (int ib = 0; ib < nbeam; ++ib, w += W64_STRIDE) {
+            double fr, fi;
+            const uint64_t dead =
+                aperture_any_f64(rec.v, hdr + (size_t)(b0 + ib) * HDR_STRIDE, vtx, vx, d, s_tab,
+                                 k, eps1, fr, fi);
+            ahead.arrived();
+            if (__builtin_amdgcn_inverse_ballot_w64(~dead)) {
+                double q[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+                for (int e = 0; e < 6; ++e)  // q += u[e] W[e]
+                    for (int n = 0; n < 4; ++n) {
+                        q[n] = __builtin_fma(u[e], w[4 * e + n], q[n]);
+                        q[4 + n] = __builtin_fma(u[6 + e], w[4 * e + n], q[4 + n]);
+                    }
+                add_mueller(m, q, __builtin_fma(fr, fr, fi * fi));
+            }
+            ahead.touch(w + (ib + 1 < nbeam ? W64_STRIDE : 0));
+            eb += ib + 1 < nbeam ? EB_STRIDE : 0;
+            rec = load_record(eb);
         }
         if (!live)
             continue;
-        const double w = weights[o];
+        const double weight = weights[o];
         double *dst = out + ((size_t)item * cells + cell) * 16;
         const bool first = (o == it.o_begin);
         for (int q = 0; q < 16; ++q)
-            dst[q] = (first ? 0.0 : dst[q]) + w * m[q];
+            dst[q] = (first ? 0.0 : dst[q]) + weight * m[q];
     }
 }
 
@@ -1772,10 +2008,9 @@ template <int NS, int JONES, int PER, int QUEUE, int FSRC = 0, int WAVES = MBS_M
 __global__ __launch_bounds__(256) MBS_MFMA_OCCUPANCY void diffract_mfma_kernel(
     const WorkItem *__restrict__ items, int n_items, int n_tiles, int cells, int n_az,
     const double *__restrict__ tab, const double *__restrict__ hdr,
-    const uint32_t *__restrict__ wb, const double *__restrict__ vtx,
-    const double *__restrict__ vdd, const int32_t *__restrict__ vflag,
-    const double *__restrict__ ebeam, const double *__restrict__ evert,
-    const PhasorNode *__restrict__ phasor, const int64_t *__restrict__ ooff,
+    const double *__restrict__ w64, const uint32_t *__restrict__ wb,
+    const double *__restrict__ vtx, const double *__restrict__ vx,
+    const double *__restrict__ ebeam, const PhasorNode *__restrict__ phasor, const int64_t *__restrict__ ooff,
     const double *__restrict__ weights, double k, double eps1, double *__restrict__ out,
     double *__restrict__ out_ns, double *__restrict__ per_orient, int *__restrict__ queue,
     const float *__restrict__ tab32, const int32_t *__restrict__ sidx = nullptr,
@@ -1802,7 +2037,7 @@ __global__ __launch_bounds__(256) MBS_MFMA_OCCUPANCY void diffract_mfma_kernel(
     const int c = live ? cell : cells - 1;  // dead lanes compute, never store
     double d[3];
     for (int q = 0; q < 3; ++q)
-        d[q] = tab[(size_t)(DT_DIR + q) * cells + c];
+        d[q] = kPhasorN * tab[(size_t)(DT_DIR + q) * cells + c];
     // this lane's u0, u1, read by the epilogue straight from its 48-byte
     // FP32 record (once per work item; staging them in LDS cost 12 KB per
     // workgroup, and one base address keeps the loads from holding twelve)
@@ -1822,9 +2057,10 @@ __global__ __launch_bounds__(256) MBS_MFMA_OCCUPANCY void diffract_mfma_kernel(
         // a 32-bit trip count: the scalar unit has no 64-bit ordered compare,
         // so a 64-bit loop test would go to the vector unit
         const int nbeam = (int)(b1 - b0);
+        const double *eb = ebeam + (size_t)b0 * EB_STRIDE;
         BeamRecord rec{};
         if (nbeam > 0)
-            rec = load_record(ebeam, b0);
+            rec = load_record(eb);
         // this lane's B words: row lane / 32, column lane % 32; the columns
         // past 24 lie outside the record and read as zero
         const int col = lane & 31;
@@ -1848,24 +2084,21 @@ __global__ __launch_bounds__(256) MBS_MFMA_OCCUPANCY void diffract_mfma_kernel(
                 fr = f.x * inv;
                 fs = f.y * (kInvSqrt2 * inv);
             } else {
-                aperture_mixed(rec.v, evert, h, vtx, vdd, vflag, d, s_tab, k, eps1, fr, fs);
+                aperture_mixed(rec.v, h, vtx, vx, d, s_tab, k, eps1, fr, fs);
             }
             const float scale = low_float(rec.v[EB_SCALE]);
-            const bool shadow = NS && high_word(rec.v[EB_KIND]) != 0;
+            const bool shadow = NS && (high_word(rec.v[EB_KIND]) & 1) != 0;
             // the next beam's record: after this one's last table read (LDS
             // reads and scalar loads share one wait counter), so that it
             // arrives while the contraction issues
-            rec = load_record(ebeam, b0 + min(ib + 1, nbeam - 1));
+            eb += ib + 1 < nbeam ? EB_STRIDE : 0;
+            rec = load_record(eb);
             if (shadow) {
                 // shadow beams (one an orientation) stay out of the no-shadow
                 // sum: added on the vector ALU to sums of their own, so that
                 // one accumulator set serves both grids
-                float u0[6], u1[6];
-                for (int q = 0; q < 6; ++q) {
-                    u0[q] = u[q];
-                    u1[q] = u[6 + q];
-                }
-                rotate_add_mixed(h, u0, u1, scale, fr, fs, jx);
+                rotate_add<float>(w64 + (size_t)b * W64_STRIDE, u, 1, fr * scale,
+                                  fs * (kSqrt2 * scale), jx);
                 continue;
             }
             const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(fr),

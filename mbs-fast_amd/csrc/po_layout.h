@@ -5,50 +5,50 @@
 
 namespace mbs {
 
-// Beam header, FP64, HDR_STRIDE doubles per beam (256 B aligned records so a
-// wave-uniform load of a header is a few 64-byte scalar loads).
+// Beam header, FP64, HDR_STRIDE doubles per beam, wave-uniform reads.  The
+// common path of the diffraction kernels reads the beam's EB record instead;
+// this serves the lanes and beams that leave it, and the spectrum source.
 enum {
     H_HOR = 0,   // aperture horizontal axis (3)
     H_A0 = 3,    // beamDir . hor
     H_VER = 4,   // aperture vertical axis (3)
     H_B0 = 7,    // beamDir . ver
     H_KC = 8,    // -k * centre (3), zero for external beams
-    H_SPARE = 11,
+    H_PHB = 11,  // max(|A|,|B|) above which some vertex phase exceeds 1e-3 rad
     H_AL = 12,   // small-phase area limit / complWave (complex)
     H_MOM = 14,  // k mX, k mY, k^2 mXX, 2 k^2 mXY, k^2 mYY (5)
-    H_PHB = 19,  // max(|A|,|B|) above which some vertex phase exceeds 1e-3 rad
-    H_T0 = 20,   // 1/2 (NT, nxDT)   (6)
-    H_T1 = 26,   // 1/2 (NP, nxDP)   (6)
-    H_JP = 32,   // complWave * J_phased (8)
-    // moments of orders 3..7 for the mixed kernels' moment form: entry a
+    // moments of orders 3, 4, 5 for the mixed kernels' moment form: entry a
     // of order n multiplies A^a B^(n-a) and holds k^n C(n,a) <x^a y^(n-a)> / n!
-    H_MOM3 = 40,  // (4)
-    H_MOM4 = 44,  // (5)
-    H_MOM5 = 49,  // (6)
-    H_MOM6 = 55,  // (7)
-    H_MOM7 = 62,  // (8)
-    HDR_USED = 70,
-    HDR_STRIDE = 72
+    H_MOM3 = 19,  // (4)
+    H_MOM4 = 23,  // (5)
+    H_MOM5 = 28,  // (6)
+    HDR_USED = 34,
+    HDR_STRIDE = 36
 };
+
+// Polarisation data of a beam, FP64: W[m][c] = s (T0[m] Jp[0][c] + T1[m]
+// Jp[1][c]), entry 4m + 2c + r for rotation component m (0..5), Jones column c
+// and r = 0 (real part) / 1 (imaginary part); T0 = 1/2 (NT, nxDT), T1 = 1/2 (NP,
+// nxDP), Jp = complWave J_phased, s the record's EB_S64.
+enum { W64_STRIDE = 24 };
 
 // MFMA B operand of one beam (mixed kernel): the complex contraction
 //   G[dir][n] += Re F'(dir) * B[0][n] + Im F'(dir) / sqrt(2) * B[1][n],
-// with column n = 4m + 2c + r for rotation component m (0..5), Jones column c
-// and r = 0 (real part) / 1 (imaginary part) of W[m][c] = s (T0[m] Jp[0][c] +
-// T1[m] Jp[1][c]), s = F / F' the beam's constant of EB_SCALE: B[0][n] = (Re W,
-// Im W), B[1][n] = sqrt(2) (-Im W, Re W).  Every B value is split into three
-// BF16 parts h + m + l (24 significant bits, nearest rounding); record entry
-// [row][n] holds four words of two parts each, the first in the low half:
-// (h, m) (h, m) (0, h) (0, l), the partners of the words the kernel makes of
-// F's own three parts.
+// columns n as the W entries above (with s the scale F / F' of the mixed class):
+// B[0][n] = (Re W, Im W), B[1][n] = sqrt(2) (-Im W, Re W).  Every B value is
+// split into three BF16 parts h + m + l (24 significant bits, nearest rounding);
+// record entry [row][n] holds four words of two parts each, the first in the low
+// half: (h, m) (h, m) (0, h) (0, l), the partners of the words the kernel makes
+// of F's own three parts.
 enum { WB_COLS = 24, WB_WORDS = 4, WB_STRIDE = 2 * WB_COLS * WB_WORDS };
 
-// Class of a beam in the mixed kernels (see "mixed precision" in
-// po_kernels.hip); the class word is the vertex count plus BEAM_CLASS times it.
+// Class of a beam (see "polygon classes" in po_kernels.hip); the class word is
+// the vertex count plus BEAM_CLASS times it.
 //   BEAM_VERTICES     any other polygon
 //   BEAM_TRAPEZOID    a triangle, or a quadrilateral with edges 0 and 2 parallel
 //   BEAM_PARALLEL     a parallelogram
-//   BEAM_MOMENTS      a polygon so small that every direction takes the moments
+//   BEAM_MOMENTS      (mixed kernels) a polygon so small that every direction
+//                     takes the moments
 //   BEAM_SLOPES       the edge sum with the slopes as given: a polygon whose
 //                     slopes or flags say something else than its vertices,
 //                     with a degenerate edge, a value that is not finite, axes
@@ -56,40 +56,43 @@ enum { WB_COLS = 24, WB_WORDS = 4, WB_STRIDE = 2 * WB_COLS * WB_WORDS };
 enum { BEAM_VERTICES, BEAM_TRAPEZOID, BEAM_PARALLEL, BEAM_MOMENTS, BEAM_SLOPES };
 enum { BEAM_CLASS = 32, BEAM_NV = 31 };
 
-// Record of the mixed kernels' aperture integral, EB_STRIDE doubles per beam:
-// beam direction b, the phase offset (-k centre . b in turns, reduced, plus
-// kTurnMagic; a quarter turn more for BEAM_TRAPEZOID and BEAM_VERTICES), two limits on edge 0's
-// |phase step| in turns (low word: below it the lane is looked at one by one;
-// high word: below it edge 0 counts as near-singular), (low word) the scale
-// s = F / F' of the class's formula and (high word) 1 / s, (low word) the class
-// word and (high word) 1 for an external beam, the beam's vertex offset (an
-// integer), and its phase vectors Q: -k / 2 pi times points of the aperture
-// (from the particle's origin) or differences of them, the phase being Q . (d -
-// b) plus the offset.  BEAM_TRAPEZOID: the middle of edge 1, half of edge 1, the
-// middle of the last edge, half of it.  BEAM_PARALLEL: the centre, half of edge
-// 0, half of edge 1.
+// Record of the aperture integral, EB_STRIDE doubles per beam.  Phases and steps
+// are in nodes, 1024 to the turn.
 enum {
-    EB_DIR = 0,
-    EB_PHASE = 3,
-    EB_LIM = 4,
-    EB_SCALE = 5,
-    EB_KIND = 6,
-    EB_VOFF = 7,
+    EB_DIR = 0,    // 1024 b, b the beam direction (3)
+    EB_PHASE = 3,  // mixed: -k centre . b, reduced to a turn, plus kNodeMagic (and a
+                   // quarter turn for BEAM_TRAPEZOID and BEAM_VERTICES)
+    EB_LIM = 4,    // mixed, two FP32: |step| of edge 0 below which a lane is looked at,
+                   // and below which it counts as singular
+    EB_SCALE = 5,  // mixed, two FP32: (F / F') / EB_S64 and 1 / (F / F'), F' what the
+                   // class's formula gives
+    EB_KIND = 6,   // the mixed class word; the FP64 class times 2, plus 1 for an
+                   // external beam
+    EB_VOFF = 7,   // the beam's vertex offset (an integer)
+    // phase vectors Q (four, 3 each): -k / 2 pi times points of the aperture (from
+    // the particle's origin) or differences of them, the phase being Q . 1024 (d - b)
+    // plus the offset.  BEAM_TRAPEZOID: the middle of edge 1, half of edge 1, the
+    // middle of the last edge, half of it.  BEAM_PARALLEL: the centre, half of edge
+    // 0, half of edge 1.  Others (mixed): -hor / 2 pi, -ver / 2 pi and the beam
+    // centre.
     EB_Q = 8,
-    EB_STRIDE = 20
+    EB_PHASE64 = 20,  // the offset for the FP64 kernels (a quarter turn more for
+                      // BEAM_TRAPEZOID)
+    EB_S64 = 21,      // their F / F'
+    EB_LOOK64 = 22,   // their limits: where a lane is looked at (|step| of edge 0, half
+    EB_SING64 = 23,   // of it, or max(|A|, |B|) by class), and singular steps
+    EB_STRIDE = 24
 };
-// EV_STRIDE doubles per vertex of a BEAM_VERTICES beam: the vertex's Q, and in
-// one slot two FP32 weights of the edge from this vertex: -(t_0 x t_e) (k / 2
-// pi)^2 and none for a quadrilateral, k dx / 2 pi and -k dy / 2 pi otherwise.
-enum { EV_Q = 0, EV_W = 3, EV_STRIDE = 4 };
 
 // Vertex records, FP64, 32 bytes: k x, k y, slope dy/dx, slope dx/dy (the
-// slopes of edge e = vertex e -> vertex e+1).  The packed vertices start where
-// the beam's class wants its edge 0: at the longest edge, or at the longer of
-// a trapezoid's parallel ones.  The edge deltas dx, dy, read
-// only by the rare near-singular branch, live in a separate array.
+// slopes of edge e = vertex e -> vertex e+1), and 32 more: the edge's dx and dy,
+// its two FP32 weights in the mixed kernels (see VX_W) and its flags.  The packed
+// vertices start where the beam's class wants its edge 0: at the longest edge,
+// or at the longer of a trapezoid's parallel ones.
 enum { V_KX = 0, V_KY = 1, V_SYX = 2, V_SXY = 3, VTX_STRIDE = 4 };
-enum { D_DX = 0, D_DY = 1, VDD_STRIDE = 2 };
+// VX_W: -(t_0 x t_e) (1024 k / 2 pi)^2 and none for a quadrilateral, k dx (1024 /
+// 2 pi)^2 and -k dy (1024 / 2 pi)^2 from five vertices on.
+enum { VX_DX = 0, VX_DY = 1, VX_W = 2, VX_FLAG = 3, VX_STRIDE = 4 };
 // Per-vertex edge flags (as the C ABI's MBS_EDGE_VALID_X / _Y): the edge
 // from this vertex has a usable dx (enters the |B| > |A| sum) / dy.
 enum { EDGE_VX = 1, EDGE_VY = 2 };

@@ -1,11 +1,9 @@
 // po_math.h -- device math for the PO diffraction kernels (gfx950).
 //
-// Phasors e^{i x} are evaluated here rather than through the device library
-// so that the hot loop's cost and accuracy are known: a table-driven
-// reduction against a 256-entry LDS table of e^{2 pi i j / 256} and short
-// Taylor polynomials (see sincos_table below).  Phases reach ~1e4 rad for the
-// largest particles; the reduction is exact to an ulp for |x| < 2^20.
-// The mixed-precision kernels' FP32 phasors are further down.
+// Phasors are evaluated here rather than through the device library so that the
+// hot loops' cost and accuracy are known: phases are counted in table nodes, reduced
+// against a table in LDS and finished by short polynomials (FP64) or shears
+// (FP32, mixed-precision kernels).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -14,14 +12,17 @@
 namespace mbs {
 
 constexpr double kPi = 3.141592653589793116;            // double(pi) = M_PI
+// 1 / (2 pi) and the rest of it
+constexpr double kInvTwoPi = 0.15915494309189533577;
+constexpr double kInvTwoPiRest = -9.8393375401186e-18;
 // Small-phase switch: every vertex phase within 1e-3 rad
 // (HandlerPO_fast.h:161-216).
 constexpr double kSmallPhase = 1e-3;
 // The mixed-precision kernels' switch.  Their sums cancel to O(phase) of a
 // single term where a lane's phase steps are small (kLookStep), so such lanes
-// take the moment form where every phase is within 0.5 rad, with polygon moments
-// to seventh order (truncation below max|phase|^8 / 8! = 9.7e-8 there).
-constexpr double kSmallPhaseMixed = 0.5;
+// take the moment form where every phase is within 0.25 rad, with polygon moments
+// to fifth order (truncation below max|phase|^6 / 6! = 3.4e-7 there).
+constexpr double kSmallPhaseMixed = 0.25;
 
 // Slope stored for an edge that is not valid in that direction (|dx| or
 // |dy| below the reference's geometric tolerance).  Its coefficient
@@ -44,23 +45,17 @@ __device__ __forceinline__ double horner(double p, double z, double c)
 }
 
 // ---------------------------------------------------------------------------
-// Table-driven phasor e^{i x}: x = j (2 pi/256) + d with j = rint(x 256/2pi),
-// |d| <= pi/256.  e^{i j 2pi/256} comes from a 256-entry table in LDS (filled
-// once per workgroup from the device library's sincos), e^{i d} from Taylor
-// polynomials (sin to d^7, cos to d^6, truncation < 1e-20), and one complex
-// product joins them.  The reduction is exact for |j| < 2^20 with
-// kTabStep1 = double(pi)/128 (an exact scaling of double(pi)): both x and
-// j*kTabStep1 are multiples of 2^-58 and |x - j*kTabStep1| < 2^-6.
+// FP64 phasors.  Phases are in nodes, 1/1024 of a turn: a phase is j + r with j =
+// rint(p) and |r| <= 1/2.  e^{2 pi i j / 1024} comes from a table in LDS, e^{i d},
+// d = 2 pi r / 1024 <= pi / 1024, from Taylor polynomials in r (sin to d^5, cos to
+// d^4: the next terms are 5e-22 and 1.2e-18), and one complex product joins them.
+// The reduction is three exact additions.  Phases in radians against a 256-entry
+// table took one constant more there and a step more in each polynomial; phases
+// in turns two moves more, for a product with 1024 whose addend is a constant too.
 // ---------------------------------------------------------------------------
-constexpr int kTabN = 256;
-constexpr double kTabInvStep = 40.743665431525205956;  // 256 / (2 pi)
-constexpr double kTabStep1 = 3.141592653589793116 / 128.0;
-constexpr double kTabStep2 = 1.2246467991473532e-16 / 128.0;
-
-// j = rint(x 256/2pi) by the addition of 1.5 2^52, whose sum carries j in its
-// low 32 bits (two's complement) and is j + 1.5 2^52 exactly for |j| < 2^51:
-// one FMA for the product and the rounding, one subtraction for j as a double.
-constexpr double kRoundMagic = 6755399441055744.0;  // 1.5 * 2^52
+constexpr int kTabN = 1024;
+// 1.5 2^52: a sum with it carries the integer nearest in its low 32 bits
+constexpr double kRoundMagic = 6755399441055744.0;
 __device__ __forceinline__ uint32_t low_bits(double t)
 {
     return (uint32_t)__builtin_bit_cast(uint64_t, t);
@@ -69,41 +64,64 @@ __device__ __forceinline__ uint32_t low_bits(double t)
 // In two halves, so that callers can issue the table reads of several arguments
 // before using any of them: reduction and table read, then polynomials and
 // product.
-__device__ __forceinline__ void sincos_reduce(double x, const double2 *__restrict__ tab,
-                                              double &d, double2 &e)
+__device__ __forceinline__ void node_reduce(double p, const double2 *__restrict__ tab, double &r,
+                                            double2 &e)
 {
-    const double t = __builtin_fma(x, kTabInvStep, kRoundMagic);
-    const double j = t - kRoundMagic;
-    d = __builtin_fma(-j, kTabStep1, x);
-    d = __builtin_fma(-j, kTabStep2, d);
+    const double t = p + kRoundMagic;
+    r = p - (t - kRoundMagic);
     e = tab[low_bits(t) & (kTabN - 1)];
 }
 
-__device__ __forceinline__ void sincos_finish(double d, double2 e, double &s, double &c)
+__device__ __forceinline__ void node_poly(double r, double &sd, double &cd)
 {
-    const double z = d * d;
-    double ps = __builtin_fma(z, -1.0 / 5040.0, 1.0 / 120.0);
-    ps = horner(ps, z, -1.0 / 6.0);
-    const double sd = __builtin_fma(d * z, ps, d);
-    double pc = __builtin_fma(z, -1.0 / 720.0, 1.0 / 24.0);
-    pc = horner(pc, z, -0.5);
-    const double cd = __builtin_fma(pc, z, 1.0);
+    constexpr double c1 = 6.28318530717958647693 / kTabN, c2 = c1 * c1;
+    const double z = r * r;
+    const double ps = __builtin_fma(z, c1 * c2 * c2 / 120.0, -c1 * c2 / 6.0);
+    sd = r * horner(ps, z, c1);
+    const double pc = __builtin_fma(z, c2 * c2 / 24.0, -0.5 * c2);
+    cd = __builtin_fma(pc, z, 1.0);
+}
+
+__device__ __forceinline__ void node_finish(double r, double2 e, double &s, double &c)
+{
+    double sd, cd;
+    node_poly(r, sd, cd);
     s = __builtin_fma(e.y, cd, e.x * sd);
     c = __builtin_fma(e.x, cd, -(e.y * sd));
+}
+
+// The sine alone.
+__device__ __forceinline__ double node_sine(double r, double2 e)
+{
+    double sd, cd;
+    node_poly(r, sd, cd);
+    return __builtin_fma(e.y, cd, e.x * sd);
+}
+
+// sin and cos of an angle in radians: to nodes in two parts, the second the
+// rounding of the product and of 1024 / (2 pi).
+__device__ __forceinline__ void sincos_reduce(double x, const double2 *__restrict__ tab,
+                                              double &r, double2 &e)
+{
+    const double p = x * (kTabN * kInvTwoPi);
+    const double rest = __builtin_fma(x, kTabN * kInvTwoPiRest,
+                                      __builtin_fma(x, kTabN * kInvTwoPi, -p));
+    node_reduce(p, tab, r, e);
+    r += rest;
 }
 
 __device__ __forceinline__ void sincos_table(double x, const double2 *__restrict__ tab,
                                              double &s, double &c)
 {
-    double d;
+    double r;
     double2 e;
-    sincos_reduce(x, tab, d, e);
-    sincos_finish(d, e, s, c);
+    sincos_reduce(x, tab, r, e);
+    node_finish(r, e, s, c);
 }
 
 // ---------------------------------------------------------------------------
-// FP32 phasors of the mixed kernels.  A phase is held in turns as an FP64
-// number with 1.5 2^22 added (kTurnMagic, carried by the phase's constant
+// FP32 phasors of the mixed kernels.  A phase is held in nodes (1/1024 turn) as
+// an FP64 number with 1.5 2^32 added (kNodeMagic, carried by the phase's constant
 // term, so the addition costs nothing): the low word of the sum is then the
 // phase modulo 4 turns in units of 2^-30 turn (5.9e-9 rad), exact to that unit
 // for phases within 2^21 turns.  Bits 20..29 select one of 1024 nodes, the 20
@@ -124,8 +142,7 @@ __device__ __forceinline__ void sincos_table(double x, const double2 *__restrict
 // FP64 reduction to radians took ten.
 // ---------------------------------------------------------------------------
 constexpr int kPhasorN = 1024;
-constexpr double kTurnMagic = 6291456.0;                 // 1.5 * 2^22
-constexpr double kInvTwoPi = 0.15915494309189533577;
+constexpr double kNodeMagic = 6442450944.0;              // 1.5 * 2^32
 constexpr float kSqrt2 = 1.41421356237309504880f;
 constexpr float kInvSqrt2 = 0.70710678118654752440f;
 // g = sqrt(2) pi (r - 2^19) 2^-30 - (node offset) / sqrt(2) for the 20-bit place
@@ -168,12 +185,12 @@ __device__ __forceinline__ float sine_finish(uint32_t u, PhasorNode e)
     return __builtin_fmaf(g, __builtin_fmaf(-g, e.s, e.c), e.s);
 }
 
-// Phase steps (in turns) up to which a lane is looked at one by one for the
+// Phase steps (in nodes) up to which a lane is looked at one by one for the
 // moment form: 0.25 rad, by edge 0's step and then the other edges' half steps.
-constexpr double kLookStep = 0.25 * kInvTwoPi;
-// Half steps (in turns) up to which sin(h) / h is taken from its series; the
-// table's relative error grows like 3e-10 / h below.
-constexpr float kSeriesStep = 1.0f / 512.0f;
+constexpr double kLookStep = 0.25 * kPhasorN * kInvTwoPi;
+// Half steps (in nodes) up to which sin(h) / h is taken from its series; the
+// table's relative error grows like 3e-7 / h below.
+constexpr float kSeriesStep = 2.0f;
 
 // The phasor of an angle in radians, of any size: reduced to half a turn
 // first.
@@ -181,7 +198,7 @@ __device__ __forceinline__ void phasor_rad(double x, const PhasorNode *__restric
                                            float &c, float &s)
 {
     const double y = x * kInvTwoPi;
-    const uint32_t u = low_bits((y - __builtin_rint(y)) + kTurnMagic);
+    const uint32_t u = low_bits(__builtin_fma(y - __builtin_rint(y), (double)kPhasorN, kNodeMagic));
     phasor_finish(u, phasor_read(u, tab), c, s);
 }
 
@@ -201,12 +218,6 @@ __device__ __forceinline__ double rcp_f64_fast(double x)
 {
     const double r = __builtin_amdgcn_rcp(x);
     return __builtin_fma(__builtin_fma(-x, r, 1.0), r, r);
-}
-
-__device__ __forceinline__ float rcp_f32(float x)
-{
-    float r = __builtin_amdgcn_rcpf(x);
-    return __builtin_fmaf(__builtin_fmaf(-x, r, 1.0f), r, r);
 }
 
 // sin(x)/x from its Taylor series through x^10; for |x| <= 0.25 the first

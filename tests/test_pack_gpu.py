@@ -93,19 +93,11 @@ def _shapes(rng):
     return out
 
 
-@pytest.mark.parametrize("variant", ["plain", "clockwise", "tiny", "small", "far", "slopes",
-                                     "doubled", "long axes"])
-def test_polygon_classes(pkg, oracle, variant):
-    """Shapes of every class on a grid with near-forward rows, as they are; with
-    the vertices reversed; scaled to where every direction (tiny) or some
-    (small) take the moments; with centres so far out that the phases leave
-    the fixed-point range; with slopes that differ from the vertices' by 1e-4;
-    with a repeated vertex; with an aperture axis longer than 1."""
-    abi = pkg.abi
+def _class_batch(abi, variant):
     fx = load_fixture("sobol_average")
     consts = abi.consts_from_fixture(fx)
     src = abi.BeamBatch.from_fixture(fx)
-    rng = np.random.default_rng(77)
+    rng, noise = np.random.default_rng(77), np.random.default_rng(78)
     shapes = _shapes(rng)
     bs = src.beam_scalars[rng.integers(0, src.n_beams, len(shapes))].copy()
     cols = {k: [] for k in ("x", "y", "syx", "sxy", "fl")}
@@ -116,6 +108,9 @@ def test_polygon_classes(pkg, oracle, variant):
             p = p[::-1]
         if variant == "doubled":
             p = np.insert(p, 1, p[1], axis=0)
+        if variant in ("noise 3e-12", "noise 3e-10"):  # past either tolerance
+            size = np.abs(p).max()
+            p = p + size * float(variant.split()[1]) * noise.uniform(-1.0, 1.0, p.shape)
         dx, dy = (np.roll(p, -1, 0) - p).T
         okx, oky = np.abs(dx) > 1e-12, np.abs(dy) > 1e-12
         syx = np.divide(dy, dx, out=np.zeros_like(dx), where=okx)
@@ -140,9 +135,21 @@ def test_polygon_classes(pkg, oracle, variant):
     if variant == "long axes":
         bs[:, abi.B_HOR:abi.B_HOR + 3] *= 1.5
     nb = len(shapes)
-    batch = abi.BeamBatch([0, nb], [1.0], bs, nv, np.arange(nb) % 5 == 4,
-                          np.r_[0, np.cumsum(nv)],
-                          *[np.concatenate(cols[k]) for k in ("x", "y", "syx", "sxy", "fl")])
+    return consts, abi.BeamBatch([0, nb], [1.0], bs, nv, np.arange(nb) % 5 == 4,
+                                 np.r_[0, np.cumsum(nv)],
+                                 *[np.concatenate(cols[k]) for k in ("x", "y", "syx", "sxy", "fl")])
+
+
+@pytest.mark.parametrize("variant", ["plain", "clockwise", "tiny", "small", "far", "slopes",
+                                     "doubled", "long axes"])
+def test_polygon_classes(pkg, oracle, variant):
+    """Shapes of every class on a grid with near-forward rows, as they are; with
+    the vertices reversed; scaled to where every direction (tiny) or some
+    (small) take the moments; with centres so far out that the phases leave
+    the fixed-point range; with slopes that differ from the vertices' by 1e-4;
+    with a repeated vertex; with an aperture axis longer than 1."""
+    abi = pkg.abi
+    consts, batch = _class_batch(abi, variant)
     theta = np.r_[0.0, np.logspace(-4, -1, 25), np.linspace(0.2, np.pi, 40)]
     grid = abi.Grid.build(theta, 9)
     o, on, _ = oracle.diffract(grid, batch, consts, noshadow=True)
@@ -158,3 +165,33 @@ def test_polygon_classes(pkg, oracle, variant):
                 # the path's bar; a far centre's phases of 4e6 rad carry 1e-9
                 # rad of their own rounding
                 assert e11 < 1e-4 and e < 1e-4
+
+
+@pytest.mark.parametrize("variant", ["plain", "clockwise", "tiny", "small", "far", "slopes",
+                                     "doubled", "long axes", "noise 3e-12", "noise 3e-10"])
+def test_polygon_classes_fp64(pkg, oracle, variant):
+    """The same shapes in FP64, and with vertices moved by 3e-12 and 3e-10 of
+    their size, which takes polygons out of one tolerance on parallel edges or
+    of both.  eps1 = 0 leaves a lane to the half-angle form only at an edge
+    coefficient of zero.  The bar is the path's, but for what the two sides'
+    own rounding allows: of phases of 4e6 rad (far), 4e6 2^-53 a step; of the
+    sum of O(1) terms that cancel to a phase of 1e-3 squared (tiny), 1e-16 / 1e-6."""
+    abi = pkg.abi
+    consts, batch = _class_batch(abi, variant)
+    bar = {"far": 1e-8, "tiny": 1e-9}.get(variant, 1e-10)
+    theta = np.r_[0.0, np.logspace(-4, -1, 25), np.linspace(0.2, np.pi, 40)]
+    grid = abi.Grid.build(theta, 9)
+    for eps1 in (consts.eps1, 0.0):
+        consts.eps1 = eps1
+        o, on, _ = oracle.diffract(grid, batch, consts, noshadow=True)
+        inc = oracle.incoherent(grid, batch, consts)
+        with pkg.engine.Context(0) as ctx:
+            ctx.set_grid(grid)
+            ctx.upload(batch, consts)
+            m, mn = ctx.mueller(abi.PREC_FP64, noshadow=True)
+            mi = ctx.mueller(abi.PREC_FP64 | abi.INCOHERENT)
+            mi = mi[0] if isinstance(mi, tuple) else mi
+        for a, b in ((m, o), (mn, on), (mi, inc)):
+            e = M.grid_l2(a, b, theta)
+            print("%s, eps1 %g: grid_l2 %.2e" % (variant, eps1, e))
+            assert e < bar
