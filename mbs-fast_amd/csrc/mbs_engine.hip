@@ -802,10 +802,9 @@ static bool plan_items(mbs_ctx *ctx, int n_tiles, int target, int work_mode,
     const int64_t nb = ctx->n_beams;
     const size_t cells = (size_t)ctx->cells;
     const int64_t want_items = std::max<int64_t>(1, (target + n_tiles - 1) / n_tiles);
-    // segment size in beams: enough items to fill the device, but at least
-    // kMinSeg beams each so the per-item writes stay negligible
-    const int64_t kMinSeg = 32;
-    int64_t seg = std::max<int64_t>(kMinSeg, (nb + want_items - 1) / std::max<int64_t>(want_items, 1));
+    // segment size in beams: the items the target asks for, but no fewer beams
+    // each than pay for one
+    int64_t seg = std::max<int64_t>(min_segment(nb, n_tiles), (nb + want_items - 1) / std::max<int64_t>(want_items, 1));
     int64_t n_seg = 0;
     for (int o = 0; o < no; ++o) {
         const int64_t n = ctx->h_ooff[o + 1] - ctx->h_ooff[o];
@@ -900,6 +899,33 @@ static void launch_diffract(int prec, int ns, int jones, int per, bool queue,
 #undef MBS_L
 }
 
+template <typename T>
+static void launch_jones_to_mueller(const T *part, const T *part_ns, const KernelArgs &a,
+                                    int n_items, const double *weights, int ns,
+                                    double *res, double *res_ns, double *per, hipStream_t s)
+{
+    const dim3 grid((a.cells + J2M_CELLS - 1) / J2M_CELLS, ns + 1);
+    // enough slices for 65,536 threads, a wave on every SIMD (181 x 32 directions,
+    // 1,988 items: 0.41 ms with two slices, 0.18 with sixteen; 721 x 48, 16 items,
+    // both grids: 18 us with two, 54 with sixteen).  By the grid alone, so that a
+    // batch planned on the host and on the device is added in the same order.
+    int slices = 2;
+    while (slices < 16 && a.cells * (int64_t)slices < 65536)
+        slices *= 2;
+    const auto launch = [&](auto kernel, int count) {
+        kernel<<<grid, J2M_CELLS * count, 0, s>>>(part, part_ns, a.items, n_items, a.cells, a.n_az,
+                                                  weights, res, res_ns, per, a.queue);
+    };
+    if (slices == 16)
+        launch(jones_to_mueller_kernel<T, 16>, 16);
+    else if (slices == 8)
+        launch(jones_to_mueller_kernel<T, 8>, 8);
+    else if (slices == 4)
+        launch(jones_to_mueller_kernel<T, 4>, 4);
+    else
+        launch(jones_to_mueller_kernel<T, 2>, 2);
+}
+
 // Launches the diffraction kernel and its reduction on the context's stream:
 // kernels only (no copies, no memsets), so the sequence can be captured in a
 // graph.  The partial sums and the work list are a.out / a.out_ns / a.items;
@@ -932,20 +958,14 @@ static int issue_diffraction(mbs_ctx *ctx, int prec, int ns, bool jones, int per
     if (jones) {
         // the mixed kernels (prec 1, 2, 4) leave FP32 Jones partials
         const bool f32 = prec == 1 || prec == 2 || prec == 4;
-        const dim3 jb((cells + rt - 1) / rt);
-        for (int q = 0; q <= ns; ++q) {
-            const double *src = q ? a.out_ns : a.out;
-            double *dst = q ? res_ns : res;
-            double *po = q ? nullptr : per_res;
-            if (f32)
-                jones_to_mueller_kernel<float><<<jb, rt, 0, s>>>(
-                    reinterpret_cast<const float *>(src), a.items, n_items, cells, ctx->n_az,
-                    ctx->weights.p, dst, po, a.queue);
-            else
-                jones_to_mueller_kernel<double><<<jb, rt, 0, s>>>(
-                    src, a.items, n_items, cells, ctx->n_az, ctx->weights.p, dst, po, a.queue);
-            HIP_TRY(ctx, hipGetLastError());
-        }
+        if (f32)
+            launch_jones_to_mueller(reinterpret_cast<const float *>(a.out),
+                                    reinterpret_cast<const float *>(a.out_ns), a, n_items,
+                                    ctx->weights.p, ns, res, res_ns, per_res, s);
+        else
+            launch_jones_to_mueller(a.out, a.out_ns, a, n_items, ctx->weights.p, ns, res,
+                                    res_ns, per_res, s);
+        HIP_TRY(ctx, hipGetLastError());
     } else {
         const int rb = (int)((mcount + rt - 1) / rt);
         reduce_mueller_kernel<<<rb, rt, 0, s>>>(a.out, n_items, cells, ctx->n_az, res);

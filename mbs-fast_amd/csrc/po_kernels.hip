@@ -624,6 +624,7 @@ __global__ void __launch_bounds__(PACK_THREADS) pack_beams_kernel(
                                                  : fmax(eps1 * edge, 2.0 * small);
         eb[EB_SING64] = cls64 == BEAM_VERTICES ? eps1 * k_node * lmax
                         : cls64 == BEAM_TRAPEZOID ? eps1 * edge : 0.0;
+        h[H_INV] = 1.0 / scale;
         s_scale[g] = scale;
         s_s64[g] = s64;
     }
@@ -1140,10 +1141,12 @@ __device__ __forceinline__ void add_jones(const double *g, const double *u, size
 
 // The moment form: F of a cell whose vertex phases are all within
 // kSmallPhaseMixed: <e^{i phi}> = sum_n i^n <phi^n> / n! to
-// fifth order, times the area limit and e^{i psi}.  Returns Re F and
-// Im F / sqrt(2).
+// fifth order, times the area limit and e^{i psi}, and times scale (in FP64: a
+// forward peak is all in such a value).  Returns the real part and the imaginary
+// part / sqrt(2).
 __device__ __forceinline__ void moments_mixed(const double *__restrict__ h, double A, double B,
-                                              double psi, const PhasorNode *__restrict__ tab,
+                                              double psi, double scale,
+                                              const PhasorNode *__restrict__ tab,
                                               float &out_r, float &out_s)
 {
     const double A2 = A * A, B2 = B * B, AB = A * B;
@@ -1157,8 +1160,8 @@ __device__ __forceinline__ void moments_mixed(const double *__restrict__ h, doub
     const double q5 = B3 * (B2 * c5[0] + AB * c5[1] + A2 * c5[2]) +
                       A3 * (B2 * c5[3] + AB * c5[4] + A2 * c5[5]);
     const double gr = 1.0 - 0.5 * p2 + q4, gi = p1 - q3 + q5;
-    const float ar = (float)(h[H_AL] * gr - h[H_AL + 1] * gi);
-    const float ai = (float)(h[H_AL] * gi + h[H_AL + 1] * gr);
+    const float ar = (float)((h[H_AL] * gr - h[H_AL + 1] * gi) * scale);
+    const float ai = (float)((h[H_AL] * gi + h[H_AL + 1] * gr) * scale);
     float c, s;
     phasor_rad(psi, tab, c, s);
     out_r = __builtin_fmaf(-ai * kSqrt2, s, ar * c);
@@ -1231,16 +1234,19 @@ __device__ __forceinline__ void fix_lanes(const double *eb, const double *__rest
     const double psi = kNode * (d[0] * h[H_KC] + d[1] * h[H_KC + 1] + d[2] * h[H_KC + 2]);
     const bool small =
         maybe && (cls == BEAM_MOMENTS || all_phases_small(vtx, nv, A, B, kSmallPhaseMixed));
-    if (singular && !small)
-        edges_mixed(vtx, vx, nv, A, B, psi, tab, k, eps1, out_r, out_s);
-    if (small)
-        moments_mixed(h, A, B, psi, tab, out_r, out_s);
-    if (singular || small) {
+    if (singular && !small) {
         const float inv = high_float(eb[EB_SCALE]);
+        edges_mixed(vtx, vx, nv, A, B, psi, tab, k, eps1, out_r, out_s);
+        out_r *= inv;
+        out_s *= inv;
+    }
+    if (small)
+        moments_mixed(h, A, B, psi, h[H_INV], tab, out_r, out_s);
+    if (singular || small) {
         // a NaN F (degenerate polygon) counts as zero
         const bool bad = __builtin_isnan(out_r);
-        out_r = bad ? 0.0f : out_r * inv;
-        out_s = bad ? 0.0f : out_s * inv;
+        out_r = bad ? 0.0f : out_r;
+        out_s = bad ? 0.0f : out_s;
     }
 }
 
@@ -1515,8 +1521,13 @@ __device__ __forceinline__ void rotate_add(const double *__restrict__ w, const T
 }
 
 // XCD-aware block -> (item, tile): consecutive workgroup ids land on the 8
-// XCDs round-robin; remapping gives each XCD a contiguous range of items so
-// the beam records of an item are shared through that XCD's L2.
+// XCDs round-robin.  On a large grid they stay in order: a few items are in
+// flight at a time, each read by every XCD, and the XCDs get equal work whatever
+// the items' sizes.  On a small one each XCD gets a contiguous range of items, so
+// that the beam records of an item pass through one L2 (in order, a thousand
+// workgroups would hold dozens of items).  11,000 beams on 1001 x 48 directions
+// (188 tiles): 3.94 ms in order, 4.16 by ranges; 59,000 on 181 x 32 (23 tiles): 1.38
+// and 1.32.
 __device__ __forceinline__ bool map_block(int n_items, int n_tiles, int &item,
                                           int &tile)
 {
@@ -1524,7 +1535,7 @@ __device__ __forceinline__ bool map_block(int n_items, int n_tiles, int &item,
     const int nblk = gridDim.x;
     const int per_xcd = (nblk + 7) / 8;
     const int bid = blockIdx.x;
-    const int logical = (bid % 8) * per_xcd + bid / 8;
+    const int logical = n_tiles >= 64 ? bid : (bid % 8) * per_xcd + bid / 8;
     if (logical >= total)
         return false;
     item = logical / n_tiles;
@@ -1535,7 +1546,7 @@ __device__ __forceinline__ bool map_block(int n_items, int n_tiles, int &item,
 // ---------------------------------------------------------------------------
 // Device work queue (work mode MBS_WORK_QUEUE).  plan_segments_kernel cuts
 // every orientation into beam segments on the device (the host plan's rule:
-// segments of max(32, ceil(n_beams / want)) beams, at least one per
+// segments of max(min_segment, ceil(n_beams / want)) beams, at least one per
 // orientation) and splits the (item, tile) units into 8 contiguous ranges,
 // one per XCD, so the units of one item stay in one XCD's L2.  A persistent
 // workgroup takes units from its XCD's range with an atomic counter and,
@@ -1543,6 +1554,23 @@ __device__ __forceinline__ bool map_block(int n_items, int n_tiles, int &item,
 // eight are empty.  Each unit still writes its own partial sums, so results
 // do not depend on which workgroup ran it.
 // ---------------------------------------------------------------------------
+// The least beams of a segment, on the host and on the device.  A segment costs its
+// workgroups a start and an end (tables, the first records, the sum's way out)
+// worth some tens of beams, and its partial grid; a launch ends with workgroups
+// idle for half a segment.  With N beams, T tiles and P workgroups at once the two
+// are N T / (P seg) x cost and seg / 2: least at a multiple of sqrt(N T / P).
+// With P = 1024 the multiple 4 is best or near it throughout (times of kernel and
+// reduction at multiples 2.7, 4 and 6.4, and with 32 beams at least): 1,900 beams on
+// 541 x 96 directions, FP64, 1.74 1.62 1.91 (1.80) ms; 11,000 on 1001 x 48, 4.48 4.23
+// 3.97 (4.92); 59,000 on 181 x 32 1.33 1.31 1.46 (1.60); 137,000 on 541 x 96 16.9 17.4
+// 17.1 (16.8).  At least four: 185 beams on 91 x 16 take 20 us with four or five,
+// 23 with eight, 50 with 32.
+__host__ __device__ inline int64_t min_segment(int64_t n_beams, int n_tiles)
+{
+    const int64_t seg = (int64_t)(sqrt((double)(n_beams * n_tiles)) / 8.0);
+    return seg > 4 ? seg : 4;
+}
+
 struct QueueCursor {
     int range = -1;   // XCD range being drained (thread 0 only)
     int tried = 0;    // ranges found empty so far
@@ -1588,7 +1616,7 @@ __global__ void __launch_bounds__(1024) plan_segments_kernel(
     __shared__ int s_base;
     const int64_t nb = ooff[n_orient];
     const int64_t seg =
-        max((int64_t)32, (nb + (int64_t)want - 1) / max((int64_t)want, (int64_t)1));
+        max(min_segment(nb, n_tiles), (nb + (int64_t)want - 1) / max((int64_t)want, (int64_t)1));
     if (threadIdx.x == 0)
         s_base = 0;
     __syncthreads();
@@ -2170,48 +2198,169 @@ __global__ void reduce_mueller_kernel(const double *__restrict__ part, int n_ite
 // Jones segments -> Mueller: items are ordered by orientation; for each
 // orientation the segment Jones sums are added in segment order, converted
 // and accumulated with the orientation weight (TracerPOTotal.cpp:5985-5994).
-template <typename T>
-__global__ void jones_to_mueller_kernel(const T *__restrict__ part,
-                                        const WorkItem *__restrict__ items,
-                                        int n_items, int cells, int n_az,
-                                        const double *__restrict__ weights,
-                                        double *__restrict__ res,
-                                        double *__restrict__ per_orient,
-                                        const int *__restrict__ queue)
+//
+// Its floor is the partials' bytes (read once; per-orientation grids written
+// once).  A thread that walks a cell's items alone waits for one load after the
+// other with too few threads in flight, so a workgroup takes 32 cells and SLICES
+// equal slices of the item list.  Of an orientation that a slice's ends cut, the
+// slices leave their parts in LDS and the slice where it ends adds them in order;
+// the slices' Mueller sums are added in order too, so the result is reproducible.
+// 1,988 items (256 orientations) on 181 x 32 directions with their grids kept: 1.42
+// -> 0.18 ms (559 MB: 3.2 TB/s); 333 items on 541 x 96: 0.19 -> 0.11 ms (5.0 TB/s).
+// blockIdx.y selects the full or the no-shadow grid.
+enum { J2M_CELLS = 32 };
+
+// The end of the run of items of orientation o that starts at i (< end).
+__device__ __forceinline__ int orientation_end(const WorkItem *__restrict__ items, int i, int end,
+                                               int o)
 {
-    const int cell = blockIdx.x * blockDim.x + threadIdx.x;
-    if (cell >= cells)
-        return;
+    // the next 32 items, one a lane of this half of the wave
+    const int at = i + (threadIdx.x & 31);
+    const uint64_t same =
+        __builtin_amdgcn_ballot_w64(at < end && items[min(at, end - 1)].o_begin == o);
+    const uint32_t half = (uint32_t)(same >> (threadIdx.x & 32));
+    if (half != 0xffffffffu)
+        return i + __builtin_ctz(~half);
+    int lo = i + 31, hi = end;  // items[lo] is of o, items[hi] is not
+    while (hi - lo > 1) {
+        const int mid = lo + (hi - lo) / 2;
+        if (items[mid].o_begin == o)
+            lo = mid;
+        else
+            hi = mid;
+    }
+    return hi;
+}
+
+// Adds the Jones partials of items [i, end) of a cell to j, in order, four
+// items' loads at a time.
+template <typename T>
+__device__ __forceinline__ void add_partials(const T *__restrict__ part, size_t stride, int i,
+                                             int end, double *j)
+{
+    struct alignas(16) Jones {
+        T v[8];
+    };
+    const T *src = part + (size_t)i * stride;
+    for (; i + 4 <= end; i += 4, src += 4 * stride) {
+        Jones p[4];
+        for (int u = 0; u < 4; ++u)
+            p[u] = *reinterpret_cast<const Jones *>(src + u * stride);
+        for (int u = 0; u < 4; ++u)
+            for (int q = 0; q < 8; ++q)
+                j[q] += p[u].v[q];
+    }
+    for (; i < end; ++i, src += stride) {
+        const Jones p = *reinterpret_cast<const Jones *>(src);
+        for (int q = 0; q < 8; ++q)
+            j[q] += p.v[q];
+    }
+}
+
+template <typename T, int SLICES>
+__global__ void __launch_bounds__(J2M_CELLS * SLICES)
+    jones_to_mueller_kernel(const T *__restrict__ part, const T *__restrict__ part_ns,
+                            const WorkItem *__restrict__ items, int n_items, int cells,
+                            int n_az, const double *__restrict__ weights,
+                            double *__restrict__ res, double *__restrict__ res_ns,
+                            double *__restrict__ per_orient, const int *__restrict__ queue)
+{
+    __shared__ double s_head[SLICES][8][J2M_CELLS], s_tail[SLICES][8][J2M_CELLS];
+    __shared__ int s_state[SLICES];
     if (queue)  // planned on the device
         n_items = queue[Q_ITEMS];
-    const size_t out_cell = abi_cell(cell, n_az, cells);
+    if (blockIdx.y) {
+        part = part_ns;
+        res = res_ns;
+        per_orient = nullptr;
+    }
+    const int l = threadIdx.x % J2M_CELLS, slice = threadIdx.x / J2M_CELLS;
+    const int first = blockIdx.x * J2M_CELLS;
+    const int cell = min(first + l, cells - 1);  // spare lanes compute, never store
+    const bool live = first + l < cells;
+    const size_t stride = (size_t)cells * 8;
+    const T *src = part + (size_t)cell * 8;
     double m[16];
     for (int q = 0; q < 16; ++q)
         m[q] = 0.0;
-    int i = 0;
-    while (i < n_items) {
-        const int o = items[i].o_begin;
-        double j[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-        while (i < n_items && items[i].o_begin == o) {
-            const T *src = part + ((size_t)i * cells + cell) * 8;
-            for (int q = 0; q < 8; ++q)
-                j[q] += src[q];
-            ++i;
-        }
-        add_mueller(m, j, weights[o]);
+    const auto convert = [&](const double *j, int o) {
         if (per_orient) {
             double po[16];
             for (int q = 0; q < 16; ++q)
                 po[q] = 0.0;
             add_mueller(po, j, weights[o]);
-            double *dst = per_orient + ((size_t)o * cells + out_cell) * 16;
-            for (int q = 0; q < 16; ++q)
-                dst[q] = po[q];
+            double *dst = per_orient + ((size_t)o * cells + abi_cell(cell, n_az, cells)) * 16;
+            for (int q = 0; q < 16; ++q) {
+                if (live)
+                    dst[q] = po[q];
+                m[q] += po[q];
+            }
+        } else {
+            add_mueller(m, j, weights[o]);
+        }
+    };
+    // this slice's items, and what it leaves: NONE, the first part of an
+    // orientation (TAIL), or nothing but a middle part of one (MIDDLE; also an
+    // empty slice, whose part is zero)
+    enum { NONE, TAIL, MIDDLE };
+    const int lo = (int)((int64_t)n_items * slice / SLICES);
+    const int hi = (int)((int64_t)n_items * (slice + 1) / SLICES);
+    int state = lo < hi ? NONE : MIDDLE;
+    int ends = -1;  // the orientation from before that ends here
+    if (lo == hi)
+        for (int q = 0; q < 8; ++q)
+            s_head[slice][q][l] = 0.0;
+    for (int i = lo; i < hi;) {
+        const int o = items[i].o_begin;
+        const int to = orientation_end(items, i, n_items, o);
+        const bool before = i == lo && i > 0 && items[i - 1].o_begin == o;
+        double j[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+        add_partials(src, stride, i, min(to, hi), j);
+        if (before) {
+            for (int q = 0; q < 8; ++q)
+                s_head[slice][q][l] = j[q];
+            if (to <= hi)
+                ends = o;
+            else
+                state = MIDDLE;
+        } else if (to > hi) {
+            for (int q = 0; q < 8; ++q)
+                s_tail[slice][q][l] = j[q];
+            state = TAIL;
+        } else {
+            convert(j, o);
+        }
+        i = to;
+    }
+    if (l == 0)
+        s_state[slice] = state;
+    __syncthreads();
+    if (ends >= 0) {
+        int from = slice - 1;
+        while (s_state[from] == MIDDLE)
+            --from;
+        double j[8];
+        for (int q = 0; q < 8; ++q)
+            j[q] = s_tail[from][q][l];
+        for (int e = from + 1; e <= slice; ++e)
+            for (int q = 0; q < 8; ++q)
+                j[q] += s_head[e][q][l];
+        convert(j, ends);
+    }
+    for (int h = 0; h < 2; ++h) {  // eight elements at a time
+        __syncthreads();
+        for (int q = 0; q < 8; ++q)
+            s_head[slice][q][l] = m[8 * h + q];
+        __syncthreads();
+        for (int i = threadIdx.x; i < 8 * J2M_CELLS; i += J2M_CELLS * SLICES) {
+            const int q = i % 8, at = i / 8;
+            double sum = 0.0;
+            for (int e = 0; e < SLICES; ++e)
+                sum += s_head[e][q][at];
+            if (first + at < cells)
+                res[abi_cell(first + at, n_az, cells) * 16 + 8 * h + q] = sum;
         }
     }
-    double *dst = res + out_cell * 16;
-    for (int q = 0; q < 16; ++q)
-        dst[q] = m[q];
 }
 
 // Azimuth (laboratory-alpha) average of an orientation-summed Mueller grid,

@@ -22,7 +22,8 @@ enum {
     H_MOM3 = 19,  // (4)
     H_MOM4 = 23,  // (5)
     H_MOM5 = 28,  // (6)
-    HDR_USED = 34,
+    H_INV = 34,   // 1 / (F / F') of the mixed class (see EB_SCALE)
+    HDR_USED = 35,
     HDR_STRIDE = 36
 };
 
