@@ -2192,12 +2192,18 @@ int mlp_ensure_rows(mbs_mlp *m, int rows)
     return MBS_OK;
 }
 
-template <int TA, int TB>
-void mlp_gemm(hipStream_t s, int M, int N, int K, const float *A, int lda, const float *B,
-              int ldb, float *C, int ldc, const float *bias, int beta)
+// 128 x 128 tiles where there is one for every CU, else 32 x 32 ones (4096 x 2896 x
+// 256, 736 tiles: 54 and 80 us; 512 x 2896 x 256, 92 tiles: 24 and 14; 4096 x 256 x
+// 256, 64 tiles: 32 and 16).
+template <int TA, int TB, int SPLIT>
+void mlp_gemm(hipStream_t s, const MlpGemm &g)
 {
-    const dim3 grid((N + 63) / 64, (M + 63) / 64);
-    mlp_gemm_kernel<TA, TB><<<grid, 256, 0, s>>>(M, N, K, A, lda, B, ldb, C, ldc, bias, beta);
+    const dim3 tiles((g.N + MLP_TILE - 1) / MLP_TILE, (g.M + MLP_TILE - 1) / MLP_TILE);
+    const dim3 small((g.N + 31) / 32, (g.M + 31) / 32);
+    if ((int64_t)tiles.x * tiles.y >= 256 || small.y > 65535)
+        mlp_tile_kernel<TA, TB><<<tiles, 256, 0, s>>>(g);
+    else
+        mlp_split_kernel<TA, TB, SPLIT><<<small, 64 * SPLIT, 0, s>>>(g);
 }
 
 // Forward pass of `rows` inputs already in a[0]; output in y.
@@ -2208,14 +2214,10 @@ int mlp_forward_dev(mbs_mlp *m, int rows)
     const float *P = m->params.p;
     for (int l = 0; l <= m->depth; ++l) {
         const int in = mlp_layer_in(m, l), out = mlp_layer_out(m, l);
-        float *dst = l < m->depth ? m->z[l].p : m->y.p;
-        mlp_gemm<0, 0>(s, rows, out, in, m->a[l].p, in, P + m->w_off[l], out, dst, out,
-                       P + m->b_off[l], 0);
-        if (l < m->depth) {
-            const size_t n = (size_t)rows * out;
-            mlp_gelu_kernel<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(n, m->z[l].p,
-                                                                        m->a[l + 1].p);
-        }
+        const bool last = l == m->depth;
+        mlp_gemm<0, 0, 1>(s, MlpGemm{rows, out, in, m->a[l].p, in, P + m->w_off[l], out,
+                                  last ? m->y.p : m->z[l].p, out, P + m->b_off[l], nullptr,
+                                  last ? nullptr : m->a[l + 1].p});
     }
     HIP_TRY(ctx, hipGetLastError());
     return MBS_OK;
@@ -2231,24 +2233,19 @@ int mlp_backward_dev(mbs_mlp *m, int rows)
     float *G = m->grads.p;
     mlp_mse_grad_kernel<<<rows, 256, 0, s>>>(rows, m->n_out, m->y.p, m->t.p, m->dy.p,
                                              m->row_sq.p);
-    const float *dcur = m->dy.p;  // gradient w.r.t. the output of layer l
+    const float *dout = m->dy.p;  // gradient w.r.t. layer l's product
     for (int l = m->depth; l >= 0; --l) {
         const int in = mlp_layer_in(m, l), out = mlp_layer_out(m, l);
-        const float *dout = dcur;
-        if (l < m->depth) {
-            const size_t n = (size_t)rows * out;
-            mlp_gelu_grad_kernel<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(n, m->z[l].p, dcur,
-                                                                             m->dz.p);
-            dout = m->dz.p;
-        }
         // dW_l = A_l^T dOut, db_l = column sums of dOut
-        mlp_gemm<1, 0>(s, in, out, rows, m->a[l].p, in, dout, out, G + m->w_off[l], out,
-                       nullptr, 0);
-        mlp_colsum_kernel<<<(out + 255) / 256, 256, 0, s>>>(rows, out, dout, G + m->b_off[l]);
-        if (l > 0) {  // dA_l = dOut W_l^T
-            mlp_gemm<0, 1>(s, rows, in, out, dout, out, P + m->w_off[l], out, m->da.p, in,
-                           nullptr, 0);
-            dcur = m->da.p;
+        mlp_gemm<1, 0, 8>(s, MlpGemm{in, out, rows, m->a[l].p, in, dout, out, G + m->w_off[l], out,
+                                  nullptr, nullptr, nullptr});
+        mlp_colsum_kernel<<<(out + 31) / 32, 32 * COLSUM_SLICES, 0, s>>>(rows, out, dout,
+                                                                         G + m->b_off[l]);
+        if (l > 0) {  // dOut of layer l - 1: (dOut W_l^T) GELU'(z_l-1)
+            float *next = dout == m->dz.p ? m->da.p : m->dz.p;
+            mlp_gemm<0, 1, 8>(s, MlpGemm{rows, in, out, dout, out, P + m->w_off[l], out, next, in,
+                                      nullptr, m->z[l - 1].p, nullptr});
+            dout = next;
         }
     }
     HIP_TRY(ctx, hipGetLastError());
