@@ -105,16 +105,22 @@ class HandlerPOGpu:
             ctx = self._context()
             ctx.upload(batch, self.consts)
             ctx.diffract(self._flags())
-            tmp = np.zeros((g.n_az, g.n_zen + 1, 16))
-            tmpn = np.zeros_like(tmp) if mnv is not None else None
+            # the engine adds a grid only once it is all on the host (both, up
+            # to 64 MiB each); anything else goes through a grid of its own
+            grids = [a for a in (mv, mnv) if a is not None]
+            direct = all(a.flags.c_contiguous and a.flags.aligned and a.flags.writeable
+                         and (len(grids) == 1 or a.nbytes <= 64 << 20) for a in grids)
+            tmp = mv if direct else np.zeros((g.n_az, g.n_zen + 1, 16))
+            tmpn = mnv if direct or mnv is None else np.zeros_like(tmp)
             ctx.accumulate(tmp, tmpn)
         except EngineError as e:
             if e.status in (abi.MBS_ERR_BAD_BEAM, abi.MBS_ERR_INVALID):
                 return False
             return self._device_failure(e)
-        mv += tmp
-        if mnv is not None:
-            mnv += tmpn
+        if not direct:
+            mv += tmp
+            if mnv is not None:
+                mnv += tmpn
         return True
 
     def HandleOrientationsToLocalGpuOnDevice(self, prepared, start, count, device, localM,
