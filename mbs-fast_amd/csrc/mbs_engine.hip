@@ -996,8 +996,10 @@ static const size_t kPartialBudget = (size_t)8 << 30;  // bytes
 // Workgroups of a persistent (work-queue) launch: 256 CUs x 8 slots.
 static const int kQueueBlocks = 2048;
 
+//  Values: the doubles of a segment's partial in a cell (8, a Jones matrix; the
+//  incoherent sum's segments keep 16, a Mueller matrix).
 static bool plan_items(mbs_ctx *ctx, int n_tiles, int target, int work_mode,
-                       std::vector<WorkItem> &items)
+                       std::vector<WorkItem> &items, int values = 8)
 {
     items.clear();
     const int no = ctx->n_orient;
@@ -1012,7 +1014,7 @@ static bool plan_items(mbs_ctx *ctx, int n_tiles, int target, int work_mode,
         const int64_t n = ctx->h_ooff[o + 1] - ctx->h_ooff[o];
         n_seg += std::max<int64_t>(1, (n + seg - 1) / seg);
     }
-    const bool segments_fit = (size_t)n_seg * cells * 8 * sizeof(double) <= kPartialBudget;
+    const bool segments_fit = (size_t)n_seg * cells * values * sizeof(double) <= kPartialBudget;
     const bool jones = work_mode == 2 || (work_mode == 0 && segments_fit && nb > 0);
     if (jones) {
         for (int o = 0; o < no; ++o) {
@@ -1262,11 +1264,12 @@ int mbs_diffract(mbs_ctx *ctx, uint32_t flags)
         n_items = ctx->queue_want + ctx->n_orient;  // the most the device plan makes
         ctx->h_items.clear();
     } else {
-        // the incoherent sum keeps per-item Mueller sums (orientation items)
-        jones = plan_items(ctx, n_tiles, target,
-                           incoh ? MBS_WORK_ORIENTATIONS
-                                 : mode == MBS_WORK_QUEUE ? MBS_WORK_SEGMENTS : mode,
-                           ctx->h_items);
+        // the incoherent sum keeps Mueller sums, of beam segments too while they fit
+        if (incoh)
+            plan_items(ctx, n_tiles, target, 0, ctx->h_items, 16);
+        jones = !incoh && plan_items(ctx, n_tiles, target,
+                                     mode == MBS_WORK_QUEUE ? MBS_WORK_SEGMENTS : mode,
+                                     ctx->h_items);
         n_items = (int)ctx->h_items.size();
     }
     const size_t mcount = (size_t)cells * 16;
