@@ -80,12 +80,13 @@ def calibrate_copy():
 
 def algorithmic_bytes(batch, cells):
     """HBM bytes one launch must move at least: the device beam records read
-    once (FP64 header 320 B, FP32 header 80 B, MFMA operand 256 B per beam;
-    vertex records 32 + 16 + 4 B per vertex), the grid tables read once
-    (15 FP64 per direction) and the Mueller grid written once (16 FP64 per
-    direction)."""
+    once (header 288 B, FP64 rotation data 192 B, aperture record 192 B, MFMA
+    operand 768 B per beam; vertex records 32 + 32 B per vertex), the grid tables
+    read once (15 FP64 per direction) and the Mueller grid written once (16 FP64
+    per direction)."""
     n_vert = int(batch.vert_offsets[-1])
-    return float(batch.n_beams) * (320 + 80 + 256) + n_vert * 52.0 + cells * (15 + 16) * 8.0
+    return float(batch.n_beams) * (288 + 192 + 192 + 768) + n_vert * 64.0 \
+        + cells * (15 + 16) * 8.0
 
 
 def cpu_model():

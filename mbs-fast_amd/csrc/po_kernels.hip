@@ -1100,25 +1100,27 @@ __device__ __forceinline__ uint64_t aperture_any_f64(const double *eb, const dou
 }
 
 // G += F' W: entry 4m + 2c + r of G and of W (po_layout.h).
-__device__ __forceinline__ void add_rotated_f64(const double *__restrict__ w, double fr, double fi,
-                                                double *g)
+template <typename T>
+__device__ __forceinline__ void add_rotated(const double *__restrict__ w, T fr, T fi, T *g)
 {
 #pragma unroll
     for (int n = 0; n < W64_STRIDE; n += 2) {
-        g[n] = __builtin_fma(fr, w[n], __builtin_fma(-fi, w[n + 1], g[n]));
-        g[n + 1] = __builtin_fma(fr, w[n + 1], __builtin_fma(fi, w[n], g[n + 1]));
+        const T wr = (T)w[n], wi = (T)w[n + 1];
+        g[n] = fr * wr + (g[n] - fi * wi);
+        g[n + 1] = fr * wi + (g[n + 1] + fi * wr);
     }
 }
 
 // The Jones sum of a lane from its G: J[i][c] = sum_m u_i[m] G[m][c]; entry m of u0,
 // u1 at m * ld.
-__device__ __forceinline__ void add_jones(const double *g, const double *u, size_t ld, double *j)
+template <typename T>
+__device__ __forceinline__ void add_jones(const T *g, const T *u, size_t ld, T *j)
 {
 #pragma unroll
     for (int m = 0; m < 12; ++m) {
-        const double um = u[m * ld];
+        const T um = u[m * ld];
         for (int n = 0; n < 4; ++n)
-            j[4 * (m / 6) + n] = __builtin_fma(um, g[4 * (m % 6) + n], j[4 * (m / 6) + n]);
+            j[4 * (m / 6) + n] = um * g[4 * (m % 6) + n] + j[4 * (m / 6) + n];
     }
 }
 
@@ -1710,11 +1712,12 @@ __device__ __forceinline__ void flush_mueller(const T *j, double w, double *dst,
 // stores into `out` must be provably disjoint from the beam records for the
 // compiler to keep reading those through the scalar cache.
 //
-// FP64 (PREC 0): the sum is kept in the directions' frame, G[m][c] += F W[m][c]
-// (24 FP64 accumulators, 48 FMAs a beam with W in scalar registers), and turned
-// into the Jones sum once per orientation or segment.  Rotating each beam (R =
-// u . T, R Jp, F R Jp) took 56 and twelve LDS reads.  PREC 1, the mixed kernel on
-// the vector ALU: FP32 sums, each beam rotated.
+// The sum is kept in the global frame, G[m][c] += F W[m][c] (24 accumulators, 48
+// FMAs a beam with W in scalar registers), and turned into the Jones sum once per
+// orientation or segment.  Rotating each beam (R = u . T, R Jp, F R Jp) took 56 and
+// twelve LDS reads.  PREC 0: FP64; PREC 1, the mixed kernel on the vector ALU: FP32
+// sums of W rounded to FP32 (137,000 beams on 541 x 96 directions: 21.2 ms,
+// where each beam rotated, with its conversions, took 32 to 33).
 template <int PREC, int NS, int JONES, int PER, int QUEUE>
 __global__ __launch_bounds__(256) MBS_OCCUPANCY void diffract_kernel(
     const WorkItem *__restrict__ items, int n_items, int n_tiles, int cells, int n_az,
@@ -1783,9 +1786,8 @@ __global__ __launch_bounds__(256) MBS_OCCUPANCY void diffract_kernel(
             b0 = it.b_begin;
             b1 = it.b_end;
         }
-        constexpr int SUMS = PREC == 1 ? 8 : W64_STRIDE;  // J, or G
-        U sum[SUMS];
-        for (int q = 0; q < SUMS; ++q)
+        U sum[W64_STRIDE];  // G
+        for (int q = 0; q < W64_STRIDE; ++q)
             sum[q] = 0;
         if constexpr (NS)
             for (int q = 0; q < 8; ++q)
@@ -1810,7 +1812,7 @@ __global__ __launch_bounds__(256) MBS_OCCUPANCY void diffract_kernel(
                     if (counts)
                         add_shadow(w, fr, fi);
                 } else if (counts) {
-                    add_rotated_f64(w, fr, fi, sum);
+                    add_rotated<double>(w, fr, fi, sum);
                 }
                 ahead.touch(w + (ib + 1 < nbeam ? W64_STRIDE : 0));
                 eb += ib + 1 < nbeam ? EB_STRIDE : 0;
@@ -1819,23 +1821,20 @@ __global__ __launch_bounds__(256) MBS_OCCUPANCY void diffract_kernel(
                 float fr, fs;
                 aperture_mixed(rec.v, h, vtx, vx, d, s_tab, k, eps1, fr, fs);
                 const float scale = low_float(rec.v[EB_SCALE]);
-                eb += ib + 1 < nbeam ? EB_STRIDE : 0;
-                rec = load_record(eb);
+                ahead.arrived();
                 fr *= scale;
                 fs *= kSqrt2 * scale;
                 if (shadow)
                     add_shadow(w, fr, fs);
                 else
-                    rotate_add<U>(w, u, ld, fr, fs, sum);
+                    add_rotated<float>(w, fr, fs, sum);
+                ahead.touch(w + (ib + 1 < nbeam ? W64_STRIDE : 0));
+                eb += ib + 1 < nbeam ? EB_STRIDE : 0;
+                rec = load_record(eb);
             }
         }
         U j[8] = {0, 0, 0, 0, 0, 0, 0, 0}, jn[8];
-        if constexpr (PREC == 1) {
-            for (int q = 0; q < 8; ++q)
-                j[q] = sum[q];
-        } else {
-            add_jones(sum, u, ld, j);
-        }
+        add_jones<U>(sum, u, ld, j);
         if constexpr (NS)  // the sum without and with the shadow beams
             for (int q = 0; q < 8; ++q) {
                 jn[q] = j[q];
