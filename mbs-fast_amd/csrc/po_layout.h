@@ -113,9 +113,9 @@ struct WorkItem {
 };
 
 // Header of the device work queue (work mode MBS_WORK_QUEUE), written by
-// plan_segments_kernel: the item count, then for each of the 8 XCDs the next
-// unit to hand out and the end of its range of units (unit = item * n_tiles
-// + tile).
-enum { Q_ITEMS = 0, Q_NEXT = 1, Q_END = 9, Q_WORDS = 17 };
+// plan_segments_kernel: the item count, then for each of the 8 XCDs the end of its
+// range of units (unit = item * n_tiles + tile), and the next unit to hand out,
+// each in a line of its own (atomics on one line are served one after the other).
+enum { Q_ITEMS = 0, Q_END = 1, Q_NEXT = 64, Q_LINE = 64, Q_WORDS = Q_NEXT + 8 * Q_LINE };
 
 }  // namespace mbs
