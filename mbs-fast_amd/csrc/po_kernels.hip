@@ -2035,6 +2035,7 @@ __device__ __forceinline__ bf16x8 split_words(uint32_t x)
 }
 
 enum { G_LD = 25 };  // LDS row stride (floats) of the per-wave G transpose
+static_assert(32 * G_LD >= 8 * 64, "the tile holds a wave's shadow sums");
 
 // G (this wave's accumulators) -> this lane's Jones sum.  Accumulator v of
 // lane l holds G[dir][n] with n = l % 32, dir = 8 (v/4) + 4 (l/32) + v % 4
@@ -2127,7 +2128,7 @@ __global__ __launch_bounds__(256) MBS_MFMA_OCCUPANCY void diffract_mfma_kernel(
             b1 = it.b_end;
         }
         f32x16 g0 = {}, g1 = {};
-        float jx[8] = {0, 0, 0, 0, 0, 0, 0, 0};  // shadow beams (NS)
+        bool cast = false;  // whether a shadow beam has left its sum in sg
         // a 32-bit trip count: the scalar unit has no 64-bit ordered compare,
         // so a 64-bit loop test would go to the vector unit
         const int nbeam = (int)(b1 - b0);
@@ -2161,18 +2162,26 @@ __global__ __launch_bounds__(256) MBS_MFMA_OCCUPANCY void diffract_mfma_kernel(
                 aperture_mixed(rec.v, h, vtx, vx, d, s_tab, k, eps1, fr, fs);
             }
             const float scale = low_float(rec.v[EB_SCALE]);
-            const bool shadow = NS && (high_word(rec.v[EB_KIND]) & 1) != 0;
+            const bool shadow = (high_word(rec.v[EB_KIND]) & 1) != 0;
             // the next beam's record: after this one's last table read (LDS
             // reads and scalar loads share one wait counter), so that it
             // arrives while the contraction issues
             eb += ib + 1 < nbeam ? EB_STRIDE : 0;
             rec = load_record(eb);
             if (shadow) {
-                // shadow beams (one an orientation) stay out of the no-shadow
-                // sum: added on the vector ALU to sums of their own, so that
-                // one accumulator set serves both grids
+                // shadow beams (one an orientation) are added on the vector ALU to a
+                // sum of their own, in this wave's part of the epilogue's tile: it
+                // keeps them out of the no-shadow sum with one accumulator set,
+                // and near the forward peak, where they are far the largest,
+                // keeps the other beams' FP32 sum from being rounded at their size
+                float jx[8];
+                for (int q = 0; q < 8; ++q)
+                    jx[q] = cast ? sg[64 * q + lane] : 0.0f;
                 rotate_add<float>(w64 + (size_t)b * W64_STRIDE, u, 1, fr * scale,
                                   fs * (kSqrt2 * scale), jx);
+                for (int q = 0; q < 8; ++q)
+                    sg[64 * q + lane] = jx[q];
+                cast = true;
                 continue;
             }
             const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(fr),
@@ -2181,13 +2190,14 @@ __global__ __launch_bounds__(256) MBS_MFMA_OCCUPANCY void diffract_mfma_kernel(
             g0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(split_words(sw[0]), bop, g0, 0, 0, 0);
             g1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(split_words(sw[1]), bop, g1, 0, 0, 0);
         }
-        float j[8], jn[8];
+        float j[8], jn[8], jx[8];
+        for (int q = 0; q < 8; ++q)
+            jx[q] = cast ? sg[64 * q + lane] : 0.0f;
         mfma_epilogue(g0, g1, sg, u, cells, j);
-        if constexpr (NS)
-            for (int q = 0; q < 8; ++q) {
-                jn[q] = j[q];
-                j[q] += jx[q];
-            }
+        for (int q = 0; q < 8; ++q) {
+            jn[q] = j[q];
+            j[q] += jx[q];
+        }
         if (!live)
             continue;
         if constexpr (JONES) {
