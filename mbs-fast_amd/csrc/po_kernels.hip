@@ -625,7 +625,7 @@ __global__ void __launch_bounds__(PACK_THREADS) pack_beams_kernel(
         eb[EB_SING64] = cls64 == BEAM_VERTICES ? eps1 * k_node * lmax
                         : cls64 == BEAM_TRAPEZOID ? eps1 * edge : 0.0;
         h[H_INV] = 1.0 / scale;
-        s_scale[g] = scale;
+        s_scale[g] = ext ? 0.0 : scale;
         s_s64[g] = s64;
     }
     __syncthreads();
@@ -647,16 +647,18 @@ __global__ void __launch_bounds__(PACK_THREADS) pack_beams_kernel(
         rotation(c, n, wr, wi);
         w64[(size_t)first * W64_STRIDE + i] = s_s64[c] * ((n & 1) ? wi : wr);
     }
-    // MFMA operand, split into three BF16 parts
+    // MFMA operand, split into three BF16 parts; a shadow beam's is zero: it is
+    // summed apart
     for (int i = threadIdx.x; i < count * (2 * WB_COLS); i += PACK_THREADS) {
         const int c = i / (2 * WB_COLS), e = i - c * (2 * WB_COLS);
         const int row = e / WB_COLS, n = e - row * WB_COLS;
         double wr, wi;
         rotation(c, n, wr, wi);
         // rows 0 and 1 multiply Re F and Im F / sqrt(2)
-        const double w = s_scale[c] * (row == 0 ? ((n & 1) ? wi : wr)
-                                                : 1.41421356237309504880 *
-                                                      ((n & 1) ? wr : -wi));
+        const double w = s_scale[c] == 0.0 ? 0.0
+                                           : s_scale[c] * (row == 0 ? ((n & 1) ? wi : wr)
+                                                                    : 1.41421356237309504880 *
+                                                                          ((n & 1) ? wr : -wi));
         const uint32_t ph = bf16_bits((float)w);
         const double r1 = w - (double)bf16_value(ph);
         const uint32_t pm = bf16_bits((float)r1);
@@ -2128,11 +2130,53 @@ __global__ __launch_bounds__(256) MBS_MFMA_OCCUPANCY void diffract_mfma_kernel(
             b1 = it.b_end;
         }
         f32x16 g0 = {}, g1 = {};
-        bool cast = false;  // whether a shadow beam has left its sum in sg
         // a 32-bit trip count: the scalar unit has no 64-bit ordered compare,
         // so a 64-bit loop test would go to the vector unit
         const int nbeam = (int)(b1 - b0);
         const double *eb = ebeam + (size_t)b0 * EB_STRIDE;
+        // Re F', Im F' / sqrt(2) of beam b
+        const auto field = [&](const BeamRecord &r, int64_t b, float &fr,
+                               float &fs) __attribute__((always_inline)) {
+            const double *h = hdr + (size_t)b * HDR_STRIDE;
+            const int slot = FSRC ? __builtin_amdgcn_readfirstlane(sidx[b]) : -1;
+            if (FSRC && slot >= 0) {
+                const float2 f = fbuf[(size_t)slot * cells + c];
+                const float inv = high_float(r.v[EB_SCALE]);
+                fr = f.x * inv;
+                fs = f.y * (kInvSqrt2 * inv);
+            } else {
+                aperture_mixed(r.v, h, vtx, vx, d, s_tab, k, eps1, fr, fs);
+            }
+        };
+        // Shadow beams (one an orientation) are added on the vector ALU to a sum
+        // of their own, kept in this wave's part of the epilogue's tile: out of
+        // the no-shadow sum with one accumulator set, and near the forward peak,
+        // where they are far the largest, out of the FP32 sum of the others.
+        // They are looked for 64 at a time ahead of the loop below, which runs
+        // over them too, with zeros for operands.  A branch in that loop held
+        // scalars that then spilled to vector lanes, 9 vector instructions a beam
+        // in a queue launch: 12.04 -> 11.10 ms (aggregate of 50 to 40,000 beams,
+        // 541 x 96), 2.20 -> 2.14 (15,000 beams, two grids), 1.21 -> 1.16
+        // (59,000 beams by orientation, 181 x 32)
+        {
+            float jx[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+            for (int ib = 0; ib < nbeam; ib += 64) {
+                bool ext = false;
+                if (ib + lane < nbeam)
+                    ext = high_word(eb[(size_t)(ib + lane) * EB_STRIDE + EB_KIND]) & 1;
+                for (uint64_t left = __ballot(ext); left; left &= left - 1) {
+                    const int64_t b = b0 + ib + __builtin_ctzll(left);
+                    const BeamRecord r = load_record(ebeam + (size_t)b * EB_STRIDE);
+                    float fr, fs;
+                    field(r, b, fr, fs);
+                    const float scale = low_float(r.v[EB_SCALE]);
+                    rotate_add<float>(w64 + (size_t)b * W64_STRIDE, u, 1, fr * scale,
+                                      fs * (kSqrt2 * scale), jx);
+                }
+            }
+            for (int q = 0; q < 8; ++q)
+                sg[64 * q + lane] = jx[q];
+        }
         BeamRecord rec{};
         if (nbeam > 0)
             rec = load_record(eb);
@@ -2150,40 +2194,13 @@ __global__ __launch_bounds__(256) MBS_MFMA_OCCUPANCY void diffract_mfma_kernel(
                 kBufferRsrcWord3);
             w += WB_STRIDE;
             const u32x4 bw = __builtin_amdgcn_raw_buffer_load_b128(wres, lane_off, 0, 0);
-            float fr, fs;  // Re F', Im F' / sqrt(2)
-            const double *h = hdr + (size_t)b * HDR_STRIDE;
-            const int slot = FSRC ? __builtin_amdgcn_readfirstlane(sidx[b]) : -1;
-            if (FSRC && slot >= 0) {
-                const float2 f = fbuf[(size_t)slot * cells + c];
-                const float inv = high_float(rec.v[EB_SCALE]);
-                fr = f.x * inv;
-                fs = f.y * (kInvSqrt2 * inv);
-            } else {
-                aperture_mixed(rec.v, h, vtx, vx, d, s_tab, k, eps1, fr, fs);
-            }
-            const float scale = low_float(rec.v[EB_SCALE]);
-            const bool shadow = (high_word(rec.v[EB_KIND]) & 1) != 0;
+            float fr, fs;
+            field(rec, b, fr, fs);
             // the next beam's record: after this one's last table read (LDS
             // reads and scalar loads share one wait counter), so that it
             // arrives while the contraction issues
             eb += ib + 1 < nbeam ? EB_STRIDE : 0;
             rec = load_record(eb);
-            if (shadow) {
-                // shadow beams (one an orientation) are added on the vector ALU to a
-                // sum of their own, in this wave's part of the epilogue's tile: it
-                // keeps them out of the no-shadow sum with one accumulator set,
-                // and near the forward peak, where they are far the largest,
-                // keeps the other beams' FP32 sum from being rounded at their size
-                float jx[8];
-                for (int q = 0; q < 8; ++q)
-                    jx[q] = cast ? sg[64 * q + lane] : 0.0f;
-                rotate_add<float>(w64 + (size_t)b * W64_STRIDE, u, 1, fr * scale,
-                                  fs * (kSqrt2 * scale), jx);
-                for (int q = 0; q < 8; ++q)
-                    sg[64 * q + lane] = jx[q];
-                cast = true;
-                continue;
-            }
             const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(fr),
                                                              __float_as_uint(fs), false, false);
             const bf16x8 bop = __builtin_bit_cast(bf16x8, bw);
@@ -2192,7 +2209,7 @@ __global__ __launch_bounds__(256) MBS_MFMA_OCCUPANCY void diffract_mfma_kernel(
         }
         float j[8], jn[8], jx[8];
         for (int q = 0; q < 8; ++q)
-            jx[q] = cast ? sg[64 * q + lane] : 0.0f;
+            jx[q] = sg[64 * q + lane];
         mfma_epilogue(g0, g1, sg, u, cells, j);
         for (int q = 0; q < 8; ++q) {
             jn[q] = j[q];

@@ -231,3 +231,29 @@ def test_segment_sums(pkg, counts, cells):
             per = ctx.per_orient()
             full = ctx.mueller(flags)[0]
             assert np.linalg.norm(per.sum(0) - full) <= tol * np.linalg.norm(full)
+
+
+@pytest.mark.parametrize("shadow", [[], [0], [63, 64], [129], list(range(130))],
+                         ids=["none", "first", "edge", "last", "all"])
+def test_shadow_beams_apart(pkg, shadow):
+    """Shadow beams are looked for 64 at a time and summed apart: at the edges of
+    these groups, among 130 beams and in every one of them, the mixed sums
+    against the FP64 ones, and the no-shadow grid, which holds none of them.
+    Sums of up to 130 FP32 terms, each off by some 2^-22: within 130 2^-22."""
+    abi = pkg.abi
+    fx = load_fixture("sobol_average")
+    src, consts = abi.BeamBatch.from_fixture(fx), abi.consts_from_fixture(fx)
+    batch = pkg.synthetic.resample(src, np.asarray([130, 3]), seed=7)
+    batch.beam_external[:] = 0
+    batch.beam_external[shadow] = 1
+    grid = abi.Grid.build(np.linspace(0.0, np.pi, 37), 6)
+    with pkg.engine.Context(0) as ctx:
+        ctx.set_grid(grid)
+        ctx.upload(batch, consts)
+        want, want_ns = ctx.mueller(abi.PREC_FP64, noshadow=True)
+        for mode in (abi.WORK_ORIENTATIONS, abi.WORK_SEGMENTS, abi.WORK_QUEUE):
+            ctx.set_work_mode(mode)
+            m, mn = ctx.mueller(abi.PREC_MIXED, noshadow=True)
+            one = ctx.mueller(abi.PREC_MIXED)[0]
+            for a, b in ((m, want), (mn, want_ns), (one, want)):
+                assert np.linalg.norm(a - b) <= 130 * 2.0 ** -22 * np.linalg.norm(b)
