@@ -1133,7 +1133,7 @@ __device__ __forceinline__ void add_jones(const T *g, const T *u, size_t ld, T *
 // and parallelograms 40 vector instructions, where the reference's branches (A,
 // B, psi, two FP64 coefficients and a select per edge, an FP64 reduction per
 // vertex) took 109, and other quadrilaterals 100 (137,000 beams of 2,000-15,000
-// an orientation on 541 x 96 directions: 17.3 ms against 27.3 for the kernel,
+// an orientation on 541 x 96 directions: 16.8 ms against 27.3 for the kernel,
 // contraction included).  From five vertices on (shadow beams, 4 to 15 in 100
 // others) the weights are the reference's dx or dy, by the larger of |A| and |B|,
 // since one edge's own step is too often small against K there.
