@@ -456,8 +456,12 @@ __global__ void __launch_bounds__(PACK_THREADS) pack_beams_kernel(
                  cz = ext ? 0.0 : s[11] * sc;
     const double k_turn = k * kInvTwoPi, k_node = kPhasorN * k_turn;
     const double tol = 1e-9 * lmax;
-    // 2 where every edge agrees closely, 1 where every edge does; the largest |vertex|
-    double agree = 2.0, reach = 0.0;
+    // 2 where every edge agrees closely, 1 where every edge does; the largest
+    // |vertex|; 1 where every value is finite
+    double agree = 2.0, reach = 0.0, finite = 1.0;
+    for (int i = 0; i < 9; ++i)
+        finite = fabs(s[i]) < __builtin_inf() ? finite : 0.0;
+    finite = fabs(k * cx) + fabs(k * cy) + fabs(k * cz) < __builtin_inf() ? finite : 0.0;
     for (int i = q; i < nv; i += PACK_GROUP) {
         const int to = (i + 1 < nv) ? i + 1 : 0;
         const double x = px[i], y = py[i], dx = px[to] - x, dy = py[to] - y;
@@ -469,8 +473,10 @@ __global__ void __launch_bounds__(PACK_THREADS) pack_beams_kernel(
                             : offx <= 1e-4 * tol && offy <= 1e-4 * tol ? 2.0 : 1.0;
         agree = fmin(agree, here);
         reach = fmax(reach, sqrt(x * x + y * y));
+        finite = fabs(k * x) + fabs(k * y) < __builtin_inf() ? finite : 0.0;
     }
     agree = group_min(agree);
+    finite = group_min(finite);
     reach = -group_min(-reach);
     const double n_hor = hor[0] * hor[0] + hor[1] * hor[1] + hor[2] * hor[2];
     const double n_ver = ver[0] * ver[0] + ver[1] * ver[1] + ver[2] * ver[2];
@@ -520,7 +526,7 @@ __global__ void __launch_bounds__(PACK_THREADS) pack_beams_kernel(
         if (fabs(w1) >= 1e-30 && fabs(w1) <= 1e30) {
             if (unit && agree >= 1.0)
                 start = from;
-            if (unit && close) {
+            if (unit && close && finite == 1.0) {
                 cls64 = form;  // else the sum over vertices, below
                 s64 = form == BEAM_PARALLEL ? -w1 : w1;
             }
@@ -531,11 +537,11 @@ __global__ void __launch_bounds__(PACK_THREADS) pack_beams_kernel(
             cls = BEAM_SLOPES;
         }
     }
-    if (cls64 == BEAM_SLOPES && unit && agree == 2.0) {
+    if (cls64 == BEAM_SLOPES && unit && agree == 2.0 && finite == 1.0) {
         cls64 = BEAM_VERTICES;
         s64 = k_node * (kPhasorN * kInvTwoPi);
     }
-    if (!(unit && fits && agree >= 1.0))
+    if (!(unit && fits && agree >= 1.0) || finite != 1.0)
         cls = BEAM_SLOPES;
     else if (fabs(skew) <= 1e-6 && 2.01 * k * reach <= kSmallPhaseMixed)
         cls = BEAM_MOMENTS;
@@ -611,7 +617,10 @@ __global__ void __launch_bounds__(PACK_THREADS) pack_beams_kernel(
             part + (cls == BEAM_TRAPEZOID || cls == BEAM_VERTICES ? kPhasorN / 4 : 0) + kNodeMagic;
         const double sing = eps_mixed * edge;
         eb[EB_LIM] = pack_floats((float)fmax(sing, kLookStep), (float)sing);
-        eb[EB_SCALE] = pack_floats((float)(scale / s64), (float)(1.0 / scale));
+        // F of a beam with a value that is not finite is NaN in every direction: the
+        // FP64 phases see to that by themselves, the mixed ones lose it as words
+        const double inverse = finite == 1.0 ? 1.0 / scale : __builtin_nan("");
+        eb[EB_SCALE] = pack_floats((float)(scale / s64), (float)inverse);
         eb[EB_KIND] = pack_words(nv + BEAM_CLASS * cls, 2 * cls64 + (ext ? 1 : 0));
         eb[EB_VOFF] = __builtin_bit_cast(double, v0);
         eb[EB_PHASE64] = part + (cls64 == BEAM_TRAPEZOID ? kPhasorN / 4 : 0);
@@ -624,7 +633,9 @@ __global__ void __launch_bounds__(PACK_THREADS) pack_beams_kernel(
                                                  : fmax(eps1 * edge, 2.0 * small);
         eb[EB_SING64] = cls64 == BEAM_VERTICES ? eps1 * k_node * lmax
                         : cls64 == BEAM_TRAPEZOID ? eps1 * edge : 0.0;
-        h[H_INV] = 1.0 / scale;
+        h[H_INV] = inverse;
+        if (finite != 1.0)  // not for the spectrum source either
+            h[H_A0] = __builtin_inf();
         s_scale[g] = ext ? 0.0 : scale;
         s_s64[g] = s64;
     }
