@@ -33,16 +33,18 @@
 #include "po_math.h"
 #include "po_layout.h"
 
-// Occupancy of the vector-ALU kernels: at least 4 waves per SIMD (128 VGPRs).
-// The FP64 kernel's common path takes about 120 with its 24 sums; the other
-// polygons' spill there.  With 3 waves and no spills it is slower (11.7 ms
-// against 9.3 for 35,800 beams on 541 x 96 directions): it waits on LDS and
-// scalar loads.
-// Builds may pass -DMBS_MIN_WAVES=N for tuning.
+// Occupancy of the vector-ALU kernels, in waves per SIMD.  FP64: at least 4 (128
+// VGPRs), which the common path takes about 120 of with its 24 sums; with 3 waves
+// and no spills it is slower (11.7 ms against 9.3 for 35,800 beams on 541 x 96
+// directions), since it waits on LDS and scalar loads.  Mixed precision: 7 (72
+// VGPRs; 6 with the shadow beams' sums, whose LDS lets no more share a CU).  Left
+// alone it takes 75 to 87 and runs at 5 or 6: 4,000 beams of six vertices and more
+// on those directions 1.75 ms, with 7 waves 1.52.
+// Builds may pass -DMBS_MIN_WAVES=N for tuning (FP64).
 #ifndef MBS_MIN_WAVES
 #define MBS_MIN_WAVES 4
 #endif
-#define MBS_OCCUPANCY __attribute__((amdgpu_waves_per_eu(MBS_MIN_WAVES, 8)))
+#define MBS_OCCUPANCY(waves) __attribute__((amdgpu_waves_per_eu(waves, 8)))
 // The MFMA kernel is held to WAVES waves per SIMD (default 5: 96 VGPRs); its
 // 29 KB of LDS per workgroup lets five workgroups share a CU.  The autotuner
 // also tries 4 and 6 for the default beam-segment kernel.
@@ -989,26 +991,37 @@ __device__ __forceinline__ void aperture_vertices_f64(const double *__restrict__
         node_reduce(p, tab, r, e);
         node_finish(r, e, sn, cs);
     };
-    double p0, s0, c0;
-    vertex(0, p0, s0, c0);
-    double pp = p0, sp = s0, cp = c0, sr = 0.0, si = 0.0;
+    // edge e, from a vertex (phase, sine and cosine p, sp, cp) to the next (n, sn, cn)
+    double sr = 0.0, si = 0.0;
     step = __builtin_inf();
-    const int n = NV > 0 ? NV : nv;
-#pragma unroll
-    for (int e = 0; e < n; ++e) {
+    const auto edge = [&](int e, double p, double sp, double cp, double n, double sn, double cn) {
         const double dx = uniform_f64(vx[e * VX_STRIDE + VX_DX]),
                      dy = uniform_f64(vx[e * VX_STRIDE + VX_DY]);
-        double pn = p0, sn = s0, cn = c0;
-        if (e + 1 < n)
-            vertex(e + 1, pn, sn, cn);
-        const double D = pn - pp;
+        const double D = n - p;
         const double w = __builtin_fma(dy, uy, dx * ux) * rcp_f64_cubic(D);
         sr = __builtin_fma(cn - cp, w, sr);
         si = __builtin_fma(sn - sp, w, si);
         step = __builtin_fmin(step, __builtin_fabs(D));
-        pp = pn;
-        sp = sn;
-        cp = cn;
+    };
+    double p0, s0, c0;
+    vertex(0, p0, s0, c0);
+    double p = p0, sp = s0, cp = c0, n, sn, cn;
+    const int last = (NV > 0 ? NV : nv) - 1;
+    int e = 0;
+    // two edges at a time (the compiler does not unroll loops that read lanes)
+#pragma unroll
+    for (; e + 2 <= last; e += 2) {
+        vertex(e + 1, n, sn, cn);
+        edge(e, p, sp, cp, n, sn, cn);
+        vertex(e + 2, p, sp, cp);
+        edge(e + 1, n, sn, cn, p, sp, cp);
+    }
+    if (e < last) {
+        vertex(last, n, sn, cn);
+        edge(e, p, sp, cp, n, sn, cn);
+        edge(last, n, sn, cn, p0, s0, c0);
+    } else {
+        edge(last, p, sp, cp, p0, s0, c0);
     }
     fr = sr;
     fi = si;
@@ -1424,23 +1437,33 @@ __device__ __forceinline__ void aperture_loop(const double *eb, const double *__
 {
     const Projection p = project(eb, d);
     const bool useB = __builtin_fabs(p.b) > __builtin_fabs(p.a);
-    const double p0 = vertex_phase(p, vtx);
-    double pp = p0;
     float sr = 0.0f, ss = 0.0f, steps = 0.0f;
-    for (int e = 0; e < nv; ++e) {
+    const auto edge = [&](int e, double from, double to) {
         const double w = vx[e * VX_STRIDE + VX_W];
         const float wx = low_float(w), wy = high_float(w);
-        double pn = p0;
-        if (e + 1 < nv)
-            pn = vertex_phase(p, vtx + (e + 1) * VTX_STRIDE);
         float c, s, ratio, f;
-        edge_terms(pp, pn, tab, c, s, ratio, f);
+        edge_terms(from, to, tab, c, s, ratio, f);
         const float coef = ratio * (useB ? wx : wy);
         sr = __builtin_fmaf(c, coef, sr);
         ss = __builtin_fmaf(s, coef, ss);
         steps = __builtin_fmaxf(steps, __builtin_fabsf(f));
-        pp = pn;
+    };
+    // two edges at a time (the compiler does not unroll loops that vote)
+    const double p0 = vertex_phase(p, vtx);
+    double from = p0;
+    int e = 0;
+    for (; e + 2 < nv; e += 2) {
+        const double mid = vertex_phase(p, vtx + (e + 1) * VTX_STRIDE);
+        edge(e, from, mid);
+        from = vertex_phase(p, vtx + (e + 2) * VTX_STRIDE);
+        edge(e + 1, mid, from);
     }
+    if (e + 1 < nv) {
+        const double mid = vertex_phase(p, vtx + (e + 1) * VTX_STRIDE);
+        edge(e, from, mid);
+        from = mid;
+    }
+    edge(nv - 1, from, p0);
     const float r = __builtin_amdgcn_rcpf((float)(useB ? p.b : p.a));
     out_r = sr * r;
     out_s = ss * r;
@@ -1741,7 +1764,8 @@ __device__ __forceinline__ void flush_mueller(const T *j, double w, double *dst,
 // sums of W rounded to FP32 (137,000 beams on 541 x 96 directions: 21.2 ms,
 // where each beam rotated, with its conversions, took 32 to 33).
 template <int PREC, int NS, int JONES, int PER, int QUEUE>
-__global__ __launch_bounds__(256) MBS_OCCUPANCY void diffract_kernel(
+__global__ __launch_bounds__(256) MBS_OCCUPANCY(PREC == 1 ? (NS ? 6 : 7) : MBS_MIN_WAVES) void
+diffract_kernel(
     const WorkItem *__restrict__ items, int n_items, int n_tiles, int cells, int n_az,
     const double *__restrict__ tab, const double *__restrict__ hdr,
     const double *__restrict__ w64, const double *__restrict__ vtx,
@@ -1903,7 +1927,7 @@ __global__ __launch_bounds__(256) MBS_OCCUPANCY void diffract_kernel(
 // reduce_mueller_kernel adds the items.  With whole orientations only, 16 of them
 // on 181 x 48 directions kept half of the device busy, each beam waiting for the one
 // before: 0.65 ms, now 0.30.
-__global__ __launch_bounds__(256) MBS_OCCUPANCY void diffract_incoherent_kernel(
+__global__ __launch_bounds__(256) MBS_OCCUPANCY(MBS_MIN_WAVES) void diffract_incoherent_kernel(
     const WorkItem *__restrict__ items, int n_items, int n_tiles, int cells,
     const double *__restrict__ tab, const double *__restrict__ hdr,
     const double *__restrict__ w64, const double *__restrict__ vtx,
