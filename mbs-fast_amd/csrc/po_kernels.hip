@@ -487,7 +487,11 @@ __global__ void __launch_bounds__(PACK_THREADS) pack_beams_kernel(
     // |phase| <= |Q| |d - b| with axes no longer than 1; comparisons written
     // so that a value that is not a number fails them
     const bool unit = n_hor <= 1.0 + 1e-6 && n_ver <= 1.0 + 1e-6 && n_bd <= 1.0 + 1e-6;
-    const bool fits = 2.5 * k_turn * (sqrt(cx * cx + cy * cy + cz * cz) + reach) < 0x1p20;
+    const double far = sqrt(cx * cx + cy * cy + cz * cz);
+    const bool fits = 2.5 * k_turn * (far + reach) < 0x1p20;
+    // the same for any axes, |d - b| <= 1 + |b|
+    const bool in_range = 1.25 * k_turn * (far + (sqrt(n_hor) + sqrt(n_ver)) * reach) *
+                              (1.0 + sqrt(n_bd)) < 0x1p20;
     // the polygon's own form, and edge 0 for it
     int form = BEAM_VERTICES, from = start;
     bool close = agree == 2.0;  // to the FP64 kernels' tolerance
@@ -544,12 +548,12 @@ __global__ void __launch_bounds__(PACK_THREADS) pack_beams_kernel(
         s64 = k_node * (kPhasorN * kInvTwoPi);
     }
     if (!(unit && fits && agree >= 1.0) || finite != 1.0)
-        cls = BEAM_SLOPES;
+        cls = in_range && finite == 1.0 && cls64 == BEAM_SLOPES ? BEAM_SLOPES : BEAM_FAR;
     else if (fabs(skew) <= 1e-6 && 2.01 * k * reach <= kSmallPhaseMixed)
         cls = BEAM_MOMENTS;
     if (cls == BEAM_VERTICES)
         scale = 1.41421356237309504880;
-    else if (cls == BEAM_SLOPES || cls == BEAM_MOMENTS)
+    else if (cls >= BEAM_MOMENTS)
         scale = 1.0;
     // phase vector in turns of a point of the aperture plane, from the beam
     // centre or from the particle's origin
@@ -618,7 +622,11 @@ __global__ void __launch_bounds__(PACK_THREADS) pack_beams_kernel(
         eb[EB_PHASE] =
             part + (cls == BEAM_TRAPEZOID || cls == BEAM_VERTICES ? kPhasorN / 4 : 0) + kNodeMagic;
         const double sing = eps_mixed * edge;
-        eb[EB_LIM] = pack_floats((float)fmax(sing, kLookStep), (float)sing);
+        // BEAM_SLOPES: max(|A|, |B|) in nodes above which some phase exceeds 0.25 rad
+        const double lim = cls == BEAM_SLOPES
+                               ? (kPhasorN * kInvTwoPi * kSmallPhaseMixed / kSmallPhase) * h[H_PHB]
+                               : fmax(sing, kLookStep);
+        eb[EB_LIM] = pack_floats((float)lim, (float)sing);
         // F of a beam with a value that is not finite is NaN in every direction: the
         // FP64 phases see to that by themselves, the mixed ones lose it as words
         const double inverse = finite == 1.0 ? 1.0 / scale : __builtin_nan("");
@@ -684,11 +692,8 @@ __global__ void __launch_bounds__(PACK_THREADS) pack_beams_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// Per-(beam, direction) evaluation, FP64.  Returns false when the aperture
-// integral is NaN (the reference skips the beam, HandlerPO.cpp:2742); else
-// adds d = F R Jp to j[8] (and to jn[8] when ACC_NS).
-//
-// The two edge-sum branches of the reference (|B| > |A|: sum over edges with
+// The edge sums as the reference has them, for beams of class BEAM_SLOPES and for
+// lanes next to a singular edge.  Its two branches (|B| > |A|: sum over edges with
 // valid dx, coefficient A + (dy/dx) B, divide by B; otherwise edges with
 // valid dy, coefficient A (dx/dy) + B, divide by -A) are evaluated by one
 // loop whose operands are selected per lane, so lanes that take different
@@ -729,188 +734,178 @@ __device__ __forceinline__ bool all_phases_small(const double *__restrict__ vtx,
     return small;
 }
 
-template <int NV>
-__device__ __forceinline__ bool all_phases_small_nv(const double *kx, const double *ky, double A,
-                                                    double B, double limit = kSmallPhase)
-{
-    bool small = true;
-#pragma unroll
-    for (int e = 0; e < NV; ++e)
-        small = small && __builtin_fabs(__builtin_fma(A, kx[e], B * ky[e])) <= limit;
-    return small;
-}
-
-// Lanes for which edge e enters the sum, as a wave mask: an edge with a
-// valid dx in the lanes of mB (|B| > |A|), with a valid dy in the others.
-// The flags are wave-uniform, so this is scalar mask arithmetic and the
-// per-lane choice costs no vector instruction.  Used by the FP64 sums; in
-// the mixed ones the extra scalar work measured slower than the two vector
-// instructions it saves.
-__device__ __forceinline__ uint64_t edge_valid_mask(int flags, uint64_t mB)
-{
-    const uint64_t mx = (flags & EDGE_VX) ? ~0ull : 0ull;
-    const uint64_t my = (flags & EDGE_VY) ? ~0ull : 0ull;
-    return (mB & mx) | (~mB & my);
-}
-
-// One edge of the aperture sum (FP64 phasors): the phasor of vertex e+1
-// (vertex 0 again for the closing edge), the edge coefficient
-// C = A + (dy/dx) B (|B| > |A|) or A (dx/dy) + B (otherwise) and its
-// contribution (e^{i phi_{e+1}} - e^{i phi_e}) / C, or the exact half-angle
-// form when |C| <= eps1.
-__device__ __forceinline__ void edge_f64(int e, int n, const double *__restrict__ vtx,
-                                         const double *__restrict__ vx, double A, double B,
-                                         double psi, bool useB, uint64_t mB,
-                                         const double2 *__restrict__ tab, double k,
-                                         double eps1, double s0, double c0, double &sp,
-                                         double &cp, double &sr, double &si, bool small)
-{
-    const double *v = vtx + (size_t)e * VTX_STRIDE;
-    // both slopes as scalars and both coefficients, then a per-lane select
-    // (a select between the two loads becomes a divergent branch around each
-    // scalar load)
-    const double syx = uniform_f64(v[V_SYX]), sxy = uniform_f64(v[V_SXY]);
-    const int f = vertex_flags(vx, e);
-    double sn = s0, cn = c0;
-    if (e + 1 < n) {
-        const double xn = __builtin_fma(B, v[VTX_STRIDE + V_KY], psi);
-        sincos_table(__builtin_fma(A, v[VTX_STRIDE + V_KX], xn), tab, sn, cn);
-    }
-    const double cc = useB ? __builtin_fma(syx, B, A) : __builtin_fma(sxy, A, B);
-    const uint64_t mvalid = edge_valid_mask(f, mB);
-    const uint64_t mbig = __builtin_amdgcn_ballot_w64(__builtin_fabs(cc) > eps1);
-    const double r = rcp_f64_fast(cc);
-    const double inv = __builtin_amdgcn_inverse_ballot_w64(mvalid & mbig) ? r : 0.0;
-    sr = __builtin_fma(cn - cp, inv, sr);
-    si = __builtin_fma(sn - sp, inv, si);
-    if (__builtin_expect(__builtin_amdgcn_inverse_ballot_w64(mvalid & ~mbig) && !small, 0)) {
-        const double *w = vx + (size_t)e * VX_STRIDE;
-        const double dd = useB ? uniform_f64(w[VX_DX]) : uniform_f64(w[VX_DY]);
-        const double2 q = stable_edge_quotient(cp, sp, cn, sn, dd, cc, k);
-        sr += q.x;
-        si += q.y;
-    }
-    sp = sn;
-    cp = cn;
-}
-
-// The edge sum of aperture_f64: both coefficients from scalar slopes, then
-// a per-lane select; the lanes an edge enters as scalar masks.
-template <int NV>
-__device__ __forceinline__ void edge_sum_f64_nv(
-    const double *syx, const double *sxy, const int *fl, const double *sv, const double *cv,
-    const double *__restrict__ vx, double A, double B, bool useB, uint64_t mB, double k,
-    double eps1, bool small, double &sr, double &si)
-{
-#pragma unroll
-    for (int e = 0; e < NV; ++e) {
-        const int f = e + 1 < NV ? e + 1 : 0;
-        const double cx = __builtin_fma(syx[e], B, A);
-        const double cy = __builtin_fma(sxy[e], A, B);
-        const double cc = useB ? cx : cy;
-        const uint64_t mvalid = edge_valid_mask(fl[e], mB);
-        const uint64_t mbig = __builtin_amdgcn_ballot_w64(__builtin_fabs(cc) > eps1);
-        const double r = rcp_f64_fast(cc);
-        const double inv = __builtin_amdgcn_inverse_ballot_w64(mvalid & mbig) ? r : 0.0;
-        sr = __builtin_fma(cv[f] - cv[e], inv, sr);
-        si = __builtin_fma(sv[f] - sv[e], inv, si);
-        const bool rare = __builtin_amdgcn_inverse_ballot_w64(mvalid & ~mbig) && !small;
-        if (__builtin_expect(rare, 0)) {
-            const double *w = vx + (size_t)e * VX_STRIDE;
-            const double dx = uniform_f64(w[VX_DX]), dy = uniform_f64(w[VX_DY]);
-            const double2 q =
-                stable_edge_quotient(cv[e], sv[e], cv[f], sv[f], useB ? dx : dy, cc, k);
-            sr += q.x;
-            si += q.y;
-        }
-    }
-}
-
 // A lane holds its direction d as 1024 d, so that phases come out in nodes.
 constexpr double kNode = 1.0 / kPhasorN;
 static_assert(kPhasorN == kTabN, "both precisions count phases in the same nodes");
 
-// Aperture integral F(beam, direction) / complWave in FP64 (A4).  NV > 0
-// is the vertex count known at compile time (the loops are unrolled, the
-// scalar loads issued up front and every vertex's table read issued before
-// the first is used); NV = 0 loops over nv.  Returns false when
-// the result is NaN (degenerate beam, skipped).
-template <int NV>
+// Nodes of a radian, and a node in radians.
+constexpr double kNodes = kPhasorN * kInvTwoPi, kPerNode = 6.28318530717958647693 / kPhasorN;
+
+// The sum over the edges as the reference's two branches have it, in FP64: G = sum
+// (e^{i phi_{e+1}} - e^{i phi_e}) / c_e, where c = A + (dy/dx) B (|B| > |A|) or A
+// (dx/dy) + B (otherwise), and edges with |c| <= limit are left to
+// singular_edges_f64.  A, B in any unit (that of c and limit); `place` gives a
+// vertex's place between nodes and table entry.  NV > 0 is the vertex count known
+// at compile time: every vertex's table read is issued before the first is used.
+// No branch for the singular edges in here: one after every edge, and the flags read
+// for it, kept an edge's loads and instructions from passing those of the one
+// before.  4,000 beams with slopes of their own on 541 x 96 directions: 2.05 ms with
+// these, 1.76 without (of five vertices, one edge a turn: 3.41, now 2.06; the former
+// kernel, which rotated each beam and kept fewer sums, 1.60 to 1.77 and 2.1 to
+// 2.2).  An invalid edge's stored slope makes its reciprocal vanish.  Returns the
+// lanes with an edge within the limit.
+template <int NV, typename Place>
+__device__ __forceinline__ uint64_t edges_f64(const double *__restrict__ vtx, int nv, double A,
+                                              double B, bool useB, double limit, Place place,
+                                              double &sr, double &si)
+{
+    uint64_t near = 0;
+    sr = si = 0.0;
+    const auto edge = [&](int e, double sp, double cp, double sn, double cn) {
+        const double *v = vtx + e * VTX_STRIDE;
+        const double cx = __builtin_fma(uniform_f64(v[V_SYX]), B, A),
+                     cy = __builtin_fma(uniform_f64(v[V_SXY]), A, B);
+        const double cc = useB ? cx : cy;
+        const bool big = __builtin_fabs(cc) > limit;
+        const double inv = big ? rcp_f64_fast(cc) : 0.0;
+        near |= __builtin_amdgcn_ballot_w64(!big);
+        sr = __builtin_fma(cn - cp, inv, sr);
+        si = __builtin_fma(sn - sp, inv, si);
+    };
+    if constexpr (NV > 0) {
+        double r[NV], sv[NV], cv[NV];
+        double2 t[NV];
+#pragma unroll
+        for (int v = 0; v < NV; ++v)
+            place(v, r[v], t[v]);
+#pragma unroll
+        for (int v = 0; v < NV; ++v)
+            node_finish(r[v], t[v], sv[v], cv[v]);
+#pragma unroll
+        for (int e = 0; e < NV; ++e) {
+            const int f = e + 1 < NV ? e + 1 : 0;
+            edge(e, sv[e], cv[e], sv[f], cv[f]);
+        }
+    } else {  // two edges at a time (the compiler does not unroll loops that vote)
+        const auto vertex = [&](int v, double &sn, double &cs) {
+            double r;
+            double2 t;
+            place(v, r, t);
+            node_finish(r, t, sn, cs);
+        };
+        double s0, c0, sn, cn;
+        vertex(0, s0, c0);
+        double sp = s0, cp = c0;
+        int e = 0;
+        for (; e + 2 < nv; e += 2) {
+            vertex(e + 1, sn, cn);
+            edge(e, sp, cp, sn, cn);
+            vertex(e + 2, sp, cp);
+            edge(e + 1, sn, cn, sp, cp);
+        }
+        if (e + 1 < nv) {
+            vertex(e + 1, sn, cn);
+            edge(e, sp, cp, sn, cn);
+            sp = sn;
+            cp = cn;
+        }
+        edge(nv - 1, sp, cp, s0, c0);
+    }
+    return near;
+}
+
+// What the edges within the limit add to the sum of edges_f64, in a lane that has
+// one: the exact half-angle form.
+template <typename Place>
+__device__ __forceinline__ void singular_edges_f64(const double *__restrict__ vtx,
+                                                   const double *__restrict__ vx, int nv,
+                                                   double a, double b, bool useB, double limit,
+                                                   double k, Place place,
+                                                   double &sr, double &si)
+{
+    for (int e = 0; e < nv; ++e) {
+        const double *v = vtx + e * VTX_STRIDE, *w = vx + e * VX_STRIDE;
+        const double cc = useB ? __builtin_fma(uniform_f64(v[V_SYX]), b, a)
+                               : __builtin_fma(uniform_f64(v[V_SXY]), a, b);
+        if (__builtin_fabs(cc) > limit || !(vertex_flags(w, 0) & (useB ? EDGE_VX : EDGE_VY)))
+            continue;
+        double r, sp, cp, sn, cn;
+        double2 t;
+        place(e, r, t);
+        node_finish(r, t, sp, cp);
+        place(e + 1 < nv ? e + 1 : 0, r, t);
+        node_finish(r, t, sn, cn);
+        const double dx = uniform_f64(w[VX_DX]), dy = uniform_f64(w[VX_DY]);
+        const double2 q = stable_edge_quotient(cp, sp, cn, sn, useB ? dx : dy, kPerNode * cc, k);
+        sr = __builtin_fma(kPerNode, q.x, sr);
+        si = __builtin_fma(kPerNode, q.y, si);
+    }
+}
+
+// Aperture integral F(beam, direction) / complWave in FP64 by the reference's
+// branches.  k0, k1, k2: 1024 (d - b), d: 1024 times the direction.  Returns
+// false when the result is NaN (degenerate beam, skipped).
 __device__ __forceinline__ bool aperture_f64(const double *__restrict__ h,
                                              const double *__restrict__ vtx,
-                                             const double *__restrict__ vx, int nv,
-                                             const double *d, const double2 *__restrict__ tab,
-                                             double k, double eps1, double &fr, double &fi)
+                                             const double *__restrict__ vx, int nv, double k0,
+                                             double k1, double k2, const double *d,
+                                             const double2 *__restrict__ tab, double k,
+                                             double eps1, double &fr, double &fi)
 {
-    // A, B: projections of k - k0 = b - d on the aperture axes
-    const double d0 = d[0] * kNode, d1 = d[1] * kNode, d2 = d[2] * kNode;
-    const double A = h[H_A0] - (d0 * h[H_HOR] + d1 * h[H_HOR + 1] + d2 * h[H_HOR + 2]);
-    const double B = h[H_B0] - (d0 * h[H_VER] + d1 * h[H_VER + 1] + d2 * h[H_VER + 2]);
-    const double psi = d0 * h[H_KC] + d1 * h[H_KC + 1] + d2 * h[H_KC + 2];
-    const bool useB = __builtin_fabs(B) > __builtin_fabs(A);
-    const uint64_t mB = __builtin_amdgcn_ballot_w64(useB);  // lanes summing the dx-valid edges
-    // psi is folded into the vertex phasors (the integral is linear in each
-    // phasor), as the reference CUDA path does (GpuDiffraction.cu:1110-1122)
-    double sr = 0.0, si = 0.0;
-    bool small;
-    if constexpr (NV > 0) {
-        // all vertex phasors first (scalar loads, then every table read), so
-        // the LDS latency of one vertex overlaps the others; then the edges
-        double kx[NV], ky[NV];
-#pragma unroll
-        for (int e = 0; e < NV; ++e) {
-            kx[e] = uniform_f64(vtx[(size_t)e * VTX_STRIDE + V_KX]);
-            ky[e] = uniform_f64(vtx[(size_t)e * VTX_STRIDE + V_KY]);
-        }
-        const double phb = uniform_f64(h[H_PHB]);
-        double dv[NV];
-        double2 ev[NV];
-#pragma unroll
-        for (int e = 0; e < NV; ++e)
-            sincos_reduce(__builtin_fma(A, kx[e], __builtin_fma(B, ky[e], psi)), tab, dv[e],
-                          ev[e]);
-        double sv[NV], cv[NV];
-#pragma unroll
-        for (int e = 0; e < NV; ++e)
-            node_finish(dv[e], ev[e], sv[e], cv[e]);
-        // the vertex phases one by one only where the beam's bound leaves
-        // the small-phase form possible, after the table reads are consumed
-        small = false;
-        if (__builtin_expect(__builtin_fabs(useB ? B : -A) <= phb, 0))
-            small = all_phases_small_nv<NV>(kx, ky, A, B);
-        double syx[NV], sxy[NV];
-        int fl[NV];
-#pragma unroll
-        for (int e = 0; e < NV; ++e) {
-            syx[e] = uniform_f64(vtx[(size_t)e * VTX_STRIDE + V_SYX]);
-            sxy[e] = uniform_f64(vtx[(size_t)e * VTX_STRIDE + V_SXY]);
-            fl[e] = vertex_flags(vx, e);
-        }
-        edge_sum_f64_nv<NV>(syx, sxy, fl, sv, cv, vx, A, B, useB, mB, k, eps1, small, sr, si);
-    } else {
-        small = false;
-        if (__builtin_expect(__builtin_fabs(useB ? B : -A) <= h[H_PHB], 0))
-            small = all_phases_small(vtx, nv, A, B);
-        double s0, c0;
-        sincos_table(__builtin_fma(A, vtx[V_KX], __builtin_fma(B, vtx[V_KY], psi)), tab, s0, c0);
-        double sp = s0, cp = c0;
-        for (int e = 0; e < nv; ++e)
-            edge_f64(e, nv, vtx, vx, A, B, psi, useB, mB, tab, k, eps1, s0, c0, sp, cp, sr, si,
-                     small);
+    // a word of the first, a middle and the last cache line of the vertices (four lie
+    // in two or three): they come beside the header, not after it
+    const double t0 = vtx[0], t1 = vtx[2 * VTX_STRIDE], t2 = vtx[nv * VTX_STRIDE - 1];
+    // the projections A, B of k - k0 = b - d on the aperture axes and psi = d . kc,
+    // times 1024 / 2 pi: a vertex's phase in nodes is a k x + b k y + c, psi folded in
+    // (the integral is linear in each phasor), as the reference CUDA path does
+    // (GpuDiffraction.cu:1110-1122).  The coefficients take the same a, b: rounded
+    // apart from the phases they would not cancel with them.
+    const double a = -kInvTwoPi * (k0 * h[H_HOR] + k1 * h[H_HOR + 1] + k2 * h[H_HOR + 2]);
+    const double b = -kInvTwoPi * (k0 * h[H_VER] + k1 * h[H_VER + 1] + k2 * h[H_VER + 2]);
+    const double c = kInvTwoPi * (d[0] * h[H_KC] + d[1] * h[H_KC + 1] + d[2] * h[H_KC + 2]);
+    const bool useB = __builtin_fabs(b) > __builtin_fabs(a);
+    asm volatile("" ::"s"(t0), "s"(t1), "s"(t2));
+    const auto place = [&](int v, double &r, double2 &t) {
+        const double *q = vtx + v * VTX_STRIDE;
+        node_reduce(__builtin_fma(a, uniform_f64(q[V_KX]),
+                                  __builtin_fma(b, uniform_f64(q[V_KY]), c)),
+                    tab, r, t);
+    };
+    const double limit = kNodes * eps1;
+    double sr, si;
+    uint64_t near;
+    if (nv == 4)
+        near = edges_f64<4>(vtx, 4, a, b, useB, limit, place, sr, si);
+    else if (nv == 3)
+        near = edges_f64<3>(vtx, 3, a, b, useB, limit, place, sr, si);
+    else
+        near = edges_f64<0>(vtx, nv, a, b, useB, limit, place, sr, si);
+    // the vertex phases one by one only where the beam's bound leaves the
+    // small-phase form possible
+    const double larger = useB ? b : -a;
+    bool small = false;
+    if (__builtin_expect(__builtin_fabs(larger) <= kNodes * h[H_PHB], 0))
+        small = all_phases_small(vtx, nv, a, b, kNodes * kSmallPhase);
+    if (__builtin_expect(near != 0, 0)) {
+        if (__builtin_amdgcn_inverse_ballot_w64(near) && !small)
+            singular_edges_f64(vtx, vx, nv, a, b, useB, limit, k, place, sr, si);
     }
-    const double nrm = rcp_f64(useB ? B : -A);
+    const double nrm = rcp_f64(kPerNode * kPerNode * larger);
     fr = sr * nrm;
     fi = si * nrm;
     if (__builtin_expect(small, 0)) {
         // small-phase moment form (HandlerPO_fast.h:161-216); the area limit
         // is stored divided by complWave
+        const double A = kPerNode * a, B = kPerNode * b;
         const double p1 = A * h[H_MOM] + B * h[H_MOM + 1];
         const double p2 = A * A * h[H_MOM + 2] + A * B * h[H_MOM + 3] + B * B * h[H_MOM + 4];
         const double gr = 1.0 - 0.5 * p2, gi = p1;
         const double ar = h[H_AL] * gr - h[H_AL + 1] * gi;
         const double ai = h[H_AL] * gi + h[H_AL + 1] * gr;
-        double sd, cd;
-        sincos_table(psi, tab, sd, cd);
+        double r, sd, cd;
+        double2 t;
+        node_reduce(c, tab, r, t);
+        node_finish(r, t, sd, cd);
         fr = ar * cd - ai * sd;
         fi = ar * sd + ai * cd;
     }
@@ -1110,15 +1105,12 @@ __device__ __forceinline__ uint64_t aperture_any_f64(const double *eb, const dou
     if (__builtin_expect(general != 0, 0)) {
         bool ok = true;
         if (__builtin_amdgcn_inverse_ballot_w64(general)) {
-            if (nv == 4)
-                ok = aperture_f64<4>(h, vtx, vx, 4, d, tab, k, eps1, fr, fi);
-            else if (nv == 3)
-                ok = aperture_f64<3>(h, vtx, vx, 3, d, tab, k, eps1, fr, fi);
-            else
-                ok = aperture_f64<0>(h, vtx, vx, nv, d, tab, k, eps1, fr, fi);
-            const double inv = 1.0 / eb[EB_S64];
-            fr *= inv;
-            fi *= inv;
+            ok = aperture_f64(h, vtx, vx, nv, k0, k1, k2, d, tab, k, eps1, fr, fi);
+            if (cls != BEAM_SLOPES) {  // whose EB_S64 is 1
+                const double inv = rcp_f64(eb[EB_S64]);
+                fr *= inv;
+                fi *= inv;
+            }
         }
         dead = __builtin_amdgcn_ballot_w64(!ok);
     }
@@ -1197,56 +1189,100 @@ __device__ __forceinline__ void moments_mixed(const double *__restrict__ h, doub
 }
 
 // The edge sum over the reference's branches, as the ABI's slopes and flags
-// define it, for any vertex count and any phase: beams of class BEAM_SLOPES,
-// and single lanes of other beams next to a singular edge.  The edge
-// coefficient is cancellation-prone and stays in FP64; edges with |C| <=
-// eps1 take the half-angle form.
-__device__ __forceinline__ void edges_mixed(const double *__restrict__ vtx,
-                                            const double *__restrict__ vx, int nv, double A,
-                                            double B, double psi,
-                                            const PhasorNode *__restrict__ tab, double k,
-                                            double eps1, float &out_r, float &out_s)
+// define it: beams of class BEAM_SLOPES and BEAM_FAR, and single lanes of other
+// beams next to a singular edge.  As edges_f64, with `word` giving a vertex's
+// phase word; the edge coefficient is cancellation-prone and stays in FP64.
+template <int NV, typename Word>
+__device__ __forceinline__ uint64_t edges_mixed(const double *__restrict__ vtx, int nv, double A,
+                                                double B, bool useB, double limit,
+                                                const PhasorNode *__restrict__ tab, Word word,
+                                                float &sr, float &ss)
 {
-    const bool useB = __builtin_fabs(B) > __builtin_fabs(A);
-    const int vmask = useB ? EDGE_VX : EDGE_VY;
-    float c0, s0;
-    phasor_rad(__builtin_fma(A, vtx[V_KX], __builtin_fma(B, vtx[V_KY], psi)), tab, c0, s0);
-    float cp = c0, sp = s0, sr = 0.0f, ss = 0.0f;
-    for (int e = 0; e < nv; ++e) {
-        const double *v = vtx + (size_t)e * VTX_STRIDE;
-        const double syx = uniform_f64(v[V_SYX]), sxy = uniform_f64(v[V_SXY]);
-        const int f = vertex_flags(vx, e);
-        float cn = c0, sn = s0;
-        if (e + 1 < nv) {
-            const double xn = __builtin_fma(B, v[VTX_STRIDE + V_KY], psi);
-            phasor_rad(__builtin_fma(A, v[VTX_STRIDE + V_KX], xn), tab, cn, sn);
-        }
-        const double cc = useB ? __builtin_fma(syx, B, A) : __builtin_fma(sxy, A, B);
-        const bool big = __builtin_fabs(cc) > eps1;
-        // an invalid edge's stored slope makes the reciprocal exactly zero
+    uint64_t near = 0;
+    sr = ss = 0.0f;
+    const auto edge = [&](int e, float cp, float sp, float cn, float sn) {
+        const double *v = vtx + e * VTX_STRIDE;
+        const double cx = __builtin_fma(uniform_f64(v[V_SYX]), B, A),
+                     cy = __builtin_fma(uniform_f64(v[V_SXY]), A, B);
+        const double cc = useB ? cx : cy;
+        const bool big = __builtin_fabs(cc) > limit;
         const float r = __builtin_amdgcn_rcpf((float)cc);
         const float inv = big ? r : 0.0f;
+        near |= __builtin_amdgcn_ballot_w64(!big);
         sr = __builtin_fmaf(cn - cp, inv, sr);
         ss = __builtin_fmaf(sn - sp, inv, ss);
-        if (__builtin_expect(!big && (f & vmask) != 0, 0)) {
-            const double *w = vx + (size_t)e * VX_STRIDE;
-            const double dd = useB ? uniform_f64(w[VX_DX]) : uniform_f64(w[VX_DY]);
-            const double2 q = stable_edge_quotient((double)cp, (double)(sp * kSqrt2), (double)cn,
-                                                   (double)(sn * kSqrt2), dd, cc, k);
-            sr += (float)q.x;
-            ss += (float)(q.y * (double)kInvSqrt2);
+    };
+    if constexpr (NV > 0) {
+        float cv[NV], sv[NV];
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            const uint32_t u = word(v);
+            phasor_finish(u, phasor_read(u, tab), cv[v], sv[v]);
         }
-        cp = cn;
-        sp = sn;
+#pragma unroll
+        for (int e = 0; e < NV; ++e) {
+            const int f = e + 1 < NV ? e + 1 : 0;
+            edge(e, cv[e], sv[e], cv[f], sv[f]);
+        }
+    } else {  // two edges at a time
+        const auto vertex = [&](int v, float &cs, float &sn) {
+            const uint32_t u = word(v);
+            phasor_finish(u, phasor_read(u, tab), cs, sn);
+        };
+        float c0, s0, cn, sn;
+        vertex(0, c0, s0);
+        float cp = c0, sp = s0;
+        int e = 0;
+        for (; e + 2 < nv; e += 2) {
+            vertex(e + 1, cn, sn);
+            edge(e, cp, sp, cn, sn);
+            vertex(e + 2, cp, sp);
+            edge(e + 1, cn, sn, cp, sp);
+        }
+        if (e + 1 < nv) {
+            vertex(e + 1, cn, sn);
+            edge(e, cp, sp, cn, sn);
+            cp = cn;
+            sp = sn;
+        }
+        edge(nv - 1, cp, sp, c0, s0);
     }
-    const float nrm = __builtin_amdgcn_rcpf(useB ? (float)B : -(float)A);
-    out_r = sr * nrm;
-    out_s = ss * nrm;
+    return near;
+}
+
+// As singular_edges_f64, a and b in nodes.
+template <typename Word>
+__device__ __forceinline__ void singular_edges_mixed(const double *__restrict__ vtx,
+                                                     const double *__restrict__ vx, int nv,
+                                                     double a, double b, bool useB, double limit,
+                                                     double k,
+                                                     const PhasorNode *__restrict__ tab,
+                                                     Word word, float &sr, float &ss)
+{
+    for (int e = 0; e < nv; ++e) {
+        const double *v = vtx + e * VTX_STRIDE, *w = vx + e * VX_STRIDE;
+        const double cc = useB ? __builtin_fma(uniform_f64(v[V_SYX]), b, a)
+                               : __builtin_fma(uniform_f64(v[V_SXY]), a, b);
+        if (__builtin_fabs(cc) > limit || !(vertex_flags(w, 0) & (useB ? EDGE_VX : EDGE_VY)))
+            continue;
+        float cp, sp, cn, sn;
+        uint32_t u = word(e);
+        phasor_finish(u, phasor_read(u, tab), cp, sp);
+        u = word(e + 1 < nv ? e + 1 : 0);
+        phasor_finish(u, phasor_read(u, tab), cn, sn);
+        const double dx = uniform_f64(w[VX_DX]), dy = uniform_f64(w[VX_DY]);
+        const double2 q = stable_edge_quotient((double)cp, (double)(sp * kSqrt2), (double)cn,
+                                               (double)(sn * kSqrt2), useB ? dx : dy, kPerNode * cc,
+                                               k);
+        sr += (float)(kPerNode * q.x);
+        ss += (float)(kPerNode * q.y * (double)kInvSqrt2);
+    }
 }
 
 // F' of the lanes that the formulas over edge 0 leave: those with small phases
 // (`maybe` those to be tested for it) by the moments, those next to a singular
-// edge, and every lane of a BEAM_SLOPES beam, by the reference's branches.
+// edge, and every lane of a BEAM_SLOPES or BEAM_FAR beam, by the reference's
+// branches.
 __device__ __forceinline__ void fix_lanes(const double *eb, const double *__restrict__ h,
                                           const double *__restrict__ vtx,
                                           const double *__restrict__ vx, int nv, int cls,
@@ -1260,13 +1296,30 @@ __device__ __forceinline__ void fix_lanes(const double *eb, const double *__rest
     const double A = k0 * h[H_HOR] + k1 * h[H_HOR + 1] + k2 * h[H_HOR + 2];
     const double B = k0 * h[H_VER] + k1 * h[H_VER + 1] + k2 * h[H_VER + 2];
     const double psi = kNode * (d[0] * h[H_KC] + d[1] * h[H_KC + 1] + d[2] * h[H_KC + 2]);
-    const bool small =
-        maybe && (cls == BEAM_MOMENTS || all_phases_small(vtx, nv, A, B, kSmallPhaseMixed));
+    bool small = maybe;
+    if (cls == BEAM_FAR)  // (the other classes' steps have told)
+        small = __builtin_fmax(__builtin_fabs(A), __builtin_fabs(B)) <=
+                (kSmallPhaseMixed / kSmallPhase) * h[H_PHB];
+    if (cls != BEAM_MOMENTS)
+        small = small && all_phases_small(vtx, nv, A, B, kSmallPhaseMixed);
     if (singular && !small) {
-        const float inv = high_float(eb[EB_SCALE]);
-        edges_mixed(vtx, vx, nv, A, B, psi, tab, k, eps1, out_r, out_s);
-        out_r *= inv;
-        out_s *= inv;
+        const double a = kNodes * A, b = kNodes * B, c = kNodes * psi;
+        const bool useB = __builtin_fabs(b) > __builtin_fabs(a);
+        const auto word = [&](int v) {  // of any size: to half a turn first
+            const double *q = vtx + v * VTX_STRIDE;
+            const double p = __builtin_fma(a, uniform_f64(q[V_KX]),
+                                           __builtin_fma(b, uniform_f64(q[V_KY]), c));
+            return low_bits(__builtin_fma(-(double)kPhasorN, __builtin_rint(kNode * p), p) +
+                            kNodeMagic);
+        };
+        float sr, ss;
+        const uint64_t near = edges_mixed<0>(vtx, nv, a, b, useB, kNodes * eps1, tab, word, sr, ss);
+        if (__builtin_amdgcn_inverse_ballot_w64(near))
+            singular_edges_mixed(vtx, vx, nv, a, b, useB, kNodes * eps1, k, tab, word, sr, ss);
+        const float nrm = __builtin_amdgcn_rcpf((float)(useB ? b : -a)) *
+                          ((float)(kNodes * kNodes) * high_float(eb[EB_SCALE]));
+        out_r = sr * nrm;
+        out_s = ss * nrm;
     }
     if (small)
         moments_mixed(h, A, B, psi, h[H_INV], tab, out_r, out_s);
@@ -1470,6 +1523,35 @@ __device__ __forceinline__ void aperture_loop(const double *eb, const double *__
     maybe = __builtin_amdgcn_ballot_w64(steps <= (float)kLookStep);
 }
 
+// The edge sum with the slopes as given, for phases within the fixed-point range
+// (BEAM_SLOPES).  Nothing of the header is read on the way: with it, every vertex's
+// phase tested for the moments, and a branch and flags for each edge, a beam waited
+// for load after load (4,000 beams on 541 x 96 directions: 1.73 ms, now 0.98; on
+// the vector ALU 1.59, now 0.97; the former kernel 1.01 and 0.95).  Lanes with a
+// singular edge, or phases that may all be small, go to fix_lanes.
+__device__ __forceinline__ void aperture_slopes(const double *eb, const double *__restrict__ vtx,
+                                                int nv, const double *d,
+                                                const PhasorNode *__restrict__ tab, double eps1,
+                                                float &out_r, float &out_s, uint64_t &singular,
+                                                uint64_t &maybe)
+{
+    const Projection p = project(eb, d);
+    const bool useB = __builtin_fabs(p.b) > __builtin_fabs(p.a);
+    const auto word = [&](int v) { return low_bits(vertex_phase(p, vtx + v * VTX_STRIDE)); };
+    float sr, ss;
+    if (nv == 4)
+        singular = edges_mixed<4>(vtx, 4, p.a, p.b, useB, kNodes * eps1, tab, word, sr, ss);
+    else if (nv == 3)
+        singular = edges_mixed<3>(vtx, 3, p.a, p.b, useB, kNodes * eps1, tab, word, sr, ss);
+    else
+        singular = edges_mixed<0>(vtx, nv, p.a, p.b, useB, kNodes * eps1, tab, word, sr, ss);
+    const float q = (float)(useB ? p.b : -p.a);
+    const float nrm = __builtin_amdgcn_rcpf(q) * (float)(kNodes * kNodes);
+    out_r = sr * nrm;
+    out_s = ss * nrm;
+    maybe = __builtin_amdgcn_ballot_w64(__builtin_fabsf(q) <= low_float(eb[EB_LIM]));
+}
+
 // F' = F / complWave / s of a beam in a direction, s = 1 / the second half of its
 // EB_SCALE, mixed precision: FP64 phases and moments, FP32 phasors and sums.  eb: the
 // beam's record (in registers).  Returns the real part and the imaginary part /
@@ -1495,8 +1577,10 @@ __device__ __forceinline__ void aperture_mixed(const double *eb, const double *_
             aperture_quad(eb, vtx, vx, d, tab, out_r, out_s, singular, maybe);
         else
             aperture_loop(eb, vtx, vx, nv, d, tab, out_r, out_s, maybe);
+    } else if (cls == BEAM_SLOPES) {
+        aperture_slopes(eb, vtx, nv, d, tab, eps1, out_r, out_s, singular, maybe);
     } else {
-        singular = cls == BEAM_SLOPES ? ~0ull : 0;
+        singular = cls == BEAM_MOMENTS ? 0 : ~0ull;
         maybe = ~0ull;
     }
     if (__builtin_expect((singular | maybe) != 0, 0)) {

@@ -52,9 +52,10 @@ enum { WB_COLS = 24, WB_WORDS = 4, WB_STRIDE = 2 * WB_COLS * WB_WORDS };
 //                     takes the moments
 //   BEAM_SLOPES       the edge sum with the slopes as given: a polygon whose
 //                     slopes or flags say something else than its vertices,
-//                     with a degenerate edge, a value that is not finite, axes
-//                     longer than 1, or phases beyond the fixed-point range
-enum { BEAM_VERTICES, BEAM_TRAPEZOID, BEAM_PARALLEL, BEAM_MOMENTS, BEAM_SLOPES };
+//                     with a degenerate edge, or axes longer than 1
+//   BEAM_FAR          (mixed kernels) the same where phases leave the fixed-point
+//                     range, and where a value is not finite
+enum { BEAM_VERTICES, BEAM_TRAPEZOID, BEAM_PARALLEL, BEAM_MOMENTS, BEAM_SLOPES, BEAM_FAR };
 enum { BEAM_CLASS = 32, BEAM_NV = 31 };
 
 // Record of the aperture integral, EB_STRIDE doubles per beam.  Phases and steps
@@ -63,8 +64,9 @@ enum {
     EB_DIR = 0,    // 1024 b, b the beam direction (3)
     EB_PHASE = 3,  // mixed: -k centre . b, reduced to a turn, plus kNodeMagic (and a
                    // quarter turn for BEAM_TRAPEZOID and BEAM_VERTICES)
-    EB_LIM = 4,    // mixed, two FP32: |step| of edge 0 below which a lane is looked at,
-                   // and below which it counts as singular
+    EB_LIM = 4,    // mixed, two FP32: |step| of edge 0 below which a lane is looked at
+                   // (BEAM_SLOPES: max(|A|, |B|), in nodes), and below which it
+                   // counts as singular
     EB_SCALE = 5,  // mixed, two FP32: (F / F') / EB_S64 and 1 / (F / F'), F' what the
                    // class's formula gives
     EB_KIND = 6,   // the mixed class word; the FP64 class times 2, plus 1 for an

@@ -12,9 +12,7 @@
 namespace mbs {
 
 constexpr double kPi = 3.141592653589793116;            // double(pi) = M_PI
-// 1 / (2 pi) and the rest of it
-constexpr double kInvTwoPi = 0.15915494309189533577;
-constexpr double kInvTwoPiRest = -9.8393375401186e-18;
+constexpr double kInvTwoPi = 0.15915494309189533577;  // 1 / (2 pi)
 // Small-phase switch: every vertex phase within 1e-3 rad
 // (HandlerPO_fast.h:161-216).
 constexpr double kSmallPhase = 1e-3;
@@ -26,13 +24,11 @@ constexpr double kSmallPhaseMixed = 0.25;
 
 // Slope stored for an edge that is not valid in that direction (|dx| or
 // |dy| below the reference's geometric tolerance).  Its coefficient
-// A + s B (or s A + B) is then at least 1e300 times the lane's larger
-// projection, so the mixed kernels' FP32 reciprocal of it is exactly zero
-// and the edge drops out of the sum with no per-lane validity test; only a
-// lane with both projections below 1e-300 (every vertex phase tiny, so it
-// takes the moment form) sees a small coefficient.  The FP64 kernels mask
-// invalid edges by their flags and never use the value.
-constexpr double kInvalidSlope = 1e300;
+// A + s B (or s A + B) is then 1e30 times the lane's larger projection, and what
+// it adds below 1e-22 of any valid edge's share, so the edge drops out of the sum
+// with no per-lane validity test; only a lane with both projections near 1e-30
+// (every vertex phase tiny, so it takes the moment form) sees a small coefficient.
+constexpr double kInvalidSlope = 1e30;
 // One Horner step p*z + c as a single three-operand v_fma_f64 with the
 // coefficient in an SGPR pair.  Written as inline assembly because the
 // compiler otherwise keeps loop-invariant FP64 coefficients in VGPRs and
@@ -96,27 +92,6 @@ __device__ __forceinline__ double node_sine(double r, double2 e)
     double sd, cd;
     node_poly(r, sd, cd);
     return __builtin_fma(e.y, cd, e.x * sd);
-}
-
-// sin and cos of an angle in radians: to nodes in two parts, the second the
-// rounding of the product and of 1024 / (2 pi).
-__device__ __forceinline__ void sincos_reduce(double x, const double2 *__restrict__ tab,
-                                              double &r, double2 &e)
-{
-    const double p = x * (kTabN * kInvTwoPi);
-    const double rest = __builtin_fma(x, kTabN * kInvTwoPiRest,
-                                      __builtin_fma(x, kTabN * kInvTwoPi, -p));
-    node_reduce(p, tab, r, e);
-    r += rest;
-}
-
-__device__ __forceinline__ void sincos_table(double x, const double2 *__restrict__ tab,
-                                             double &s, double &c)
-{
-    double r;
-    double2 e;
-    sincos_reduce(x, tab, r, e);
-    node_finish(r, e, s, c);
 }
 
 // ---------------------------------------------------------------------------
