@@ -944,6 +944,23 @@ static bool plan_items(mbs_ctx *ctx, int n_tiles, int target, int work_mode,
     return false;
 }
 
+// Work items of the incoherent sum, which keeps a Mueller grid each: beam segments
+// (while they fit the budget) if the longest orientation has at least four beams
+// for every orientation there is, else runs of whole orientations.  Splitting an
+// orientation saves its workgroups up to 0.7 us a beam; each item more costs the
+// reduction, which adds them one after the other, 0.2 to 0.5 us, and 128 bytes a
+// direction.  Segments and whole orientations: one of 300 beams on 181 x 48
+// directions 55 and 228 us, 16 of 300 0.35 and 0.47 ms, 30 of 60 on 91 x 16 84 and 73
+// us, 100 of 20 105 and 73, 500 of 230 1.82 and 1.44 ms; 5,000 of 8 on 181 x 48 6.9
+// and 5.5 ms, with 5.6 GB of partial grids against 2.1.
+static int incoherent_mode(const mbs_ctx *ctx)
+{
+    int64_t longest = 0;
+    for (int o = 0; o < ctx->n_orient; ++o)
+        longest = std::max(longest, ctx->h_ooff[o + 1] - ctx->h_ooff[o]);
+    return longest >= 4 * (int64_t)ctx->n_orient ? MBS_WORK_AUTO : MBS_WORK_ORIENTATIONS;
+}
+
 template <int PREC, int NS, int JONES, int PER, int Q>
 static void launch_one(const KernelArgs &a, int blocks, hipStream_t s)
 {
@@ -1166,9 +1183,8 @@ int mbs_diffract(mbs_ctx *ctx, uint32_t flags)
         n_items = ctx->queue_want + ctx->n_orient;  // the most the device plan makes
         ctx->h_items.clear();
     } else {
-        // the incoherent sum keeps Mueller sums, of beam segments too while they fit
         if (incoh)
-            plan_items(ctx, n_tiles, target, 0, ctx->h_items, 16);
+            plan_items(ctx, n_tiles, target, incoherent_mode(ctx), ctx->h_items, 16);
         jones = !incoh && plan_items(ctx, n_tiles, target,
                                      mode == MBS_WORK_QUEUE ? MBS_WORK_SEGMENTS : mode,
                                      ctx->h_items);
