@@ -45,6 +45,18 @@ _i64p = C.POINTER(C.c_int64)
 _u8p = C.POINTER(C.c_uint8)
 
 
+# Device bytes of an uploaded batch (csrc/po_layout.h): the input block and the
+# packed records, per beam and per vertex
+BEAM_DEVICE_BYTES = (BEAM_SCALARS * 8 + 4 + 4 + 8) + (36 + 24 + 24) * 8 + 2 * 24 * 4 * 4
+VERTEX_DEVICE_BYTES = (4 * 8 + 1) + (4 + 4) * 8
+
+
+def device_bytes(n_beams, n_vert):
+    """Device memory that a batch of n_beams beams with n_vert vertices in all takes
+    once it is uploaded (without partial sums and results)."""
+    return n_beams * BEAM_DEVICE_BYTES + n_vert * VERTEX_DEVICE_BYTES
+
+
 class mbs_beam_batch(C.Structure):
     _fields_ = [("n_orient", C.c_int32), ("n_beams", C.c_int32),
                 ("orient_offsets", _i64p), ("weights", _dp),

@@ -93,6 +93,7 @@ struct mbs_ctx {
     Part<uint8_t> ef_in;
     DevBuf<double> hdr, w64, vtx, vx;
     DevBuf<uint32_t> wb;          // MFMA operand of the mixed kernels
+    bool wb_held = false;         // a captured graph may read wb: it stays
     DevBuf<double> ebeam;         // aperture records
     DevBuf<PhasorNode> phasor;    // phasor nodes of the mixed kernels
     DevBuf<double2> turns;        // phasors of the FP64 kernels
@@ -191,6 +192,39 @@ static int fail(mbs_ctx *ctx, int code, const char *fmt, ...)
             return fail((ctx), MBS_ERR_DEVICE, "%s failed: %s", #call,            \
                         hipGetErrorString(e_));                                   \
     } while (0)
+
+// Device memory of a context.  Where there is none left, the MFMA operand (768 bytes a
+// beam, more than a third of a batch) gives up its own, if that is enough: without it
+// the mixed kernels take the vector ALU until the next upload.  So a batch needs no
+// more than its input and 928 bytes a beam (four vertices): 1,364 with the input, and
+// 2,132 with the operand.  An operand that mbs_diffract_noalloc has handed to a launch
+// stays, since a graph may hold that launch, until an upload moves the other records
+// too.
+template <typename T>
+static hipError_t room(mbs_ctx *ctx, DevBuf<T> &buf, size_t n)
+{
+    hipError_t e = buf.ensure(n);
+    if (e == hipSuccess)
+        return e;
+    (void)hipGetLastError();  // told here, not by the next launch
+    size_t free_bytes = 0, total = 0;
+    if (e == hipErrorOutOfMemory && ctx->wb.p && !ctx->wb_held &&
+        hipMemGetInfo(&free_bytes, &total) == hipSuccess &&
+        free_bytes + ctx->wb.cap * sizeof(uint32_t) >= n * sizeof(T)) {
+        (void)hipStreamSynchronize(ctx->stream);  // a launch may still read it
+        ctx->wb.release();
+        e = buf.ensure(n);
+        if (e != hipSuccess)
+            (void)hipGetLastError();
+    }
+    return e;
+}
+
+// Whether the batch's MFMA operand is there.
+static bool have_operand(const mbs_ctx *ctx)
+{
+    return ctx->wb.cap >= (size_t)std::max(ctx->n_beams, 1) * WB_STRIDE;
+}
 
 // Scratch memory of mbs_diffract_noalloc (work list and partial sums): one
 // fixed array per device, held until the process ends.  In host code
@@ -432,12 +466,12 @@ int mbs_set_grid(mbs_ctx *ctx, const mbs_grid *g)
     ctx->n_zen1 = g->n_zen + 1;
     ctx->cells = (int)cells;
     ctx->az_step = g->az_step;
-    HIP_TRY(ctx, ctx->theta.ensure(ctx->n_zen1));
-    HIP_TRY(ctx, ctx->vf.ensure((size_t)cells * 3));
-    HIP_TRY(ctx, ctx->tab.ensure((size_t)cells * DT_COUNT));
-    HIP_TRY(ctx, ctx->tab32.ensure((size_t)cells * DT32_COUNT));
-    HIP_TRY(ctx, ctx->phasor.ensure(kPhasorN));
-    HIP_TRY(ctx, ctx->turns.ensure(kTabN));
+    HIP_TRY(ctx, room(ctx, ctx->theta, ctx->n_zen1));
+    HIP_TRY(ctx, room(ctx, ctx->vf, (size_t)cells * 3));
+    HIP_TRY(ctx, room(ctx, ctx->tab, (size_t)cells * DT_COUNT));
+    HIP_TRY(ctx, room(ctx, ctx->tab32, (size_t)cells * DT32_COUNT));
+    HIP_TRY(ctx, room(ctx, ctx->phasor, kPhasorN));
+    HIP_TRY(ctx, room(ctx, ctx->turns, kTabN));
     HIP_TRY(ctx, hipMemcpyAsync(ctx->theta.p, g->theta, sizeof(double) * ctx->n_zen1,
                                 hipMemcpyHostToDevice, ctx->stream));
     HIP_TRY(ctx, hipMemcpyAsync(ctx->vf.p, g->vf, sizeof(double) * cells * 3,
@@ -489,7 +523,8 @@ static int launch_pack(mbs_ctx *ctx, int nb, const mbs_consts &c, double scale, 
         sg * c.inv_compl_wave[1], c.compl_wave[0], c.compl_wave[1], rescale ? scale : 1.0,
         rescale ? ctx->sc_raw.p : nullptr, ctx->sc_path.p, ctx->sc_sign.p, ctx->sc_aoff.p,
         ctx->sc_apath.p, ctx->sc_cabs, ctx->sc_k, c.eps1, mixed_eps(c), ctx->hdr.p, ctx->w64.p,
-        ctx->vtx.p, ctx->vx.p, ctx->wb.p, ctx->ebeam.p);
+        ctx->vtx.p, ctx->vx.p, ctx->wb.cap < (size_t)nb * WB_STRIDE ? nullptr : ctx->wb.p,
+        ctx->ebeam.p);
     HIP_TRY(ctx, hipGetLastError());
     return MBS_OK;
 }
@@ -663,7 +698,11 @@ static int upload_impl(mbs_ctx *ctx, const mbs_beam_batch *bt, const mbs_consts 
     HIP_TRY(ctx, hipSetDevice(ctx->device));
     size_t off[11];
     const size_t total = stage_layout(no, nb, nvert, off);
-    HIP_TRY(ctx, ctx->input.ensure(total));
+    if (total > ctx->input.cap || (size_t)nb * HDR_STRIDE > ctx->hdr.cap ||
+        (size_t)nb * EB_STRIDE > ctx->ebeam.cap || (size_t)nb * W64_STRIDE > ctx->w64.cap ||
+        (size_t)nvert * VTX_STRIDE > ctx->vtx.cap || (size_t)nvert * VX_STRIDE > ctx->vx.cap)
+        ctx->wb_held = false;
+    HIP_TRY(ctx, room(ctx, ctx->input, total));
     unsigned char *in = ctx->input.p;
     ctx->ooff.p = (int64_t *)(in + off[0]);
     ctx->weights.p = (double *)(in + off[1]);
@@ -676,12 +715,14 @@ static int upload_impl(mbs_ctx *ctx, const mbs_beam_batch *bt, const mbs_consts 
     ctx->syx_in.p = (double *)(in + off[8]);
     ctx->sxy_in.p = (double *)(in + off[9]);
     ctx->ef_in.p = (uint8_t *)(in + off[10]);
-    HIP_TRY(ctx, ctx->hdr.ensure((size_t)nb * HDR_STRIDE));
-    HIP_TRY(ctx, ctx->ebeam.ensure((size_t)nb * EB_STRIDE));
-    HIP_TRY(ctx, ctx->w64.ensure((size_t)nb * W64_STRIDE));
-    HIP_TRY(ctx, ctx->vtx.ensure((size_t)nvert * VTX_STRIDE));
-    HIP_TRY(ctx, ctx->vx.ensure((size_t)nvert * VX_STRIDE));
-    HIP_TRY(ctx, ctx->wb.ensure((size_t)std::max(nb, 1) * WB_STRIDE));
+    HIP_TRY(ctx, room(ctx, ctx->hdr, (size_t)nb * HDR_STRIDE));
+    HIP_TRY(ctx, room(ctx, ctx->ebeam, (size_t)nb * EB_STRIDE));
+    HIP_TRY(ctx, room(ctx, ctx->w64, (size_t)nb * W64_STRIDE));
+    HIP_TRY(ctx, room(ctx, ctx->vtx, (size_t)nvert * VTX_STRIDE));
+    HIP_TRY(ctx, room(ctx, ctx->vx, (size_t)nvert * VX_STRIDE));
+    // (without room for the operand the mixed kernels take the vector ALU)
+    if (ctx->wb.ensure((size_t)std::max(nb, 1) * WB_STRIDE) != hipSuccess)
+        (void)hipGetLastError();
     hipStream_t s = ctx->stream;
     if (ctx->timing)
         HIP_TRY(ctx, hipEventRecord(ctx->ev[0], s));
@@ -835,11 +876,11 @@ extern "C" int mbs_upload_beam_scaling(mbs_ctx *ctx, const mbs_beam_scaling *sc)
         if (sc->abs_offsets[b + 1] < sc->abs_offsets[b])
             return fail(ctx, MBS_ERR_INVALID, "abs_offsets decrease at %d", b);
     HIP_TRY(ctx, hipSetDevice(ctx->device));
-    HIP_TRY(ctx, ctx->sc_raw.ensure((size_t)nb * 8));
-    HIP_TRY(ctx, ctx->sc_path.ensure(nb));
-    HIP_TRY(ctx, ctx->sc_sign.ensure(nb));
-    HIP_TRY(ctx, ctx->sc_aoff.ensure((size_t)nb + 1));
-    HIP_TRY(ctx, ctx->sc_apath.ensure((size_t)na));
+    HIP_TRY(ctx, room(ctx, ctx->sc_raw, (size_t)nb * 8));
+    HIP_TRY(ctx, room(ctx, ctx->sc_path, nb));
+    HIP_TRY(ctx, room(ctx, ctx->sc_sign, nb));
+    HIP_TRY(ctx, room(ctx, ctx->sc_aoff, (size_t)nb + 1));
+    HIP_TRY(ctx, room(ctx, ctx->sc_apath, (size_t)na));
     hipStream_t s = ctx->stream;
     if (nb > 0) {
         HIP_TRY(ctx, hipMemcpyAsync(ctx->sc_raw.p, sc->raw_jones, sizeof(double) * 8 * nb,
@@ -1148,7 +1189,7 @@ int mbs_diffract(mbs_ctx *ctx, uint32_t flags)
     const bool mfma = !(flags & MBS_NO_MFMA) && !(tn.valid && !tn.mfma);
     const bool incoh = (flags & MBS_INCOHERENT) != 0;
     const bool spec = (flags & MBS_SPECTRUM) != 0;
-    const int prec = incoh ? 3 : spec ? 4 : base ? (mfma ? 2 : 1) : 0;
+    int prec = incoh ? 3 : spec ? 4 : base ? (mfma ? 2 : 1) : 0;
     const int ns = (flags & MBS_NOSHADOW) ? 1 : 0;
     const int per = (flags & MBS_PER_ORIENT) ? 1 : 0;
     if (flags & ~(uint32_t)(MBS_PREC_MIXED | MBS_NOSHADOW | MBS_PER_ORIENT | MBS_NO_MFMA |
@@ -1191,11 +1232,11 @@ int mbs_diffract(mbs_ctx *ctx, uint32_t flags)
         n_items = (int)ctx->h_items.size();
     }
     const size_t mcount = (size_t)cells * 16;
-    HIP_TRY(ctx, ctx->res.ensure(mcount));
+    HIP_TRY(ctx, room(ctx, ctx->res, mcount));
     if (ns)
-        HIP_TRY(ctx, ctx->res_ns.ensure(mcount));
+        HIP_TRY(ctx, room(ctx, ctx->res_ns, mcount));
     if (per)
-        HIP_TRY(ctx, ctx->per_orient.ensure((size_t)ctx->n_orient * mcount));
+        HIP_TRY(ctx, room(ctx, ctx->per_orient, (size_t)ctx->n_orient * mcount));
     hipStream_t s = ctx->stream;
     if (n_items == 0) {
         const int zb = (int)((mcount + 255) / 256);
@@ -1209,15 +1250,22 @@ int mbs_diffract(mbs_ctx *ctx, uint32_t flags)
         return MBS_OK;
     }
     const size_t pstride = (size_t)cells * (jones ? 8 : 16);
-    HIP_TRY(ctx, ctx->part.ensure((size_t)n_items * pstride));
+    HIP_TRY(ctx, room(ctx, ctx->part, (size_t)n_items * pstride));
     if (ns)
-        HIP_TRY(ctx, ctx->part_ns.ensure((size_t)n_items * pstride));
-    HIP_TRY(ctx, ctx->items.ensure(n_items));
+        HIP_TRY(ctx, room(ctx, ctx->part_ns, (size_t)n_items * pstride));
+    HIP_TRY(ctx, room(ctx, ctx->items, n_items));
     if (queue)
-        HIP_TRY(ctx, ctx->queue.ensure(Q_WORDS));
+        HIP_TRY(ctx, room(ctx, ctx->queue, Q_WORDS));
     else
         HIP_TRY(ctx, hipMemcpyAsync(ctx->items.p, ctx->h_items.data(),
                                     sizeof(WorkItem) * n_items, hipMemcpyHostToDevice, s));
+    if (!have_operand(ctx)) {  // there was no memory for it
+        if (prec == 4)
+            return fail(ctx, MBS_ERR_CAPACITY,
+                        "MBS_SPECTRUM: no device memory for the MFMA operand of %d beams",
+                        ctx->n_beams);
+        prec = prec == 2 ? 1 : prec;
+    }
     KernelArgs a;
     batch_args(ctx, prec, n_items, n_tiles, a);
     a.waves = tn.valid ? tn.waves : 0;
@@ -1318,7 +1366,8 @@ int mbs_diffract_noalloc(mbs_ctx *ctx, uint32_t flags, double *d_m_full, double 
         return fail(ctx, MBS_ERR_DEVICE, "no scratch address for device %d: %s", ctx->device,
                     hipGetErrorString(serr));
     const int base = (flags & MBS_PREC_MIXED) ? 1 : 0;
-    const int prec = base ? ((flags & MBS_NO_MFMA) ? 1 : 2) : 0;
+    const int prec = base ? ((flags & MBS_NO_MFMA) || !have_operand(ctx) ? 1 : 2) : 0;
+    ctx->wb_held = ctx->wb_held || prec == 2;
     HIP_TRY(ctx, hipSetDevice(ctx->device));
     int rc = ensure_tables(ctx);
     if (rc)
@@ -1579,7 +1628,7 @@ int mbs_azimuth_average(mbs_ctx *ctx, int noshadow, double *rows)
         return fail(ctx, MBS_ERR_INVALID, "no-shadow result was not requested (MBS_NOSHADOW)");
     HIP_TRY(ctx, hipSetDevice(ctx->device));
     const size_t n = (size_t)ctx->n_zen1 * 18;
-    HIP_TRY(ctx, ctx->avg_rows.ensure(n));
+    HIP_TRY(ctx, room(ctx, ctx->avg_rows, n));
     azimuth_average_kernel<<<ctx->n_zen1, 64, 0, ctx->stream>>>(
         noshadow ? ctx->res_ns.p : ctx->res.p, ctx->theta.p, ctx->n_az, ctx->n_zen1 - 1,
         ctx->az_step, ctx->avg_rows.p);
@@ -1595,7 +1644,7 @@ int mbs_azimuth_average_per_orient(mbs_ctx *ctx, double *rows)
         return fail(ctx, MBS_ERR_INVALID, "per-orientation result was not requested");
     HIP_TRY(ctx, hipSetDevice(ctx->device));
     const size_t n = (size_t)ctx->n_orient * ctx->n_zen1 * 18;
-    HIP_TRY(ctx, ctx->avg_rows.ensure(n));
+    HIP_TRY(ctx, room(ctx, ctx->avg_rows, n));
     azimuth_average_kernel<<<dim3(ctx->n_zen1, ctx->n_orient), 64, 0, ctx->stream>>>(
         ctx->per_orient.p, ctx->theta.p, ctx->n_az, ctx->n_zen1 - 1, ctx->az_step,
         ctx->avg_rows.p);
@@ -1637,8 +1686,8 @@ static int upsample_pass(mbs_ctx *ctx, const UpLines &g, int lines, const double
         return fail(ctx, MBS_ERR_CAPACITY, "upsampling: too many factors (%d -> %d)", g.n_in,
                     g.n_out);
     hipStream_t s = ctx->stream;
-    HIP_TRY(ctx, ctx->up_roots_in.ensure(g.n_in));
-    HIP_TRY(ctx, ctx->up_roots_out.ensure(g.n_out));
+    HIP_TRY(ctx, room(ctx, ctx->up_roots_in, g.n_in));
+    HIP_TRY(ctx, room(ctx, ctx->up_roots_out, g.n_out));
     up_roots_kernel<<<(g.n_in + 255) / 256, 256, 0, s>>>(g.n_in, ctx->up_roots_in.p);
     up_roots_kernel<<<(g.n_out + 255) / 256, 256, 0, s>>>(g.n_out, ctx->up_roots_out.p);
     HIP_TRY(ctx, hipGetLastError());
@@ -1681,7 +1730,7 @@ int mbs_upsample_result(mbs_ctx *ctx, int noshadow, int32_t n_az_out, int32_t n_
     const size_t mid = (size_t)n_az * (n_zen_out + 1) * 16;
     const size_t out = (size_t)n_az_out * (n_zen_out + 1) * 16;
     if (up_zen) {
-        HIP_TRY(ctx, ctx->up_a.ensure(mid));
+        HIP_TRY(ctx, room(ctx, ctx->up_a, mid));
         UpLines g{1, 2 * n_zen, 2 * n_zen_out, 2 * n_zen_out, n_zen + 1, n_zen, n_zen_out};
         int rc = upsample_pass(ctx, g, n_az * 8, cur, ctx->up_a.p);
         if (rc)
@@ -1689,7 +1738,7 @@ int mbs_upsample_result(mbs_ctx *ctx, int noshadow, int32_t n_az_out, int32_t n_
         cur = ctx->up_a.p;
     }
     if (up_az) {
-        HIP_TRY(ctx, ctx->up_b.ensure(out));
+        HIP_TRY(ctx, room(ctx, ctx->up_b, out));
         UpLines g{0, n_az, n_az_out, n_az_out, n_zen_out + 1, 0, 0};
         int rc = upsample_pass(ctx, g, (n_zen_out + 1) * 8, cur, ctx->up_b.p);
         if (rc)
@@ -1698,8 +1747,8 @@ int mbs_upsample_result(mbs_ctx *ctx, int noshadow, int32_t n_az_out, int32_t n_
     }
     if (rows_out) {
         const size_t n = (size_t)(n_zen_out + 1) * 18;
-        HIP_TRY(ctx, ctx->up_theta.ensure(n_zen_out + 1));
-        HIP_TRY(ctx, ctx->avg_rows.ensure(n));
+        HIP_TRY(ctx, room(ctx, ctx->up_theta, n_zen_out + 1));
+        HIP_TRY(ctx, room(ctx, ctx->avg_rows, n));
         HIP_TRY(ctx, hipMemcpyAsync(ctx->up_theta.p, theta_out, sizeof(double) * (n_zen_out + 1),
                                     hipMemcpyHostToDevice, ctx->stream));
         azimuth_average_kernel<<<n_zen_out + 1, 64, 0, ctx->stream>>>(
@@ -1734,7 +1783,7 @@ int mbs_orientation_set(mbs_ctx *ctx, int kind, int32_t n, uint32_t seed, double
                     "symmetry domain must satisfy 0 < beta <= pi and 0 < gamma <= 2*pi");
     HIP_TRY(ctx, hipSetDevice(ctx->device));
     const size_t count = (size_t)n * MBS_ORIENT_STRIDE;
-    HIP_TRY(ctx, ctx->orient.ensure(count));
+    HIP_TRY(ctx, room(ctx, ctx->orient, count));
     orientation_set_kernel<<<(n + 255) / 256, 256, 0, ctx->stream>>>(
         kind, n, seed, std::cos(beta_sym), gamma_sym, ctx->orient.p);
     HIP_TRY(ctx, hipGetLastError());
@@ -1774,13 +1823,13 @@ int mbs_aperture_fft(mbs_ctx *ctx, const int64_t *beams, int32_t n_beams, int32_
     int logn = 0;
     while ((1 << logn) < n)
         ++logn;
-    HIP_TRY(ctx, ctx->fft_grid.ensure((size_t)n_beams * n * n));
-    HIP_TRY(ctx, ctx->fft_rec.ensure((size_t)n_beams * FB_STRIDE));
-    HIP_TRY(ctx, ctx->fft_beams.ensure(n_beams));
+    HIP_TRY(ctx, room(ctx, ctx->fft_grid, (size_t)n_beams * n * n));
+    HIP_TRY(ctx, room(ctx, ctx->fft_rec, (size_t)n_beams * FB_STRIDE));
+    HIP_TRY(ctx, room(ctx, ctx->fft_beams, n_beams));
     hipStream_t s = ctx->stream;
     HIP_TRY(ctx, hipMemcpyAsync(ctx->fft_beams.p, beams, sizeof(int64_t) * n_beams,
                                 hipMemcpyHostToDevice, s));
-    HIP_TRY(ctx, ctx->fft_tw.ensure(n));
+    HIP_TRY(ctx, room(ctx, ctx->fft_tw, n));
     fft_twiddle_kernel<<<(n + 255) / 256, 256, 0, s>>>(n, ctx->fft_tw.p);
     fft_setup_kernel<<<(n_beams + 63) / 64, 64, 0, s>>>(n_beams, ctx->fft_beams.p, ctx->nv.p,
                                                        ctx->voff.p, ctx->vx_in.p, ctx->vy_in.p,
@@ -1806,8 +1855,8 @@ int mbs_aperture_fft(mbs_ctx *ctx, const int64_t *beams, int32_t n_beams, int32_
     ctx->fft_batch = n_beams;
     if (n_points > 0) {
         const size_t np = (size_t)n_beams * n_points;
-        HIP_TRY(ctx, ctx->fft_ab.ensure((size_t)n_points * 2));
-        HIP_TRY(ctx, ctx->fft_out.ensure(np * 2));
+        HIP_TRY(ctx, room(ctx, ctx->fft_ab, (size_t)n_points * 2));
+        HIP_TRY(ctx, room(ctx, ctx->fft_out, np * 2));
         HIP_TRY(ctx, hipMemcpyAsync(ctx->fft_ab.p, ab, sizeof(double) * 2 * n_points,
                                     hipMemcpyHostToDevice, s));
         fft_sample_kernel<<<(unsigned)((np + 255) / 256), 256, 0, s>>>(
@@ -1896,13 +1945,13 @@ int mbs_spectrum_source(mbs_ctx *ctx, const mbs_spectrum_params *p, mbs_spectrum
     for (hipEvent_t &e : ctx->fft_ev)
         if (!e)
             HIP_TRY(ctx, hipEventCreate(&e));
-    HIP_TRY(ctx, ctx->spec_sidx.ensure(nb));
+    HIP_TRY(ctx, room(ctx, ctx->spec_sidx, nb));
     std::vector<int32_t> sidx(nb, -1);
     std::vector<double> scan((size_t)nb * 5);
     std::vector<int32_t> nv(nb);
     std::vector<double> area(nb);
     if (nb > 0) {
-        HIP_TRY(ctx, ctx->spec_scan.ensure((size_t)nb * 5));
+        HIP_TRY(ctx, room(ctx, ctx->spec_scan, (size_t)nb * 5));
         HIP_TRY(ctx, hipEventRecord(ctx->fft_ev[0], s));
         spectrum_scan_kernel<<<nb, 256, 0, s>>>(nb, ctx->hdr.p, ctx->tab.p, cells, ctx->nv.p,
                                                 ctx->voff.p, ctx->vx_in.p, ctx->vy_in.p,
@@ -1979,17 +2028,17 @@ int mbs_spectrum_source(mbs_ctx *ctx, const mbs_spectrum_params *p, mbs_spectrum
     HIP_TRY(ctx, hipMemcpyAsync(ctx->spec_sidx.p, sidx.data(), nb * sizeof(int32_t),
                                 hipMemcpyHostToDevice, s));
     if (ns > 0) {
-        HIP_TRY(ctx, ctx->spec_beam.ensure(ns));
-        HIP_TRY(ctx, ctx->spec_logn.ensure(ns));
-        HIP_TRY(ctx, ctx->spec_band.ensure(ns));
-        HIP_TRY(ctx, ctx->spec_cph.ensure(max_n + 1));
-        HIP_TRY(ctx, ctx->spec_h.ensure(ns));
-        HIP_TRY(ctx, ctx->spec_off.ensure(ns));
-        HIP_TRY(ctx, ctx->spec_rec.ensure((size_t)ns * SP_STRIDE));
-        HIP_TRY(ctx, ctx->spec_grid.ensure((size_t)total));
-        HIP_TRY(ctx, ctx->spec_f.ensure((size_t)ns * cells));
-        HIP_TRY(ctx, ctx->fft_tw.ensure(max_n));
-        HIP_TRY(ctx, ctx->spec_deap.ensure(max_n));
+        HIP_TRY(ctx, room(ctx, ctx->spec_beam, ns));
+        HIP_TRY(ctx, room(ctx, ctx->spec_logn, ns));
+        HIP_TRY(ctx, room(ctx, ctx->spec_band, ns));
+        HIP_TRY(ctx, room(ctx, ctx->spec_cph, max_n + 1));
+        HIP_TRY(ctx, room(ctx, ctx->spec_h, ns));
+        HIP_TRY(ctx, room(ctx, ctx->spec_off, ns));
+        HIP_TRY(ctx, room(ctx, ctx->spec_rec, (size_t)ns * SP_STRIDE));
+        HIP_TRY(ctx, room(ctx, ctx->spec_grid, (size_t)total));
+        HIP_TRY(ctx, room(ctx, ctx->spec_f, (size_t)ns * cells));
+        HIP_TRY(ctx, room(ctx, ctx->fft_tw, max_n));
+        HIP_TRY(ctx, room(ctx, ctx->spec_deap, max_n));
         HIP_TRY(ctx, hipMemcpyAsync(ctx->spec_beam.p, sb.data(), ns * sizeof(int32_t),
                                     hipMemcpyHostToDevice, s));
         HIP_TRY(ctx, hipMemcpyAsync(ctx->spec_logn.p, sl.data(), ns * sizeof(int32_t),
@@ -2322,15 +2371,15 @@ int mlp_ensure_rows(mbs_mlp *m, int rows)
     m->z.resize(m->depth);
     m->a.resize(m->depth + 1);
     for (int l = 0; l <= m->depth; ++l)
-        HIP_TRY(ctx, m->a[l].ensure((size_t)rows * mlp_layer_in(m, l)));
+        HIP_TRY(ctx, room(ctx, m->a[l], (size_t)rows * mlp_layer_in(m, l)));
     for (int l = 0; l < m->depth; ++l)
-        HIP_TRY(ctx, m->z[l].ensure((size_t)rows * m->width));
-    HIP_TRY(ctx, m->y.ensure((size_t)rows * m->n_out));
-    HIP_TRY(ctx, m->t.ensure((size_t)rows * m->n_out));
-    HIP_TRY(ctx, m->dy.ensure((size_t)rows * m->n_out));
-    HIP_TRY(ctx, m->da.ensure((size_t)rows * m->width));
-    HIP_TRY(ctx, m->dz.ensure((size_t)rows * m->width));
-    HIP_TRY(ctx, m->row_sq.ensure(rows));
+        HIP_TRY(ctx, room(ctx, m->z[l], (size_t)rows * m->width));
+    HIP_TRY(ctx, room(ctx, m->y, (size_t)rows * m->n_out));
+    HIP_TRY(ctx, room(ctx, m->t, (size_t)rows * m->n_out));
+    HIP_TRY(ctx, room(ctx, m->dy, (size_t)rows * m->n_out));
+    HIP_TRY(ctx, room(ctx, m->da, (size_t)rows * m->width));
+    HIP_TRY(ctx, room(ctx, m->dz, (size_t)rows * m->width));
+    HIP_TRY(ctx, room(ctx, m->row_sq, rows));
     m->cap_rows = rows;
     return MBS_OK;
 }
@@ -2574,9 +2623,9 @@ int mbs_mlp_train(mbs_mlp *m, const float *x, const float *t, int32_t n, int32_t
     if (rc)
         return rc;
     hipStream_t s = ctx->stream;
-    HIP_TRY(ctx, m->x_all.ensure((size_t)n * m->n_in));
-    HIP_TRY(ctx, m->t_all.ensure((size_t)n * m->n_out));
-    HIP_TRY(ctx, m->idx.ensure(n));
+    HIP_TRY(ctx, room(ctx, m->x_all, (size_t)n * m->n_in));
+    HIP_TRY(ctx, room(ctx, m->t_all, (size_t)n * m->n_out));
+    HIP_TRY(ctx, room(ctx, m->idx, n));
     HIP_TRY(ctx, hipMemcpyAsync(m->x_all.p, x, sizeof(float) * n * m->n_in,
                                 hipMemcpyHostToDevice, s));
     HIP_TRY(ctx, hipMemcpyAsync(m->t_all.p, t, sizeof(float) * n * m->n_out,

@@ -668,8 +668,10 @@ __global__ void __launch_bounds__(PACK_THREADS) pack_beams_kernel(
         rotation(c, n, wr, wi);
         w64[(size_t)first * W64_STRIDE + i] = s_s64[c] * ((n & 1) ? wi : wr);
     }
-    // MFMA operand, split into three BF16 parts; a shadow beam's is zero: it is
-    // summed apart
+    // MFMA operand (if there was memory for it), split into three BF16 parts; a shadow
+    // beam's is zero: it is summed apart
+    if (!wb)
+        return;
     for (int i = threadIdx.x; i < count * (2 * WB_COLS); i += PACK_THREADS) {
         const int c = i / (2 * WB_COLS), e = i - c * (2 * WB_COLS);
         const int row = e / WB_COLS, n = e - row * WB_COLS;

@@ -142,7 +142,8 @@ class HandlerPOGpu:
     def SelectGpuOrientationBatchSize(self, prepared, start, maxCount):
         """HandlerPO::SelectGpuOrientationBatchSize (HandlerPO.h:145-147): the
         largest count from ``start`` whose device working set fits in 80 % of
-        free device memory (partials + packed beams), at least 1."""
+        free device memory (partials + the uploaded and the packed beams,
+        ``abi.device_bytes``), at least 1."""
         from .engine import lib
         import ctypes as C
         fr, tot = C.c_int64(), C.c_int64()
@@ -151,11 +152,11 @@ class HandlerPOGpu:
         budget = 0.8 * fr.value
         cells = self.grid.cells
         n = max(1, maxCount)
-        oo = prepared.orient_offsets
+        oo, vo = prepared.orient_offsets, prepared.vert_offsets
         while n > 1:
             end = min(prepared.n_orient, start + n)
-            beams = int(oo[end] - oo[start])
-            need = beams * (36 + 40 + 14 + 6 * 31) * 8 + 64 * cells * 16 * 8 * 2
+            b0, b1 = int(oo[start]), int(oo[end])
+            need = abi.device_bytes(b1 - b0, int(vo[b1] - vo[b0])) + 64 * cells * 16 * 8 * 2
             if need <= budget:
                 break
             n //= 2
