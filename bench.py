@@ -78,15 +78,16 @@ def calibrate_copy():
     print(json.dumps({"calibrate_copy_bytes": n, "launches": 3}))
 
 
-def algorithmic_bytes(batch, cells):
-    """HBM bytes one launch must move at least: the device beam records read
-    once (header 288 B, FP64 rotation data 192 B, aperture record 192 B, MFMA
-    operand 768 B per beam; vertex records 32 + 32 B per vertex), the grid tables
-    read once (15 FP64 per direction) and the Mueller grid written once (16 FP64
-    per direction)."""
-    n_vert = int(batch.vert_offsets[-1])
-    return float(batch.n_beams) * (288 + 192 + 192 + 768) + n_vert * 64.0 \
-        + cells * (15 + 16) * 8.0
+def algorithmic_bytes(batch, cells, kernel):
+    """HBM bytes one launch of a kernel ("mfma", "valu" or "fp64") must move at
+    least: each beam's aperture record (192 B) and what it multiplies F by (MFMA
+    operand 768 B, shadow beams and the other two kernels the FP64 polarisation
+    data of 192 B), the grid tables read once (3 FP64 and 12 FP32 per direction,
+    FP64 kernel 15 FP64) and the Mueller grid written once (16 FP64 per direction).
+    Headers and vertices, which only some polygons and lanes read, are not in it."""
+    operands = int((np.asarray(batch.beam_external) == 0).sum()) if kernel == "mfma" else 0
+    tables = 15 * 8.0 if kernel == "fp64" else 3 * 8.0 + 12 * 4.0
+    return batch.n_beams * (192 + 192.0) + operands * (768 - 192.0) + cells * (tables + 128.0)
 
 
 def cpu_model():
@@ -496,7 +497,6 @@ def run(args):
     grid = syn.config2_grid()
     flops_b, ne = unit_flops(batch)
     flops_launch = float(flops_b.sum()) * grid.cells
-    alg_bytes = algorithmic_bytes(batch, grid.cells)
     units = float(batch.n_beams) * grid.cells
     hip = Hip()
     ctx = eng.Context(0)
@@ -521,11 +521,11 @@ def run(args):
     results = {}
     traffic = measured_traffic()
 
-    def leg(name, flags, peak, mode=None, graph=False):
+    def leg(name, flags, peak, mode=None, graph=False, mfma=True):
         """Times args.steps calls of mbs_diffract(flags): wall per step, and
         the main kernel's mean duration from the engine's events (graph
         replay brackets the whole sequence, so the kernel time comes from an
-        eager pass of the same shape first)."""
+        eager pass of the same shape first).  mfma: what the tuner chose."""
         if mode is not None:
             ctx.set_work_mode(mode)
         kernel_ms = []
@@ -552,6 +552,9 @@ def run(args):
         kms = float(np.mean(kernel_ms))
         # the committed counter figures of this leg's kernel and launch shape
         tb = traffic.get(name)
+        kernel = "fp64" if not flags & abi.PREC_MIXED else \
+            "valu" if flags & abi.NO_MFMA or not mfma else "mfma"
+        alg_bytes = algorithmic_bytes(batch, grid.cells, kernel)
         results[name] = {
             "value": units * args.steps / wall,
             "ms_per_step": 1e3 * wall / args.steps,
@@ -578,7 +581,7 @@ def run(args):
     tune = ctx.autotune(abi.PREC_MIXED)
     tune_s = time.perf_counter() - t0
     best = min(tune, key=lambda e: e[3])
-    leg("mixed", abi.PREC_MIXED, FP32_PEAK, graph=True)
+    leg("mixed", abi.PREC_MIXED, FP32_PEAK, graph=True, mfma=bool(best[2]))
     results["mixed"]["tuned"] = {"target_blocks": best[0], "work_mode": best[1],
                                  "mfma": bool(best[2]), "waves_per_simd": best[4],
                                  "candidates": len(tune),
