@@ -124,8 +124,19 @@ typedef struct mbs_consts {
 #define MBS_NOSHADOW 4u       /* also accumulate the no-shadow Mueller grid     */
 #define MBS_PER_ORIENT 8u     /* also keep one Mueller grid per orientation     */
 #define MBS_NO_MFMA 16u       /* mixed precision: rotation and coherent sum on
-                                 the vector ALU instead of the MFMA contraction
-                                 (same arithmetic, for comparison)              */
+                                 the vector ALU instead of the MFMA contraction.
+                                 The same aperture integrals; but the beam's
+                                 polarisation data are rounded once to FP32
+                                 (MFMA: three-part BF16 factors), and the shadow
+                                 beams enter the FP32 sum of the others, unless
+                                 MBS_NOSHADOW asks for the two apart (MFMA: always
+                                 a sum of their own).  So the full grid may differ
+                                 in its last FP32 digits from the MFMA one, and
+                                 with MBS_NOSHADOW from the one without.
+                                 mbs_autotune may choose this form for
+                                 MBS_PREC_MIXED, and a batch whose MFMA operand
+                                 (768 bytes a beam) found no device memory takes
+                                 it                                             */
 #define MBS_INCOHERENT 32u    /* FP64 sum of every beam's own Mueller matrix,
                                  sum_o w_o sum_b Mueller(d_b), instead of the
                                  Mueller matrix of the coherent sum; its M11 is
@@ -138,7 +149,9 @@ typedef struct mbs_consts {
                                  their FFT spectra, the others the direct
                                  integral.  Not with MBS_PER_ORIENT or
                                  MBS_INCOHERENT; needs a current
-                                 mbs_spectrum_source (MBS_ERR_INVALID)         */
+                                 mbs_spectrum_source (MBS_ERR_INVALID) and the
+                                 batch's MFMA operand (MBS_ERR_CAPACITY where it
+                                 found no device memory)                       */
 
 typedef struct mbs_ctx mbs_ctx;
 
