@@ -39,7 +39,10 @@
 // directions), since it waits on LDS and scalar loads.  Mixed precision: 7 (72
 // VGPRs; 6 with the shadow beams' sums, whose LDS lets no more share a CU).  Left
 // alone it takes 75 to 87 and runs at 5 or 6: 4,000 beams of six vertices and more
-// on those directions 1.75 ms, with 7 waves 1.52.
+// on those directions 1.75 ms, with 7 waves 1.52.  Where workgroups take whole
+// orientations, 6: the launch ends with the longest, alone on its CU or not (30
+// orientations of 800 beams on 181 x 48 directions 0.99 ms with 7, 0.95 with 6 or 5;
+// 300 of 230 2.35, 2.34 and 2.47).
 // Builds may pass -DMBS_MIN_WAVES=N for tuning (FP64).
 #ifndef MBS_MIN_WAVES
 #define MBS_MIN_WAVES 4
@@ -1850,7 +1853,7 @@ __device__ __forceinline__ void flush_mueller(const T *j, double w, double *dst,
 // sums of W rounded to FP32 (137,000 beams on 541 x 96 directions: 21.2 ms,
 // where each beam rotated, with its conversions, took 32 to 33).
 template <int PREC, int NS, int JONES, int PER, int QUEUE>
-__global__ __launch_bounds__(256) MBS_OCCUPANCY(PREC == 1 ? (NS ? 6 : 7) : MBS_MIN_WAVES) void
+__global__ __launch_bounds__(256) MBS_OCCUPANCY(PREC == 1 ? (NS || !JONES ? 6 : 7) : MBS_MIN_WAVES) void
 diffract_kernel(
     const WorkItem *__restrict__ items, int n_items, int n_tiles, int cells, int n_az,
     const double *__restrict__ tab, const double *__restrict__ hdr,
