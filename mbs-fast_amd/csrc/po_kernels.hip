@@ -35,7 +35,7 @@
 
 // Occupancy of the vector-ALU kernels, in waves per SIMD.  FP64: at least 4 (128
 // VGPRs), which the common path takes about 120 of with its 24 sums; with 3 waves
-// and no spills it is slower (11.7 ms against 9.3 for 35,800 beams on 541 x 96
+// and no spills it is slower (9.5 ms against 8.65 for 35,800 beams on 541 x 96
 // directions), since it waits on LDS and scalar loads.  Mixed precision: 7 (72
 // VGPRs; 6 with the shadow beams' sums, whose LDS lets no more share a CU).  Left
 // alone it takes 75 to 87 and runs at 5 or 6: 4,000 beams of six vertices and more
@@ -193,7 +193,7 @@ __global__ void grid_tables_kernel(const double *__restrict__ theta,
 // for 59,000 and 2.57 ms for 137,000; this form takes 13, 53 and 105 us.  The
 // polygon is staged in LDS, the lanes of a group
 // take the vertices in turn and add their sums by butterflies, and an edge's
-// share of a moment is a 4-point Gauss rule: over the triangle (0, P, Q) a
+// share of a moment is a 3-point Gauss rule: over the triangle (0, P, Q) a
 // monomial of degree n integrates to det(P, Q) / (n + 2) times its mean along
 // PQ, which three nodes give exactly to degree 5.  The record goes through LDS
 // so that its stores are contiguous.
@@ -1652,9 +1652,11 @@ __device__ __forceinline__ void rotate_add(const double *__restrict__ w, const T
 // flight at a time, each read by every XCD, and the XCDs get equal work whatever
 // the items' sizes.  On a small one each XCD gets a contiguous range of items, so
 // that the beam records of an item pass through one L2 (in order, a thousand
-// workgroups would hold dozens of items).  11,000 beams on 1001 x 48 directions
-// (188 tiles): 3.94 ms in order, 4.16 by ranges; 59,000 on 181 x 32 (23 tiles): 1.38
-// and 1.32.
+// workgroups would hold dozens of items).  In order, 11,000 to 59,000 beams in 2 to
+// 256 orientations are 4 to 10 % slower in mixed precision and 0 to 6 % in FP64 on 12
+// to 46 tiles (59,000 on 23: 1.11 and 1.06 ms); at 68, 91, 136 and 188 tiles neither
+// order wins in most, and they lie within 4 % of each other (59,000 on 188: 7.21 and
+// 7.25 ms; 5,870 near-forward beams on them, FP64, 1.54 and 1.61).
 __device__ __forceinline__ bool map_block(int n_items, int n_tiles, int &item,
                                           int &tile)
 {
@@ -1688,12 +1690,14 @@ __device__ __forceinline__ bool map_block(int n_items, int n_tiles, int &item,
 // worth some tens of beams, and its partial grid; a launch ends with workgroups
 // idle for half a segment.  With N beams, T tiles and P workgroups at once the two
 // are N T / (P seg) x cost and seg / 2: least at a multiple of sqrt(N T / P).
-// With P = 1024 the multiple 4 is best or near it throughout (times of kernel and
-// reduction at multiples 2.7, 4 and 6.4, and with 32 beams at least): 1,900 beams on
-// 541 x 96 directions, FP64, 1.74 1.62 1.91 (1.80) ms; 11,000 on 1001 x 48, 4.48 4.23
-// 3.97 (4.92); 59,000 on 181 x 32 1.33 1.31 1.46 (1.60); 137,000 on 541 x 96 16.9 17.4
-// 17.1 (16.8).  At least four: 185 beams on 91 x 16 take 20 us with four or five,
-// 23 with eight, 50 with 32.
+// With P = 1024 that is the multiple 4 for costs of some 30 beams.  The optimum is
+// flat: kernel and reduction with 2.7 and with 6.4 against 4, over 1,900 to 136,000
+// beams in 1 to 256 orientations on 12 to 203 tiles, take on the mean (least to most)
+// mixed 1.01 (0.97 to 1.09) and 1.01 (0.96 to 1.09), FP64 1.01 (0.97 to 1.09) and 1.00
+// (0.93 to 1.07), mixed on the vector ALU 1.00 (0.96 to 1.04) and 1.03 (0.97 to 1.09),
+// the incoherent sum 1.04 (0.99 to 1.17) and 0.98 (0.85 to 1.02): one rule for all, and
+// not the best for each.  At least four: 185 beams on 91 x 16 take 20 us with four or
+// five, 23 with eight, 50 with 32.
 __host__ __device__ inline int64_t min_segment(int64_t n_beams, int n_tiles)
 {
     const int64_t seg = (int64_t)(sqrt((double)(n_beams * n_tiles)) / 8.0);
