@@ -221,8 +221,8 @@ def bench_config3(pkg, args):
     """The batched non-convex aggregate at its stated batch (opt-in,
     --config3): 16,384 orientations with beam counts log-uniform over
     50..40,000 (a synthetic resample of the 8-column aggregate's traced beams,
-    tests/golden/config3_aggregate.npz; ~1e8 beams, ~130 GB of device
-    records) on configuration 2's 541 x 96 grid.  One eager beam-segment
+    tests/golden/config3_aggregate.npz; ~1e8 beams, ~220 GB of device
+    memory) on configuration 2's 541 x 96 grid.  One eager beam-segment
     launch, then the persistent work-queue launch captured as a graph and
     replayed twice; every replay must equal the eager result bit for bit."""
     abi, syn, eng = pkg.abi, pkg.synthetic, pkg.engine

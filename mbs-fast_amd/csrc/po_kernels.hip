@@ -949,9 +949,11 @@ __device__ __forceinline__ bool aperture_f64(const double *__restrict__ h,
 // coefficients and a select per edge, four phasors with an extra constant and a
 // longer polynomial each) took 214; other polygons the sum over their vertices with
 // the reference's weights.  35,800 beams of 2,000-15,000 an orientation on 541 x 96
-// directions: 8.8 ms against 12.7 for the kernel, which the vector ALU bounds (150
-// instructions a beam and wave on average; four waves a SIMD leave it 80 % busy).
-// The error against extended precision is 0.25 to 0.4 of the branches'.
+// directions: 8.65 ms against 12.7 for the kernel, which the vector ALU bounds (144
+// instructions a beam and wave over 139,000 beams; four waves a SIMD leave it 84 %
+// busy).  The error against extended precision is 0.04 to 0.4 of the branches' on the
+// mean over draws, workload by workload, and single draws go either way (30 fixed
+// orientations on 91 x 16 directions: 0.39 on the mean, 2.8 at the most).
 
 // 1/x to full FP64 precision from the hardware estimate e (1 + e + e^2).
 __device__ __forceinline__ double rcp_f64_cubic(double x)
