@@ -867,7 +867,11 @@ __device__ __forceinline__ bool aperture_f64(const double *__restrict__ h,
     // apart from the phases they would not cancel with them.
     const double a = -kInvTwoPi * (k0 * h[H_HOR] + k1 * h[H_HOR + 1] + k2 * h[H_HOR + 2]);
     const double b = -kInvTwoPi * (k0 * h[H_VER] + k1 * h[H_VER + 1] + k2 * h[H_VER + 2]);
-    const double c = kInvTwoPi * (d[0] * h[H_KC] + d[1] * h[H_KC + 1] + d[2] * h[H_KC + 2]);
+    double c = kInvTwoPi * (d[0] * h[H_KC] + d[1] * h[H_KC + 1] + d[2] * h[H_KC + 2]);
+    // Without its whole turns (exact), so that a vertex's phase, a hundred times
+    // smaller then, is rounded that much finer: the rounding stands over an edge's own
+    // small step (1 % of the kernel with slopes of their own, 1.76 -> 1.78 ms)
+    c = __builtin_fma(-kPhasorN, __builtin_rint(kNode * c), c);
     const bool useB = __builtin_fabs(b) > __builtin_fabs(a);
     asm volatile("" ::"s"(t0), "s"(t1), "s"(t2));
     const auto place = [&](int v, double &r, double2 &t) {
