@@ -820,7 +820,9 @@ __device__ __forceinline__ uint64_t edges_f64(const double *__restrict__ vtx, in
 }
 
 // What the edges within the limit add to the sum of edges_f64, in a lane that has
-// one: the exact half-angle form.
+// one: the exact half-angle form, which reads the next vertex's phasor only where the
+// edge is longer than it serves.  (Edges found by a mask first, theirs alone visited:
+// the mask costs the common path registers and 2 to 10 %.)
 template <typename Place>
 __device__ __forceinline__ void singular_edges_f64(const double *__restrict__ vtx,
                                                    const double *__restrict__ vx, int nv,
@@ -834,14 +836,18 @@ __device__ __forceinline__ void singular_edges_f64(const double *__restrict__ vt
                                : __builtin_fma(uniform_f64(v[V_SXY]), a, b);
         if (__builtin_fabs(cc) > limit || !(vertex_flags(w, 0) & (useB ? EDGE_VX : EDGE_VY)))
             continue;
-        double r, sp, cp, sn, cn;
+        double r, sp, cp;
         double2 t;
         place(e, r, t);
         node_finish(r, t, sp, cp);
-        place(e + 1 < nv ? e + 1 : 0, r, t);
-        node_finish(r, t, sn, cn);
         const double dx = uniform_f64(w[VX_DX]), dy = uniform_f64(w[VX_DY]);
-        const double2 q = stable_edge_quotient(cp, sp, cn, sn, useB ? dx : dy, kPerNode * cc, k);
+        const double delta = useB ? dx : dy, c = kPerNode * cc;
+        double sn = sp, cn = cp;
+        if (!(__builtin_fabs(k * c * delta) <= kHalfAngle)) {  // (no half-angle form)
+            place(e + 1 < nv ? e + 1 : 0, r, t);
+            node_finish(r, t, sn, cn);
+        }
+        const double2 q = stable_edge_quotient(cp, sp, cn, sn, delta, c, k);
         sr = __builtin_fma(kPerNode, q.x, sr);
         si = __builtin_fma(kPerNode, q.y, si);
     }
@@ -881,20 +887,22 @@ __device__ __forceinline__ bool aperture_f64(const double *__restrict__ h,
                     tab, r, t);
     };
     const double limit = kNodes * eps1;
-    double sr, si;
-    uint64_t near;
-    if (nv == 4)
-        near = edges_f64<4>(vtx, 4, a, b, useB, limit, place, sr, si);
-    else if (nv == 3)
-        near = edges_f64<3>(vtx, 3, a, b, useB, limit, place, sr, si);
-    else
-        near = edges_f64<0>(vtx, nv, a, b, useB, limit, place, sr, si);
     // the vertex phases one by one only where the beam's bound leaves the
     // small-phase form possible
     const double larger = useB ? b : -a;
     bool small = false;
     if (__builtin_expect(__builtin_fabs(larger) <= kNodes * h[H_PHB], 0))
         small = all_phases_small(vtx, nv, a, b, kNodes * kSmallPhase);
+    double sr = 0.0, si = 0.0;
+    uint64_t near = 0;
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(!small) != 0, 1)) {
+        if (nv == 4)
+            near = edges_f64<4>(vtx, 4, a, b, useB, limit, place, sr, si);
+        else if (nv == 3)
+            near = edges_f64<3>(vtx, 3, a, b, useB, limit, place, sr, si);
+        else
+            near = edges_f64<0>(vtx, nv, a, b, useB, limit, place, sr, si);
+    }
     if (__builtin_expect(near != 0, 0)) {
         if (__builtin_amdgcn_inverse_ballot_w64(near) && !small)
             singular_edges_f64(vtx, vx, nv, a, b, useB, limit, k, place, sr, si);
@@ -1107,6 +1115,11 @@ __device__ __forceinline__ uint64_t aperture_any_f64(const double *eb, const dou
     }
     // next to a singular edge, and where every phase is small: the branches
     if (__builtin_expect(look != 0, 0)) {
+        // a word of each cache line that the branches read of the polygon, so that
+        // they come together and not one after the other
+        const double t0 = vtx[0], t1 = vtx[2 * VTX_STRIDE], t2 = vtx[nv * VTX_STRIDE - 1];
+        const double t3 = vx[0], t4 = vx[2 * VX_STRIDE], t5 = vx[nv * VX_STRIDE - 1];
+        asm volatile("" ::"s"(t0), "s"(t1), "s"(t2), "s"(t3), "s"(t4), "s"(t5));
         const double A = -kNode * (k0 * h[H_HOR] + k1 * h[H_HOR + 1] + k2 * h[H_HOR + 2]);
         const double B = -kNode * (k0 * h[H_VER] + k1 * h[H_VER + 1] + k2 * h[H_VER + 2]);
         const bool leaves = !(__builtin_fabs(step) > eb[EB_SING64]) || div == 0.0 ||

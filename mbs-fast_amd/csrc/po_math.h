@@ -207,6 +207,9 @@ __device__ __forceinline__ double sinc_series(double x)
     return __builtin_fma(z, p, 1.0);
 }
 
+// |k c delta| up to which stable_edge_quotient reads the first phasor alone.
+constexpr double kHalfAngle = 0.25;
+
 // add_stable_edge_quotient (src/handler/HandlerPO_fast.h:235-264): the exact
 // half-angle form of exp(i phaseStart)(exp(i k c delta) - 1)/c for an edge
 // coefficient c at or near zero.  Returns the increment (real part in .x,
@@ -222,7 +225,7 @@ __device__ __forceinline__ double2 stable_edge_quotient(double pr, double pi, do
                                                         double k)
 {
     const double z = k * cc * delta;
-    if (__builtin_fabs(z) <= 0.25) {
+    if (__builtin_fabs(z) <= kHalfAngle) {
         const double sh = sinc_series(0.5 * z);
         const double lr = -0.5 * k * k * cc * delta * delta * sh * sh;
         const double li = k * delta * sinc_series(z);
